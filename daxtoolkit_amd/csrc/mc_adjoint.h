@@ -205,8 +205,6 @@ __device__ __forceinline__ int64_t edge_vid(const GatherCtx& c, int dx, int dy, 
   return vid < c.n_adj ? vid : -1;
 }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 // (S_p, dL/dg_p) at p = (x,j,k) + (dx,dy,dz): over the 3 edges leaving p
 // (lower halves of their records) and the 3 edges entering p (upper halves),
 // summed in that order.

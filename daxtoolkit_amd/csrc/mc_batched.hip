@@ -39,7 +39,7 @@ constexpr int kBatchGenTile = 256;
 
 // Launch shapes of the batch forward, picked by dax_hip_mc_batch_autotune
 // and cached per batch shape class: classify unroll (row words per wave
-// step) and persistent blocks per CU, threads per scan tile (the tile's
+// step, a float4 load in flight per thread for two of them) and persistent blocks per CU, threads per scan tile (the tile's
 // 1024 words over 256, 512 or 1024 threads), generate blocks per CU and
 // its XCD-contiguous tile order.
 struct BatchTuning {
@@ -105,7 +105,7 @@ constexpr int64_t kBatchMagic = 0x4441584842415443LL;  // "DAXHBATC"
 constexpr size_t kBatchHeaderBytes = 256;
 static_assert(sizeof(BatchHeader) <= kBatchHeaderBytes, "header fits its reserved bytes");
 
-template <int UNROLL>
+template <int LOADS>
 __global__ __launch_bounds__(256) void k_batch_classify(const VolGeom* __restrict__ vols,
                                                         const TileRef* __restrict__ tiles,
                                                         int64_t ntiles,
@@ -113,17 +113,17 @@ __global__ __launch_bounds__(256) void k_batch_classify(const VolGeom* __restric
                                                         uint64_t* __restrict__ bits,
                                                         unsigned long long* __restrict__ zero_buf,
                                                         int64_t zero_words) {
+  __shared__ FlatLds<kBatchGenTile> sh;
   const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = gtid; i < zero_words; i += nthreads) zero_buf[i] = 0ull;
-  const int wv = threadIdx.x >> 6;
   for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const TileRef tr = tiles[t];
     const VolGeom g = vols[tr.vol];
     const int64_t w_end = min((int64_t)tr.w0 + kBatchGenTile, g.nwords);
-    for (int64_t w0 = tr.w0 + (int64_t)wv * UNROLL; w0 < w_end;
-         w0 += (int64_t)(blockDim.x >> 6) * UNROLL)
-      classify_words<UNROLL, false>(g, fields + g.field_off, bits + g.word_off, w0, w_end);
+    classify_flat<kBatchGenTile, LOADS>(g, fields + g.field_off, bits + g.word_off,
+                                        (uint32_t)tr.w0, (uint32_t)w_end, sh);
+    __syncthreads();  // LDS reused by the next tile
   }
 }
 
@@ -310,15 +310,15 @@ int batch_classify(const BatchHeader& h, const BatchPtrs& p, const float* d_fiel
   const dim3 grid((unsigned)persistent_blocks(t.cls_blocks)), blk(256);
   switch (t.cls_unroll) {
     case 8:
-      k_batch_classify<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
+      k_batch_classify<4><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
                                                p.status, zero_words);
       break;
     case 32:
-      k_batch_classify<32><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
+      k_batch_classify<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
                                                 p.status, zero_words);
       break;
     default:
-      k_batch_classify<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
+      k_batch_classify<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
                                                 p.status, zero_words);
   }
   DAXHIP_LAUNCH_CHECK("k_batch_classify");

@@ -31,7 +31,7 @@ namespace mc {
 
 // Classify row words [w_lo, w_hi) (w_lo a multiple of 4 for the float4 form)
 // and clear zero_words words of count/scan state.
-template <int UNROLL, bool ALIGNED>
+template <int UNROLL>
 __global__ __launch_bounds__(256) void k_classify(VolGeom g, const float* __restrict__ field,
                                                   uint64_t* __restrict__ bits,
                                                   unsigned long long* __restrict__ zero_buf,
@@ -39,7 +39,24 @@ __global__ __launch_bounds__(256) void k_classify(VolGeom g, const float* __rest
   const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (gtid < zero_words) zero_buf[gtid] = 0ull;
   const int64_t w0 = w_lo + (gtid >> 6) * UNROLL;
-  classify_words<UNROLL, ALIGNED>(g, field + g.field_off, bits + g.word_off, w0, w_hi);
+  classify_words<UNROLL>(g, field + g.field_off, bits + g.word_off, w0, w_hi);
+}
+
+// Rows that are not whole 64-point words, or a field that is not 16-byte
+// aligned: TW words per block.  Bound by HBM.
+template <int TW>
+__global__ __launch_bounds__(256) void k_classify_flat(VolGeom g, const float* __restrict__ field,
+                                                       uint64_t* __restrict__ bits,
+                                                       unsigned long long* __restrict__ zero_buf,
+                                                       int64_t zero_words, int64_t w_lo,
+                                                       int64_t w_hi) {
+  __shared__ FlatLds<TW> sh;
+  const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (gtid < zero_words) zero_buf[gtid] = 0ull;
+  const int64_t w0 = w_lo + (int64_t)blockIdx.x * TW;
+  if (w0 >= w_hi) return;  // a block that only clears
+  classify_flat<TW, kFlatLoads>(g, field + g.field_off, bits + g.word_off, (uint32_t)w0,
+                                (uint32_t)min(w0 + TW, w_hi), sh);
 }
 
 template <int UNROLL>
@@ -356,9 +373,9 @@ __global__ __launch_bounds__(256) void k_classify_plane(VolGeom g, FieldPlane pl
 // Tuning: per grid shape, the classify variant, scan sub-tiles and generate
 // tile words.  Defaults are used until dax_hip_mc_autotune (or
 // dax_hip_mc_set_tuning) records a choice for a shape.
-// The defaults are the 512^3 workload's autotuned choice (classify falls
-// back to one float per lane, 16 words per wave, on rows that are not
-// 64-point aligned).
+// The defaults are the 512^3 workload's autotuned choice (the classify
+// variants are for rows of whole 64-point words; other rows are read as a
+// flat stream, k_classify_flat).
 struct Tuning {
   int cls_unroll = 4;   // words (vec 1) or 256-point chunks (vec 4) per wave
   int cls_vec = 4;      // floats per lane per load
@@ -606,32 +623,40 @@ int launch_bits(const VolGeom& g, const float* field, char* ws, const Workspace&
   uint64_t* bits = (uint64_t*)(ws + L.off_bits);
   unsigned long long* status = (unsigned long long*)(ws + L.off_status);
   const int64_t zero_words = zero ? L.ntiles + (int64_t)(sizeof(Ctrl) / 8) : 0;
-  const bool aligned = (g.nx % 64) == 0;
-  const bool aligned16 = aligned && (g.field_off % 4) == 0 && ((uintptr_t)field % 16) == 0 &&
-                         (w_lo % 4) == 0;
-  const int vec = aligned16 ? tu.cls_vec : 1;
-  const int unroll = (vec == 1 && tu.cls_vec != 1) ? 16 : tu.cls_unroll;
+  const bool aligned = (g.nx % 64) == 0 && (g.field_off % 4) == 0 &&
+                       ((uintptr_t)field % 16) == 0 && (w_lo % 4) == 0;
+  if (!aligned) {
+    // 8192 points, 8 float4 loads per thread, for rows of full or half words;
+    // shorter rows hold fewer points per word, so four times the words
+    const int tw = g.nx > 32 ? 128 : 512;
+    const int64_t blocks = std::max<int64_t>(
+        std::max(ceil_div(w_hi - w_lo, tw), ceil_div(zero_words, 256)), 1);
+    const dim3 grid((unsigned)blocks), block(256);
+    if (tw == 128)
+      k_classify_flat<128><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi);
+    else
+      k_classify_flat<512><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi);
+    DAXHIP_LAUNCH_CHECK("k_classify_flat");
+    return DAX_HIP_OK;
+  }
+  const int vec = tu.cls_vec, unroll = tu.cls_unroll;
   const int64_t units = vec == 4 ? ceil_div(w_hi - w_lo, 4) : w_hi - w_lo;  // chunks or words
   const int64_t waves = ceil_div(units, unroll);
   int64_t blocks = std::max<int64_t>(ceil_div(waves * 64, 256), ceil_div(zero_words, 256));
   blocks = std::max<int64_t>(blocks, 1);
   const dim3 grid((unsigned)blocks), block(256);
-#define DAXHIP_CLS(U, A) \
-  k_classify<U, A><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi)
+#define DAXHIP_CLS(U) \
+  k_classify<U><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi)
 #define DAXHIP_CLS4(U) \
   k_classify_v4<U><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi)
   if (vec == 4) {
     if (unroll == 2) DAXHIP_CLS4(2);
     else if (unroll == 4) DAXHIP_CLS4(4);
     else DAXHIP_CLS4(8);
-  } else if (aligned) {
-    if (unroll == 8) DAXHIP_CLS(8, true);
-    else if (unroll == 32) DAXHIP_CLS(32, true);
-    else DAXHIP_CLS(16, true);
   } else {
-    if (unroll == 8) DAXHIP_CLS(8, false);
-    else if (unroll == 32) DAXHIP_CLS(32, false);
-    else DAXHIP_CLS(16, false);
+    if (unroll == 8) DAXHIP_CLS(8);
+    else if (unroll == 32) DAXHIP_CLS(32);
+    else DAXHIP_CLS(16);
   }
 #undef DAXHIP_CLS
 #undef DAXHIP_CLS4
@@ -1217,9 +1242,9 @@ int dax_hip_mc_autotune(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   Tuning best = tuning_for(nx, ny, nz);
   EventPair ev;
 
-  // classify variants
-  std::vector<std::pair<int, int>> cls = {{8, 1}, {16, 1}, {32, 1}};
-  if (nx % 64 == 0) cls.insert(cls.end(), {{2, 4}, {4, 4}, {8, 4}});
+  // classify variants (one for rows that are not whole words)
+  std::vector<std::pair<int, int>> cls = {{best.cls_unroll, best.cls_vec}};
+  if (nx % 64 == 0) cls = {{8, 1}, {16, 1}, {32, 1}, {2, 4}, {4, 4}, {8, 4}};
   float best_ms[3] = {1e30f, 1e30f, 1e30f};
   for (auto uv : cls) {
     Tuning t = best;
