@@ -36,6 +36,11 @@ struct TileRef {
 // generate (and classify) tiles.  The launch shapes over them are tuned.
 constexpr int kBatchScanTile = 1024;
 constexpr int kBatchGenTile = 256;
+// Threads per generate tile: one per word; a batch has tiles enough, so more
+// waves per tile only stage the same words for fewer outputs each (256 volumes
+// of 32..160 points an axis, forward + adjoint: 1077 us, 1133 with 512
+// threads, 1250 with 1024).
+constexpr int kBatchGenThreads = 256;
 
 // Launch shapes of the batch forward, picked by dax_hip_mc_batch_autotune
 // and cached per batch shape class: classify unroll (row words per wave
@@ -150,14 +155,14 @@ __global__ __launch_bounds__(NT) void k_batch_count_scan(
   }
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_batch_generate(
+template <bool dedup>
+__global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
     const float* __restrict__ fields, const uint64_t* __restrict__ bits,
     const uint32_t* __restrict__ base_v, const uint32_t* __restrict__ base_t,
     const Ctrl* __restrict__ ctrl, OutPtrs out, unsigned flags, int64_t cap_points,
     int64_t cap_tris, int64_t* __restrict__ counts, int xcd) {
   extern __shared__ uint64_t s_dyn[];
-  const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
   const bool normals = (flags & DAX_HIP_MC_NORMALS) != 0 && out.normals != nullptr;
   const uint64_t total_v = ctrl->total_v, total_t = ctrl->total_t;
   const uint64_t n_points = dedup ? total_v : 3ull * total_t;
@@ -171,9 +176,9 @@ __global__ __launch_bounds__(kScanThreads) void k_batch_generate(
     const TileRef tr = tiles[xcd ? xcd_tile(b, ntiles) : b];
     const VolGeom g = vols[tr.vol];
     const int64_t vbv = base_v[g.word_off], vbt = base_t[g.word_off];
-    generate_tile<kBatchGenTile>(g, FieldArray{fields + g.field_off}, bits + g.word_off,
-                                 base_v + g.word_off, base_t + g.word_off, tr.w0, out, dedup,
-                                 normals, vbv, vbt, s_dyn);
+    generate_tile<kBatchGenTile, kBatchGenThreads, FieldArray, dedup>(
+        g, FieldArray{fields + g.field_off}, bits + g.word_off, base_v + g.word_off,
+        base_t + g.word_off, tr.w0, out, normals, vbv, vbt, s_dyn);
     __syncthreads();  // LDS reused by the next tile
   }
 }
@@ -347,11 +352,16 @@ int batch_scan(const BatchHeader& h, const BatchPtrs& p, const BatchTuning& t, h
 int batch_generate(const BatchHeader& h, const BatchPtrs& p, const float* d_fields,
                    unsigned flags, const OutPtrs& o, int64_t cap_points, int64_t cap_tris,
                    int64_t* d_counts, const BatchTuning& t, hipStream_t s) {
-  const size_t lds = GenLayout<kBatchGenTile>((int)h.max_wpr).bytes();
-  k_batch_generate<<<dim3((unsigned)std::min<int64_t>(persistent_blocks(t.gen_blocks), h.ngen)),
-                     dim3(kScanThreads), lds, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
-                                                   p.bv, p.bt, p.ctrl, o, flags, cap_points,
-                                                   cap_tris, d_counts, t.gen_xcd);
+  const size_t lds = GenLayout<kBatchGenTile, kBatchGenThreads>((int)h.max_wpr).bytes();
+  const dim3 grid((unsigned)std::min<int64_t>(persistent_blocks(t.gen_blocks), h.ngen));
+  if (flags & DAX_HIP_MC_DEDUP)
+    k_batch_generate<true><<<grid, dim3(kBatchGenThreads), lds, s>>>(
+        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, p.bv, p.bt, p.ctrl, o, flags, cap_points,
+        cap_tris, d_counts, t.gen_xcd);
+  else
+    k_batch_generate<false><<<grid, dim3(kBatchGenThreads), lds, s>>>(
+        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, p.bv, p.bt, p.ctrl, o, flags, cap_points,
+        cap_tris, d_counts, t.gen_xcd);
   DAXHIP_LAUNCH_CHECK("k_batch_generate");
   return DAX_HIP_OK;
 }

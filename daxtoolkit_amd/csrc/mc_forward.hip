@@ -274,14 +274,13 @@ __global__ __launch_bounds__(256) void k_bases(VolGeom g, CountSrc cs) {
   cs.base_t[g.word_off + w] = (uint32_t)(p >> 32);
 }
 
-template <int TW, class Src>
-__global__ __launch_bounds__(kScanThreads, 5) void k_generate(
+template <int TW, int NT, class Src, bool dedup>
+__global__ __launch_bounds__(NT, 4) void k_generate(
     VolGeom g, Src field, const uint64_t* __restrict__ bits, CountSrc cs,
     const Ctrl* __restrict__ ctrl, OutPtrs out, unsigned flags, int64_t cap_points,
     int64_t cap_tris, int64_t* __restrict__ counts, int xcd_order, int64_t tile_lo,
     int64_t ntiles, const uint32_t* __restrict__ order) {
   extern __shared__ uint64_t s_dyn[];
-  const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
   const bool normals = (flags & DAX_HIP_MC_NORMALS) != 0 && out.normals != nullptr;
   const uint64_t total_v = ctrl->total_v, total_t = ctrl->total_t;
   const uint64_t n_points = dedup ? total_v : 3ull * total_t;
@@ -304,9 +303,9 @@ __global__ __launch_bounds__(kScanThreads, 5) void k_generate(
   const int64_t tile =
       ordered ? (int64_t)(ord & ~kOrderHasOutput)
               : tile_lo + (xcd_order ? xcd_tile(blockIdx.x, ntiles) : (int64_t)blockIdx.x);
-  generate_tile<TW, Src, true>(g, field, bits + g.word_off, nullptr, nullptr, tile * TW, out,
-                               dedup, normals, 0, 0, s_dyn, cs, emit,
-                               ordered && (ord & kOrderHasOutput) != 0u);
+  generate_tile<TW, NT, Src, dedup, true>(g, field, bits + g.word_off, nullptr, nullptr, tile * TW,
+                                          out, normals, 0, 0, s_dyn, cs, emit,
+                                          ordered && (ord & kOrderHasOutput) != 0u);
 }
 
 // Slice classify: a wave per kPlaneRowsPerWave grid rows.  Along a row the
@@ -373,25 +372,47 @@ __global__ __launch_bounds__(256) void k_classify_plane(VolGeom g, FieldPlane pl
 // Tuning: per grid shape, the classify variant, scan sub-tiles and generate
 // tile words.  Defaults are used until dax_hip_mc_autotune (or
 // dax_hip_mc_set_tuning) records a choice for a shape.
-// The defaults are the 512^3 workload's autotuned choice (the classify
-// variants are for rows of whole 64-point words; other rows are read as a
-// flat stream, k_classify_flat).
+// The classify variants are for rows of whole 64-point words; other rows are
+// read as a flat stream, k_classify_flat.
 struct Tuning {
   int cls_unroll = 4;   // words (vec 1) or 256-point chunks (vec 4) per wave
   int cls_vec = 4;      // floats per lane per load
   int scan_sub = 8;     // count tiles (waves) per count block
   int gen_tile = 512;   // generate tile words
   int gen_xcd = 0;      // 1: each XCD takes a contiguous range of generate tiles
+  bool operator==(const Tuning& o) const {
+    return cls_unroll == o.cls_unroll && cls_vec == o.cls_vec && scan_sub == o.scan_sub &&
+           gen_tile == o.gen_tile && gen_xcd == o.gen_xcd;
+  }
 };
 
 std::mutex g_tune_mu;
 Tuning g_tune_default;
 std::map<std::tuple<int64_t, int64_t, int64_t>, Tuning> g_tune_cache;
 
+// The launch shape of a volume without a choice of its own, while the default
+// is the built-in one.  Generate tiles: 64 words (spread over the waves
+// launch_generate_src gives them) up to 2^20 words, 256 beyond, where the
+// dispatch order of tiles of at least a count tile pays (forward, 64 / 256
+// words: 256^3 points 59 / 65 us, 384^3 105 / 109, 512^3 194 / 176; dense
+// 640^3 367 / 375).  A tile stages two rows beyond its own, so rows of more
+// than 32 words take tiles of at least two rows.  Count blocks: one wave up to
+// 2^16 words, to spread over more CUs (100 x 90 x 110 points: forward 37 / 38
+// / 40 us with 1 / 4 / 8 waves), four beyond (256^3: 68 / 67 / 69).
+Tuning shape_tuning(int64_t nx, int64_t ny, int64_t nz) {
+  Tuning t;
+  const int64_t wpr = ceil_div(nx, 64), words = wpr * ny * nz;
+  t.gen_tile = words <= (1 << 20) ? 64 : 256;
+  while (t.gen_tile < 1024 && wpr > 32 && t.gen_tile < 2 * wpr) t.gen_tile *= 2;
+  t.scan_sub = words <= (1 << 16) ? 1 : 4;
+  return t;
+}
+
 Tuning tuning_for(int64_t nx, int64_t ny, int64_t nz) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune_cache.find(std::make_tuple(nx, ny, nz));
-  return it == g_tune_cache.end() ? g_tune_default : it->second;
+  if (it != g_tune_cache.end()) return it->second;
+  return g_tune_default == Tuning{} ? shape_tuning(nx, ny, nz) : g_tune_default;
 }
 
 bool valid_tuning(const Tuning& t) {
@@ -736,22 +757,28 @@ int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu
 }
 
 // Generate tiles of TW words [t_lo, t_hi) (all when t_hi < 0).
-template <int TW, class Src>
+template <int TW, int NT, class Src>
 int launch_generate_tw(const VolGeom& g, const Src& field, const char* ws, const Workspace& L,
                        unsigned flags, const OutPtrs& o, int64_t cap_points, int64_t cap_tris,
                        int64_t* counts, const Tuning& tu, hipStream_t s, int64_t t_lo,
                        int64_t t_hi) {
   const int xcd = tu.gen_xcd;
-  const size_t lds = GenLayout<TW>(g.wpr).bytes();
+  const size_t lds = GenLayout<TW, NT>(g.wpr).bytes();
   const int64_t all = ceil_div(g.nwords, (int64_t)TW);
   if (t_hi < 0) t_hi = all;
   const int64_t ntiles = std::max<int64_t>(t_hi - t_lo, 1);
   const CountSrc cs = count_src(ws, L, tu);
   const uint32_t* order =
       (t_lo == 0 && t_hi == all) ? (const uint32_t*)(ws + L.off_order) : nullptr;
-  k_generate<TW, Src><<<dim3((unsigned)ntiles), dim3(kScanThreads), lds, s>>>(
-      g, field, (const uint64_t*)(ws + L.off_bits), cs, (const Ctrl*)(ws + L.off_ctrl), o, flags,
-      cap_points, cap_tris, counts, xcd, t_lo, ntiles, order);
+#define DAXHIP_GEN(DEDUP)                                                                        \
+  k_generate<TW, NT, Src, DEDUP><<<dim3((unsigned)ntiles), dim3(NT), lds, s>>>(                  \
+      g, field, (const uint64_t*)(ws + L.off_bits), cs, (const Ctrl*)(ws + L.off_ctrl), o, flags, \
+      cap_points, cap_tris, counts, xcd, t_lo, ntiles, order)
+  if (flags & DAX_HIP_MC_DEDUP)
+    DAXHIP_GEN(true);
+  else
+    DAXHIP_GEN(false);
+#undef DAXHIP_GEN
   DAXHIP_LAUNCH_CHECK("k_generate");
   return DAX_HIP_OK;
 }
@@ -761,23 +788,29 @@ int launch_generate_src(const VolGeom& g, const Src& field, const char* ws, cons
                         unsigned flags, const OutPtrs& o, int64_t cap_points, int64_t cap_tris,
                         int64_t* counts, const Tuning& tu, hipStream_t s, int64_t t_lo = 0,
                         int64_t t_hi = -1) {
+#define DAXHIP_GEN_TW(TW, NT)                                                                  \
+  launch_generate_tw<TW, NT>(g, field, ws, L, flags, o, cap_points, cap_tris, counts, tu, s, t_lo, \
+                             t_hi)
   switch (tu.gen_tile) {
     case 64:
-      return launch_generate_tw<64>(g, field, ws, L, flags, o, cap_points, cap_tris, counts, tu,
-                                    s, t_lo, t_hi);
+      // A wave per tile runs its rounds one after another, so few tiles leave
+      // the chip waiting on chains: four waves share a tile's outputs up to
+      // 2^18 words, two up to 2^20 (128^3 points: 43 / 28 / 18 us with one /
+      // two / four waves, 256^3 47 / 39 / 39, 384^3 58 / 56 / 67, 512^3 84 /
+      // 105 / 155).
+      if (g.nwords <= (1 << 18)) return DAXHIP_GEN_TW(64, 256);
+      if (g.nwords <= (1 << 20)) return DAXHIP_GEN_TW(64, 128);
+      return DAXHIP_GEN_TW(64, 64);
     case 128:
-      return launch_generate_tw<128>(g, field, ws, L, flags, o, cap_points, cap_tris, counts,
-                                     tu, s, t_lo, t_hi);
+      return DAXHIP_GEN_TW(128, 128);
     case 256:
-      return launch_generate_tw<256>(g, field, ws, L, flags, o, cap_points, cap_tris, counts,
-                                     tu, s, t_lo, t_hi);
+      return DAXHIP_GEN_TW(256, 256);
     case 1024:
-      return launch_generate_tw<1024>(g, field, ws, L, flags, o, cap_points, cap_tris, counts,
-                                      tu, s, t_lo, t_hi);
+      return DAXHIP_GEN_TW(1024, 1024);
     default:
-      return launch_generate_tw<512>(g, field, ws, L, flags, o, cap_points, cap_tris, counts,
-                                     tu, s, t_lo, t_hi);
+      return DAXHIP_GEN_TW(512, 512);
   }
+#undef DAXHIP_GEN_TW
 }
 
 int launch_generate(const VolGeom& g, const float* field, const char* ws, const Workspace& L,

@@ -895,21 +895,118 @@ __device__ __forceinline__ void write_order_units(uint64_t reg, uint32_t K, uint
   if (threadIdx.x == 0) order[0] = tag;
 }
 
-// LDS layout of a generate tile of TW words (wpr known at run time).
-constexpr int kMaxGenThreads = 256;
-template <int TW>
+// What one wave of a generate tile keeps of a round of up to 64 active cells:
+// the cells' table entries, the vertex ids of their 12 edges, their first
+// triangle within the round, and the round's triangle -> cell map.
+struct GenWave {
+  uint64_t table[64];
+  uint32_t ids[12][64];
+  uint16_t first[64];
+  uint16_t cell[64];           // word << 6 | bit
+  uint8_t tri_cell[5 * 64];    // at most 5 triangles per cell
+  uint8_t word_mark[64];
+};
+
+// LDS layout of a generate tile of TW words and NT threads (wpr known at run
+// time): bits (3 planes), active cells, vertex bases (2 planes), triangle
+// bases, the waves' rounds.
+template <int TW, int NT>
 struct GenLayout {
-  static constexpr int kRoundTris = 5 * kMaxGenThreads;  // triangles of one round of cells
+  static constexpr int kWaves = NT / 64;
   int segb, segv;
   __host__ __device__ GenLayout(int wpr) : segb(TW + 2 * wpr + 2), segv(TW + wpr + 2) {}
-  // u64: bits (3 planes), case table, active cells; u32: vertex bases
-  // (2 planes), triangle bases, active-cell slots, scan scratch, round
-  // offsets and cell info; u8: the round's triangle -> cell map
-  __host__ __device__ size_t bytes() const {
-    return (size_t)(3 * segb + 256 + TW) * 8 +
-           (size_t)(2 * segv + 2 * (TW + 1) + 32 + 2 * kMaxGenThreads + 1) * 4 + kRoundTris;
+  __host__ __device__ size_t wave_offset() const {
+    return ((size_t)(3 * segb + TW) * 8 + (size_t)(2 * segv + TW + 1) * 4 + 7) / 8 * 8;
   }
+  __host__ __device__ size_t bytes() const { return wave_offset() + kWaves * sizeof(GenWave); }
 };
+
+// Orders the LDS accesses of a wave's lanes among themselves (a wave's LDS
+// operations execute in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Inclusive prefix maximum over the lanes of a wave (wave_incl_scan's steps).
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+  return v;
+}
+
+// Bits b, b+1, ... of the word A followed by the word A1 (b < 64).
+__device__ __forceinline__ uint32_t bit_window(uint64_t A, uint64_t A1, int b) {
+  const uint32_t d0 = (uint32_t)A, d1 = (uint32_t)(A >> 32), d2 = (uint32_t)A1;
+  const bool up = b >= 32;
+  return __builtin_amdgcn_alignbit(up ? d2 : d1, up ? d1 : d0, (uint32_t)b & 31u);
+}
+
+// Case and edge ids of the active cell at bit b of a row word.  Rows of words
+// r_yz: r00 the cell's own, r10 / r20 one and two rows up, r01 / r11 / r21
+// the same a plane up, r02 / r12 two planes up (each with its next word along
+// x, 0 past the row's end).  A row without a neighbour in y (z) is passed as
+// its own neighbour, so its edges in that direction vanish.  An edge's id is
+// the base of its lower endpoint's word plus its rank among the word's
+// active edges; the ranks count bits below b only, which are inside the
+// grid, so they need no row-end masks, and the endpoint at b + 1 = 64, bit 0
+// of the next word, follows the word's last edge in the numbering.  x2: the
+// row has a point b + 2.
+struct RowPair {
+  uint64_t a, a1;  // a word and the next one along x
+};
+__device__ __forceinline__ uint32_t rank_below(uint64_t a, uint64_t y, uint64_t z, uint64_t m) {
+  return (uint32_t)(popc((a ^ (a >> 1)) & m) + popc((a ^ y) & m) + popc((a ^ z) & m));
+}
+__device__ __forceinline__ int cell_edges(const RowPair& r00, const RowPair& r10,
+                                          const RowPair& r20, const RowPair& r01,
+                                          const RowPair& r11, uint64_t r21, uint64_t r02,
+                                          uint64_t r12, int b, bool x2, uint32_t base00,
+                                          uint32_t base10,
+                                          uint32_t base01, uint32_t base11, uint32_t* id) {
+  const uint64_t m = (1ull << b) - 1ull;
+  const uint32_t w00 = bit_window(r00.a, r00.a1, b), w10 = bit_window(r10.a, r10.a1, b);
+  const uint32_t w01 = bit_window(r01.a, r01.a1, b), w11 = bit_window(r11.a, r11.a1, b);
+  const uint32_t w20 = bit_window(r20.a, r20.a1, b), w02 = bit_window(r02, 0ull, b);
+  // flags of the points b (bit 0) and b + 1 (bit 1) of a row
+  const uint32_t x00 = w00 ^ (w00 >> 1), y00 = w00 ^ w10, z00 = w00 ^ w01;
+  const uint32_t x10 = w10 ^ (w10 >> 1), y10 = w10 ^ w20, z10 = w10 ^ w11;
+  const uint32_t x01 = w01 ^ (w01 >> 1), y01 = w01 ^ w11, z01 = w01 ^ w02;
+  const uint32_t e00 = base00 + rank_below(r00.a, r10.a, r01.a, m);
+  const uint32_t e10 = base10 + rank_below(r10.a, r20.a, r11.a, m);
+  const uint32_t e01 = base01 + rank_below(r01.a, r11.a, r02, m);
+  const uint32_t e11 = base11 + rank_below(r11.a, r21, r12, m);
+  const uint32_t n00 = e00 + (x00 & 1u) + (y00 & 1u) + (z00 & 1u);  // first id at b + 1
+  const uint32_t n10 = e10 + (x10 & 1u) + (y10 & 1u) + (z10 & 1u);
+  const uint32_t n01 = e01 + (x01 & 1u) + (y01 & 1u) + (z01 & 1u);
+  const uint32_t one = x2 ? 1u : 0u;  // x-edges at b + 1 exist
+  const uint32_t t00 = (x00 >> 1) & one, t10 = (x10 >> 1) & one, t01 = (x01 >> 1) & one;
+  id[0] = e00;
+  id[3] = e00 + (x00 & 1u);
+  id[8] = e00 + (x00 & 1u) + (y00 & 1u);
+  id[1] = n00 + t00;
+  id[9] = n00 + t00 + ((y00 >> 1) & 1u);
+  id[2] = e10;
+  id[11] = e10 + (x10 & 1u) + (y10 & 1u);
+  id[10] = n10 + t10 + ((y10 >> 1) & 1u);
+  id[4] = e01;
+  id[7] = e01 + (x01 & 1u);
+  id[5] = n01 + t01;
+  id[6] = e11;
+  return (int)((w00 & 3u) | ((w10 & 2u) << 1) | ((w10 & 1u) << 3) | ((w01 & 3u) << 4) |
+               ((w11 & 2u) << 5) | ((w11 & 1u) << 7));
+}
+
+// 12 contiguous bytes.
+template <class T>
+__device__ __forceinline__ void store3(T* p, T a, T b, T c) {
+  const T v[3] = {a, b, c};
+  __builtin_memcpy(p, v, 12);
+}
 
 // Edge flags of the word at LDS index lw of plane sA (its +z plane sC) with
 // position p; branch-free (the +x word is read and masked).
@@ -918,18 +1015,6 @@ __device__ __forceinline__ void lds_flags(const VolGeom& g, const uint64_t* sA, 
                                           uint64_t& fz) {
   const uint64_t A = sA[lw], A1n = sA[lw + 1], B = sA[lw + g.wpr], C = sC[lw];
   edge_flags(p, A, p.q + 1 < g.wpr ? A1n : 0ull, B, C, fx, fy, fz);
-}
-
-__device__ __forceinline__ WordPos make_pos(const VolGeom& g, int q, int j, int k) {
-  WordPos p;
-  p.q = q;
-  p.j = j;
-  p.k = k;
-  p.has_y = j + 1 < g.ny;
-  p.has_z = k + 1 < g.nz;
-  p.pmask = low_mask(g.nx - q * 64);
-  p.xmask = low_mask(g.nx - 1 - q * 64);
-  return p;
 }
 
 // Exclusive scan of one value per thread over the block (thread order);
@@ -1004,34 +1089,44 @@ __device__ __forceinline__ unsigned long long word_bases_nb(const CountSrc& cs, 
   return past ? bp : full;
 }
 
-// One generate tile: words [w_begin, w_begin + TW) of a volume.
+// One generate tile: words [w_begin, w_begin + TW) of a volume, a block of NT
+// threads.
 //   1. stage bits (planes k, k+1, k+2), vertex bases (k, k+1), triangle bases
-//   2. per word: active-cell mask; block scan of the active-cell counts
-//      gives every active cell a slot
-//   3. one thread per output vertex: word by binary search over the vertex
+//   2. a thread per word: active-cell mask.  The last barrier: from here each
+//      wave works alone
+//   3. a thread per output vertex: word by binary search over the vertex
 //      bases, edge by popcount select; coordinates, normal, records
-//   4. rounds of up to blockDim active cells: one thread per cell (word by
-//      binary search over the slots, cell by popcount select) forms its
-//      case; a block scan of NumFaces gives its first triangle and the cell
-//      marks its triangles' entries of the round's triangle -> cell map; one
-//      thread per triangle turns the triangle's edges into vertex ids through
-//      the edge flags, formed where they are read from the staged bits
+//   4. each wave takes a run of words with its share of the tile's triangles,
+//      in rounds of 64 active cells: words mark their first cell's lane, a
+//      prefix maximum gives every lane its word and a popcount select its
+//      cell; the lane forms the cell's case and the ids of all 12 edges at
+//      once (cell_edges: a third of the operations of ranking each triangle
+//      corner by itself), then a lane per triangle picks three of them
+//
+// What bounds it: VALU issue and the chain of loads (staging, then the field
+// values of a vertex).  The waves share the staged words but no barriers, so
+// the chains of different waves overlap.  A block of 256 threads with rounds
+// between barriers took, with 512-word tiles, 63 us at 37 x 29 x 33 points, 86
+// at 256^3 (475 K vertices) and 88 at 512^3 (957 K); this one, with the tiles
+// gen_shape picks, 13, 36 and 62.
 //
 // FROM_COUNTS: the bases come from the count kernel's per-word prefixes and
 // count-tile prefixes (cs) instead of bv / bt; the tile writes the bases of
 // its words (and, for the last tile, entry nwords) to cs.base_v / base_t,
 // and with emit false only that.  has_output skips the check for a tile
 // without output (one round trip).
-template <int TW, class Src, bool FROM_COUNTS = false>
+template <int TW, int NT, class Src, bool dedup, bool FROM_COUNTS = false>
 __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
                                               const uint64_t* __restrict__ b,
                                               const uint32_t* __restrict__ bv,
                                               const uint32_t* __restrict__ bt, int64_t w_begin,
-                                              const OutPtrs& out, bool dedup, bool normals,
+                                              const OutPtrs& out, bool normals,
                                               int64_t vol_base_v, int64_t vol_base_t,
                                               uint64_t* s_dyn, const CountSrc& cs = CountSrc{},
                                               bool emit = true, bool has_output = false) {
-  const int tid = threadIdx.x, nt = blockDim.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  static_assert(NT >= TW, "a thread per word");
+  constexpr int nt = NT, nwaves = NT / 64;
   const int nw = (int)min((int64_t)TW, g.nwords - w_begin);
   if constexpr (FROM_COUNTS) {
     // count tiles without output (has_output: known not to be the case):
@@ -1057,20 +1152,15 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
       return;  // uniform: no output in this tile
   }
 
-  const GenLayout<TW> L(g.wpr);
+  const GenLayout<TW, NT> L(g.wpr);
   uint64_t* s_b0 = s_dyn;
   uint64_t* s_b1 = s_b0 + L.segb;
   uint64_t* s_b2 = s_b1 + L.segb;
-  uint64_t* s_case = s_b2 + L.segb;
-  uint64_t* s_act = s_case + 256;
+  uint64_t* s_act = s_b2 + L.segb;
   uint32_t* s_v0 = reinterpret_cast<uint32_t*>(s_act + TW);
   uint32_t* s_v1 = s_v0 + L.segv;
   uint32_t* s_t = s_v1 + L.segv;
-  uint32_t* s_cs = s_t + TW + 1;
-  uint32_t* s_w = s_cs + TW + 1;                     // scan scratch (<= 16 waves)
-  uint32_t* s_rfirst = s_w + 32;                     // [nt + 1]
-  uint32_t* s_rinfo = s_rfirst + kMaxGenThreads + 1;  // [nt]: li << 16 | bit << 8 | case
-  uint8_t* s_tcell = reinterpret_cast<uint8_t*>(s_rinfo + kMaxGenThreads);  // [kRoundTris]
+  GenWave& W = reinterpret_cast<GenWave*>(reinterpret_cast<char*>(s_dyn) + L.wave_offset())[tid >> 6];
 
   // staging: each thread issues the loads of up to kStageU of its words
   // (clamped indices, every load unconditional) before storing any of them,
@@ -1137,7 +1227,6 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
     }
     for (int i = tid; i <= nw; i += nt) s_t[i] = bt[w_begin + i];
   }
-  for (int i = tid; i < 256; i += nt) s_case[i] = c_case_table[i];
   __syncthreads();
   const uint32_t tv0 = s_v0[0], tv1 = s_v0[nw];
   const uint32_t tt0 = s_t[0], tt1 = s_t[nw];
@@ -1153,44 +1242,22 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
     if (!emit || (tv0 == tv1 && tt0 == tt1)) return;  // bases only, or no output here
   }
 
-  // 2. per word (each thread a run of consecutive words): active cells
-  const int wpt = (TW + nt - 1) / nt;
-  uint32_t ncell = 0;
-  {
-    const int i0 = tid * wpt;
-    if (i0 < nw) {
-      WordIter it;
-      it.init(g, (int)(w_begin + i0));
-      for (int u = 0; u < wpt && i0 + u < nw; ++u) {
-        const int li = i0 + u;
-        const WordPos p = it.pos(g);
-        const bool nx1 = p.q + 1 < g.wpr;
-        CellPlanes cp;
-        cell_planes(p, s_b0[li], nx1 ? s_b0[li + 1] : 0ull, s_b0[li + g.wpr],
-                    nx1 ? s_b0[li + g.wpr + 1] : 0ull, s_b1[li], nx1 ? s_b1[li + 1] : 0ull,
-                    s_b1[li + g.wpr], nx1 ? s_b1[li + g.wpr + 1] : 0ull, cp);
-        s_act[li] = cp.active;
-        ncell += (uint32_t)popc(cp.active);
-        it.next(g);
-      }
-    }
-  }
-  uint32_t n_cells;
-  {
-    uint32_t run = block_excl_scan(ncell, n_cells, s_w);
-    const int i0 = tid * wpt;
-    for (int u = 0; u < wpt && i0 + u < nw; ++u) {
-      s_cs[i0 + u] = run;
-      run += (uint32_t)popc(s_act[i0 + u]);
-    }
-    if (tid == 0) s_cs[nw] = n_cells;
+  // 2. active cells of the thread's word
+  if (tid < nw) {
+    const WordPos p = word_pos(g, w_begin + tid);
+    const bool nx1 = p.q + 1 < g.wpr;
+    CellPlanes cp;
+    cell_planes(p, s_b0[tid], nx1 ? s_b0[tid + 1] : 0ull, s_b0[tid + g.wpr],
+                nx1 ? s_b0[tid + g.wpr + 1] : 0ull, s_b1[tid], nx1 ? s_b1[tid + 1] : 0ull,
+                s_b1[tid + g.wpr], nx1 ? s_b1[tid + g.wpr + 1] : 0ull, cp);
+    s_act[tid] = cp.active;
   }
   __syncthreads();
 
   // 3. vertices (dedup: one per active edge, in id order).  A thread's
   //    first vertex is located and its field values loaded here, and
   //    finished after the triangle rounds: the loads' latency overlaps the
-  //    rounds' LDS work (their barriers wait for LDS operations only).
+  //    rounds' LDS work.
   const int nV = (int)(tv1 - tv0);
   auto locate = [&](int vl, int& x, int& y, int& z, int& axis) {
     const int li = find_word(s_v0, nw, tv0 + (uint32_t)vl);
@@ -1206,14 +1273,8 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
   auto store_vertex = [&](int vl, int axis, const float xyz[3], const float nrm[3], float w,
                           int32_t pa, int32_t pb) {
     const int64_t gv = (int64_t)tv0 + vl;
-    out.vertices[3 * gv + 0] = xyz[0];
-    out.vertices[3 * gv + 1] = xyz[1];
-    out.vertices[3 * gv + 2] = xyz[2];
-    if (normals) {
-      out.normals[3 * gv + 0] = nrm[0];
-      out.normals[3 * gv + 1] = nrm[1];
-      out.normals[3 * gv + 2] = nrm[2];
-    }
+    store3(out.vertices + 3 * gv, xyz[0], xyz[1], xyz[2]);
+    if (normals) store3(out.normals + 3 * gv, nrm[0], nrm[1], nrm[2]);
     if (out.edges) out.edges[gv] = ((uint32_t)axis << 30) | (uint32_t)pa;
     if (out.interp_first) out.interp_first[gv] = (int32_t)pa;
     if (out.interp_second) out.interp_second[gv] = (int32_t)pb;
@@ -1228,77 +1289,103 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
     point_loads(g, f, fx0, fy0, fz0, fax, normals, fl, fpa, fpb);
   }
 
-  // 4. triangles
-  uint32_t carry = 0;
-  for (uint32_t c0 = 0; c0 < n_cells; c0 += (uint32_t)nt) {  // uniform
-    const uint32_t slot = c0 + (uint32_t)tid;
-    uint32_t nf = 0;
-    if (slot < n_cells) {
-      const int li = find_word(s_cs, nw, slot);
-      const int bit = select_bit(s_act[li], (int)(slot - s_cs[li]));
-      const WordPos p = word_pos(g, w_begin + li);
-      const bool nx1 = p.q + 1 < g.wpr;
-      CellPlanes cp;
-      cell_planes(p, s_b0[li], nx1 ? s_b0[li + 1] : 0ull, s_b0[li + g.wpr],
-                  nx1 ? s_b0[li + g.wpr + 1] : 0ull, s_b1[li], nx1 ? s_b1[li + 1] : 0ull,
-                  s_b1[li + g.wpr], nx1 ? s_b1[li + g.wpr + 1] : 0ull, cp);
-      const int cs = cell_case(cp, bit);
-      nf = (uint32_t)(s_case[cs] >> 60);
-      s_rinfo[tid] = ((uint32_t)li << 16) | ((uint32_t)bit << 8) | (uint32_t)cs;
+  // 4. triangles: the wave's words are those whose first triangle lies in its
+  //    share of the tile's (lanes 0 and 1 search its ends)
+  const int n_tri = (int)(tt1 - tt0);
+  int wa = 0, wb = nw;
+  if constexpr (nwaves > 1) {
+    const uint32_t part = (uint32_t)(tid >> 6) + (lane == 1 ? 1u : 0u);
+    const uint32_t want = tt0 + part * (uint32_t)n_tri / (uint32_t)nwaves;
+    int lo = 0, hi = nw;  // first word whose base is at least `want`
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      const bool below = s_t[mid] < want;
+      lo = below ? mid + 1 : lo;
+      hi = below ? hi : mid;
     }
-    uint32_t round_tris;
-    const uint32_t first = block_excl_scan(nf, round_tris, s_w);
-    for (uint32_t t = 0; t < nf; ++t) s_tcell[first + t] = (uint8_t)tid;  // <= 5 per cell
-    s_rfirst[tid] = first;
-    __syncthreads();
-    for (uint32_t tl = (uint32_t)tid; tl < round_tris; tl += (uint32_t)nt) {
-      const int c = (int)s_tcell[tl];
-      const uint32_t info = s_rinfo[c];
-      const int li = (int)(info >> 16), bit = (int)((info >> 8) & 0xff), cs = (int)(info & 0xff);
-      const int visit = (int)(tl - s_rfirst[c]);
+    wa = __builtin_amdgcn_readlane(lo, 0);
+    wb = part == (uint32_t)nwaves ? nw : lo;
+    wb = __builtin_amdgcn_readlane(wb, 1);
+  }
+  int64_t tri = n_tri > 0 && wa < wb ? (int64_t)s_t[wa] : 0;
+  for (int c = wa; c < wb && n_tri > 0; c += 64) {  // wave-uniform
+    const uint64_t act_l = c + lane < wb ? s_act[c + lane] : 0ull;
+    const uint32_t nc = (uint32_t)popc(act_l);
+    const uint32_t inc = wave_incl_scan(nc), n_cells = wave_last(inc), start = inc - nc;
+    for (uint32_t c0 = 0; c0 < n_cells; c0 += 64u) {
+      W.word_mark[lane] = 0;
+      wave_lds_sync();
+      if (nc != 0u && start < c0 + 64u && inc > c0)
+        W.word_mark[max(start, c0) - c0] = (uint8_t)(lane + 1);
+      wave_lds_sync();
+      const int wl = (int)wave_incl_max((uint32_t)W.word_mark[lane]) - 1;
+      const uint32_t slot = c0 + (uint32_t)lane;
+      const bool valid = slot < n_cells;
+      const uint32_t wstart = (uint32_t)__shfl((int)start, wl, 64);
+      const int li = c + wl;
+      const int bit = select_bit(s_act[li], valid ? (int)(slot - wstart) : 0);
       const WordPos p = word_pos(g, w_begin + li);
-      const uint64_t packed = s_case[cs];
-      const int64_t t = (int64_t)tt0 + carry + tl;
-      int32_t ids[3];
+      const bool nx1 = p.q + 1 < g.wpr, hy2 = p.j + 2 < g.ny, hz2 = p.k + 2 < g.nz;
+      const int l1 = li + g.wpr, l2 = hy2 ? l1 + g.wpr : l1;
+      const uint64_t* s_z2 = hz2 ? s_b2 : s_b1;
+      auto pair = [&](const uint64_t* row, int i) {
+        const uint64_t n = row[i + 1];
+        return RowPair{row[i], nx1 ? n : 0ull};
+      };
+      uint32_t id[12];
+      const int cs = cell_edges(pair(s_b0, li), pair(s_b0, l1), pair(s_b0, l2), pair(s_b1, li),
+                                pair(s_b1, l1), s_b1[l2], s_z2[li], s_z2[l1], bit,
+                                p.q * 64 + bit + 2 < g.nx, s_v0[li], s_v0[l1], s_v1[li], s_v1[l1],
+                                id);
+      const uint64_t table = c_case_table[cs];
+      const uint32_t nf = valid ? (uint32_t)(table >> 60) : 0u;
+      const uint32_t finc = wave_incl_scan(nf), round_tris = wave_last(finc), ffirst = finc - nf;
+      W.table[lane] = table;
+      W.first[lane] = (uint16_t)ffirst;
+      if (dedup) {
 #pragma unroll
-      for (int v = 0; v < 3; ++v) {
-        const int e = (int)((packed >> (4 * (3 * visit + v))) & 0xF);
-        const int code = (int)((kEdgeCodes >> (5 * e)) & 31u);
-        const int dx = code & 1, dy = (code >> 1) & 1, dz = (code >> 2) & 1, axis = code >> 3;
-        const int x = p.q * 64 + bit + dx;
-        if (dedup) {
-          const int qq = x >> 6, bb = x & 63;
-          const int lw2 = li + (qq - p.q) + dy * g.wpr;  // <= nw + wpr
-          const WordPos p2 = make_pos(g, qq, p.j + dy, p.k + dz);
-          uint64_t fx, fy, fz;
-          lds_flags(g, dz ? s_b1 : s_b0, dz ? s_b2 : s_b1, lw2, p2, fx, fy, fz);
-          const uint32_t base = (dz ? s_v1 : s_v0)[lw2];
-          ids[v] = (int32_t)((int64_t)base + edge_rank(fx, fy, fz, bb, axis) - vol_base_v);
-        } else {
-          const int64_t corner = 3 * t + v;
-          float xyz[3], nrm[3], w;
-          int32_t pa, pb;
-          emit_point(g, f, x, p.j + dy, p.k + dz, axis, normals, xyz, nrm, w, pa, pb);
-          out.vertices[3 * corner + 0] = xyz[0];
-          out.vertices[3 * corner + 1] = xyz[1];
-          out.vertices[3 * corner + 2] = xyz[2];
-          if (normals) {
-            out.normals[3 * corner + 0] = nrm[0];
-            out.normals[3 * corner + 1] = nrm[1];
-            out.normals[3 * corner + 2] = nrm[2];
-          }
-          if (out.interp_first) out.interp_first[corner] = (int32_t)pa;
-          if (out.interp_second) out.interp_second[corner] = (int32_t)pb;
-          if (out.interp_weight) out.interp_weight[corner] = w;
-          ids[v] = (int32_t)(corner - 3 * vol_base_t);
-        }
+        for (int e = 0; e < 12; ++e) W.ids[e][lane] = id[e];
+      } else {
+        W.cell[lane] = (uint16_t)((li << 6) | bit);
       }
-      out.conn[3 * t + 0] = ids[0];
-      out.conn[3 * t + 1] = ids[1];
-      out.conn[3 * t + 2] = ids[2];
+#pragma unroll
+      for (uint32_t t = 0; t < 5u; ++t)
+        if (t < nf) W.tri_cell[ffirst + t] = (uint8_t)lane;
+      wave_lds_sync();
+      for (uint32_t tl = (uint32_t)lane; tl < round_tris; tl += 64u) {
+        const int cl = (int)W.tri_cell[tl];
+        const uint32_t visit = tl - W.first[cl];
+        const uint32_t es = (uint32_t)(W.table[cl] >> (12u * visit));
+        const int64_t t = tri + tl;
+        int32_t ids[3];
+        if (dedup) {
+#pragma unroll
+          for (int v = 0; v < 3; ++v)
+            ids[v] = (int32_t)((int64_t)W.ids[(es >> (4 * v)) & 15u][cl] - vol_base_v);
+        } else {
+          const int cw = (int)W.cell[cl] >> 6, cb = (int)W.cell[cl] & 63;
+          const WordPos pc = word_pos(g, w_begin + cw);
+#pragma unroll
+          for (int v = 0; v < 3; ++v) {
+            const int code = (int)((kEdgeCodes >> (5 * ((es >> (4 * v)) & 15u))) & 31u);
+            const int64_t corner = 3 * t + v;
+            float xyz[3], nrm[3], w;
+            int32_t pa, pb;
+            emit_point(g, f, pc.q * 64 + cb + (code & 1), pc.j + ((code >> 1) & 1),
+                       pc.k + ((code >> 2) & 1), code >> 3, normals, xyz, nrm, w, pa, pb);
+            store3(out.vertices + 3 * corner, xyz[0], xyz[1], xyz[2]);
+            if (normals) store3(out.normals + 3 * corner, nrm[0], nrm[1], nrm[2]);
+            if (out.interp_first) out.interp_first[corner] = (int32_t)pa;
+            if (out.interp_second) out.interp_second[corner] = (int32_t)pb;
+            if (out.interp_weight) out.interp_weight[corner] = w;
+            ids[v] = (int32_t)(corner - 3 * vol_base_t);
+          }
+        }
+        store3(out.conn + 3 * t, ids[0], ids[1], ids[2]);
+      }
+      tri += round_tris;
+      wave_lds_sync();  // the round's LDS is reused
     }
-    carry += round_tris;
-    __syncthreads();  // s_rfirst / s_rinfo / s_tcell reused by the next round
   }
 
   if (first) {
