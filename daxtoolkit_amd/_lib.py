@@ -136,6 +136,10 @@ _SIGNATURES = {
                                                  C.c_int]),
     "dax_hip_mc_slice": (C.c_int, [i64, i64, i64, vp, vp, vp, vp, C.c_uint, vp, sz, vp, vp, vp,
                                    vp, vp, vp, vp, i64, i64, vp, vp]),
+    "dax_hip_mc_slice_count": (C.c_int, [i64, i64, i64, vp, vp, vp, vp, vp, sz, P_i64, P_i64, vp]),
+    "dax_hip_mc_slice_generate": (C.c_int, [i64, i64, i64, vp, vp, vp, vp, C.c_uint, vp, sz, vp,
+                                            vp, vp, vp, vp, vp, vp, i64, i64, vp, vp]),
+    "dax_hip_mc_count": (C.c_int, [vp, i64, i64, i64, f32, vp, sz, P_i64, P_i64, vp]),
     "dax_hip_mc_bits": (C.c_int, [vp, i64, i64, i64, f32, vp, sz, vp]),
     "dax_hip_mc_scan": (C.c_int, [i64, i64, i64, vp, sz, vp]),
     "dax_hip_mc_generate": (C.c_int, [vp, i64, i64, i64, vp, vp, f32, C.c_uint, vp, sz,

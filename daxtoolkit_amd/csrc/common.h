@@ -32,6 +32,23 @@ struct TempBuf {
   int alloc(size_t bytes) { return temp_alloc(&p, bytes, s); }
 };
 
+// Eight 64-bit words of pinned host memory that kernels write results into, so
+// that a size reaches the host with the end of the kernel that has it: no
+// copy launch and no staging buffer between.  From a fixed table of slots
+// (one page, kept until the process ends), held by one call at a time; `p` is
+// null when every slot is taken or there is no pinned memory, and the caller
+// then copies.  A slot is reused only after its holder has synchronised.
+struct HostSlot {
+  int64_t* p = nullptr;
+  HostSlot();
+  ~HostSlot();
+  HostSlot(const HostSlot&) = delete;
+  HostSlot& operator=(const HostSlot&) = delete;
+
+ private:
+  int index_ = -1;
+};
+
 #define DAXHIP_CHECK(expr)                                  \
   do {                                                      \
     hipError_t _e = (expr);                                 \

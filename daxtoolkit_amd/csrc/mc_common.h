@@ -263,7 +263,7 @@ __device__ __forceinline__ uint64_t pack_status(uint32_t v, uint32_t t, uint64_t
 // Control block at the end of the workspace.
 struct Ctrl {
   uint32_t tile_counter;
-  uint32_t pad;
+  uint32_t tpb_shift;  // log2 of the count tiles per count block of the last scan
   unsigned long long total_v;  // 64-bit totals: vertices (active edges), triangles
   unsigned long long total_t;
 };

@@ -171,6 +171,13 @@ struct GenOrder {
   uint32_t* gorder;  // the gather tiles' order: entry 0 cleared (the adjoint writes it)
 };
 
+// Where the scan reports {T, U} besides the control block (each may be null):
+// device memory, and pinned host memory.
+struct ScanOut {
+  int64_t* counts;
+  int64_t* host;
+};
+
 constexpr int kTsumThreads = 1024;
 constexpr int kTsumWaves = kTsumThreads / 64;
 constexpr uint32_t kOrderStage = 16384;  // 64 KiB of LDS
@@ -187,7 +194,8 @@ template <bool LARGE>
 __global__ __launch_bounds__(kTsumThreads) void k_scan_tsums(const unsigned long long* __restrict__ bsum,
                                                              unsigned long long* __restrict__ bpre,
                                                              int64_t n, Ctrl* __restrict__ ctrl,
-                                                             GenOrder go) {
+                                                             GenOrder go, int tpb_shift,
+                                                             ScanOut so) {
   constexpr int kWaves = kTsumWaves;
   // the scan's wave sums, then the dispatch order's LDS window
   __shared__ uint32_t s_stage[kOrderStage];
@@ -251,6 +259,15 @@ __global__ __launch_bounds__(kTsumThreads) void k_scan_tsums(const unsigned long
     bpre[n] = (cv & 0xffffffffull) | (ct << 32);
     ctrl->total_v = cv;
     ctrl->total_t = ct;
+    ctrl->tpb_shift = (uint32_t)tpb_shift;
+    if (so.counts) {
+      so.counts[0] = (int64_t)ct;
+      so.counts[1] = (int64_t)cv;
+    }
+    if (so.host) {
+      __hip_atomic_store(so.host, (int64_t)ct, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(so.host + 1, (int64_t)cv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 
   if (units)
@@ -266,7 +283,9 @@ __global__ __launch_bounds__(kTsumThreads) void k_scan_tsums(const unsigned long
 }
 
 // Bases of every row word (and entry nwords): tile prefix + local prefix.
-__global__ __launch_bounds__(256) void k_bases(VolGeom g, CountSrc cs) {
+__global__ __launch_bounds__(256) void k_bases(VolGeom g, CountSrc cs,
+                                               const Ctrl* __restrict__ ctrl) {
+  cs.tpb_shift = (int)ctrl->tpb_shift;
   const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (w > g.nwords) return;
   const unsigned long long p = word_bases(cs, w);
@@ -283,6 +302,7 @@ __global__ __launch_bounds__(NT, 4) void k_generate(
   extern __shared__ uint64_t s_dyn[];
   const bool normals = (flags & DAX_HIP_MC_NORMALS) != 0 && out.normals != nullptr;
   const uint64_t total_v = ctrl->total_v, total_t = ctrl->total_t;
+  cs.tpb_shift = (int)ctrl->tpb_shift;
   const uint64_t n_points = dedup ? total_v : 3ull * total_t;
   if (blockIdx.x == 0 && threadIdx.x == 0 && counts) {
     counts[0] = (int64_t)total_t;
@@ -692,15 +712,19 @@ int gen_tile_words(const Tuning& tu) {
              : 512;
 }
 
-// Where the generate kernel reads the word bases; a count block holds two
-// count tiles per wave, with the waves of launch_scan's dispatch (1, 2, 8,
-// else 4).
-CountSrc count_src(const char* ws, const Workspace& L, const Tuning& tu) {
+// A count block holds two count tiles per wave, with the waves of
+// launch_scan's dispatch (1, 2, 8, else 4).
+int tiles_per_block_shift(const Tuning& tu) {
+  return tu.scan_sub == 1 ? 1 : (tu.scan_sub == 2 ? 2 : (tu.scan_sub == 8 ? 4 : 3));
+}
+
+// Where the generate kernel reads the word bases (the tiles per count block
+// come from the control block: the scan may have run under another tuning).
+CountSrc count_src(const char* ws, const Workspace& L) {
   char* wsm = const_cast<char*>(ws);
   return CountSrc{(const uint32_t*)(ws + L.off_counts),
                   (const unsigned long long*)(ws + L.off_tsum),
-                  (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles,
-                  tu.scan_sub == 1 ? 1 : (tu.scan_sub == 2 ? 2 : (tu.scan_sub == 8 ? 4 : 3)),
+                  (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0,
                   (uint32_t*)(wsm + L.off_base_v), (uint32_t*)(wsm + L.off_base_t)};
 }
 
@@ -709,7 +733,7 @@ CountSrc count_src(const char* ws, const Workspace& L, const Tuning& tu) {
 // word's bases (calls that stop before the generate kernel, which otherwise
 // stores them).
 int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu, hipStream_t s,
-                bool bases = false) {
+                bool bases = false, ScanOut so = ScanOut{nullptr, nullptr}) {
   const uint64_t* bits = (const uint64_t*)(ws + L.off_bits);
   uint32_t* lpre = (uint32_t*)(ws + L.off_counts);
   unsigned long long* tloc = (unsigned long long*)(ws + L.off_tsum);
@@ -744,13 +768,15 @@ int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu
   const GenOrder go{tc.gcls, g.nwords, tw, tc.tw > 0, units ? (uint32_t)sp : 0u,
                     (uint32_t*)(ws + L.off_order), (uint32_t*)(ws + L.off_gorder)};
   if (ceil_div(ceil_div(g.nwords, (int64_t)tw), (int64_t)kTsumThreads) > kOrderRegTiles)
-    k_scan_tsums<true><<<1, dim3(kTsumThreads), 0, s>>>(bsum, bpre, nblocks, (Ctrl*)(ws + L.off_ctrl), go);
+    k_scan_tsums<true><<<1, dim3(kTsumThreads), 0, s>>>(
+        bsum, bpre, nblocks, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
   else
-    k_scan_tsums<false><<<1, dim3(kTsumThreads), 0, s>>>(bsum, bpre, nblocks, (Ctrl*)(ws + L.off_ctrl), go);
+    k_scan_tsums<false><<<1, dim3(kTsumThreads), 0, s>>>(
+        bsum, bpre, nblocks, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
   DAXHIP_LAUNCH_CHECK("k_scan_tsums");
   if (bases) {
     k_bases<<<dim3((unsigned)ceil_div(g.nwords + 1, 256)), dim3(256), 0, s>>>(
-        g, count_src(ws, L, tu));
+        g, count_src(ws, L), (const Ctrl*)(ws + L.off_ctrl));
     DAXHIP_LAUNCH_CHECK("k_bases");
   }
   return DAX_HIP_OK;
@@ -767,7 +793,7 @@ int launch_generate_tw(const VolGeom& g, const Src& field, const char* ws, const
   const int64_t all = ceil_div(g.nwords, (int64_t)TW);
   if (t_hi < 0) t_hi = all;
   const int64_t ntiles = std::max<int64_t>(t_hi - t_lo, 1);
-  const CountSrc cs = count_src(ws, L, tu);
+  const CountSrc cs = count_src(ws, L);
   const uint32_t* order =
       (t_lo == 0 && t_hi == all) ? (const uint32_t*)(ws + L.off_order) : nullptr;
 #define DAXHIP_GEN(DEDUP)                                                                        \
@@ -857,10 +883,33 @@ int check_outputs(const VolGeom& g, const float* field, unsigned flags, const fl
   return DAX_HIP_OK;
 }
 
-__global__ void k_write_counts(const Ctrl* ctrl, int64_t* counts, unsigned flags) {
-  const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
-  counts[0] = (int64_t)ctrl->total_t;
-  counts[1] = dedup ? (int64_t)ctrl->total_v : 3 * (int64_t)ctrl->total_t;
+// T and U within the int32 dax::Id range.
+int check_totals(int64_t t, int64_t u) {
+  if (u > 0x7fffffffLL || 3 * t > 0x7fffffffLL) {
+    set_error("dax_hip_mc: %lld triangles / %lld points exceed the int32 dax::Id range",
+              (long long)t, (long long)u);
+    return DAX_HIP_EXEC_ERROR;
+  }
+  return DAX_HIP_OK;
+}
+
+// Count + scan of classified bits, with {T, U} read back (synchronous).
+int count_sync(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu, int64_t* h_tris,
+               int64_t* h_points, hipStream_t s) {
+  int64_t c[2] = {0, 0};
+  HostSlot slot;
+  int rc;
+  if ((rc = launch_scan(g, ws, L, tu, s, false, ScanOut{nullptr, slot.p}))) return rc;
+  unsigned long long vt[2];
+  if (!slot.p)
+    DAXHIP_CHECK(hipMemcpyAsync(vt, ws + L.off_ctrl + offsetof(Ctrl, total_v), sizeof(vt),
+                                hipMemcpyDeviceToHost, s));
+  DAXHIP_CHECK(hipStreamSynchronize(s));
+  c[0] = slot.p ? ((volatile int64_t*)slot.p)[0] : (int64_t)vt[1];
+  c[1] = slot.p ? ((volatile int64_t*)slot.p)[1] : (int64_t)vt[0];
+  *h_tris = c[0];
+  *h_points = c[1];
+  return check_totals(c[0], c[1]);
 }
 
 }  // namespace
@@ -932,12 +981,25 @@ int dax_hip_mc_classify(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   char* ws = (char*)d_workspace;
   const Tuning tu = tuning_for(nx, ny, nz);
   if ((rc = launch_bits(g, d_field, ws, L, tu, s))) return rc;
-  if ((rc = launch_scan(g, ws, L, tu, s, true))) return rc;
-  if (d_counts) {
-    k_write_counts<<<1, 1, 0, s>>>((const Ctrl*)(ws + L.off_ctrl), d_counts, DAX_HIP_MC_DEDUP);
-    DAXHIP_LAUNCH_CHECK("k_write_counts");
+  return launch_scan(g, ws, L, tu, s, true, ScanOut{d_counts, nullptr});
+}
+
+int dax_hip_mc_count(const float* d_field, int64_t nx, int64_t ny, int64_t nz, float iso,
+                     void* d_workspace, size_t workspace_bytes, int64_t* h_tris,
+                     int64_t* h_points, void* stream) {
+  VolGeom g;
+  int rc = make_geom(nx, ny, nz, nullptr, nullptr, iso, g);
+  if (rc) return rc;
+  Workspace L;
+  if ((rc = check_ws(g, workspace_bytes, L, d_workspace))) return rc;
+  if (!d_field || !h_tris || !h_points) {
+    set_error("dax_hip_mc_count: field, h_tris and h_points are required");
+    return DAX_HIP_BAD_VALUE;
   }
-  return DAX_HIP_OK;
+  hipStream_t s = (hipStream_t)stream;
+  const Tuning tu = tuning_for(nx, ny, nz);
+  if ((rc = launch_bits(g, d_field, (char*)d_workspace, L, tu, s))) return rc;
+  return count_sync(g, (char*)d_workspace, L, tu, h_tris, h_points, s);
 }
 
 int dax_hip_mc_forward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
@@ -1041,12 +1103,49 @@ int dax_hip_mc_slice_classify(int64_t nx, int64_t ny, int64_t nz, const float* h
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)d_workspace;
   if ((rc = launch_bits_plane(g, pl, ws, L, s))) return rc;
-  if ((rc = launch_scan(g, ws, L, tuning_for(nx, ny, nz), s, true))) return rc;
-  if (d_counts) {
-    k_write_counts<<<1, 1, 0, s>>>((const Ctrl*)(ws + L.off_ctrl), d_counts, DAX_HIP_MC_DEDUP);
-    DAXHIP_LAUNCH_CHECK("k_write_counts");
+  return launch_scan(g, ws, L, tuning_for(nx, ny, nz), s, true, ScanOut{d_counts, nullptr});
+}
+
+int dax_hip_mc_slice_count(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
+                           const float* h_spacing3, const float* h_plane_origin3,
+                           const float* h_plane_normal3, void* d_workspace,
+                           size_t workspace_bytes, int64_t* h_tris, int64_t* h_points,
+                           void* stream) {
+  VolGeom g;
+  FieldPlane pl;
+  int rc = make_slice(nx, ny, nz, h_origin3, h_spacing3, h_plane_origin3, h_plane_normal3, g, pl);
+  if (rc) return rc;
+  Workspace L;
+  if ((rc = check_ws(g, workspace_bytes, L, d_workspace))) return rc;
+  if (!h_tris || !h_points) {
+    set_error("dax_hip_mc_slice_count: h_tris and h_points are required");
+    return DAX_HIP_BAD_VALUE;
   }
-  return DAX_HIP_OK;
+  hipStream_t s = (hipStream_t)stream;
+  if ((rc = launch_bits_plane(g, pl, (char*)d_workspace, L, s))) return rc;
+  return count_sync(g, (char*)d_workspace, L, tuning_for(nx, ny, nz), h_tris, h_points, s);
+}
+
+int dax_hip_mc_slice_generate(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
+                              const float* h_spacing3, const float* h_plane_origin3,
+                              const float* h_plane_normal3, unsigned flags,
+                              const void* d_workspace, size_t workspace_bytes, float* d_vertices,
+                              float* d_normals, int32_t* d_conn, uint32_t* d_edges,
+                              int32_t* d_interp_first, int32_t* d_interp_second,
+                              float* d_interp_weight, int64_t cap_points, int64_t cap_tris,
+                              int64_t* d_counts, void* stream) {
+  VolGeom g;
+  FieldPlane pl;
+  int rc = make_slice(nx, ny, nz, h_origin3, h_spacing3, h_plane_origin3, h_plane_normal3, g, pl);
+  if (rc) return rc;
+  Workspace L;
+  if ((rc = check_ws(g, workspace_bytes, L, (void*)d_workspace))) return rc;
+  static const float kNoField = 0.0f;  // the slice reads no field
+  if ((rc = check_outputs(g, &kNoField, flags, d_vertices, d_conn, d_edges, d_counts))) return rc;
+  OutPtrs o{d_vertices, d_normals, d_conn, d_edges, d_interp_first, d_interp_second,
+            d_interp_weight};
+  return launch_generate_src(g, pl, (const char*)d_workspace, L, flags, o, cap_points, cap_tris,
+                             d_counts, tuning_for(nx, ny, nz), (hipStream_t)stream);
 }
 
 int dax_hip_mc_slice(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
@@ -1081,11 +1180,7 @@ int dax_hip_mc_read_counts(const int64_t* d_counts, int64_t cap_points, int64_t 
   DAXHIP_CHECK(hipStreamSynchronize((hipStream_t)stream));
   if (h_tris) *h_tris = c[0];
   if (h_points) *h_points = c[1];
-  if (c[1] > 0x7fffffffLL || 3 * c[0] > 0x7fffffffLL) {
-    set_error("dax_hip_mc: %lld triangles / %lld points exceed the int32 dax::Id range",
-              (long long)c[0], (long long)c[1]);
-    return DAX_HIP_EXEC_ERROR;
-  }
+  if (const int rc = check_totals(c[0], c[1])) return rc;
   if (c[0] > cap_tris || c[1] > cap_points) {
     set_error("dax_hip_mc: output needs %lld triangles / %lld points, capacity %lld / %lld",
               (long long)c[0], (long long)c[1], (long long)cap_tris, (long long)cap_points);

@@ -1046,7 +1046,7 @@ struct CountSrc {
   const unsigned long long* __restrict__ tloc;
   const unsigned long long* __restrict__ bpre;
   int64_t n_ctiles;
-  int tpb_shift;  // log2 of the count tiles per count block
+  int tpb_shift;  // log2 of the count tiles per count block (from the control block)
   uint32_t* __restrict__ base_v;
   uint32_t* __restrict__ base_t;
 };

@@ -84,6 +84,38 @@ hipMemPool_t pool_of(int dev, int* rc) {  // g_pool_mu held
 }
 }  // namespace
 
+namespace {
+constexpr int kHostSlots = 64;
+std::mutex g_slot_mu;
+int64_t* g_slots = nullptr;       // guarded by g_slot_mu, as are the next two
+bool g_slots_tried = false;
+uint64_t g_slots_used = 0;        // bit i: slot i is held
+static_assert(kHostSlots == 64, "one bit per slot");
+}  // namespace
+
+HostSlot::HostSlot() {
+  std::lock_guard<std::mutex> lock(g_slot_mu);
+  if (!g_slots_tried) {
+    g_slots_tried = true;
+    void* m = nullptr;
+    if (hipHostMalloc(&m, (size_t)kHostSlots * 64, hipHostMallocPortable | hipHostMallocMapped) ==
+        hipSuccess)
+      g_slots = (int64_t*)m;
+    else
+      (void)hipGetLastError();
+  }
+  if (!g_slots || ~g_slots_used == 0ull) return;
+  index_ = __builtin_ctzll(~g_slots_used);
+  g_slots_used |= 1ull << index_;
+  p = g_slots + 8 * index_;
+}
+
+HostSlot::~HostSlot() {
+  if (index_ < 0) return;
+  std::lock_guard<std::mutex> lock(g_slot_mu);
+  g_slots_used &= ~(1ull << index_);
+}
+
 int temp_alloc(void** p, size_t bytes, hipStream_t s) {
   *p = nullptr;
   int dev = 0;

@@ -237,28 +237,50 @@ def forward_phases(field: torch.Tensor, iso: float, buf: ForwardBuffers, origin=
         events[3].record()
 
 
+def _sized_outputs(T: int, U: int, device, dedup: bool, normals: bool, edges: bool, interp: bool):
+    """Outputs for T triangles and U points (of duplicate removal); at least
+    one row each, so that every pointer is valid."""
+    if not dedup:
+        U = 3 * T
+    n, t = max(U, 1), max(T, 1)
+    f32 = lambda *shape: torch.empty(shape, dtype=torch.float32, device=device)
+    i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=device)
+    return U, [f32(n, 3), f32(n, 3) if normals else None, i32(t, 3), i32(n) if edges else None,
+               i32(n) if interp else None, i32(n) if interp else None,
+               f32(n) if interp else None]
+
+
+def _sized_contour(T: int, U: int, outs, ws, counts, dims) -> Contour:
+    """The Contour of filled outputs (cut to their sizes where one row stands for none)."""
+    v, n, c, e, first, second, w = outs
+    if U == 0:
+        v, n, e, first, second, w = (x if x is None else x[:0] for x in (v, n, e, first, second, w))
+    return Contour(vertices=v, connectivity=c if T else c[:0], normals=n, edges=e,
+                   interp_first=first, interp_second=second, interp_weight=w, workspace=ws,
+                   counts=counts, grid_points=dims[0] * dims[1] * dims[2])
+
+
 def forward(field: torch.Tensor, iso: float, origin=(0, 0, 0), spacing=(1, 1, 1),
             dedup: bool = True, normals: bool = True, edges: bool = False,
             interp: bool = False) -> Contour:
-    """Classify, size the outputs, then run the full forward."""
+    """Classify and count, size the outputs, then generate from the same
+    classification.  Synchronous."""
+    import ctypes
     nx, ny, nz = _check_field(field)
-    ws, cnt = classify(field, iso)
-    T, U = read_counts(cnt)
-    if not dedup:
-        U = 3 * T
-    buf = ForwardBuffers(nx, ny, nz, max(U, 1), max(T, 1), field.device, normals=normals,
-                         edges=edges and dedup, interp=interp)
-    forward_into(field, iso, buf, origin, spacing, dedup, normals)
-    T2, U2 = read_counts(buf.counts, buf.cap_points, buf.cap_tris)
-    assert (T2, U2) == (T, U), (T2, U2, T, U)
-    return Contour(
-        vertices=buf.vertices[:U], connectivity=buf.conn[:T],
-        normals=None if buf.normals is None else buf.normals[:U],
-        edges=None if buf.edges is None else buf.edges[:U],
-        interp_first=None if buf.interp_first is None else buf.interp_first[:U],
-        interp_second=None if buf.interp_second is None else buf.interp_second[:U],
-        interp_weight=None if buf.interp_weight is None else buf.interp_weight[:U],
-        workspace=buf.workspace, counts=buf.counts, grid_points=nx * ny * nz)
+    dev, s = field.device, _stream()
+    ws = new_workspace(nx, ny, nz, dev)
+    counts = torch.empty(2, dtype=torch.int64, device=dev)
+    t, u = ctypes.c_int64(), ctypes.c_int64()
+    _lib.call("dax_hip_mc_count", field.data_ptr(), nx, ny, nz, float(iso), ws.data_ptr(),
+              ws.numel(), ctypes.byref(t), ctypes.byref(u), s)
+    T = int(t.value)
+    U, outs = _sized_outputs(T, int(u.value), dev, dedup, normals, edges and dedup, interp)
+    flags = (MC_DEDUP if dedup else 0) | (MC_NORMALS if normals else 0)
+    _lib.call("dax_hip_mc_generate", field.data_ptr(), nx, ny, nz, _f3(origin), _f3(spacing),
+              float(iso), flags, ws.data_ptr(), ws.numel(), *(_ptr(x) for x in outs), max(U, 1),
+              max(T, 1), counts.data_ptr(), s)
+    _lib.call("dax_hip_synchronize", s)
+    return _sized_contour(T, U, outs, ws, counts, (nx, ny, nz))
 
 
 def slice_into(dims, plane_origin, plane_normal, buf: ForwardBuffers, origin=(0, 0, 0),
@@ -283,28 +305,22 @@ def slice(dims, plane_origin, plane_normal, origin=(0, 0, 0), spacing=(1, 1, 1),
     plane_origin with normal plane_normal, as Dax's SliceCount then
     SliceGenerate (dax/worklet/Slice.h:28-173) produce it: count, size the
     outputs, generate.  No field is read."""
+    import ctypes
     nx, ny, nz = (int(v) for v in dims)
+    s = _stream()
     ws = new_workspace(nx, ny, nz, device)
-    cnt = torch.empty(2, dtype=torch.int64, device=device)
-    _lib.call("dax_hip_mc_slice_classify", nx, ny, nz, _f3(origin), _f3(spacing),
-              _f3(plane_origin), _f3(plane_normal), ws.data_ptr(), ws.numel(), cnt.data_ptr(),
-              _stream())
-    T, U = read_counts(cnt)
-    if not dedup:
-        U = 3 * T
-    buf = ForwardBuffers(nx, ny, nz, max(U, 1), max(T, 1), device, normals=normals,
-                         edges=dedup, interp=interp)
-    slice_into((nx, ny, nz), plane_origin, plane_normal, buf, origin, spacing, dedup, normals)
-    T2, U2 = read_counts(buf.counts, buf.cap_points, buf.cap_tris)
-    assert (T2, U2) == (T, U), (T2, U2, T, U)
-    return Contour(
-        vertices=buf.vertices[:U], connectivity=buf.conn[:T],
-        normals=None if buf.normals is None else buf.normals[:U],
-        edges=None if buf.edges is None else buf.edges[:U],
-        interp_first=None if buf.interp_first is None else buf.interp_first[:U],
-        interp_second=None if buf.interp_second is None else buf.interp_second[:U],
-        interp_weight=None if buf.interp_weight is None else buf.interp_weight[:U],
-        workspace=buf.workspace, counts=buf.counts, grid_points=nx * ny * nz)
+    counts = torch.empty(2, dtype=torch.int64, device=device)
+    plane = (_f3(origin), _f3(spacing), _f3(plane_origin), _f3(plane_normal))
+    t, u = ctypes.c_int64(), ctypes.c_int64()
+    _lib.call("dax_hip_mc_slice_count", nx, ny, nz, *plane, ws.data_ptr(), ws.numel(),
+              ctypes.byref(t), ctypes.byref(u), s)
+    T = int(t.value)
+    U, outs = _sized_outputs(T, int(u.value), device, dedup, normals, dedup, interp)
+    flags = (MC_DEDUP if dedup else 0) | (MC_NORMALS if normals else 0)
+    _lib.call("dax_hip_mc_slice_generate", nx, ny, nz, *plane, flags, ws.data_ptr(), ws.numel(),
+              *(_ptr(x) for x in outs), max(U, 1), max(T, 1), counts.data_ptr(), s)
+    _lib.call("dax_hip_synchronize", s)
+    return _sized_contour(T, U, outs, ws, counts, (nx, ny, nz))
 
 
 def _cells_contour(prefix: str, nv: int, cells: torch.Tensor, field: torch.Tensor,

@@ -283,7 +283,7 @@ class DispatcherGenerateInterpolatedCells<dax::worklet::SliceGenerate, CountHand
     if (!this->PrepareOutputs(outputGrid, (const int64_t*)counts.Data, T, U, conn, cpts, normals,
                               first, second, weight))
       return;
-    internal::HipCheck(dax_hip_mc_slice(d[0], d[1], d[2], origin, spacing, porig, pnorm,
+    internal::HipCheck(dax_hip_mc_slice_generate(d[0], d[1], d[2], origin, spacing, porig, pnorm,
                                         this->Flags(), ws.Data, ws.Bytes, cpts, normals, conn,
                                         nullptr, first, second, weight, U, T,
                                         (int64_t*)counts.Data, nullptr));

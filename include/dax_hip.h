@@ -238,6 +238,21 @@ int dax_hip_mc_slice(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
                      float* d_interp_weight, int64_t cap_points, int64_t cap_tris,
                      int64_t* d_counts, void* stream);
 
+/* The slice in two calls, as dax_hip_mc_count and dax_hip_mc_generate. */
+int dax_hip_mc_slice_count(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
+                           const float* h_spacing3, const float* h_plane_origin3,
+                           const float* h_plane_normal3, void* d_workspace,
+                           size_t workspace_bytes, int64_t* h_tris, int64_t* h_points,
+                           void* stream);
+int dax_hip_mc_slice_generate(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
+                              const float* h_spacing3, const float* h_plane_origin3,
+                              const float* h_plane_normal3, unsigned flags,
+                              const void* d_workspace, size_t workspace_bytes, float* d_vertices,
+                              float* d_normals, int32_t* d_conn, uint32_t* d_edges,
+                              int32_t* d_interp_first, int32_t* d_interp_second,
+                              float* d_interp_weight, int64_t cap_points, int64_t cap_tris,
+                              int64_t* d_counts, void* stream);
+
 /* Marching tetrahedra on an unstructured tetrahedral grid: replaces
  * DispatcherMapCell<MarchingTetrahedraCount> +
  * DispatcherGenerateInterpolatedCells<MarchingTetrahedraGenerate>
@@ -415,6 +430,14 @@ int dax_hip_mc_generate(const float* d_field, int64_t nx, int64_t ny, int64_t nz
 int dax_hip_mc_classify(const float* d_field, int64_t nx, int64_t ny, int64_t nz, float iso,
                         void* d_workspace, size_t workspace_bytes, int64_t* d_counts,
                         void* stream);
+
+/* The same two steps for a caller that sizes its outputs next (synchronous):
+ * *h_tris = T, *h_points = U with duplicate removal; DAX_HIP_EXEC_ERROR if
+ * either leaves the int32 dax::Id range.  Follow with dax_hip_mc_generate on
+ * the same workspace, which also stores the words' bases. */
+int dax_hip_mc_count(const float* d_field, int64_t nx, int64_t ny, int64_t nz, float iso,
+                     void* d_workspace, size_t workspace_bytes, int64_t* h_tris,
+                     int64_t* h_points, void* stream);
 
 /* After dax_hip_mc_classify on the same workspace: the per-cell outputs of
  * the reference's count step.  Any pointer may be NULL.
