@@ -95,6 +95,23 @@ __device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
   return s;
 }
 
+// Exclusive scan of one value per thread over the block (thread order);
+// returns the thread's offset and the block total.
+__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t& total, uint32_t* s_w) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  const uint32_t inc = wave_incl_scan(v);
+  if (lane == 63) s_w[wv] = inc;
+  __syncthreads();
+  uint32_t off = 0, tot = 0;
+  for (int q = 0; q < nwv; ++q) {
+    if (q < wv) off += s_w[q];
+    tot += s_w[q];
+  }
+  __syncthreads();
+  total = tot;
+  return off + inc - v;
+}
+
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

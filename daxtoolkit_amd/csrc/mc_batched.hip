@@ -126,8 +126,9 @@ __global__ __launch_bounds__(256) void k_batch_classify(const VolGeom* __restric
     const TileRef tr = tiles[t];
     const VolGeom g = vols[tr.vol];
     const int64_t w_end = min((int64_t)tr.w0 + kBatchGenTile, g.nwords);
-    classify_flat<kBatchGenTile, LOADS>(g, fields + g.field_off, bits + g.word_off,
-                                        (uint32_t)tr.w0, (uint32_t)w_end, sh);
+    classify_flat<kBatchGenTile, LOADS>(flat_rows(g), fields + g.field_off, bits + g.word_off,
+                                        (uint32_t)tr.w0, (uint32_t)w_end, sh,
+                                        [&](float v) { return v > g.iso; });
     __syncthreads();  // LDS reused by the next tile
   }
 }

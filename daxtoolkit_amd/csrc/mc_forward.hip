@@ -55,8 +55,9 @@ __global__ __launch_bounds__(256) void k_classify_flat(VolGeom g, const float* _
   if (gtid < zero_words) zero_buf[gtid] = 0ull;
   const int64_t w0 = w_lo + (int64_t)blockIdx.x * TW;
   if (w0 >= w_hi) return;  // a block that only clears
-  classify_flat<TW, kFlatLoads>(g, field + g.field_off, bits + g.word_off, (uint32_t)w0,
-                                (uint32_t)min(w0 + TW, w_hi), sh);
+  classify_flat<TW, kFlatLoads>(flat_rows(g), field + g.field_off, bits + g.word_off,
+                                (uint32_t)w0, (uint32_t)min(w0 + TW, w_hi), sh,
+                                [&](float v) { return v > g.iso; });
 }
 
 template <int UNROLL>

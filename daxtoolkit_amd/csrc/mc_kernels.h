@@ -10,6 +10,7 @@
 //                triangle with coalesced writes
 #pragma once
 
+#include "bit_stream.h"
 #include "mc_common.h"
 
 namespace daxhip {
@@ -78,94 +79,9 @@ __device__ __forceinline__ void classify_words(const VolGeom& g, const float* __
   if (lane < UNROLL && w0 + lane < w_end) bits[w0 + lane] = mine;
 }
 
-// OR of the 16 lanes' nibbles (4 bits, lane l of a row at bits 4l .. 4l+3)
-// in lane 15 of every 16-lane row, in steps of 1, 2, 4 and 8 lanes.
-__device__ __forceinline__ uint64_t row_nibbles(uint32_t nib, int lane) {
-  const int sh = 4 * (lane & 15);
-  uint32_t lo = sh < 32 ? nib << sh : 0u;
-  uint32_t hi = sh >= 32 ? nib << (sh - 32) : 0u;
-  lo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, 0x111, 0xf, 0xf, false);
-  hi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, 0x111, 0xf, 0xf, false);
-  lo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, 0x112, 0xf, 0xf, false);
-  hi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, 0x112, 0xf, 0xf, false);
-  lo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, 0x114, 0xf, 0xf, false);
-  hi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, 0x114, 0xf, 0xf, false);
-  lo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, 0x118, 0xf, 0xf, false);
-  hi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, 0x118, 0xf, 0xf, false);
-  return ((uint64_t)hi << 32) | lo;
-}
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// classify of row words [w0, w_end) of any rows (at most TW words, a block
-// of 256 threads).  The words' points are one contiguous run of the field,
-// so it is read as a flat stream of aligned float4s, whatever the rows'
-// extents and the field's alignment; its bits go to LDS in stream order and
-// each thread cuts its row words out of two neighbouring stream words.  A
-// lane per point of a row word instead leaves the lanes past a row's end
-// idle and takes four times the load instructions: 301 x 257 x 190 points
-// took 35 us that way and take 12 (4.9 TB/s), 256 volumes of 32..160 points
-// an axis (0.9 GB) 645 us and 180 (5.1 TB/s).
-template <int TW>
-struct FlatLds {
-  uint64_t w[TW + 4];  // stream words of at most 64 TW + 3 points, read one past the end
-};
-constexpr int kFlatLoads = 8;  // float4 loads in flight per thread
-
-template <int TW, int LOADS>
-__device__ __forceinline__ void classify_flat(const VolGeom& g, const float* __restrict__ f,
-                                              uint64_t* __restrict__ bits, uint32_t w0,
-                                              uint32_t w_end, FlatLds<TW>& sh) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int32_t P = g.nx * g.ny * g.nz;
-  auto first_point = [&](uint32_t w, uint32_t& q) -> int32_t {
-    const uint32_t row = fast_div(w, g.div_wpr);
-    q = w - row * (uint32_t)g.wpr;
-    return (int32_t)(row * (uint32_t)g.nx + 64u * q);
-  };
-  uint32_t qa, qb;
-  const int32_t p0 = first_point(w0, qa);
-  const int32_t pl = first_point(w_end - 1, qb);
-  const int32_t p1 = pl + min(64, g.nx - (int32_t)(64u * qb));
-  // stream position 0 is the 16-byte boundary at or below point p0
-  const int32_t e0 = p0 - (int32_t)((reinterpret_cast<uintptr_t>(f + p0) >> 2) & 3u);
-  const int32_t n4 = (p1 - e0 + 3) >> 2;
-  for (int32_t b = 0; b < n4; b += LOADS * 256) {
-    f32x4 v[LOADS];
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-      const int32_t i = b + u * 256 + tid;
-      const int64_t e = (int64_t)e0 + 4 * (int64_t)i;
-      v[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (i < n4) {
-        if (e >= 0 && e + 4 <= P) {
-          v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(f + e));
-        } else {  // the stream's first or last float4 crosses the field's ends
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (e + c >= 0 && e + c < P) v[u][c] = f[e + c];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-      const int32_t i = b + u * 256 + tid;
-      const uint32_t nib = (uint32_t)(v[u].x > g.iso) | ((uint32_t)(v[u].y > g.iso) << 1) |
-                           ((uint32_t)(v[u].z > g.iso) << 2) | ((uint32_t)(v[u].w > g.iso) << 3);
-      const uint64_t word = row_nibbles(nib, lane);
-      // the last stream word may be partly past n4: its bits are cut off below
-      if ((lane & 15) == 15 && (i & ~15) < n4) sh.w[i >> 4] = word;
-    }
-  }
-  __syncthreads();
-  for (uint32_t w = w0 + (uint32_t)tid; w < w_end; w += 256u) {
-    uint32_t q;
-    const uint32_t s = (uint32_t)(first_point(w, q) - e0);
-    const uint64_t lo = sh.w[s >> 6], hi = sh.w[(s >> 6) + 1];
-    const int r = (int)(s & 63u);
-    const uint64_t m = r ? (lo >> r) | (hi << (64 - r)) : lo;
-    bits[w] = m & low_mask(g.nx - (int)(64u * q));
-  }
+// The volume's points as rows of a flat array (bit_stream.h).
+__device__ __forceinline__ FlatRows flat_rows(const VolGeom& g) {
+  return FlatRows{g.nx, g.wpr, g.nx * g.ny * g.nz, g.div_wpr};
 }
 
 // classify, float4 per lane (rows of a multiple of 64 points): a wave reads
@@ -1015,23 +931,6 @@ __device__ __forceinline__ void lds_flags(const VolGeom& g, const uint64_t* sA, 
                                           uint64_t& fz) {
   const uint64_t A = sA[lw], A1n = sA[lw + 1], B = sA[lw + g.wpr], C = sC[lw];
   edge_flags(p, A, p.q + 1 < g.wpr ? A1n : 0ull, B, C, fx, fy, fz);
-}
-
-// Exclusive scan of one value per thread over the block (thread order);
-// returns the thread's offset and the block total.
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t& total, uint32_t* s_w) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-  const uint32_t inc = wave_incl_scan(v);
-  if (lane == 63) s_w[wv] = inc;
-  __syncthreads();
-  uint32_t off = 0, tot = 0;
-  for (int q = 0; q < nwv; ++q) {
-    if (q < wv) off += s_w[q];
-    tot += s_w[q];
-  }
-  __syncthreads();
-  total = tot;
-  return off + inc - v;
 }
 
 // Where the generate kernel of the single-volume forward takes its word

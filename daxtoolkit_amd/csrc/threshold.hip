@@ -20,6 +20,7 @@
 // a cell count times); Threshold's are 0 or 1.
 #include <algorithm>
 
+#include "bit_stream.h"
 #include "common.h"
 
 namespace daxhip {
@@ -31,8 +32,7 @@ constexpr int kZRun = 16;         // planes one thread marches through
 // How prepare laid out the workspace (its first int): per-cell offsets and
 // per-point ranks (any counts, any grid), or bit words (counts 0/1 on a
 // uniform grid: a bit per cell and per point, 64 to a word along x, with
-// per-word exclusive popcount prefixes).  The kernels of both layouts are
-// launched; each returns at once unless the workspace holds its layout.
+// exclusive popcount prefixes).
 constexpr int kModeCells = 0, kModeBits = 1;
 
 __device__ __forceinline__ bool in_range(float v, float lo, float hi) {
@@ -150,65 +150,6 @@ __global__ __launch_bounds__(kTX* kTY) void k_count_uniform4(const float* __rest
     }
     const unsigned both = a & b, kept = both & (both >> 1);  // cell q: points q and q+1
     store_counts256(s_cnt[threadIdx.y], kept, out, min(256, cx - xw));
-    out += cplane;
-    a = b;
-  }
-}
-
-// Bits 0..15 of x moved to bits 0, 4, 8, ..., 60.
-__device__ __forceinline__ uint64_t spread16(uint64_t x) {
-  x &= 0xFFFFull;
-  x = (x | (x << 24)) & 0x000000FF000000FFull;
-  x = (x | (x << 12)) & 0x000F000F000F000Full;
-  x = (x | (x << 6)) & 0x0303030303030303ull;
-  x = (x | (x << 3)) & 0x1111111111111111ull;
-  return x;
-}
-
-// k_count_uniform4 that also writes the cell words of the bit-word layout: a
-// wave covers cells 256 * blockIdx.x .. +255 of its row, i.e. words
-// 4 * blockIdx.x .. +3; lane l holds cells 4l .. 4l+3, so word q is the four
-// ballots of the lanes' bits, each spread to every fourth bit.
-__global__ __launch_bounds__(kTX* kTY) void k_threshold_words4(
-    const float* __restrict__ f, int nx, int ny, int nz, float lo, float hi, int wcx,
-    int32_t* __restrict__ counts, uint64_t* __restrict__ cbits, int32_t* __restrict__ cpop) {
-  const int cx = nx - 1, cy = ny - 1, cz = nz - 1;
-  const int lane = threadIdx.x;
-  const int x0 = 4 * (blockIdx.x * kTX + lane), j = blockIdx.y * kTY + threadIdx.y;
-  const int k0 = blockIdx.z * kZRun;
-  if (j >= cy || k0 >= cz) return;  // whole waves (one row per wave)
-  __shared__ __align__(16) int32_t s_cnt[kTY][256];
-  const unsigned valid = x0 >= cx ? 0u : (x0 + 4 <= cx ? 0xFu : (1u << (cx - x0)) - 1u);
-  const int64_t sy = nx, sz = (int64_t)nx * ny;
-  const float* p = f + sy * j + sz * k0;
-  unsigned a = range_bits5(p, x0, nx, lo, hi) & range_bits5(p + sy, x0, nx, lo, hi);
-  const int k1 = min(k0 + kZRun, cz);
-  const int xw = 256 * (int)blockIdx.x;  // the wave's first cell
-  int32_t* out = counts + xw + (int64_t)cx * (j + (int64_t)cy * k0);
-  const int64_t cplane = (int64_t)cx * cy;
-  // point plane k + 1 is loaded while plane k is processed (k + 1 <= k1 <= nz - 1)
-  p += sz;
-  Row5 n0 = load_row5(p, x0, nx), n1 = load_row5(p + sy, x0, nx);
-  for (int k = k0; k < k1; ++k) {
-    const unsigned b = row5_bits(n0, lo, hi) & row5_bits(n1, lo, hi);
-    if (k + 1 < k1) {
-      p += sz;
-      n0 = load_row5(p, x0, nx);
-      n1 = load_row5(p + sy, x0, nx);
-    }
-    const unsigned both = a & b, kept = both & (both >> 1) & valid;
-    store_counts256(s_cnt[threadIdx.y], kept, out, min(256, cx - xw));
-    const uint64_t b0 = __ballot(kept & 1u), b1 = __ballot((kept >> 1) & 1u);
-    const uint64_t b2 = __ballot((kept >> 2) & 1u), b3 = __ballot((kept >> 3) & 1u);
-    const int wx = 4 * (int)blockIdx.x + lane;
-    if (lane < 4 && wx < wcx) {
-      const int sh = 16 * lane;
-      const uint64_t w = spread16(b0 >> sh) | spread16(b1 >> sh) << 1 | spread16(b2 >> sh) << 2 |
-                         spread16(b3 >> sh) << 3;
-      const int64_t wi = ((int64_t)j + (int64_t)cy * k) * wcx + wx;
-      cbits[wi] = w;
-      cpop[wi] = __popcll(w);
-    }
     out += cplane;
     a = b;
   }
@@ -432,10 +373,15 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // ---- bit-word layout (uniform grids, counts 0/1) ----
 // Cell words: cell row (j, k) has wcx = ceil(cx / 64) words, word index
 // (j + cy * k) * wcx + w.  Point words: point row (j, k) has wpx =
-// ceil(nx / 64) words, index (j + ny * k) * wpx + w.
+// ceil(nx / 64) words, index (j + ny * k) * wpx + w.  Words come in tiles of
+// kWordTile: a word's exclusive popcount prefix is its prefix within the
+// tile plus the tile's.
+constexpr int kWordTile = 256;
+
 struct BitGeom {
   int nx, ny, nz, cx, cy, cz, wcx, wpx;
   int64_t n_cwords, n_pwords;
+  mc::FastDiv div_wcx, div_cy, div_cx, div_wpx, div_ny, div_nx;
 };
 
 inline BitGeom bit_geom(int nx, int ny, int nz) {
@@ -450,232 +396,321 @@ inline BitGeom bit_geom(int nx, int ny, int nz) {
   b.wpx = (nx + 63) / 64;
   b.n_cwords = (int64_t)b.wcx * b.cy * b.cz;
   b.n_pwords = (int64_t)b.wpx * ny * nz;
+  b.div_wcx = mc::make_fast_div((uint32_t)b.wcx);
+  b.div_cy = mc::make_fast_div((uint32_t)b.cy);
+  b.div_cx = mc::make_fast_div((uint32_t)b.cx);
+  b.div_wpx = mc::make_fast_div((uint32_t)b.wpx);
+  b.div_ny = mc::make_fast_div((uint32_t)ny);
+  b.div_nx = mc::make_fast_div((uint32_t)nx);
   return b;
 }
 
-// The row kernels run a wave per grid row (4 waves per block), looping over
-// the row's words; lane l stands for bit l of a word.
-constexpr int kRowWaves = 4;
-
-__device__ __forceinline__ int wave_row() {
-  return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kRowWaves + (threadIdx.x >> 6)));
+__host__ __device__ __forceinline__ FlatRows cell_rows(const BitGeom& g) {
+  return FlatRows{g.cx, g.wcx, g.cx * g.cy * g.cz, g.div_wcx};
+}
+__host__ __device__ __forceinline__ FlatRows point_rows(const BitGeom& g) {
+  return FlatRows{g.nx, g.wpx, g.nx * g.ny * g.nz, g.div_wpx};
 }
 
-// Cell row r = j + cy * k: per word the ballot of count != 0 over its 64
-// cells and its popcount; *general = 1 if a count is outside {0, 1}.
-__global__ __launch_bounds__(64 * kRowWaves) void k_cell_bits(BitGeom g,
-                                                              const int32_t* __restrict__ counts,
-                                                              uint64_t* __restrict__ cbits,
-                                                              int32_t* __restrict__ cpop,
-                                                              int32_t* __restrict__ general) {
-  const int r = wave_row(), lane = threadIdx.x & 63;
-  if (r >= g.cy * g.cz) return;  // whole waves
-  const int32_t* row = counts + (int64_t)r * g.cx;
+// Words, exclusive popcount prefixes within the tiles and the tiles' (sums,
+// then exclusive prefixes) of the cells or the points.
+struct WordSet {
+  uint64_t* bits;
+  int32_t* pre;
+  int32_t* tile;
+};
+
+// Bits of the points whose value is in range: the field read once as a flat
+// stream.  Bound by HBM (512^3: 88 us, 6.1 TB/s).
+__global__ __launch_bounds__(256) void k_range_bits(FlatRows rows, int64_t nwords,
+                                                    const float* __restrict__ f, float lo,
+                                                    float hi, uint64_t* __restrict__ pbits) {
+  __shared__ FlatLds<128> sh;
+  const int64_t w0 = (int64_t)blockIdx.x * 128;
+  classify_flat<128, kFlatLoads>(rows, f, pbits, (uint32_t)w0, (uint32_t)min(w0 + 128, nwords), sh,
+                                 [&](float v) { return in_range(v, lo, hi); });
+}
+
+// Bits of the non-zero counts; *general = 1 if a count is outside {0, 1}.
+__global__ __launch_bounds__(256) void k_count_bits(FlatRows rows, int64_t nwords,
+                                                    const int32_t* __restrict__ counts,
+                                                    uint64_t* __restrict__ cbits,
+                                                    int32_t* __restrict__ general) {
+  __shared__ FlatLds<128> sh;
+  const int64_t w0 = (int64_t)blockIdx.x * 128;
   bool bad = false;
-  for (int w0 = 0; w0 < g.wcx; w0 += 4) {  // four words' loads in flight
-    int32_t cnt[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int x = (w0 + q) * 64 + lane;
-      cnt[q] = x < g.cx ? row[x] : 0;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (w0 + q >= g.wcx) break;
-      const uint64_t bits = __ballot(cnt[q] != 0);
-      bad = bad || cnt[q] < 0 || cnt[q] > 1;
-      if (lane == 0) {
-        cbits[(int64_t)r * g.wcx + w0 + q] = bits;
-        cpop[(int64_t)r * g.wcx + w0 + q] = __popcll(bits);
-      }
-    }
-  }
+  classify_flat<128, kFlatLoads>(rows, reinterpret_cast<const float*>(counts), cbits, (uint32_t)w0,
+                                 (uint32_t)min(w0 + 128, nwords), sh, [&](float v) {
+                                   const int32_t c = __builtin_bit_cast(int32_t, v);
+                                   bad = bad || c < 0 || c > 1;
+                                   return c != 0;
+                                 });
   if (bad) *general = 1;
 }
 
-// Point row (j, k): point (i, j, k) is used when a cell of cell rows j-1, j
-// in cell planes k-1, k at x = i-1 or i is kept, i.e. the word is the OR over
-// those four cell rows of c | c << 1 | (the previous word's bit 63).  Writes
-// the words, their popcounts and, if `mask`, the int32 mask of the row.
-__global__ __launch_bounds__(64 * kRowWaves) void k_mask_bits(BitGeom g,
-                                                              const uint64_t* __restrict__ cbits,
-                                                              uint64_t* __restrict__ mbits,
-                                                              int32_t* __restrict__ mpop,
-                                                              int32_t* __restrict__ mask) {
-  const int pr = wave_row(), lane = threadIdx.x & 63;
-  if (pr >= g.ny * g.nz) return;  // whole waves
-  const int j = pr % g.ny, k = pr / g.ny;
-  // the four cell rows (j-1 or j, k-1 or k); a missing one reads row 0 and is
-  // masked out
-  const uint64_t* rows[4];
-  uint64_t keep[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int jc = j - 1 + (q & 1), kc = k - 1 + (q >> 1);
-    const bool ok = kc >= 0 && kc < g.cz && jc >= 0 && jc < g.cy;
-    rows[q] = cbits + (ok ? ((int64_t)jc + (int64_t)g.cy * kc) * g.wcx : 0);
-    keep[q] = ok ? ~0ull : 0ull;
+// The tile's words (word w of thread threadIdx.x, 0 past the end): LDS copy,
+// popcount prefixes and the tile's sum.  s_w holds kWordTile + 1 words.
+__device__ __forceinline__ void store_tile(const WordSet& ws, int64_t w, int64_t nwords,
+                                           uint64_t word, bool store_bits, uint64_t* s_w,
+                                           uint32_t* s_scan) {
+  s_w[threadIdx.x] = word;
+  uint32_t total;
+  const uint32_t pre = block_excl_scan((uint32_t)__popcll(word), total, s_scan);
+  if (w < nwords) {
+    if (store_bits) ws.bits[w] = word;
+    ws.pre[w] = (int32_t)pre;
   }
-  uint64_t carry[4] = {0, 0, 0, 0};  // bit 63 of each cell row's previous word
-  // with 16-byte aligned rows the mask goes out 4 words (256 points) at a
-  // time, lane l writing points 4l .. 4l+3 as one 16-byte store
-  const bool vec = mask && (g.nx & 3) == 0 && ((uintptr_t)mask & 15u) == 0;
-  int32_t* mrow = mask ? mask + (int64_t)pr * g.nx : nullptr;
-  for (int w0 = 0; w0 < g.wpx; w0 += 4) {
-    uint64_t m4[4];
+  if (threadIdx.x == 0) ws.tile[blockIdx.x] = (int32_t)total;
+}
+
+// Cell words from the point words: a cell is kept when its eight points are
+// in range, so a word is the AND over its four point rows of p & p >> 1.
+// Also the counts as int32: with a column of threads marching over z and
+// keeping flags in registers, reads and writes mixed, this and the field
+// took 277 us at 512^3; the field's stream and this take 88 + 110.
+__global__ __launch_bounds__(kWordTile) void k_cell_words(BitGeom g,
+                                                          const uint64_t* __restrict__ pbits,
+                                                          WordSet ws,
+                                                          int32_t* __restrict__ counts) {
+  __shared__ uint64_t s_w[kWordTile + 1];
+  __shared__ uint32_t s_scan[kWordTile / 64];
+  const uint32_t w0 = blockIdx.x * kWordTile, w = w0 + threadIdx.x;
+  uint64_t word = 0ull;
+  if (w < (uint32_t)g.n_cwords) {
+    const uint32_t row = mc::fast_div(w, g.div_wcx);
+    const int wx = (int)(w - row * (uint32_t)g.wcx);
+    const uint32_t k = mc::fast_div(row, g.div_cy), j = row - k * (uint32_t)g.cy;
+    const bool next = wx + 1 < g.wpx;
+    word = mc::low_mask(g.cx - 64 * wx);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int wx = w0 + t;
-      uint64_t m = 0;
+    for (uint32_t q = 0; q < 4u; ++q) {
+      const uint64_t* p = pbits + ((int64_t)(j + (q & 1u)) + (int64_t)g.ny * (k + (q >> 1))) * g.wpx + wx;
+      const uint64_t a = p[0], a1 = next ? p[1] : 0ull;
+      word &= a & mc::shr1(a, a1);
+    }
+  }
+  store_tile(ws, w, g.n_cwords, word, true, s_w, s_scan);
+  store_words_i32(cell_rows(g), g.div_cx, s_w, w0,
+                  (uint32_t)min((int64_t)w0 + kWordTile, g.n_cwords), counts);
+}
+
+// Popcount prefixes of words already there.
+__global__ __launch_bounds__(kWordTile) void k_word_prefix(WordSet ws, int64_t nwords) {
+  __shared__ uint64_t s_w[kWordTile + 1];
+  __shared__ uint32_t s_scan[kWordTile / 64];
+  const int64_t w = (int64_t)blockIdx.x * kWordTile + threadIdx.x;
+  store_tile(ws, w, nwords, w < nwords ? ws.bits[w] : 0ull, false, s_w, s_scan);
+}
+
+// Point words: point (i, j, k) is used when a cell of cell rows j-1, j in
+// cell planes k-1, k at x = i-1 or i is kept, i.e. the word is the OR over
+// those four cell rows of c | c << 1 | (the previous word's bit 63).  With
+// `mask`, also the int32 mask, streamed out: a wave per point row took 311 us
+// at 512^3 (537 MB of mask), this takes 105.
+__global__ __launch_bounds__(kWordTile) void k_mask_words(BitGeom g,
+                                                          const uint64_t* __restrict__ cbits,
+                                                          WordSet ws, int32_t* __restrict__ mask) {
+  __shared__ uint64_t s_w[kWordTile + 1];
+  __shared__ uint32_t s_scan[kWordTile / 64];
+  const uint32_t w0 = blockIdx.x * kWordTile, w = w0 + threadIdx.x;
+  uint64_t m = 0ull;
+  if (w < (uint32_t)g.n_pwords) {
+    const uint32_t row = mc::fast_div(w, g.div_wpx);
+    const int wx = (int)(w - row * (uint32_t)g.wpx);
+    const int k = (int)mc::fast_div(row, g.div_ny), j = (int)row - k * g.ny;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint64_t c = (wx < g.wcx ? rows[q][wx] : 0) & keep[q];  // wx <= wcx
-        m |= c | (c << 1) | carry[q];
-        carry[q] = c >> 63;
-      }
-      m4[t] = wx < g.wpx ? m : 0;
-      if (lane == 0 && wx < g.wpx) {
-        mbits[(int64_t)pr * g.wpx + wx] = m;
-        mpop[(int64_t)pr * g.wpx + wx] = __popcll(m);
+    for (int q = 0; q < 4; ++q) {
+      const int jc = j - 1 + (q & 1), kc = k - 1 + (q >> 1);
+      if (kc < 0 || kc >= g.cz || jc < 0 || jc >= g.cy) continue;
+      const uint64_t* r = cbits + ((int64_t)jc + (int64_t)g.cy * kc) * g.wcx;
+      const uint64_t c = wx < g.wcx ? r[wx] : 0ull;     // wx <= wcx
+      const uint64_t prev = wx > 0 ? r[wx - 1] : 0ull;  // wx - 1 < wcx
+      m |= c | (c << 1) | (prev >> 63);
+    }
+  }
+  store_tile(ws, w, g.n_pwords, m, true, s_w, s_scan);
+  if (mask)
+    store_words_i32(point_rows(g), g.div_nx, s_w, w0,
+                    (uint32_t)min((int64_t)w0 + kWordTile, g.n_pwords), mask);
+}
+
+__device__ __forceinline__ uint32_t read_lane(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ uint64_t read_lane64(uint64_t v, int l) {
+  return (uint64_t)read_lane((uint32_t)v, l) | ((uint64_t)read_lane((uint32_t)(v >> 32), l) << 32);
+}
+// Set bits of the wave-uniform m below the lane's.
+__device__ __forceinline__ uint32_t bits_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// The kept cells' corner ids: a wave takes 64 cell words, each lane loading
+// one word and what its cells need (the four point rows' words and
+// prefixes), then goes through the words that hold a cell with a lane per
+// cell.  All corners of a kept cell are used points, so along x a corner's
+// rank is its left neighbour's plus one.  A thread per output cell searching
+// the words' prefixes took 139 us at 512^3 (4.4 M cells), this takes 44.
+__global__ __launch_bounds__(256) void k_emit_words(BitGeom g, WordSet cells, WordSet pts,
+                                                    bool dedup, int64_t n_out, bool vec,
+                                                    int32_t* __restrict__ conn) {
+  const int lane = threadIdx.x & 63;
+  const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint64_t c = w < g.n_cwords ? cells.bits[w] : 0ull;
+  uint64_t todo = __ballot(c != 0ull);
+  if (!todo) return;
+  uint32_t first = 0u, pid = 0u;
+  uint64_t mw[4] = {0ull, 0ull, 0ull, 0ull};
+  uint32_t mo[4] = {0u, 0u, 0u, 0u};
+  if (c) {
+    const uint32_t row = mc::fast_div((uint32_t)w, g.div_wcx), wx = (uint32_t)w - row * (uint32_t)g.wcx;
+    const uint32_t k = mc::fast_div(row, g.div_cy), j = row - k * (uint32_t)g.cy;
+    first = (uint32_t)(cells.tile[w / kWordTile] + cells.pre[w]);
+    pid = 64u * wx + (uint32_t)g.nx * (j + (uint32_t)g.ny * k);
+    if (dedup) {
+#pragma unroll
+      for (uint32_t q = 0; q < 4u; ++q) {
+        const uint32_t pw = (j + (q & 1u) + (uint32_t)g.ny * (k + (q >> 1))) * (uint32_t)g.wpx + wx;
+        mw[q] = pts.bits[pw];
+        mo[q] = (uint32_t)(pts.tile[pw / kWordTile] + pts.pre[pw]);
       }
     }
-    if (!mask) continue;
-    if (vec) {
-      const int x = w0 * 64 + 4 * lane;  // points x .. x+3, all in word w0 + lane / 16
-      if (x < g.nx) {
-        const uint64_t m = m4[lane >> 4];
-        const int sh = x & 63;
-        int4 v;
-        v.x = (int)((m >> sh) & 1u);
-        v.y = (int)((m >> (sh + 1)) & 1u);
-        v.z = (int)((m >> (sh + 2)) & 1u);
-        v.w = (int)((m >> (sh + 3)) & 1u);
-        *(int4*)(mrow + x) = v;
+  }
+  while (todo) {  // wave-uniform
+    const int l = __builtin_ctzll(todo);
+    todo &= todo - 1ull;
+    const uint64_t cw = read_lane64(c, l);
+    const int64_t t = (int64_t)read_lane(first, l) + bits_below(cw);
+    uint32_t r[4];
+    if (dedup) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) r[q] = read_lane(mo[q], l) + bits_below(read_lane64(mw[q], l));
+    } else {
+      const uint32_t p = read_lane(pid, l) + (uint32_t)lane;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        r[q] = p + (uint32_t)g.nx * ((uint32_t)(q & 1) + (uint32_t)g.ny * (uint32_t)(q >> 1));
+    }
+    if (((cw >> lane) & 1ull) && t < n_out) {
+      const int32_t id[8] = {(int32_t)r[0], (int32_t)r[0] + 1, (int32_t)r[1] + 1, (int32_t)r[1],
+                             (int32_t)r[2], (int32_t)r[2] + 1, (int32_t)r[3] + 1, (int32_t)r[3]};
+      int32_t* dst = conn + 8 * t;
+      if (vec) {
+        reinterpret_cast<i32x4*>(dst)[0] = i32x4{id[0], id[1], id[2], id[3]};
+        reinterpret_cast<i32x4*>(dst)[1] = i32x4{id[4], id[5], id[6], id[7]};
+      } else {
+#pragma unroll
+        for (int v = 0; v < 8; ++v) dst[v] = id[v];
+      }
+    }
+  }
+}
+
+// The used points' coordinates (origin + spacing * ijk) or values (`words`
+// 4-byte words of `in`) at their ranks: a wave takes kCompactWords point
+// words and goes through those that hold a used point four at a time, a lane
+// per point, so that four words' loads are in flight.  A thread per used
+// point searching the prefixes took 80 us at 512^3 (4.5 M points), this takes
+// 30.
+constexpr int kCompactWords = 32;
+__global__ __launch_bounds__(256) void k_compact_words(BitGeom g, WordSet pts, int64_t n_used,
+                                                       float ox, float oy, float oz, float hx,
+                                                       float hy, float hz,
+                                                       float* __restrict__ coords,
+                                                       const uint32_t* __restrict__ in, int words,
+                                                       uint32_t* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int64_t w = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kCompactWords + lane;
+  const uint64_t m = lane < kCompactWords && w < g.n_pwords ? pts.bits[w] : 0ull;
+  uint64_t todo = __ballot(m != 0ull);
+  if (!todo) return;
+  uint32_t first = 0u, x0 = 0u, j = 0u, k = 0u;
+  if (m) {
+    const uint32_t row = mc::fast_div((uint32_t)w, g.div_wpx);
+    x0 = 64u * ((uint32_t)w - row * (uint32_t)g.wpx);
+    k = mc::fast_div(row, g.div_ny);
+    j = row - k * (uint32_t)g.ny;
+    first = (uint32_t)(pts.tile[w / kWordTile] + pts.pre[w]);
+  }
+  while (todo) {  // wave-uniform
+    int l[4];
+    uint64_t mw[4];
+    int64_t u[4];
+    bool ok[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      l[b] = todo ? __builtin_ctzll(todo) : 0;
+      mw[b] = todo ? read_lane64(m, l[b]) : 0ull;
+      todo &= todo - (todo ? 1ull : 0ull);
+      u[b] = (int64_t)read_lane(first, l[b]) + bits_below(mw[b]);
+      ok[b] = ((mw[b] >> lane) & 1ull) && u[b] < n_used;
+    }
+    if (coords) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        if (!ok[b]) continue;
+        const float v[3] = {ox + hx * (float)(int)(read_lane(x0, l[b]) + (uint32_t)lane),
+                            oy + hy * (float)(int)read_lane(j, l[b]),
+                            oz + hz * (float)(int)read_lane(k, l[b])};
+        __builtin_memcpy(coords + 3 * u[b], v, 12);
       }
     } else {
+      int64_t p[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int x = (w0 + t) * 64 + lane;
-        if (x < g.nx) mrow[x] = (int32_t)((m4[t] >> lane) & 1u);
+      for (int b = 0; b < 4; ++b)
+        p[b] = (int64_t)(read_lane(x0, l[b]) + (uint32_t)lane) +
+               (int64_t)g.nx * (read_lane(j, l[b]) + (int64_t)g.ny * read_lane(k, l[b]));
+      for (int q = 0; q < words; ++q) {
+        uint32_t v[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) v[b] = ok[b] ? in[p[b] * words + q] : 0u;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          if (ok[b]) out[u[b] * words + q] = v[b];
       }
     }
   }
 }
 
-// The point words without the int32 mask: a lane per word (32-bit index
-// arithmetic; every point word has its own independent loads).
-__global__ __launch_bounds__(256) void k_mask_words(BitGeom g, const uint64_t* __restrict__ cbits,
-                                                    uint64_t* __restrict__ mbits,
-                                                    int32_t* __restrict__ mpop) {
-  const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= (uint32_t)g.n_pwords) return;
-  const uint32_t prow = w / (uint32_t)g.wpx;
-  const int wx = (int)(w - prow * (uint32_t)g.wpx);
-  const int j = (int)(prow % (uint32_t)g.ny), k = (int)(prow / (uint32_t)g.ny);
-  uint64_t m = 0;
+// Exclusive scans of the tiles' sums, block 0 the cells', block 1 the
+// points'; the totals go to the header and, with `host`, to pinned memory
+// with the flag of counts outside {0, 1}.
+constexpr int kSumThreads = 1024;
+__global__ __launch_bounds__(kSumThreads) void k_scan_word_tiles(int32_t* __restrict__ ctile,
+                                                                 int64_t nc,
+                                                                 int32_t* __restrict__ ptile,
+                                                                 int64_t np,
+                                                                 int32_t* __restrict__ hdr,
+                                                                 int64_t* __restrict__ host) {
+  __shared__ uint32_t s_scan[kSumThreads / 64];
+  int32_t* t = blockIdx.x == 0 ? ctile : ptile;
+  const int64_t n = blockIdx.x == 0 ? nc : np;
+  constexpr int V = 8;
+  uint32_t carry = 0u;
+  for (int64_t c0 = 0; c0 < n; c0 += kSumThreads * V) {
+    const int64_t b = c0 + (int64_t)threadIdx.x * V;
+    uint32_t v[V], sum = 0u;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int jc = j - 1 + (q & 1), kc = k - 1 + (q >> 1);
-    if (kc < 0 || kc >= g.cz || jc < 0 || jc >= g.cy) continue;
-    const uint64_t* r = cbits + ((int64_t)jc + (int64_t)g.cy * kc) * g.wcx;
-    const uint64_t c = wx < g.wcx ? r[wx] : 0;     // wx <= wcx
-    const uint64_t prev = wx > 0 ? r[wx - 1] : 0;  // wx - 1 < wcx
-    m |= c | (c << 1) | (prev >> 63);
-  }
-  mbits[w] = m;
-  mpop[w] = __popcll(m);
-}
-
-// Rank of point (i, j, k) among the used points.
-__device__ __forceinline__ int32_t bit_rank(const BitGeom& g, const uint64_t* __restrict__ mbits,
-                                            const int32_t* __restrict__ moff, int i, int j, int k) {
-  const int64_t w = ((int64_t)j + (int64_t)g.ny * k) * g.wpx + (i >> 6);
-  const uint64_t below = (1ull << (i & 63)) - 1ull;
-  return moff[w] + __popcll(mbits[w] & below);
-}
-
-// Last word w with off[w] <= v (off: exclusive prefix of the words'
-// popcounts, off[0] = 0 <= v): the word holding the v-th set bit.
-__device__ __forceinline__ int64_t word_of(const int32_t* __restrict__ off, int64_t n, int64_t v) {
-  int64_t lo = 0, hi = n;
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if ((int64_t)off[mid] <= v)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
-// Position of the k-th set bit of m (k < popcount(m)).
-__device__ __forceinline__ int nth_bit(uint64_t m, int k) {
-  int lo = 0, hi = 63;  // largest i with popc(m & ((1 << i) - 1)) <= k
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (__popcll(m & ((1ull << mid) - 1ull)) <= k)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
-// A thread per output cell t: its cell is the t-th kept cell (word by binary
-// search over the cell words' prefixes, then the bit); it writes the 8
-// corner ids (ranks with dedup).
-__global__ __launch_bounds__(256) void k_emit_rank(BitGeom g, const int32_t* __restrict__ mode,
-                                                   const uint64_t* __restrict__ cbits,
-                                                   const int32_t* __restrict__ coff,
-                                                   const uint64_t* __restrict__ mbits,
-                                                   const int32_t* __restrict__ moff, bool dedup,
-                                                   int64_t n_out, int32_t* __restrict__ conn) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n_out || *mode != kModeBits) return;
-  const int64_t w = word_of(coff, g.n_cwords, t);
-  const uint64_t bits = cbits[w];
-  const int r = (int)(t - coff[w]);
-  if (r >= __popcll(bits)) return;  // prefixes not of these words
-  const int b = nth_bit(bits, r);
-  const int64_t row = w / g.wcx;
-  const int wx = (int)(w - row * g.wcx);
-  const int j = (int)(row % g.cy), k = (int)(row / g.cy), i = wx * 64 + b;
-  static constexpr int corner[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0},
-                                       {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
-  int32_t* dst = conn + t * 8;
+    for (int q = 0; q < V; ++q) {
+      v[q] = b + q < n ? (uint32_t)t[b + q] : 0u;
+      sum += v[q];
+    }
+    uint32_t total, run = carry + block_excl_scan(sum, total, s_scan);
+    carry += total;
 #pragma unroll
-  for (int v = 0; v < 8; ++v) {
-    const int pi = i + corner[v][0], pj = j + corner[v][1], pk = k + corner[v][2];
-    dst[v] = dedup ? bit_rank(g, mbits, moff, pi, pj, pk)
-                   : (int32_t)(pi + (int64_t)g.nx * (pj + (int64_t)g.ny * pk));
+    for (int q = 0; q < V; ++q) {
+      if (b + q < n) t[b + q] = (int32_t)run;
+      run += v[q];
+    }
   }
-}
-
-// A thread per used point u: its point is the u-th used one; writes its
-// coordinates (origin + spacing * ijk) or values (`words` 4-byte words).
-__global__ __launch_bounds__(256) void k_compact_rank(
-    BitGeom g, const int32_t* __restrict__ mode, const uint64_t* __restrict__ mbits,
-    const int32_t* __restrict__ moff, int64_t n_used, float ox, float oy, float oz, float hx,
-    float hy, float hz, float* __restrict__ coords, const uint32_t* __restrict__ in, int words,
-    uint32_t* __restrict__ out) {
-  const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n_used || *mode != kModeBits) return;
-  const int64_t w = word_of(moff, g.n_pwords, u);
-  const uint64_t m = mbits[w];
-  const int r = (int)(u - moff[w]);
-  if (r >= __popcll(m)) return;  // prefixes not of these words
-  const int b = nth_bit(m, r);
-  const int64_t prow = w / g.wpx;
-  const int wx = (int)(w - prow * g.wpx);
-  const int i = wx * 64 + b;
-  if (coords) {
-    const int j = (int)(prow % g.ny), k = (int)(prow / g.ny);
-    coords[3 * u] = ox + hx * (float)i;
-    coords[3 * u + 1] = oy + hy * (float)j;
-    coords[3 * u + 2] = oz + hz * (float)k;
-  } else {
-    const int64_t p = prow * g.nx + i;
-    for (int q = 0; q < words; ++q) out[u * words + q] = in[p * words + q];
+  if (threadIdx.x == 0) {
+    hdr[6 + blockIdx.x] = (int32_t)carry;
+    if (host) {
+      __hip_atomic_store(host + blockIdx.x, (int64_t)carry, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+      if (blockIdx.x == 0)
+        __hip_atomic_store(host + 2, (int64_t)hdr[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
@@ -708,12 +743,6 @@ __global__ __launch_bounds__(256) void k_count_total_i64(const int32_t* __restri
   }
 }
 
-__global__ void k_set_sizes(int32_t* __restrict__ hdr, int32_t cells, int32_t points) {
-  if (threadIdx.x == 0) {
-    hdr[6] = cells;
-    hdr[7] = points;
-  }
-}
 __global__ void k_set_header(int32_t* __restrict__ hdr, int mode, int nx, int ny, int nz,
                              int ranked) {
   if (threadIdx.x == 0) {
@@ -743,21 +772,45 @@ inline TopoWs topo_ws(int64_t n_cells, int64_t n_points) {
   return w;
 }
 
-// The bit-word layout inside regions A and B, if it fits there.
+// The bit-word layout inside regions A (cells) and B (points: the in-range
+// points' words besides), if it fits there.
 struct BitWs {
-  size_t cbits, coff, mbits, moff;
+  size_t cbits, cpre, ctile, mbits, mpre, mtile, pbits;
+  int64_t nct, nmt;  // word tiles
   bool fits;
 };
 
 inline BitWs bit_ws(const TopoWs& w, const BitGeom& g) {
   BitWs b;
+  b.nct = ceil_div(g.n_cwords, (int64_t)kWordTile);
+  b.nmt = ceil_div(g.n_pwords, (int64_t)kWordTile);
   b.cbits = w.off_a;
-  b.coff = b.cbits + align_up((size_t)g.n_cwords * 8, 256);
+  b.cpre = b.cbits + (size_t)g.n_cwords * 8;
+  b.ctile = b.cpre + (size_t)g.n_cwords * 4;
   b.mbits = w.off_b;
-  b.moff = b.mbits + align_up((size_t)g.n_pwords * 8, 256);
-  b.fits = b.coff + (size_t)g.n_cwords * 4 <= w.off_b && b.moff + (size_t)g.n_pwords * 4 <= w.bytes;
+  b.pbits = b.mbits + (size_t)g.n_pwords * 8;
+  b.mpre = b.pbits + (size_t)g.n_pwords * 8;
+  b.mtile = b.mpre + (size_t)g.n_pwords * 4;
+  b.fits = b.ctile + (size_t)b.nct * 4 <= w.off_b && b.mtile + (size_t)b.nmt * 4 <= w.bytes;
   return b;
 }
+
+inline WordSet cell_set(const void* ws, const BitWs& b) {
+  char* p = (char*)const_cast<void*>(ws);
+  return WordSet{(uint64_t*)(p + b.cbits), (int32_t*)(p + b.cpre), (int32_t*)(p + b.ctile)};
+}
+inline WordSet point_set(const void* ws, const BitWs& b) {
+  char* p = (char*)const_cast<void*>(ws);
+  return WordSet{(uint64_t*)(p + b.mbits), (int32_t*)(p + b.mpre), (int32_t*)(p + b.mtile)};
+}
+
+// What a prepare found, as the workspace's header holds it: the layout,
+// whether the points were ranked, and the sizes.  The fill calls take it from
+// the caller; the generate calls read the header back.
+struct Plan {
+  int64_t mode, ranked, cells, points, nx, ny, nz, reserved;
+};
+static_assert(sizeof(Plan) == 64, "eight int64 of the C-ABI's plan");
 
 struct Geometry {  // a uniform grid (cells == nullptr) or an unstructured one
   const int32_t* cells;
@@ -771,80 +824,115 @@ inline bool uniform_ok(int64_t nx, int64_t ny, int64_t nz) {
          nz <= 65535 * (int64_t)kZRun && nx * ny * nz <= 0x7fffffffLL;
 }
 
-// words_ready: the cell words and popcounts of the bit-word layout are
-// already in the workspace (k_threshold_words4) and the counts are 0/1.
-int prepare(const Geometry& g, const int32_t* d_counts, unsigned flags, void* d_ws,
-            size_t ws_bytes, int32_t* d_mask, int64_t* h_cells, int64_t* h_points,
-            hipStream_t s, bool words_ready = false) {
+// ThresholdCount of a uniform grid (checked arguments).
+int count_uniform(const float* d_field, int64_t nx, int64_t ny, int64_t nz, float min_value,
+                  float max_value, int32_t* d_counts, hipStream_t s) {
+  const int cx = (int)nx - 1, cy = (int)ny - 1, cz = (int)nz - 1;
+  if ((nx & 3) == 0 && ((uintptr_t)d_field & 15u) == 0) {
+    k_count_uniform4<<<dim3((unsigned)ceil_div(nx, 4 * kTX), (unsigned)ceil_div(cy, kTY),
+                            (unsigned)ceil_div(cz, kZRun)),
+                       dim3(kTX, kTY), 0, s>>>(
+        d_field, (int)nx, (int)ny, (int)nz, min_value, max_value, d_counts);
+    DAXHIP_LAUNCH_CHECK("k_count_uniform4");
+    return DAX_HIP_OK;
+  }
+  k_count_uniform<<<dim3((unsigned)ceil_div(cx, kTX), (unsigned)ceil_div(cy, kTY),
+                         (unsigned)ceil_div(cz, kZRun)),
+                    dim3(kTX, kTY), 0, s>>>(d_field, (int)nx, (int)ny, (int)nz,
+                                                              min_value, max_value, d_counts);
+  DAXHIP_LAUNCH_CHECK("k_count_uniform");
+  return DAX_HIP_OK;
+}
+
+// Cell words of a uniform grid from its in-range points or from its counts,
+// the point words and the totals, read back together.  *general: a count
+// outside {0, 1} was found, and nothing else holds.
+int prepare_bits(const BitGeom& bg, const BitWs& bw, char* ws, const float* d_field, float lo,
+                 float hi, int32_t* d_counts, unsigned flags, int32_t* d_mask, int64_t* cells,
+                 int64_t* points, bool* general, hipStream_t s) {
   const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
-  const bool mask_optional = (flags & DAX_HIP_TOPOLOGY_MASK_OPTIONAL) != 0;
+  int32_t* hdr = (int32_t*)ws;
+  const WordSet cs = cell_set(ws, bw), ps = point_set(ws, bw);
+  const dim3 b(kWordTile), gc((unsigned)bw.nct);
+  k_set_header<<<1, 64, 0, s>>>(hdr, kModeBits, bg.nx, bg.ny, bg.nz, dedup ? 1 : 0);
+  DAXHIP_LAUNCH_CHECK("k_set_header");
+  if (d_field) {
+    uint64_t* pbits = (uint64_t*)(ws + bw.pbits);
+    k_range_bits<<<dim3((unsigned)ceil_div(bg.n_pwords, 128)), dim3(256), 0, s>>>(
+        point_rows(bg), bg.n_pwords, d_field, lo, hi, pbits);
+    DAXHIP_LAUNCH_CHECK("k_range_bits");
+    k_cell_words<<<gc, b, 0, s>>>(bg, pbits, cs, d_counts);
+    DAXHIP_LAUNCH_CHECK("k_cell_words");
+  } else {
+    k_count_bits<<<dim3((unsigned)ceil_div(bg.n_cwords, 128)), dim3(256), 0, s>>>(
+        cell_rows(bg), bg.n_cwords, d_counts, cs.bits, hdr + 1);
+    DAXHIP_LAUNCH_CHECK("k_count_bits");
+    k_word_prefix<<<gc, b, 0, s>>>(cs, bg.n_cwords);
+    DAXHIP_LAUNCH_CHECK("k_word_prefix");
+  }
+  if (dedup) {
+    k_mask_words<<<dim3((unsigned)bw.nmt), b, 0, s>>>(
+        bg, cs.bits, ps, (flags & DAX_HIP_TOPOLOGY_MASK_OPTIONAL) ? nullptr : d_mask);
+    DAXHIP_LAUNCH_CHECK("k_mask_words");
+  }
+  HostSlot slot;
+  k_scan_word_tiles<<<dedup ? 2 : 1, kSumThreads, 0, s>>>(cs.tile, bw.nct, ps.tile, bw.nmt, hdr,
+                                                          slot.p);
+  DAXHIP_LAUNCH_CHECK("k_scan_word_tiles");
+  int32_t h[kHeaderInts] = {};
+  if (!slot.p)
+    DAXHIP_CHECK(hipMemcpyAsync(h, hdr, sizeof(h), hipMemcpyDeviceToHost, s));
+  DAXHIP_CHECK(hipStreamSynchronize(s));
+  const volatile int64_t* v = slot.p;
+  *cells = v ? v[0] : h[6];
+  *points = !dedup ? 0 : (v ? v[1] : h[7]);
+  *general = (v ? v[2] : h[1]) != 0;
+  return DAX_HIP_OK;
+}
+
+// Prepare from the caller's counts, or (d_field) from a field's range with
+// the counts written.  The bit-word layout where it holds, else per-cell
+// offsets and per-point ranks.
+int prepare(const Geometry& g, const float* d_field, float lo, float hi, int32_t* d_counts,
+            unsigned flags, void* d_ws, size_t ws_bytes, int32_t* d_mask, Plan* plan,
+            hipStream_t s) {
+  const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
   const TopoWs w = topo_ws(g.n_cells, g.n_points);
-  if (!d_counts || !h_cells || !h_points || !d_ws || ws_bytes < w.bytes || (dedup && !d_mask) ||
+  if (!d_counts || !plan || !d_ws || ws_bytes < w.bytes || (dedup && !d_mask) ||
       (flags & ~(unsigned)(DAX_HIP_MC_DEDUP | DAX_HIP_TOPOLOGY_MASK_OPTIONAL))) {
     set_error("topology prepare: bad arguments (workspace of %zu bytes needed)", w.bytes);
     return DAX_HIP_BAD_VALUE;
   }
-  *h_cells = 0;
-  *h_points = 0;
+  *plan = Plan{kModeCells, dedup ? 1 : 0, 0, 0, g.nx, g.ny, g.nz, 0};
   char* ws = (char*)d_ws;
   int32_t* hdr = (int32_t*)ws;
   const dim3 b(256);
   int rc = DAX_HIP_OK;
-  if (!words_ready) {
-    k_set_header<<<1, 64, 0, s>>>(hdr, kModeCells, g.nx, g.ny, g.nz, dedup ? 1 : 0);
-    DAXHIP_LAUNCH_CHECK("k_set_header");
-  }
   if (!g.cells) {
-    // counts 0/1 on a uniform grid: the bit-word layout
     const BitGeom bg = bit_geom(g.nx, g.ny, g.nz);
     const BitWs bw = bit_ws(w, bg);
     if (bw.fits) {
-      uint64_t* cbits = (uint64_t*)(ws + bw.cbits);
-      int32_t* coff = (int32_t*)(ws + bw.coff);
-      if (!words_ready) {
-        k_cell_bits<<<dim3((unsigned)ceil_div((int64_t)bg.cy * bg.cz, kRowWaves)),
-                      dim3(64 * kRowWaves), 0, s>>>(bg, d_counts, cbits, coff, hdr + 1);
-        DAXHIP_LAUNCH_CHECK("k_cell_bits");
-      }
-      int32_t total = 0, general = 0;
-      if ((rc = dax_hip_scan_exclusive_i32(coff, coff, bg.n_cwords, &total, s))) return rc;
-      if (!words_ready) {
-        DAXHIP_CHECK(hipMemcpyAsync(&general, hdr + 1, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        DAXHIP_CHECK(hipStreamSynchronize(s));
-      }
+      int64_t cells = 0, points = 0;
+      bool general = false;
+      if ((rc = prepare_bits(bg, bw, ws, d_field, lo, hi, d_counts, flags, d_mask, &cells, &points,
+                             &general, s)))
+        return rc;
       if (!general) {
-        if ((int64_t)total * 8 > 0x7fffffffLL) {
-          set_error("topology prepare: %lld output cells exceed 2^31 ids", (long long)total);
+        if (cells * 8 > 0x7fffffffLL) {
+          set_error("topology prepare: %lld output cells exceed 2^31 ids", (long long)cells);
           return DAX_HIP_BAD_VALUE;
         }
-        k_set_header<<<1, 64, 0, s>>>(hdr, kModeBits, g.nx, g.ny, g.nz, dedup ? 1 : 0);
-        DAXHIP_LAUNCH_CHECK("k_set_header");
-        *h_cells = total;
-        if (!dedup) {
-          k_set_sizes<<<1, 64, 0, s>>>(hdr, total, 0);
-          DAXHIP_LAUNCH_CHECK("k_set_sizes");
-          return DAX_HIP_OK;
-        }
-        uint64_t* mbits = (uint64_t*)(ws + bw.mbits);
-        int32_t* moff = (int32_t*)(ws + bw.moff);
-        if (mask_optional) {
-          k_mask_words<<<dim3((unsigned)ceil_div(bg.n_pwords, 256)), b, 0, s>>>(bg, cbits, mbits,
-                                                                                moff);
-          DAXHIP_LAUNCH_CHECK("k_mask_words");
-        } else {
-          k_mask_bits<<<dim3((unsigned)ceil_div((int64_t)bg.ny * bg.nz, kRowWaves)),
-                        dim3(64 * kRowWaves), 0, s>>>(bg, cbits, mbits, moff, d_mask);
-          DAXHIP_LAUNCH_CHECK("k_mask_bits");
-        }
-        int32_t used = 0;
-        if ((rc = dax_hip_scan_exclusive_i32(moff, moff, bg.n_pwords, &used, s))) return rc;
-        k_set_sizes<<<1, 64, 0, s>>>(hdr, total, used);
-        DAXHIP_LAUNCH_CHECK("k_set_sizes");
-        *h_points = used;
+        plan->mode = kModeBits;
+        plan->cells = cells;
+        plan->points = points;
         return DAX_HIP_OK;
       }
+    } else if (d_field) {
+      if ((rc = count_uniform(d_field, g.nx, g.ny, g.nz, lo, hi, d_counts, s))) return rc;
     }
   }
+  k_set_header<<<1, 64, 0, s>>>(hdr, kModeCells, g.nx, g.ny, g.nz, dedup ? 1 : 0);
+  DAXHIP_LAUNCH_CHECK("k_set_header");
   // any counts: per-cell offsets and per-point ranks.  The exact sum and the
   // sign of every count are checked first: the scan below is int32.
   {
@@ -875,7 +963,7 @@ int prepare(const Geometry& g, const int32_t* d_counts, unsigned flags, void* d_
   int32_t* rank = (int32_t*)(ws + w.off_b);
   int32_t total = 0;
   if ((rc = dax_hip_scan_exclusive_i32(d_counts, offs, g.n_cells, &total, s))) return rc;
-  *h_cells = total;
+  plan->cells = total;
   if (!dedup) return DAX_HIP_OK;
   const dim3 gp((unsigned)ceil_div(g.n_points, 256));
   if (g.cells) {
@@ -904,13 +992,25 @@ int prepare(const Geometry& g, const int32_t* d_counts, unsigned flags, void* d_
   }
   int32_t used = 0;
   if ((rc = dax_hip_scan_exclusive_i32(d_mask, rank, g.n_points, &used, s))) return rc;
-  *h_points = used;
+  plan->points = used;
   return DAX_HIP_OK;
 }
 
+// The plan a prepare left in the workspace's header (synchronous).
+int read_plan(const void* d_ws, Plan* plan, hipStream_t s) {
+  int32_t h[kHeaderInts];
+  DAXHIP_CHECK(hipMemcpyAsync(h, d_ws, sizeof(h), hipMemcpyDeviceToHost, s));
+  DAXHIP_CHECK(hipStreamSynchronize(s));
+  *plan = Plan{h[0], h[5], h[6], h[7], h[2], h[3], h[4], 0};
+  return DAX_HIP_OK;
+}
+
+// Fills the output grid; `given` is the caller's plan, or null to read the
+// header's.
 int generate(const Geometry& g, const float* d_points, const float* origin, const float* spacing,
              const int32_t* d_counts, unsigned flags, const void* d_ws, size_t ws_bytes,
-             const int32_t* d_mask, int32_t* d_conn, float* d_coords, hipStream_t s) {
+             const int32_t* d_mask, const Plan* given, int32_t* d_conn, float* d_coords,
+             hipStream_t s) {
   const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
   const TopoWs w = topo_ws(g.n_cells, g.n_points);
   if (!d_counts || !d_ws || ws_bytes < w.bytes || !d_conn || (dedup && (!d_mask || !d_coords)) ||
@@ -928,17 +1028,18 @@ int generate(const Geometry& g, const float* d_points, const float* origin, cons
     if (spacing) h[d] = spacing[d];
   }
   const dim3 b(256);
-  // the layout prepare chose (the kernels also check it) and whether it
-  // ranked the points
-  int32_t head[kHeaderInts];
-  DAXHIP_CHECK(hipMemcpyAsync(head, hdr, sizeof(head), hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
-  const int32_t mode = head[0];
-  if (dedup && !head[5]) {
+  // the layout prepare chose, whether it ranked the points, the sizes
+  Plan plan;
+  if (given) {
+    plan = *given;
+  } else if (const int rc = read_plan(d_ws, &plan, s)) {
+    return rc;
+  }
+  if (dedup && !plan.ranked) {
     set_error("topology generate: duplicate removal after a prepare without it");
     return DAX_HIP_BAD_VALUE;
   }
-  if (mode == kModeCells) {
+  if (plan.mode == kModeCells) {
     k_emit<<<dim3((unsigned)ceil_div(g.n_cells, 1024)), b, 0, s>>>(
         hdr, g.nv, g.cells, g.n_cells, g.nx, g.ny, d_counts, aligned16(d_counts), offs,
         dedup ? rank : nullptr, d_conn);
@@ -952,29 +1053,55 @@ int generate(const Geometry& g, const float* d_points, const float* origin, cons
   } else if (!g.cells) {
     const BitGeom bg = bit_geom(g.nx, g.ny, g.nz);
     const BitWs bw = bit_ws(w, bg);
-    if (!bw.fits) {
+    if (!bw.fits || plan.nx != g.nx || plan.ny != g.ny || plan.nz != g.nz) {
       set_error("topology generate: workspace of another grid");
       return DAX_HIP_BAD_VALUE;
     }
-    {
-      const uint64_t* cbits = (const uint64_t*)(ws + bw.cbits);
-      const int32_t* coff = (const int32_t*)(ws + bw.coff);
-      const uint64_t* mbits = (const uint64_t*)(ws + bw.mbits);
-      const int32_t* moff = (const int32_t*)(ws + bw.moff);
-      const int64_t n_out = head[6], n_used = head[7];
-      if (n_out > 0) {
-        k_emit_rank<<<dim3((unsigned)ceil_div(n_out, 256)), b, 0, s>>>(
-            bg, hdr, cbits, coff, mbits, moff, dedup, n_out, d_conn);
-        DAXHIP_LAUNCH_CHECK("k_emit_rank");
-      }
-      if (dedup && n_used > 0) {
-        k_compact_rank<<<dim3((unsigned)ceil_div(n_used, 256)), b, 0, s>>>(
-            bg, hdr, mbits, moff, n_used, o[0], o[1], o[2], h[0], h[1], h[2], d_coords, nullptr,
-            0, nullptr);
-        DAXHIP_LAUNCH_CHECK("k_compact_rank");
-      }
+    const WordSet cs = cell_set(ws, bw), ps = point_set(ws, bw);
+    if (plan.cells > 0) {
+      k_emit_words<<<dim3((unsigned)ceil_div(bg.n_cwords, 256)), b, 0, s>>>(
+          bg, cs, ps, dedup, plan.cells, aligned16(d_conn), d_conn);
+      DAXHIP_LAUNCH_CHECK("k_emit_words");
+    }
+    if (dedup && plan.points > 0) {
+      k_compact_words<<<dim3((unsigned)ceil_div(bg.n_pwords, 4 * kCompactWords)), b, 0, s>>>(
+          bg, ps, plan.points, o[0], o[1], o[2], h[0], h[1], h[2], d_coords, nullptr, 0, nullptr);
+      DAXHIP_LAUNCH_CHECK("k_compact_words");
     }
   }
+  return DAX_HIP_OK;
+}
+
+// CompactPointField (checked arguments).
+int compact_field(const void* d_in, int words, int64_t n_points, const TopoWs& w, const char* ws,
+                  const int32_t* d_mask, const Plan& plan, void* d_out, hipStream_t s) {
+  if (!plan.ranked) {
+    set_error("dax_hip_topology_compact_point_field: the prepare step did not remove duplicates");
+    return DAX_HIP_BAD_VALUE;
+  }
+  if (plan.mode == kModeBits) {
+    const BitGeom bg = bit_geom((int)plan.nx, (int)plan.ny, (int)plan.nz);
+    const BitWs bw = bit_ws(w, bg);
+    if (plan.nx * plan.ny * plan.nz != n_points || !bw.fits) {
+      set_error("dax_hip_topology_compact_point_field: workspace of another grid");
+      return DAX_HIP_BAD_VALUE;
+    }
+    if (plan.points > 0) {
+      k_compact_words<<<dim3((unsigned)ceil_div(bg.n_pwords, 4 * kCompactWords)), dim3(256), 0, s>>>(
+          bg, point_set(ws, bw), plan.points, 0, 0, 0, 0, 0, 0, nullptr, (const uint32_t*)d_in,
+          words, (uint32_t*)d_out);
+      DAXHIP_LAUNCH_CHECK("k_compact_words");
+    }
+    return DAX_HIP_OK;
+  }
+  if (!d_mask) {
+    set_error("dax_hip_topology_compact_point_field: the point mask is needed for this layout");
+    return DAX_HIP_BAD_VALUE;
+  }
+  k_compact_values<<<dim3((unsigned)ceil_div(n_points, 1024)), dim3(256), 0, s>>>(
+      (const uint32_t*)d_in, words, n_points, d_mask, aligned16(d_mask),
+      (const int32_t*)(ws + w.off_b), (const int32_t*)ws, (uint32_t*)d_out);
+  DAXHIP_LAUNCH_CHECK("k_compact_values");
   return DAX_HIP_OK;
 }
 
@@ -994,21 +1121,7 @@ int dax_hip_threshold_count_uniform(const float* d_field, int64_t nx, int64_t ny
               (long long)nx, (long long)ny, (long long)nz);
     return DAX_HIP_BAD_VALUE;
   }
-  const int cx = (int)nx - 1, cy = (int)ny - 1, cz = (int)nz - 1;
-  if ((nx & 3) == 0 && ((uintptr_t)d_field & 15u) == 0) {
-    k_count_uniform4<<<dim3((unsigned)ceil_div(nx, 4 * kTX), (unsigned)ceil_div(cy, kTY),
-                            (unsigned)ceil_div(cz, kZRun)),
-                       dim3(kTX, kTY), 0, (hipStream_t)stream>>>(
-        d_field, (int)nx, (int)ny, (int)nz, min_value, max_value, d_counts);
-    DAXHIP_LAUNCH_CHECK("k_count_uniform4");
-    return DAX_HIP_OK;
-  }
-  k_count_uniform<<<dim3((unsigned)ceil_div(cx, kTX), (unsigned)ceil_div(cy, kTY),
-                         (unsigned)ceil_div(cz, kZRun)),
-                    dim3(kTX, kTY), 0, (hipStream_t)stream>>>(d_field, (int)nx, (int)ny, (int)nz,
-                                                              min_value, max_value, d_counts);
-  DAXHIP_LAUNCH_CHECK("k_count_uniform");
-  return DAX_HIP_OK;
+  return count_uniform(d_field, nx, ny, nz, min_value, max_value, d_counts, (hipStream_t)stream);
 }
 
 int dax_hip_threshold_count_cells(const int32_t* d_cells, int nv, int64_t n_cells,
@@ -1039,62 +1152,88 @@ int dax_hip_threshold_count_cells(const int32_t* d_cells, int nv, int64_t n_cell
   return DAX_HIP_OK;
 }
 
+// Geometry of a uniform grid the entry points accept.
+#define DAXHIP_UNIFORM_GEOMETRY(name)                                                              \
+  if (!uniform_ok(nx, ny, nz)) {                                                                   \
+    set_error("%s: unsupported grid %lld x %lld x %lld", name, (long long)nx, (long long)ny,       \
+              (long long)nz);                                                                      \
+    return DAX_HIP_BAD_VALUE;                                                                      \
+  }                                                                                                \
+  const Geometry g{nullptr, 8, (nx - 1) * (ny - 1) * (nz - 1), nx * ny * nz, (int)nx, (int)ny,     \
+                   (int)nz}
+
+int dax_hip_threshold_plan_uniform(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
+                                   float min_value, float max_value, unsigned flags,
+                                   int32_t* d_counts, void* d_workspace, size_t workspace_bytes,
+                                   int32_t* d_point_mask, int64_t* h_plan8, void* stream) {
+  DAXHIP_UNIFORM_GEOMETRY("dax_hip_threshold_plan_uniform");
+  if (!d_field) {
+    set_error("dax_hip_threshold_plan_uniform: field is NULL");
+    return DAX_HIP_BAD_VALUE;
+  }
+  return prepare(g, d_field, min_value, max_value, d_counts, flags, d_workspace, workspace_bytes,
+                 d_point_mask, (Plan*)h_plan8, (hipStream_t)stream);
+}
+
 int dax_hip_threshold_prepare_uniform(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
                                       float min_value, float max_value, unsigned flags,
                                       int32_t* d_counts, void* d_workspace,
                                       size_t workspace_bytes, int32_t* d_point_mask,
                                       int64_t* h_cells, int64_t* h_points, void* stream) {
-  if (!uniform_ok(nx, ny, nz) || !d_field || !d_counts) {
-    set_error("dax_hip_threshold_prepare_uniform: bad arguments (grid %lld x %lld x %lld)",
-              (long long)nx, (long long)ny, (long long)nz);
+  Plan plan;
+  if (!h_cells || !h_points) {
+    set_error("dax_hip_threshold_prepare_uniform: h_cells and h_points are required");
     return DAX_HIP_BAD_VALUE;
   }
-  const Geometry g{nullptr, 8, (nx - 1) * (ny - 1) * (nz - 1), nx * ny * nz, (int)nx, (int)ny,
-                   (int)nz};
-  const TopoWs w = topo_ws(g.n_cells, g.n_points);
-  const BitGeom bg = bit_geom(g.nx, g.ny, g.nz);
-  const BitWs bw = bit_ws(w, bg);
-  hipStream_t s = (hipStream_t)stream;
-  const bool fused = (nx & 3) == 0 && ((uintptr_t)d_field & 15u) == 0 && bw.fits &&
-                     d_workspace && workspace_bytes >= w.bytes;
-  if (!fused) {  // ThresholdCount, then the generic prepare
-    int rc = dax_hip_threshold_count_uniform(d_field, nx, ny, nz, min_value, max_value, d_counts,
-                                             stream);
-    if (rc) return rc;
-    return prepare(g, d_counts, flags, d_workspace, workspace_bytes, d_point_mask, h_cells,
-                   h_points, s);
-  }
-  char* ws = (char*)d_workspace;
-  const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
-  k_set_header<<<1, 64, 0, s>>>((int32_t*)ws, kModeCells, g.nx, g.ny, g.nz, dedup ? 1 : 0);
-  DAXHIP_LAUNCH_CHECK("k_set_header");
-  k_threshold_words4<<<dim3((unsigned)ceil_div(nx, 4 * kTX), (unsigned)ceil_div(bg.cy, kTY),
-                            (unsigned)ceil_div(bg.cz, kZRun)),
-                       dim3(kTX, kTY), 0, s>>>(d_field, (int)nx, (int)ny, (int)nz, min_value,
-                                               max_value, bg.wcx, d_counts,
-                                               (uint64_t*)(ws + bw.cbits),
-                                               (int32_t*)(ws + bw.coff));
-  DAXHIP_LAUNCH_CHECK("k_threshold_words4");
-  return prepare(g, d_counts, flags, d_workspace, workspace_bytes, d_point_mask, h_cells, h_points,
-                 s, true);
+  *h_cells = *h_points = 0;
+  const int rc = dax_hip_threshold_plan_uniform(d_field, nx, ny, nz, min_value, max_value, flags,
+                                                d_counts, d_workspace, workspace_bytes,
+                                                d_point_mask, (int64_t*)&plan, stream);
+  if (rc) return rc;
+  *h_cells = plan.cells;
+  *h_points = plan.points;
+  return DAX_HIP_OK;
 }
 
 size_t dax_hip_topology_workspace_bytes(int64_t n_cells, int64_t n_points) {
   return topo_ws(n_cells, n_points).bytes;
 }
 
+int dax_hip_topology_plan_uniform(int64_t nx, int64_t ny, int64_t nz, const int32_t* d_counts,
+                                  unsigned flags, void* d_workspace, size_t workspace_bytes,
+                                  int32_t* d_point_mask, int64_t* h_plan8, void* stream) {
+  DAXHIP_UNIFORM_GEOMETRY("dax_hip_topology_prepare_uniform");
+  return prepare(g, nullptr, 0.0f, 0.0f, const_cast<int32_t*>(d_counts), flags, d_workspace,
+                 workspace_bytes, d_point_mask, (Plan*)h_plan8, (hipStream_t)stream);
+}
+
 int dax_hip_topology_prepare_uniform(int64_t nx, int64_t ny, int64_t nz, const int32_t* d_counts,
                                      unsigned flags, void* d_workspace, size_t workspace_bytes,
                                      int32_t* d_point_mask, int64_t* h_cells, int64_t* h_points,
                                      void* stream) {
-  if (!uniform_ok(nx, ny, nz)) {
-    set_error("dax_hip_topology_prepare_uniform: unsupported grid");
+  Plan plan;
+  if (!h_cells || !h_points) {
+    set_error("dax_hip_topology_prepare_uniform: h_cells and h_points are required");
     return DAX_HIP_BAD_VALUE;
   }
-  const Geometry g{nullptr, 8, (nx - 1) * (ny - 1) * (nz - 1), nx * ny * nz, (int)nx, (int)ny,
-                   (int)nz};
-  return prepare(g, d_counts, flags, d_workspace, workspace_bytes, d_point_mask, h_cells, h_points,
-                 (hipStream_t)stream);
+  *h_cells = *h_points = 0;
+  const int rc = dax_hip_topology_plan_uniform(nx, ny, nz, d_counts, flags, d_workspace,
+                                               workspace_bytes, d_point_mask, (int64_t*)&plan,
+                                               stream);
+  if (rc) return rc;
+  *h_cells = plan.cells;
+  *h_points = plan.points;
+  return DAX_HIP_OK;
+}
+
+int dax_hip_topology_fill_uniform(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
+                                  const float* h_spacing3, const int32_t* d_counts,
+                                  unsigned flags, const void* d_workspace, size_t workspace_bytes,
+                                  const int32_t* d_point_mask, const int64_t* h_plan8,
+                                  int32_t* d_conn, float* d_coords, void* stream) {
+  DAXHIP_UNIFORM_GEOMETRY("dax_hip_topology_generate_uniform");
+  return generate(g, nullptr, h_origin3, h_spacing3, d_counts, flags, d_workspace, workspace_bytes,
+                  d_point_mask, (const Plan*)h_plan8, d_conn, d_coords, (hipStream_t)stream);
 }
 
 int dax_hip_topology_generate_uniform(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
@@ -1102,14 +1241,23 @@ int dax_hip_topology_generate_uniform(int64_t nx, int64_t ny, int64_t nz, const 
                                       unsigned flags, const void* d_workspace,
                                       size_t workspace_bytes, const int32_t* d_point_mask,
                                       int32_t* d_conn, float* d_coords, void* stream) {
-  if (!uniform_ok(nx, ny, nz)) {
-    set_error("dax_hip_topology_generate_uniform: unsupported grid");
+  return dax_hip_topology_fill_uniform(nx, ny, nz, h_origin3, h_spacing3, d_counts, flags,
+                                       d_workspace, workspace_bytes, d_point_mask, nullptr, d_conn,
+                                       d_coords, stream);
+}
+
+int dax_hip_topology_plan_cells(const int32_t* d_cells, int nv, int64_t n_cells, int64_t n_points,
+                                const int32_t* d_counts, unsigned flags, void* d_workspace,
+                                size_t workspace_bytes, int32_t* d_point_mask, int64_t* h_plan8,
+                                void* stream) {
+  if (nv < 1 || nv > 8 || n_cells < 1 || n_points < 1 || n_points > 0x7fffffffLL ||
+      n_cells > 0x7fffffffLL / nv || !d_cells) {
+    set_error("dax_hip_topology_prepare_cells: bad arguments");
     return DAX_HIP_BAD_VALUE;
   }
-  const Geometry g{nullptr, 8, (nx - 1) * (ny - 1) * (nz - 1), nx * ny * nz, (int)nx, (int)ny,
-                   (int)nz};
-  return generate(g, nullptr, h_origin3, h_spacing3, d_counts, flags, d_workspace, workspace_bytes,
-                  d_point_mask, d_conn, d_coords, (hipStream_t)stream);
+  const Geometry g{d_cells, nv, n_cells, n_points, 0, 0, 0};
+  return prepare(g, nullptr, 0.0f, 0.0f, const_cast<int32_t*>(d_counts), flags, d_workspace,
+                 workspace_bytes, d_point_mask, (Plan*)h_plan8, (hipStream_t)stream);
 }
 
 int dax_hip_topology_prepare_cells(const int32_t* d_cells, int nv, int64_t n_cells,
@@ -1117,22 +1265,26 @@ int dax_hip_topology_prepare_cells(const int32_t* d_cells, int nv, int64_t n_cel
                                    void* d_workspace, size_t workspace_bytes,
                                    int32_t* d_point_mask, int64_t* h_cells, int64_t* h_points,
                                    void* stream) {
-  if (nv < 1 || nv > 8 || n_cells < 1 || n_points < 1 || n_points > 0x7fffffffLL ||
-      n_cells > 0x7fffffffLL / nv || !d_cells) {
-    set_error("dax_hip_topology_prepare_cells: bad arguments");
+  Plan plan;
+  if (!h_cells || !h_points) {
+    set_error("dax_hip_topology_prepare_cells: h_cells and h_points are required");
     return DAX_HIP_BAD_VALUE;
   }
-  const Geometry g{d_cells, nv, n_cells, n_points, 0, 0, 0};
-  return prepare(g, d_counts, flags, d_workspace, workspace_bytes, d_point_mask, h_cells, h_points,
-                 (hipStream_t)stream);
+  *h_cells = *h_points = 0;
+  const int rc = dax_hip_topology_plan_cells(d_cells, nv, n_cells, n_points, d_counts, flags,
+                                             d_workspace, workspace_bytes, d_point_mask,
+                                             (int64_t*)&plan, stream);
+  if (rc) return rc;
+  *h_cells = plan.cells;
+  *h_points = plan.points;
+  return DAX_HIP_OK;
 }
 
-int dax_hip_topology_generate_cells(const int32_t* d_cells, int nv, int64_t n_cells,
-                                    const float* d_points, int64_t n_points,
-                                    const int32_t* d_counts, unsigned flags,
-                                    const void* d_workspace, size_t workspace_bytes,
-                                    const int32_t* d_point_mask, int32_t* d_conn,
-                                    float* d_coords, void* stream) {
+int dax_hip_topology_fill_cells(const int32_t* d_cells, int nv, int64_t n_cells,
+                                const float* d_points, int64_t n_points, const int32_t* d_counts,
+                                unsigned flags, const void* d_workspace, size_t workspace_bytes,
+                                const int32_t* d_point_mask, const int64_t* h_plan8,
+                                int32_t* d_conn, float* d_coords, void* stream) {
   if (nv < 1 || nv > 8 || n_cells < 1 || n_points < 1 || n_points > 0x7fffffffLL ||
       n_cells > 0x7fffffffLL / nv || !d_cells ||
       ((flags & DAX_HIP_MC_DEDUP) && !d_points)) {
@@ -1141,13 +1293,24 @@ int dax_hip_topology_generate_cells(const int32_t* d_cells, int nv, int64_t n_ce
   }
   const Geometry g{d_cells, nv, n_cells, n_points, 0, 0, 0};
   return generate(g, d_points, nullptr, nullptr, d_counts, flags, d_workspace, workspace_bytes,
-                  d_point_mask, d_conn, d_coords, (hipStream_t)stream);
+                  d_point_mask, (const Plan*)h_plan8, d_conn, d_coords, (hipStream_t)stream);
 }
 
-int dax_hip_topology_compact_point_field(const void* d_in, size_t value_bytes, int64_t n_cells,
-                                         int64_t n_points, const int32_t* d_point_mask,
-                                         const void* d_workspace, size_t workspace_bytes,
-                                         void* d_out, void* stream) {
+int dax_hip_topology_generate_cells(const int32_t* d_cells, int nv, int64_t n_cells,
+                                    const float* d_points, int64_t n_points,
+                                    const int32_t* d_counts, unsigned flags,
+                                    const void* d_workspace, size_t workspace_bytes,
+                                    const int32_t* d_point_mask, int32_t* d_conn,
+                                    float* d_coords, void* stream) {
+  return dax_hip_topology_fill_cells(d_cells, nv, n_cells, d_points, n_points, d_counts, flags,
+                                     d_workspace, workspace_bytes, d_point_mask, nullptr, d_conn,
+                                     d_coords, stream);
+}
+
+int dax_hip_topology_fill_point_field(const void* d_in, size_t value_bytes, int64_t n_cells,
+                                      int64_t n_points, const int32_t* d_point_mask,
+                                      const void* d_workspace, size_t workspace_bytes,
+                                      const int64_t* h_plan8, void* d_out, void* stream) {
   const TopoWs w = topo_ws(n_cells, n_points);
   if (value_bytes == 0 || value_bytes % 4 || value_bytes > 1024 || n_points < 0 ||
       n_points > 0x7fffffffLL || !d_workspace || workspace_bytes < w.bytes ||
@@ -1158,40 +1321,22 @@ int dax_hip_topology_compact_point_field(const void* d_in, size_t value_bytes, i
   }
   if (n_points == 0) return DAX_HIP_OK;
   hipStream_t s = (hipStream_t)stream;
-  const char* ws = (const char*)d_workspace;
-  int32_t hdr[kHeaderInts];
-  DAXHIP_CHECK(hipMemcpyAsync(hdr, ws, sizeof(hdr), hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
-  if (!hdr[5]) {
-    set_error("dax_hip_topology_compact_point_field: the prepare step did not remove duplicates");
-    return DAX_HIP_BAD_VALUE;
+  Plan plan;
+  if (h_plan8) {
+    plan = *(const Plan*)h_plan8;
+  } else if (const int rc = read_plan(d_workspace, &plan, s)) {
+    return rc;
   }
-  const int words = (int)(value_bytes / 4);
-  if (hdr[0] == kModeBits) {
-    const BitGeom bg = bit_geom(hdr[2], hdr[3], hdr[4]);
-    const BitWs bw = bit_ws(w, bg);
-    if ((int64_t)hdr[2] * hdr[3] * hdr[4] != n_points || !bw.fits) {
-      set_error("dax_hip_topology_compact_point_field: workspace of another grid");
-      return DAX_HIP_BAD_VALUE;
-    }
-    const int64_t n_used = hdr[7];
-    if (n_used > 0) {
-      k_compact_rank<<<dim3((unsigned)ceil_div(n_used, 256)), dim3(256), 0, s>>>(
-          bg, (const int32_t*)ws, (const uint64_t*)(ws + bw.mbits), (const int32_t*)(ws + bw.moff),
-          n_used, 0, 0, 0, 0, 0, 0, nullptr, (const uint32_t*)d_in, words, (uint32_t*)d_out);
-      DAXHIP_LAUNCH_CHECK("k_compact_rank");
-    }
-    return DAX_HIP_OK;
-  }
-  if (!d_point_mask) {
-    set_error("dax_hip_topology_compact_point_field: the point mask is needed for this layout");
-    return DAX_HIP_BAD_VALUE;
-  }
-  k_compact_values<<<dim3((unsigned)ceil_div(n_points, 1024)), dim3(256), 0, s>>>(
-      (const uint32_t*)d_in, words, n_points, d_point_mask, aligned16(d_point_mask),
-      (const int32_t*)(ws + w.off_b), (const int32_t*)ws, (uint32_t*)d_out);
-  DAXHIP_LAUNCH_CHECK("k_compact_values");
-  return DAX_HIP_OK;
+  return compact_field(d_in, (int)(value_bytes / 4), n_points, w, (const char*)d_workspace,
+                       d_point_mask, plan, d_out, s);
+}
+
+int dax_hip_topology_compact_point_field(const void* d_in, size_t value_bytes, int64_t n_cells,
+                                         int64_t n_points, const int32_t* d_point_mask,
+                                         const void* d_workspace, size_t workspace_bytes,
+                                         void* d_out, void* stream) {
+  return dax_hip_topology_fill_point_field(d_in, value_bytes, n_cells, n_points, d_point_mask,
+                                           d_workspace, workspace_bytes, nullptr, d_out, stream);
 }
 
 }  // extern "C"

@@ -40,6 +40,7 @@ class Topology:
     workspace: Optional[torch.Tensor] = None   # the prepare step's (ranks of the used points)
     num_input_cells: int = 0
     _mask_buffer: Optional[torch.Tensor] = None  # what prepare was given for the mask
+    _plan: Optional[ctypes.Array] = None         # the prepare step's findings (dax_hip.h)
 
     @property
     def num_cells(self) -> int:
@@ -59,10 +60,10 @@ class Topology:
         if v.element_size() * v.shape[1] % 4:
             raise ValueError("point values of a multiple of 4 bytes")
         out = torch.empty((max(self.num_points, 1), v.shape[1]), dtype=v.dtype, device=v.device)
-        _lib.call("dax_hip_topology_compact_point_field", v.data_ptr(),
+        _lib.call("dax_hip_topology_fill_point_field", v.data_ptr(),
                   v.element_size() * v.shape[1], self.num_input_cells, P,
                   self._mask_buffer.data_ptr(), self.workspace.data_ptr(), self.workspace.numel(),
-                  out.data_ptr(), _stream())
+                  self._plan, out.data_ptr(), _stream())
         res = out[: self.num_points]
         return res.reshape(-1) if values.dim() == 1 else res.reshape((self.num_points,) +
                                                                      tuple(values.shape[1:]))
@@ -99,9 +100,10 @@ def threshold_count(field: torch.Tensor, lo: float, hi: float,
     return counts[:C]
 
 
-def _generate(counts, dims, cells, points, origin, spacing, dedup, ws, mask, T, U,
+def _generate(counts, dims, cells, points, origin, spacing, dedup, ws, mask, plan,
               mask_valid=True) -> Topology:
     dev = counts.device
+    T, U = int(plan[2]), int(plan[3])
     if cells is None:
         nx, ny, nz = (int(v) for v in dims)
         C, P, V = (nx - 1) * (ny - 1) * (nz - 1), nx * ny * nz, 8
@@ -115,17 +117,18 @@ def _generate(counts, dims, cells, points, origin, spacing, dedup, ws, mask, T, 
     cptr = coords.data_ptr() if dedup else None
     if T > 0:
         if cells is None:
-            _lib.call("dax_hip_topology_generate_uniform", nx, ny, nz, _f3(origin), _f3(spacing),
-                      counts.data_ptr(), flags, ws.data_ptr(), ws.numel(), mptr,
+            _lib.call("dax_hip_topology_fill_uniform", nx, ny, nz, _f3(origin), _f3(spacing),
+                      counts.data_ptr(), flags, ws.data_ptr(), ws.numel(), mptr, plan,
                       conn.data_ptr(), cptr, _stream())
         else:
-            _lib.call("dax_hip_topology_generate_cells", cells.data_ptr(), V, C,
+            _lib.call("dax_hip_topology_fill_cells", cells.data_ptr(), V, C,
                       points.data_ptr() if points is not None else None, P, counts.data_ptr(),
-                      flags, ws.data_ptr(), ws.numel(), mptr, conn.data_ptr(), cptr, _stream())
+                      flags, ws.data_ptr(), ws.numel(), mptr, plan, conn.data_ptr(), cptr,
+                      _stream())
     return Topology(counts=counts[:C], connectivity=conn[:T],
                     points=coords[:U] if dedup else None,
                     point_mask=mask if (dedup and mask_valid) else None,
-                    workspace=ws, num_input_cells=C, _mask_buffer=mask)
+                    workspace=ws, num_input_cells=C, _mask_buffer=mask, _plan=plan)
 
 
 def generate_topology(counts: torch.Tensor, dims=None, cells: Optional[torch.Tensor] = None,
@@ -138,7 +141,7 @@ def generate_topology(counts: torch.Tensor, dims=None, cells: Optional[torch.Ten
         raise ValueError("counts must be a contiguous int32 tensor")
     dev = counts.device
     lib = _lib.load()
-    t, u = ctypes.c_int64(), ctypes.c_int64()
+    plan = (ctypes.c_int64 * 8)()
     flags = MC_DEDUP if dedup else 0
     if cells is None:
         nx, ny, nz = (int(v) for v in dims)
@@ -157,14 +160,12 @@ def generate_topology(counts: torch.Tensor, dims=None, cells: Optional[torch.Ten
     mask = torch.empty(P, dtype=torch.int32, device=dev) if dedup else None
     mptr = mask.data_ptr() if dedup else None
     if cells is None:
-        _lib.call("dax_hip_topology_prepare_uniform", nx, ny, nz, counts.data_ptr(), flags,
-                  ws.data_ptr(), ws.numel(), mptr, ctypes.byref(t), ctypes.byref(u), _stream())
+        _lib.call("dax_hip_topology_plan_uniform", nx, ny, nz, counts.data_ptr(), flags,
+                  ws.data_ptr(), ws.numel(), mptr, plan, _stream())
     else:
-        _lib.call("dax_hip_topology_prepare_cells", cells.data_ptr(), V, C, P, counts.data_ptr(),
-                  flags, ws.data_ptr(), ws.numel(), mptr, ctypes.byref(t), ctypes.byref(u),
-                  _stream())
-    return _generate(counts, dims, cells, points, origin, spacing, dedup, ws, mask,
-                     int(t.value), int(u.value))
+        _lib.call("dax_hip_topology_plan_cells", cells.data_ptr(), V, C, P, counts.data_ptr(),
+                  flags, ws.data_ptr(), ws.numel(), mptr, plan, _stream())
+    return _generate(counts, dims, cells, points, origin, spacing, dedup, ws, mask, plan)
 
 
 def threshold(field: torch.Tensor, lo: float, hi: float, cells: Optional[torch.Tensor] = None,
@@ -189,9 +190,9 @@ def threshold(field: torch.Tensor, lo: float, hi: float, cells: Optional[torch.T
                      device=dev)
     mask = torch.empty(P, dtype=torch.int32, device=dev) if dedup else None
     flags = (MC_DEDUP if dedup else 0) | (0 if point_mask else TOPOLOGY_MASK_OPTIONAL)
-    t, u = ctypes.c_int64(), ctypes.c_int64()
-    _lib.call("dax_hip_threshold_prepare_uniform", field.data_ptr(), nx, ny, nz, float(lo),
+    plan = (ctypes.c_int64 * 8)()
+    _lib.call("dax_hip_threshold_plan_uniform", field.data_ptr(), nx, ny, nz, float(lo),
               float(hi), flags, counts.data_ptr(), ws.data_ptr(), ws.numel(),
-              mask.data_ptr() if dedup else None, ctypes.byref(t), ctypes.byref(u), _stream())
-    return _generate(counts, (nx, ny, nz), None, None, origin, spacing, dedup, ws, mask,
-                     int(t.value), int(u.value), mask_valid=point_mask)
+              mask.data_ptr() if dedup else None, plan, _stream())
+    return _generate(counts, (nx, ny, nz), None, None, origin, spacing, dedup, ws, mask, plan,
+                     mask_valid=point_mask)

@@ -340,10 +340,9 @@ size_t dax_hip_topology_workspace_bytes(int64_t n_cells, int64_t n_points);
 /* ThresholdCount and the prepare step in one call on a uniform grid (the
  * reference's Threshold pipeline, Benchmarks/Threshold/Pipeline.h:163-190):
  * d_counts as dax_hip_threshold_count_uniform, then as
- * dax_hip_topology_prepare_uniform on them.  With rows of 16-byte aligned
- * float4s (nx % 4 == 0) the count kernel also forms the bit-word layout's
- * cell words.  With DAX_HIP_TOPOLOGY_MASK_OPTIONAL, d_point_mask may be
- * left unwritten where that layout is used; pass the buffer anyway. */
+ * dax_hip_topology_prepare_uniform on them.  With
+ * DAX_HIP_TOPOLOGY_MASK_OPTIONAL, d_point_mask may be left unwritten where
+ * the library does not need it; pass the buffer anyway. */
 int dax_hip_threshold_prepare_uniform(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
                                       float min_value, float max_value, unsigned flags,
                                       int32_t* d_counts, void* d_workspace,
@@ -378,6 +377,38 @@ int dax_hip_topology_compact_point_field(const void* d_in, size_t value_bytes, i
                                          int64_t n_points, const int32_t* d_point_mask,
                                          const void* d_workspace, size_t workspace_bytes,
                                          void* d_out, void* stream);
+
+/* The same steps with the prepare's findings in the caller's hands: the plan
+ * calls are the prepare calls with h_plan8 (eight int64: [2] = T, [3] = U, the
+ * rest the library's own) in place of the two sizes, and the fill calls are
+ * generate / compact_point_field taking that plan instead of reading the
+ * workspace's header back (NULL: read it), so they queue their kernels and
+ * return. */
+int dax_hip_threshold_plan_uniform(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
+                                   float min_value, float max_value, unsigned flags,
+                                   int32_t* d_counts, void* d_workspace, size_t workspace_bytes,
+                                   int32_t* d_point_mask, int64_t* h_plan8, void* stream);
+int dax_hip_topology_plan_uniform(int64_t nx, int64_t ny, int64_t nz, const int32_t* d_counts,
+                                  unsigned flags, void* d_workspace, size_t workspace_bytes,
+                                  int32_t* d_point_mask, int64_t* h_plan8, void* stream);
+int dax_hip_topology_fill_uniform(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
+                                  const float* h_spacing3, const int32_t* d_counts,
+                                  unsigned flags, const void* d_workspace, size_t workspace_bytes,
+                                  const int32_t* d_point_mask, const int64_t* h_plan8,
+                                  int32_t* d_conn, float* d_coords, void* stream);
+int dax_hip_topology_plan_cells(const int32_t* d_cells, int nv, int64_t n_cells, int64_t n_points,
+                                const int32_t* d_counts, unsigned flags, void* d_workspace,
+                                size_t workspace_bytes, int32_t* d_point_mask, int64_t* h_plan8,
+                                void* stream);
+int dax_hip_topology_fill_cells(const int32_t* d_cells, int nv, int64_t n_cells,
+                                const float* d_points, int64_t n_points, const int32_t* d_counts,
+                                unsigned flags, const void* d_workspace, size_t workspace_bytes,
+                                const int32_t* d_point_mask, const int64_t* h_plan8,
+                                int32_t* d_conn, float* d_coords, void* stream);
+int dax_hip_topology_fill_point_field(const void* d_in, size_t value_bytes, int64_t n_cells,
+                                      int64_t n_points, const int32_t* d_point_mask,
+                                      const void* d_workspace, size_t workspace_bytes,
+                                      const int64_t* h_plan8, void* d_out, void* stream);
 
 /* VTK legacy ASCII files of an output grid held in host memory: the format
  * of the reference benchmarks' PrintContentsToStream
