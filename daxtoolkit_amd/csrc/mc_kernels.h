@@ -545,25 +545,6 @@ __device__ __forceinline__ int find_word(const uint32_t* s, int n, uint32_t v) {
   return lo;
 }
 
-// Position of the k-th set bit of m (k < popcount(m)): the half of m that
-// holds it, then halving steps on 32 bits.
-__device__ __forceinline__ int select_bit(uint64_t m, int k) {
-  const uint32_t lo = (uint32_t)m;
-  const int nlo = __popc(lo);
-  const bool up = k >= nlo;
-  uint32_t x = up ? (uint32_t)(m >> 32) : lo;
-  int r = up ? k - nlo : k, pos = up ? 32 : 0;
-#pragma unroll
-  for (int w = 16; w > 0; w >>= 1) {
-    const int c = __popc(x & ((1u << w) - 1u));
-    const bool hi = r >= c;
-    r = hi ? r - c : r;
-    x = hi ? x >> w : x;
-    pos += hi ? w : 0;
-  }
-  return pos;
-}
-
 // Edge codes of the 12 cell edges, 5 bits each (edge_code).
 __host__ __device__ constexpr uint64_t edge_codes_packed() {
   uint64_t r = 0;
@@ -836,24 +817,6 @@ struct GenLayout {
   }
   __host__ __device__ size_t bytes() const { return wave_offset() + kWaves * sizeof(GenWave); }
 };
-
-// Orders the LDS accesses of a wave's lanes among themselves (a wave's LDS
-// operations execute in order; this keeps the compiler from moving them).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// Inclusive prefix maximum over the lanes of a wave (wave_incl_scan's steps).
-__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
-  return v;
-}
 
 // Bits b, b+1, ... of the word A followed by the word A1 (b < 64).
 __device__ __forceinline__ uint32_t bit_window(uint64_t A, uint64_t A1, int b) {

@@ -336,11 +336,13 @@ def _cells_contour(prefix: str, nv: int, cells: torch.Tensor, field: torch.Tenso
         raise ValueError("points must be a contiguous float32 [P, 3] tensor")
     dev = field.device
     C = int(cells.shape[0])
-    counts = torch.empty(max(C, 1), dtype=torch.int32, device=dev)
-    offsets = torch.empty(max(C, 1), dtype=torch.int32, device=dev)
+    lib = _lib.load()
+    ws = torch.empty(max(int(lib.dax_hip_cells_workspace_bytes(C)), 1), dtype=torch.uint8,
+                     device=dev)
     t = ctypes.c_int64()
-    _lib.call(f"{prefix}_count", cells.data_ptr(), C, field.data_ptr(), P, float(iso),
-              counts.data_ptr(), offsets.data_ptr(), ctypes.byref(t), _stream())
+    s = _stream()
+    _lib.call(f"{prefix}_count_cells", cells.data_ptr(), C, field.data_ptr(), P, float(iso),
+              ws.data_ptr(), ws.numel(), ctypes.byref(t), s)
     T = int(t.value)
     n = max(3 * T, 1)
     verts = torch.empty((n, 3), dtype=torch.float32, device=dev)
@@ -348,13 +350,14 @@ def _cells_contour(prefix: str, nv: int, cells: torch.Tensor, field: torch.Tenso
     first = torch.empty(n, dtype=torch.int32, device=dev)
     second = torch.empty(n, dtype=torch.int32, device=dev)
     weight = torch.empty(n, dtype=torch.float32, device=dev)
-    nbytes = int(getattr(_lib.load(), f"{prefix}_scratch_bytes")(T)) if dedup else 0
+    nbytes = int(getattr(lib, f"{prefix}_scratch_bytes")(T)) if dedup else 0
     scratch = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     u = ctypes.c_int64()
-    _lib.call(f"{prefix}_generate", cells.data_ptr(), C, field.data_ptr(), points.data_ptr(), P,
-              float(iso), MC_DEDUP if dedup else 0, counts.data_ptr(), offsets.data_ptr(), T,
-              scratch.data_ptr(), scratch.numel(), verts.data_ptr(), conn.data_ptr(),
-              first.data_ptr(), second.data_ptr(), weight.data_ptr(), ctypes.byref(u), _stream())
+    _lib.call(f"{prefix}_generate_cells", cells.data_ptr(), C, field.data_ptr(),
+              points.data_ptr(), P, float(iso), MC_DEDUP if dedup else 0, ws.data_ptr(),
+              ws.numel(), T, scratch.data_ptr(), scratch.numel(), verts.data_ptr(),
+              conn.data_ptr(), first.data_ptr(), second.data_ptr(), weight.data_ptr(),
+              ctypes.byref(u), s)
     U = int(u.value)
     return Contour(vertices=verts[:U], connectivity=conn[:3 * T].view(T, 3), normals=None,
                    edges=None, interp_first=first[:U], interp_second=second[:U],

@@ -306,6 +306,31 @@ int dax_hip_mc_hex_generate(const int32_t* d_hexes, int64_t n_hexes, const float
                             int32_t* d_conn, int32_t* d_first, int32_t* d_second,
                             float* d_weight, int64_t* h_points, void* stream);
 
+/* The same two steps of both shapes without a count and an offset per cell:
+ * count_cells (synchronous) keeps what generate_cells needs in d_workspace
+ * (dax_hip_cells_workspace_bytes of the cell count); outputs, flags, scratch
+ * and errors as above. */
+size_t dax_hip_cells_workspace_bytes(int64_t n_cells);
+int dax_hip_mt_count_cells(const int32_t* d_tets, int64_t n_tets, const float* d_field,
+                           int64_t n_points, float iso, void* d_workspace, size_t workspace_bytes,
+                           int64_t* h_tris, void* stream);
+int dax_hip_mt_generate_cells(const int32_t* d_tets, int64_t n_tets, const float* d_field,
+                              const float* d_points, int64_t n_points, float iso, unsigned flags,
+                              const void* d_workspace, size_t workspace_bytes, int64_t n_tris,
+                              void* d_scratch, size_t scratch_bytes, float* d_vertices,
+                              int32_t* d_conn, int32_t* d_first, int32_t* d_second,
+                              float* d_weight, int64_t* h_points, void* stream);
+int dax_hip_mc_hex_count_cells(const int32_t* d_hexes, int64_t n_hexes, const float* d_field,
+                               int64_t n_points, float iso, void* d_workspace,
+                               size_t workspace_bytes, int64_t* h_tris, void* stream);
+int dax_hip_mc_hex_generate_cells(const int32_t* d_hexes, int64_t n_hexes, const float* d_field,
+                                  const float* d_points, int64_t n_points, float iso,
+                                  unsigned flags, const void* d_workspace, size_t workspace_bytes,
+                                  int64_t n_tris, void* d_scratch, size_t scratch_bytes,
+                                  float* d_vertices, int32_t* d_conn, int32_t* d_first,
+                                  int32_t* d_second, float* d_weight, int64_t* h_points,
+                                  void* stream);
+
 /* Threshold (dax/worklet/Threshold.h:30-110) through DispatcherMapCell and
  * DispatcherGenerateTopology (dax/cont/DispatcherGenerateTopology.h:146-256).
  *
