@@ -153,6 +153,7 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   g.field_off = 0;
   g.word_off = 0;
   g.nwords = (int64_t)g.wpr * ny * nz;
+  g.tile_off = 0;
   set_geom_divs(g);
   const Workspace L = workspace_layout(g.nwords);
   if (!d_workspace || workspace_bytes < L.bytes) {

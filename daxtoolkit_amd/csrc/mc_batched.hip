@@ -3,18 +3,16 @@
 // counterpart (Dax runs one grid per dispatcher call).
 //
 // Layout: the volumes' fields are concatenated (volume v at field_off[v]);
-// their row words are concatenated in volume order (word_off[v]).  Scan and
-// generate tiles never straddle a volume; tile tables map tile -> (volume,
-// first local word).  One global exclusive scan over all words gives every
-// word its vertex/triangle base; subtracting the base of the volume's first
-// word makes the numbering per volume -- a segmented scan without segment
-// flags.  Outputs are concatenated in volume order; connectivity is local to
-// each volume; per-volume {first triangle, first point} offsets are written
-// beside the counts.
+// their row words are concatenated in volume order (word_off[v]).  Tiles of
+// 256 row words never straddle a volume; a table maps tile -> (volume, first
+// local word).  Every tile is counted as two count tiles, whose prefixes run
+// over all tiles; subtracting the prefix of the volume's first tile makes the
+// numbering per volume -- a segmented scan without segment flags.  Outputs
+// are concatenated in volume order; connectivity is local to each volume;
+// per-volume {first triangle, first point} offsets are written beside the
+// counts.
 //
-// Each phase is one persistent launch (grid = a few blocks per CU, looping
-// over tiles); the four launches of a forward are graph-capturable (no host
-// read-back, scan state cleared by a kernel).
+// The four launches of a forward are graph-capturable (no host read-back).
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -32,9 +30,7 @@ struct TileRef {
   int32_t w0;  // first row word, local to the volume
 };
 
-// Tile tables are built at prepare: 1024-word scan tiles, 256-word
-// generate (and classify) tiles.  The launch shapes over them are tuned.
-constexpr int kBatchScanTile = 1024;
+// The tile table is built at prepare.  The launch shapes over it are tuned.
 constexpr int kBatchGenTile = 256;
 // Threads per generate tile: one per word; a batch has tiles enough, so more
 // waves per tile only stage the same words for fewer outputs each (256 volumes
@@ -44,9 +40,9 @@ constexpr int kBatchGenThreads = 256;
 
 // Launch shapes of the batch forward, picked by dax_hip_mc_batch_autotune
 // and cached per batch shape class: classify unroll (row words per wave
-// step, a float4 load in flight per thread for two of them) and persistent blocks per CU, threads per scan tile (the tile's
-// 1024 words over 256, 512 or 1024 threads), generate blocks per CU and
-// its XCD-contiguous tile order.
+// step, a float4 load in flight per thread for two of them) and persistent blocks per CU, threads per count block (a wave per
+// tile), generate's XCD-contiguous tile order.  gen_blocks is kept for callers
+// that set it: generate runs a block per tile.
 struct BatchTuning {
   int32_t cls_unroll, cls_blocks, scan_threads, gen_blocks, gen_xcd, pad;
 };
@@ -60,28 +56,24 @@ bool valid_batch_tuning(const BatchTuning& t) {
 }
 
 struct BatchLayout {
-  size_t off_vols, off_scan_tiles, off_gen_tiles, off_bits, off_base_v, off_base_t, off_status,
-      off_ctrl, bytes;
-  int64_t nvols, nwords, nscan, ngen;
+  size_t off_vols, off_gen_tiles, off_bits, off_base_v, off_base_t, off_vol_first, off_lpre,
+      off_tloc, off_bsum, off_bpre, off_ctrl, bytes;
+  int64_t nvols, nwords, ngen;
 };
 
 BatchLayout batch_layout(int64_t nvols, const int64_t* dims) {
   BatchLayout L;
   L.nvols = nvols;
   L.nwords = 0;
-  L.nscan = 0;
   L.ngen = 0;
   for (int64_t v = 0; v < nvols; ++v) {
     const int64_t w = ceil_div(dims[3 * v], 64) * dims[3 * v + 1] * dims[3 * v + 2];
     L.nwords += w;
-    L.nscan += ceil_div(w, kBatchScanTile);
     L.ngen += ceil_div(w, kBatchGenTile);
   }
   size_t off = 0;
   L.off_vols = off;
   off = align_up(off + (size_t)nvols * sizeof(VolGeom), 256);
-  L.off_scan_tiles = off;
-  off = align_up(off + (size_t)L.nscan * sizeof(TileRef), 256);
   L.off_gen_tiles = off;
   off = align_up(off + (size_t)L.ngen * sizeof(TileRef), 256);
   L.off_bits = off;
@@ -90,8 +82,17 @@ BatchLayout batch_layout(int64_t nvols, const int64_t* dims) {
   off = align_up(off + (size_t)(L.nwords + 1) * 4, 256);
   L.off_base_t = off;
   off = align_up(off + (size_t)(L.nwords + 1) * 4, 256);
-  L.off_status = off;
-  off += (size_t)L.nscan * 8;
+  L.off_vol_first = off;
+  off = align_up(off + (size_t)nvols * 4, 256);
+  L.off_lpre = off;
+  off = align_up(off + (size_t)L.ngen * kBatchGenTile * 4, 256);
+  // two count tiles per tile, and the entry after the last of a full block
+  L.off_tloc = off;
+  off = align_up(off + (size_t)(2 * L.ngen + 1) * 8, 256);
+  L.off_bsum = off;
+  off = align_up(off + (size_t)(L.ngen + 1) * 8, 256);
+  L.off_bpre = off;
+  off = align_up(off + (size_t)(L.ngen + 1) * 8, 256);
   L.off_ctrl = off;
   off = align_up(off + sizeof(Ctrl), 256);
   L.bytes = off;
@@ -101,9 +102,9 @@ BatchLayout batch_layout(int64_t nvols, const int64_t* dims) {
 // Header at the start of the workspace: the layout, so launches need only
 // the workspace pointer after prepare.
 struct BatchHeader {
-  int64_t magic, nvols, nwords, nscan, ngen, max_wpr;
-  size_t off_vols, off_scan_tiles, off_gen_tiles, off_bits, off_base_v, off_base_t, off_status,
-      off_ctrl, bytes;
+  int64_t magic, nvols, nwords, ngen, max_wpr;
+  size_t off_vols, off_gen_tiles, off_bits, off_base_v, off_base_t, off_vol_first, off_lpre,
+      off_tloc, off_bsum, off_bpre, off_ctrl, bytes;
   BatchTuning tune;
 };
 constexpr int64_t kBatchMagic = 0x4441584842415443LL;  // "DAXHBATC"
@@ -115,13 +116,8 @@ __global__ __launch_bounds__(256) void k_batch_classify(const VolGeom* __restric
                                                         const TileRef* __restrict__ tiles,
                                                         int64_t ntiles,
                                                         const float* __restrict__ fields,
-                                                        uint64_t* __restrict__ bits,
-                                                        unsigned long long* __restrict__ zero_buf,
-                                                        int64_t zero_words) {
+                                                        uint64_t* __restrict__ bits) {
   __shared__ FlatLds<kBatchGenTile> sh;
-  const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = gtid; i < zero_words; i += nthreads) zero_buf[i] = 0ull;
   for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const TileRef tr = tiles[t];
     const VolGeom g = vols[tr.vol];
@@ -133,36 +129,70 @@ __global__ __launch_bounds__(256) void k_batch_classify(const VolGeom* __restric
   }
 }
 
-template <int NT>
-__global__ __launch_bounds__(NT) void k_batch_count_scan(
+// Count: a wave per tile (two count tiles), WAVES tiles per block.  No block
+// waits for another (a single pass with decoupled look-back over 1024-word
+// tiles took 200 us for 256 volumes of 32..160 points an axis; this and the
+// scan of the block sums take 34 + 6).
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_batch_count(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
-    const uint64_t* __restrict__ bits, uint32_t* __restrict__ base_v,
-    uint32_t* __restrict__ base_t, unsigned long long* __restrict__ status,
-    Ctrl* __restrict__ ctrl) {
-  __shared__ ScanShared sh;
-  constexpr int WPT = kBatchScanTile / NT;
-  __shared__ uint32_t s_pk[ScanTileLds<NT, WPT>::kSize];
-  __shared__ int64_t s_tile;
-  while (true) {
-    __syncthreads();  // s_tile and sh reused across iterations
-    if (threadIdx.x == 0) s_tile = (int64_t)atomicAdd(&ctrl->tile_counter, 1u);
-    __syncthreads();
-    const int64_t t = s_tile;
-    if (t >= ntiles) break;
+    const uint64_t* __restrict__ bits, uint32_t* __restrict__ lpre,
+    unsigned long long* __restrict__ tloc, unsigned long long* __restrict__ bsum) {
+  constexpr int kBlockTiles = 2 * WAVES;
+  __shared__ unsigned long long s_ts[kBlockTiles];
+  const int wv = threadIdx.x >> 6;
+  const int64_t blk = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t t = blk * WAVES + wv;
+  unsigned long long s0 = 0ull, s1 = 0ull;
+  if (t < ntiles) {
     const TileRef tr = tiles[t];
     const VolGeom g = vols[tr.vol];
-    count_scan_tile<NT, WPT>(g, bits + g.word_off, base_v, base_t, status, ctrl, t, tr.w0, sh,
-                             s_pk);
+    const int64_t pair = tr.w0 / kBatchGenTile;
+    count_tile_pair(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, pair, 2 * pair + 2,
+                    s0, s1);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_ts[2 * wv] = s0;
+    s_ts[2 * wv + 1] = s1;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long run = 0ull;
+    for (int i = 0; i < kBlockTiles; ++i) {
+      const int64_t tile = blk * kBlockTiles + i;
+      if (tile <= 2 * ntiles) tloc[tile] = run;
+      run = add_vt(run, s_ts[i]);
+    }
+    bsum[blk] = run;
   }
 }
 
+__global__ __launch_bounds__(kTsumThreads) void k_batch_scan(
+    const unsigned long long* __restrict__ bsum, unsigned long long* __restrict__ bpre, int64_t n,
+    unsigned long long* __restrict__ tloc, int64_t n_ctiles, Ctrl* __restrict__ ctrl,
+    int tpb_shift) {
+  __shared__ uint32_t s_v[kTsumThreads / 64], s_t[kTsumThreads / 64];
+  unsigned long long cv, ct;
+  scan_block_sums(bsum, bpre, n, s_v, s_t, cv, ct);
+  if (threadIdx.x == 0) {
+    if ((n_ctiles & ((1 << tpb_shift) - 1)) == 0) tloc[n_ctiles] = 0ull;
+    ctrl->total_v = cv;
+    ctrl->total_t = ct;
+    ctrl->tpb_shift = (uint32_t)tpb_shift;
+  }
+}
+
+// Generate, a block per tile (persistent blocks looping over the tiles, four
+// per CU: forward of 256 volumes 400 us, this 368).  The tile at a volume's
+// start also writes the volume's {first triangle, first point} in the
+// concatenated outputs and its first vertex for the adjoint.
 template <bool dedup>
 __global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
-    const float* __restrict__ fields, const uint64_t* __restrict__ bits,
-    const uint32_t* __restrict__ base_v, const uint32_t* __restrict__ base_t,
+    const float* __restrict__ fields, const uint64_t* __restrict__ bits, CountSrc all,
     const Ctrl* __restrict__ ctrl, OutPtrs out, unsigned flags, int64_t cap_points,
-    int64_t cap_tris, int64_t* __restrict__ counts, int xcd) {
+    int64_t cap_tris, int64_t* __restrict__ counts, int64_t* __restrict__ vol_offsets,
+    uint32_t* __restrict__ vol_first, int xcd) {
   extern __shared__ uint64_t s_dyn[];
   const bool normals = (flags & DAX_HIP_MC_NORMALS) != 0 && out.normals != nullptr;
   const uint64_t total_v = ctrl->total_v, total_t = ctrl->total_t;
@@ -171,54 +201,67 @@ __global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
     counts[0] = (int64_t)total_t;
     counts[1] = (int64_t)n_points;
   }
-  if (total_v > 0x7fffffffull || 3ull * total_t > 0x7fffffffull) return;
-  if ((int64_t)total_t > cap_tris || (int64_t)n_points > cap_points) return;
-  for (int64_t b = blockIdx.x; b < ntiles; b += gridDim.x) {
-    const TileRef tr = tiles[xcd ? xcd_tile(b, ntiles) : b];
-    const VolGeom g = vols[tr.vol];
-    const int64_t vbv = base_v[g.word_off], vbt = base_t[g.word_off];
-    generate_tile<kBatchGenTile, kBatchGenThreads, FieldArray, dedup>(
-        g, FieldArray{fields + g.field_off}, bits + g.word_off, base_v + g.word_off,
-        base_t + g.word_off, tr.w0, out, normals, vbv, vbt, s_dyn);
-    __syncthreads();  // LDS reused by the next tile
+  // too many ids for dax::Id or too little room: the bases only
+  const bool emit = total_v <= 0x7fffffffull && 3ull * total_t <= 0x7fffffffull &&
+                    (int64_t)total_t <= cap_tris && (int64_t)n_points <= cap_points;
+  const TileRef tr = tiles[xcd ? xcd_tile_runs(blockIdx.x, ntiles) : (int64_t)blockIdx.x];
+  const VolGeom g = vols[tr.vol];
+  CountSrc cs = all;
+  cs.lpre += g.tile_off * kBatchGenTile;
+  cs.n_ctiles = 2 * ceil_div(g.nwords, (int64_t)kBatchGenTile);
+  cs.ct0 = 2 * g.tile_off;
+  cs.base_v += g.word_off;
+  cs.base_t += g.word_off;
+  const unsigned long long vol = ctile_prefix(cs, 0);
+  const int64_t vbv = (int64_t)(uint32_t)vol, vbt = (int64_t)(vol >> 32);
+  if (tr.w0 == 0 && threadIdx.x == 0) {
+    vol_first[tr.vol] = (uint32_t)vbv;
+    if (vol_offsets) {
+      vol_offsets[2 * tr.vol + 0] = vbt;
+      vol_offsets[2 * tr.vol + 1] = dedup ? vbv : 3 * vbt;
+    }
   }
-}
-
-// Per-volume {first triangle, first point} in the concatenated outputs.
-__global__ void k_batch_offsets(const VolGeom* __restrict__ vols, int64_t nvols,
-                                const uint32_t* __restrict__ base_v,
-                                const uint32_t* __restrict__ base_t, unsigned flags,
-                                int64_t* __restrict__ vol_offsets) {
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nvols) return;
-  const int64_t w = vols[v].word_off;
-  const bool dedup = (flags & DAX_HIP_MC_DEDUP) != 0;
-  vol_offsets[2 * v + 0] = base_t[w];
-  vol_offsets[2 * v + 1] = dedup ? (int64_t)base_v[w] : 3 * (int64_t)base_t[w];
+  generate_tile<kBatchGenTile, kBatchGenThreads, FieldArray, dedup>(
+      g, FieldArray{fields + g.field_off}, bits + g.word_off, tr.w0, out, normals, vbv, vbt, s_dyn,
+      cs, emit, false);
 }
 
 // ---- batched adjoint --------------------------------------------------------
-// Same tile table as generate: a block takes a tile of row words, first the
-// adjoint records of the tile's vertices (global ids base_v[w0] ..
-// base_v[w_end]), then, in a second launch (a block per tile), dL/dfield of
-// the tile's points; tiles whose endpoint records do not fit are listed and
-// redone as spans by a third launch.
+// The adjoint records of all vertices, then, in a second launch (a block per
+// tile of generate's table), dL/dfield of the tile's points; tiles whose
+// endpoint records do not fit are listed and redone as spans by a third launch.
+// A thread per vertex; its volume by binary search over the volumes' first
+// vertices, then the wave takes its volumes one at a time (one, as a rule),
+// so that the geometry stays in scalar registers.  A block per tile of words
+// instead leaves most lanes idle (73 vertices per tile in 256 volumes of
+// 32..160 points an axis: 80 us; this: 58).
 __global__ __launch_bounds__(256) void k_batch_vertex_adjoint(
-    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
-    const float* __restrict__ fields, const uint32_t* __restrict__ base_v,
-    const uint32_t* __restrict__ edges, const float* __restrict__ dldx,
-    const float* __restrict__ dldn, const int64_t* __restrict__ counts, int64_t n_points,
-    VertexAdj* __restrict__ out, uint32_t* __restrict__ list) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) list[0] = 0u;
+    const VolGeom* __restrict__ vols, int64_t nvols, const uint32_t* __restrict__ vol_first,
+    const float* __restrict__ fields, const uint32_t* __restrict__ edges,
+    const float* __restrict__ dldx, const float* __restrict__ dldn,
+    const int64_t* __restrict__ counts, int64_t n_points, VertexAdj* __restrict__ out,
+    uint32_t* __restrict__ list) {
+  const int64_t u = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (u == 0) list[0] = 0u;
   const int64_t U = counts ? min(counts[1], n_points) : n_points;
-  for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const TileRef tr = tiles[t];
-    const VolGeom g = vols[tr.vol];
-    const int64_t w_end = min((int64_t)tr.w0 + kBatchGenTile, g.nwords);
-    const int64_t u0 = base_v[g.word_off + tr.w0];
-    const int64_t u1 = min((int64_t)base_v[g.word_off + w_end], U);
-    for (int64_t u = u0 + threadIdx.x; u < u1; u += blockDim.x)
-      vertex_adjoint(g, fields, edges, dldx, dldn, u, out);
+  int64_t vol = -1;
+  if (u < U) {  // the last volume whose first vertex is at most u
+    int64_t lo = 0, hi = nvols;
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) >> 1;
+      if ((int64_t)vol_first[mid] <= u)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    vol = lo;
+  }
+  uint64_t todo = __ballot(vol >= 0);
+  while (todo) {
+    const int v = __builtin_amdgcn_readlane((int)vol, __builtin_ctzll(todo));
+    const bool mine = (int)vol == v;
+    if (mine) vertex_adjoint(vols[v], fields, edges, dldx, dldn, u, out);
+    todo &= ~__ballot(mine);
   }
 }
 
@@ -292,77 +335,94 @@ std::tuple<int64_t, int, int64_t> batch_class(const BatchHeader& h) {
 // Device pointers of a prepared workspace.
 struct BatchPtrs {
   const VolGeom* vols;
-  const TileRef* scan_tiles;
   const TileRef* gen_tiles;
   uint64_t* bits;
   uint32_t* bv;
   uint32_t* bt;
-  unsigned long long* status;
+  uint32_t* vol_first;
+  uint32_t* lpre;
+  unsigned long long* tloc;
+  unsigned long long* bsum;
+  unsigned long long* bpre;
   Ctrl* ctrl;
 };
 
 BatchPtrs batch_ptrs(const BatchHeader& h, void* d_workspace) {
   char* body = (char*)d_workspace + kBatchHeaderBytes;
-  return BatchPtrs{(const VolGeom*)(body + h.off_vols), (const TileRef*)(body + h.off_scan_tiles),
-                   (const TileRef*)(body + h.off_gen_tiles), (uint64_t*)(body + h.off_bits),
-                   (uint32_t*)(body + h.off_base_v), (uint32_t*)(body + h.off_base_t),
-                   (unsigned long long*)(body + h.off_status), (Ctrl*)(body + h.off_ctrl)};
+  return BatchPtrs{(const VolGeom*)(body + h.off_vols),
+                   (const TileRef*)(body + h.off_gen_tiles),
+                   (uint64_t*)(body + h.off_bits),
+                   (uint32_t*)(body + h.off_base_v),
+                   (uint32_t*)(body + h.off_base_t),
+                   (uint32_t*)(body + h.off_vol_first),
+                   (uint32_t*)(body + h.off_lpre),
+                   (unsigned long long*)(body + h.off_tloc),
+                   (unsigned long long*)(body + h.off_bsum),
+                   (unsigned long long*)(body + h.off_bpre),
+                   (Ctrl*)(body + h.off_ctrl)};
 }
 
-// Classify (which also clears the scan's status and control words).
 int batch_classify(const BatchHeader& h, const BatchPtrs& p, const float* d_fields,
                    const BatchTuning& t, hipStream_t s) {
-  const int64_t zero_words = h.nscan + (int64_t)(sizeof(Ctrl) / 8);
   const dim3 grid((unsigned)persistent_blocks(t.cls_blocks)), blk(256);
   switch (t.cls_unroll) {
     case 8:
-      k_batch_classify<4><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
-                                               p.status, zero_words);
+      k_batch_classify<4><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits);
       break;
     case 32:
-      k_batch_classify<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
-                                                p.status, zero_words);
+      k_batch_classify<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits);
       break;
     default:
-      k_batch_classify<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits,
-                                                p.status, zero_words);
+      k_batch_classify<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, d_fields, p.bits);
   }
   DAXHIP_LAUNCH_CHECK("k_batch_classify");
   return DAX_HIP_OK;
 }
 
+// log2 of the count tiles per count block.
+int batch_count_shift(const BatchTuning& t) {
+  return t.scan_threads == 1024 ? 5 : (t.scan_threads == 512 ? 4 : 3);
+}
+
 int batch_scan(const BatchHeader& h, const BatchPtrs& p, const BatchTuning& t, hipStream_t s) {
-  const dim3 grid((unsigned)std::min<int64_t>(persistent_blocks(4), h.nscan));
-  switch (t.scan_threads) {
-    case 512:
-      k_batch_count_scan<512><<<grid, dim3(512), 0, s>>>(p.vols, p.scan_tiles, h.nscan, p.bits,
-                                                         p.bv, p.bt, p.status, p.ctrl);
+  const int waves = t.scan_threads / 64;
+  const int64_t blocks = ceil_div(h.ngen, (int64_t)waves);
+  const dim3 grid((unsigned)blocks), blk((unsigned)t.scan_threads);
+  switch (waves) {
+    case 8:
+      k_batch_count<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
+                                            p.bsum);
       break;
-    case 1024:
-      k_batch_count_scan<1024><<<grid, dim3(1024), 0, s>>>(p.vols, p.scan_tiles, h.nscan, p.bits,
-                                                           p.bv, p.bt, p.status, p.ctrl);
+    case 16:
+      k_batch_count<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
+                                             p.bsum);
       break;
     default:
-      k_batch_count_scan<256><<<grid, dim3(256), 0, s>>>(p.vols, p.scan_tiles, h.nscan, p.bits,
-                                                         p.bv, p.bt, p.status, p.ctrl);
+      k_batch_count<4><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
+                                            p.bsum);
   }
-  DAXHIP_LAUNCH_CHECK("k_batch_count_scan");
+  DAXHIP_LAUNCH_CHECK("k_batch_count");
+  k_batch_scan<<<1, dim3(kTsumThreads), 0, s>>>(p.bsum, p.bpre, blocks, p.tloc, 2 * h.ngen, p.ctrl,
+                                                batch_count_shift(t));
+  DAXHIP_LAUNCH_CHECK("k_batch_scan");
   return DAX_HIP_OK;
 }
 
 int batch_generate(const BatchHeader& h, const BatchPtrs& p, const float* d_fields,
                    unsigned flags, const OutPtrs& o, int64_t cap_points, int64_t cap_tris,
-                   int64_t* d_counts, const BatchTuning& t, hipStream_t s) {
+                   int64_t* d_counts, int64_t* d_vol_offsets, const BatchTuning& t,
+                   hipStream_t s) {
+  const CountSrc cs{p.lpre, p.tloc, p.bpre, 0, 0, batch_count_shift(t), p.bv, p.bt};
   const size_t lds = GenLayout<kBatchGenTile, kBatchGenThreads>((int)h.max_wpr).bytes();
-  const dim3 grid((unsigned)std::min<int64_t>(persistent_blocks(t.gen_blocks), h.ngen));
+  const dim3 grid((unsigned)h.ngen);
   if (flags & DAX_HIP_MC_DEDUP)
     k_batch_generate<true><<<grid, dim3(kBatchGenThreads), lds, s>>>(
-        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, p.bv, p.bt, p.ctrl, o, flags, cap_points,
-        cap_tris, d_counts, t.gen_xcd);
+        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points, cap_tris,
+        d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
   else
     k_batch_generate<false><<<grid, dim3(kBatchGenThreads), lds, s>>>(
-        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, p.bv, p.bt, p.ctrl, o, flags, cap_points,
-        cap_tris, d_counts, t.gen_xcd);
+        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points, cap_tris,
+        d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
   DAXHIP_LAUNCH_CHECK("k_batch_generate");
   return DAX_HIP_OK;
 }
@@ -392,8 +452,7 @@ int dax_hip_mc_batch_prepare(int64_t n_volumes, const int64_t* h_dims3,
     return DAX_HIP_BAD_VALUE;
   }
   std::vector<VolGeom> vols((size_t)n_volumes);
-  std::vector<TileRef> scan_tiles, gen_tiles;
-  scan_tiles.reserve((size_t)L.nscan);
+  std::vector<TileRef> gen_tiles;
   gen_tiles.reserve((size_t)L.ngen);
   int64_t word_off = 0;
   for (int64_t v = 0; v < n_volumes; ++v) {
@@ -417,7 +476,7 @@ int dax_hip_mc_batch_prepare(int64_t n_volumes, const int64_t* h_dims3,
     g.word_off = word_off;
     g.nwords = (int64_t)g.wpr * ny * nz;
     set_geom_divs(g);
-    for (int64_t w = 0; w < g.nwords; w += kBatchScanTile) scan_tiles.push_back({(int32_t)v, (int32_t)w});
+    g.tile_off = (int64_t)gen_tiles.size();
     for (int64_t w = 0; w < g.nwords; w += kBatchGenTile) gen_tiles.push_back({(int32_t)v, (int32_t)w});
     word_off += g.nwords;
   }
@@ -425,17 +484,19 @@ int dax_hip_mc_batch_prepare(int64_t n_volumes, const int64_t* h_dims3,
   h.magic = kBatchMagic;
   h.nvols = n_volumes;
   h.nwords = L.nwords;
-  h.nscan = L.nscan;
   h.ngen = L.ngen;
   h.max_wpr = 1;
   for (const VolGeom& g : vols) h.max_wpr = std::max<int64_t>(h.max_wpr, g.wpr);
   h.off_vols = L.off_vols;
-  h.off_scan_tiles = L.off_scan_tiles;
   h.off_gen_tiles = L.off_gen_tiles;
   h.off_bits = L.off_bits;
   h.off_base_v = L.off_base_v;
   h.off_base_t = L.off_base_t;
-  h.off_status = L.off_status;
+  h.off_vol_first = L.off_vol_first;
+  h.off_lpre = L.off_lpre;
+  h.off_tloc = L.off_tloc;
+  h.off_bsum = L.off_bsum;
+  h.off_bpre = L.off_bpre;
   h.off_ctrl = L.off_ctrl;
   h.bytes = L.bytes;
   h.tune = kBatchTuningDefault;
@@ -450,8 +511,6 @@ int dax_hip_mc_batch_prepare(int64_t n_volumes, const int64_t* h_dims3,
   DAXHIP_CHECK(hipMemcpyAsync(ws, &h, sizeof(h), hipMemcpyHostToDevice, s));
   DAXHIP_CHECK(hipMemcpyAsync(body + L.off_vols, vols.data(), vols.size() * sizeof(VolGeom),
                               hipMemcpyHostToDevice, s));
-  DAXHIP_CHECK(hipMemcpyAsync(body + L.off_scan_tiles, scan_tiles.data(),
-                              scan_tiles.size() * sizeof(TileRef), hipMemcpyHostToDevice, s));
   DAXHIP_CHECK(hipMemcpyAsync(body + L.off_gen_tiles, gen_tiles.data(),
                               gen_tiles.size() * sizeof(TileRef), hipMemcpyHostToDevice, s));
   DAXHIP_CHECK(hipStreamSynchronize(s));
@@ -461,7 +520,7 @@ int dax_hip_mc_batch_prepare(int64_t n_volumes, const int64_t* h_dims3,
 
 size_t dax_hip_mc_batch_header_bytes(void) { return sizeof(BatchHeader); }
 
-// The batch forward: four persistent launches, graph-capturable.  h_header is
+// The batch forward: four launches, graph-capturable.  h_header is
 // the header returned by prepare.  d_counts {T, U} totals; d_vol_offsets
 // [n][2] {first triangle, first point} of each volume.
 int dax_hip_mc_batch_forward(const float* d_fields, const void* h_header, void* d_workspace,
@@ -490,18 +549,12 @@ int dax_hip_mc_batch_forward(const float* d_fields, const void* h_header, void* 
   if ((rc = batch_classify(*h, p, d_fields, t, s))) return rc;
   if ((rc = batch_scan(*h, p, t, s))) return rc;
   OutPtrs o{d_vertices, d_normals, d_conn, d_edges, nullptr, nullptr, nullptr};
-  if ((rc = batch_generate(*h, p, d_fields, flags, o, cap_points, cap_tris, d_counts, t, s)))
-    return rc;
-  if (d_vol_offsets) {
-    k_batch_offsets<<<dim3((unsigned)ceil_div(h->nvols, 256)), dim3(256), 0, s>>>(
-        p.vols, h->nvols, p.bv, p.bt, flags, d_vol_offsets);
-    DAXHIP_LAUNCH_CHECK("k_batch_offsets");
-  }
-  return DAX_HIP_OK;
+  return batch_generate(*h, p, d_fields, flags, o, cap_points, cap_tris, d_counts, d_vol_offsets, t,
+                        s);
 }
 
 // Launch shapes of a prepared batch: {classify unroll, classify blocks per
-// CU, scan threads per tile, generate blocks per CU, generate XCD order}.
+// CU, threads per count block, generate blocks per CU, generate XCD order}.
 int dax_hip_mc_batch_set_tuning(void* h_header, const int* h_params5) {
   BatchHeader* h = (BatchHeader*)h_header;
   if (!h || h->magic != kBatchMagic || !h_params5) {
@@ -583,7 +636,7 @@ int dax_hip_mc_batch_autotune(const float* d_fields, void* h_header, void* d_wor
         best.cls_blocks = bpc;
       }
     }
-  // scan: each timed launch follows a classify that resets its state
+  // scan: each timed launch follows a classify, as in the forward
   for (int nt : {256, 512, 1024}) {
     BatchTuning t = best;
     t.scan_threads = nt;
@@ -603,22 +656,21 @@ int dax_hip_mc_batch_autotune(const float* d_fields, void* h_header, void* d_wor
   // generate over one classify + scan
   if ((rc = batch_classify(*h, p, d_fields, best, s))) goto done;
   if ((rc = batch_scan(*h, p, best, s))) goto done;
-  for (int bpc : {2, 4, 8})
-    for (int xcd : {0, 1}) {
+  for (int xcd : {0, 1}) {
       BatchTuning t = best;
-      t.gen_blocks = bpc;
       t.gen_xcd = xcd;
-      if ((rc = batch_generate(*h, p, d_fields, flags, o, cap_points, cap_tris, d_counts, t, s)))
+      if ((rc = batch_generate(*h, p, d_fields, flags, o, cap_points, cap_tris, d_counts, nullptr, t,
+                               s)))
         goto done;
       (void)hipEventRecord(e0, s);
       for (int r = 0; r < reps; ++r)
-        if ((rc = batch_generate(*h, p, d_fields, flags, o, cap_points, cap_tris, d_counts, t, s)))
+        if ((rc = batch_generate(*h, p, d_fields, flags, o, cap_points, cap_tris, d_counts, nullptr, t,
+                               s)))
           goto done;
       (void)hipEventRecord(e1, s);
       const float ms = elapsed() / reps;
       if (ms < best_ms[2]) {
         best_ms[2] = ms;
-        best.gen_blocks = bpc;
         best.gen_xcd = xcd;
       }
     }
@@ -682,15 +734,13 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
   const TileRef* gen_tiles = (const TileRef*)(body + h->off_gen_tiles);
   const uint64_t* bits = (const uint64_t*)(body + h->off_bits);
   const uint32_t* bv = (const uint32_t*)(body + h->off_base_v);
-  const int grid = (int)std::min<int64_t>(persistent_blocks(4), h->ngen);
   uint32_t* list =
       n_points > 0 ? (uint32_t*)((char*)d_scratch + gather_list_offset(n_points)) : nullptr;
   const size_t lds = gather_lds_bytes((int)h->max_wpr);
   if (n_points > 0) {
-    k_batch_vertex_adjoint<<<dim3(grid), dim3(256), 0, s>>>(vols, gen_tiles, h->ngen, d_fields,
-                                                            bv, d_edges, d_dl_dvertices,
-                                                            d_dl_dnormals, d_counts, n_points,
-                                                            (VertexAdj*)d_scratch, list);
+    k_batch_vertex_adjoint<<<dim3((unsigned)ceil_div(n_points, 256)), dim3(256), 0, s>>>(
+        vols, h->nvols, (const uint32_t*)(body + h->off_vol_first), d_fields, d_edges,
+        d_dl_dvertices, d_dl_dnormals, d_counts, n_points, (VertexAdj*)d_scratch, list);
     DAXHIP_LAUNCH_CHECK("k_batch_vertex_adjoint");
   }
   k_batch_point_gather<<<dim3((unsigned)h->ngen), dim3(kGatherThreads), lds, s>>>(

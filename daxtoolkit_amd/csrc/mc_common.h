@@ -21,10 +21,8 @@
 namespace daxhip {
 namespace mc {
 
-constexpr int kTileWords = 1024;     // row words per scan tile
+constexpr int kTileWords = 1024;     // the workspace's word arrays are padded to this
 constexpr int kCountTile = 128;      // row words per count tile: its prefixes fit 16 bits
-constexpr int kScanThreads = 256;    // threads of the count/scan and generate blocks
-constexpr int kWordsPerThread = kTileWords / kScanThreads;
 constexpr int kMaxWpr = 256;         // nx <= 16384
 constexpr int kGatherTileWords = 256;  // row words per tile of the adjoint's gather
 
@@ -58,6 +56,7 @@ struct VolGeom {
   int64_t field_off;  // first field element of the volume
   int64_t word_off;   // first row word of the volume
   int64_t nwords;     // wpr*ny*nz
+  int64_t tile_off;   // first 256-word tile of the volume in its batch (0 alone)
   FastDiv div_wpr, div_ny, div_nx;
   // Spacings that are powers of two (bit d): then x / (2h) == x * (rcp_h/2)
   // and x / h == x * rcp_h exactly in IEEE arithmetic.
@@ -249,20 +248,9 @@ __device__ __forceinline__ void edge_select(uint64_t fx, uint64_t fy, uint64_t f
   axis = r < bx ? 0 : (r < bx + by ? 1 : 2);
 }
 
-// Decoupled look-back tile status: flag in bits 62-63 (0 = not ready,
-// 1 = aggregate, 2 = inclusive prefix), triangle count in bits 31-61, vertex
-// count in bits 0-30.  Totals above 2^31-1 overflow dax::Id anyway; the
-// 64-bit totals accumulated beside the scan detect that case.
-constexpr uint64_t kStatusAgg = 1ull;
-constexpr uint64_t kStatusPrefix = 2ull;
-
-__device__ __forceinline__ uint64_t pack_status(uint32_t v, uint32_t t, uint64_t flag) {
-  return (flag << 62) | ((uint64_t)(t & 0x7fffffffu) << 31) | (uint64_t)(v & 0x7fffffffu);
-}
-
 // Control block at the end of the workspace.
 struct Ctrl {
-  uint32_t tile_counter;
+  uint32_t pad;
   uint32_t tpb_shift;  // log2 of the count tiles per count block of the last scan
   unsigned long long total_v;  // 64-bit totals: vertices (active edges), triangles
   unsigned long long total_t;
@@ -280,7 +268,7 @@ struct Ctrl {
 // (0: none), then the generate tiles in dispatch order; off_gorder: the
 // same for the adjoint's gather tiles.
 struct Workspace {
-  size_t off_bits, off_base_v, off_base_t, off_status, off_ctrl, off_counts, off_tsum, off_bsum,
+  size_t off_bits, off_base_v, off_base_t, off_ctrl, off_counts, off_tsum, off_bsum,
       off_tpre, off_gcls, off_tcls, off_order, off_gorder, bytes;
   int64_t nwords, ntiles, n_ctiles;
 };
@@ -296,8 +284,6 @@ inline Workspace workspace_layout(int64_t nwords) {
   off = align_up(off + (size_t)(nwords + 1) * 4, 256);
   w.off_base_t = off;
   off = align_up(off + (size_t)(nwords + 1) * 4, 256);
-  w.off_status = off;  // status then ctrl: one contiguous block zeroed per run
-  off = off + (size_t)w.ntiles * 8;
   w.off_ctrl = off;
   off = align_up(off + sizeof(Ctrl), 256);
   w.off_counts = off;  // packed per-word counts

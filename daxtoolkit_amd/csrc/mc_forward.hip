@@ -29,17 +29,13 @@
 namespace daxhip {
 namespace mc {
 
-// Classify row words [w_lo, w_hi) (w_lo a multiple of 4 for the float4 form)
-// and clear zero_words words of count/scan state.
+// Classify the volume's row words.
 template <int UNROLL>
 __global__ __launch_bounds__(256) void k_classify(VolGeom g, const float* __restrict__ field,
                                                   uint64_t* __restrict__ bits,
-                                                  unsigned long long* __restrict__ zero_buf,
-                                                  int64_t zero_words, int64_t w_lo, int64_t w_hi) {
+                                                  int64_t nwords) {
   const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gtid < zero_words) zero_buf[gtid] = 0ull;
-  const int64_t w0 = w_lo + (gtid >> 6) * UNROLL;
-  classify_words<UNROLL>(g, field + g.field_off, bits + g.word_off, w0, w_hi);
+  classify_words<UNROLL>(g, field + g.field_off, bits + g.word_off, (gtid >> 6) * UNROLL, nwords);
 }
 
 // Rows that are not whole 64-point words, or a field that is not 16-byte
@@ -47,29 +43,21 @@ __global__ __launch_bounds__(256) void k_classify(VolGeom g, const float* __rest
 template <int TW>
 __global__ __launch_bounds__(256) void k_classify_flat(VolGeom g, const float* __restrict__ field,
                                                        uint64_t* __restrict__ bits,
-                                                       unsigned long long* __restrict__ zero_buf,
-                                                       int64_t zero_words, int64_t w_lo,
-                                                       int64_t w_hi) {
+                                                       int64_t nwords) {
   __shared__ FlatLds<TW> sh;
-  const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gtid < zero_words) zero_buf[gtid] = 0ull;
-  const int64_t w0 = w_lo + (int64_t)blockIdx.x * TW;
-  if (w0 >= w_hi) return;  // a block that only clears
+  const int64_t w0 = (int64_t)blockIdx.x * TW;
   classify_flat<TW, kFlatLoads>(flat_rows(g), field + g.field_off, bits + g.word_off,
-                                (uint32_t)w0, (uint32_t)min(w0 + TW, w_hi), sh,
+                                (uint32_t)w0, (uint32_t)min(w0 + TW, nwords), sh,
                                 [&](float v) { return v > g.iso; });
 }
 
 template <int UNROLL>
 __global__ __launch_bounds__(256) void k_classify_v4(VolGeom g, const float* __restrict__ field,
                                                      uint64_t* __restrict__ bits,
-                                                     unsigned long long* __restrict__ zero_buf,
-                                                     int64_t zero_words, int64_t w_lo,
-                                                     int64_t w_hi) {
+                                                     int64_t nwords) {
   const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gtid < zero_words) zero_buf[gtid] = 0ull;
-  const int64_t c0 = w_lo / 4 + (gtid >> 6) * UNROLL;
-  classify_chunks_v4<UNROLL>(g, field + g.field_off, bits + g.word_off, c0, w_hi);
+  classify_chunks_v4<UNROLL>(g, field + g.field_off, bits + g.word_off, (gtid >> 6) * UNROLL,
+                             nwords);
 }
 
 // ---- count and scan --------------------------------------------------------
@@ -119,7 +107,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_count(VolGeom g, const uint64_t*
     unsigned long long run = 0ull;
     for (int i = 0; i < kBlockTiles; ++i) {
       const int64_t tile = blk * kBlockTiles + i;
-      if (tile < n_ctiles) tloc[tile] = run;
+      if (tile <= n_ctiles) tloc[tile] = run;  // the entry after the last: the totals
       run = add_vt(run, s_ts[i]);
     }
     bsum[blk] = run;
@@ -179,30 +167,27 @@ struct ScanOut {
   int64_t* host;
 };
 
-constexpr int kTsumThreads = 1024;
-constexpr int kTsumWaves = kTsumThreads / 64;
 constexpr uint32_t kOrderStage = 16384;  // 64 KiB of LDS
-constexpr int kTsumPerThread = 4;        // block sums per thread and round
 
-// One block scans the n count-block sums (v | t << 32, each below 2^32)
-// 4096 at a time: four consecutive sums per thread, wave scans of the
-// thread totals' halves, the block's wave sums in 64 bits, 64-bit carries
-// between rounds.  The same block then
-// writes the two dispatch orders.
+// One block scans the count blocks' sums (scan_block_sums), completes the tile
+// prefixes and writes the two dispatch orders.
 // LARGE: some thread's chunk exceeds kOrderRegTiles tiles (a separate
 // instance, so the common one stays small).
 template <bool LARGE>
 __global__ __launch_bounds__(kTsumThreads) void k_scan_tsums(const unsigned long long* __restrict__ bsum,
                                                              unsigned long long* __restrict__ bpre,
-                                                             int64_t n, Ctrl* __restrict__ ctrl,
+                                                             int64_t n,
+                                                             unsigned long long* __restrict__ tloc,
+                                                             int64_t n_ctiles,
+                                                             Ctrl* __restrict__ ctrl,
                                                              GenOrder go, int tpb_shift,
                                                              ScanOut so) {
-  constexpr int kWaves = kTsumWaves;
+  constexpr int kWaves = kTsumThreads / 64;
   // the scan's wave sums, then the dispatch order's LDS window
   __shared__ uint32_t s_stage[kOrderStage];
   uint32_t* s_v = s_stage;
   uint32_t* s_t = s_stage + kWaves;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x;
   const uint32_t ng = (uint32_t)ceil_div(go.nwords, (int64_t)go.tw);
   const uint32_t Kg = order_chunk(ng, kTsumThreads);
   const bool ordered = go.gen_classes;  // uniform
@@ -213,51 +198,11 @@ __global__ __launch_bounds__(kTsumThreads) void k_scan_tsums(const unsigned long
       units ? load_unit_classes(go.gcls, Ku, nunits, go.unit_sp)
             : (ordered ? load_classes(go.gcls, (uint32_t)tid * Kg, Kg, ng) : 0ull);
 
-  unsigned long long cv = 0, ct = 0;  // 64-bit carries
-  constexpr int kPer = kTsumPerThread;
-  for (int64_t e0 = 0; e0 < n; e0 += kPer * kTsumThreads) {
-    const int64_t e = e0 + (int64_t)kPer * tid;  // the thread's kPer consecutive sums
-    uint32_t v[kPer], t[kPer], sv = 0u, st = 0u;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const unsigned long long x = e + i < n ? bsum[e + i] : 0ull;
-      v[i] = (uint32_t)x;
-      t[i] = (uint32_t)(x >> 32);
-      sv += v[i];
-      st += t[i];
-    }
-    // a round's sums stay below 2^32 only for the wave partials (a count
-    // block holds at most 3 * 2^17 vertices); the cross-wave totals are
-    // formed in 64 bits
-    const uint32_t iv = wave_incl_scan(sv), it = wave_incl_scan(st);
-    if (lane == 63) {
-      s_v[wv] = iv;
-      s_t[wv] = it;
-    }
-    __syncthreads();
-    unsigned long long ov = 0, ot = 0, rv = 0, rt = 0;
-#pragma unroll
-    for (int q = 0; q < kWaves; ++q) {
-      if (q < wv) {
-        ov += s_v[q];
-        ot += s_t[q];
-      }
-      rv += s_v[q];
-      rt += s_t[q];
-    }
-    __syncthreads();
-    unsigned long long pv = cv + ov + iv - sv, pt = ct + ot + it - st;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      if (e + i < n) bpre[e + i] = (pv & 0xffffffffull) | (pt << 32);
-      pv += v[i];
-      pt += t[i];
-    }
-    cv += rv;
-    ct += rt;
-  }
+  unsigned long long cv, ct;
+  scan_block_sums(bsum, bpre, n, s_v, s_t, cv, ct);
   if (tid == 0) {
-    bpre[n] = (cv & 0xffffffffull) | (ct << 32);
+    // the count blocks wrote it unless the last one is full
+    if ((n_ctiles & ((1 << tpb_shift) - 1)) == 0) tloc[n_ctiles] = 0ull;
     ctrl->total_v = cv;
     ctrl->total_t = ct;
     ctrl->tpb_shift = (uint32_t)tpb_shift;
@@ -324,9 +269,8 @@ __global__ __launch_bounds__(NT, 4) void k_generate(
   const int64_t tile =
       ordered ? (int64_t)(ord & ~kOrderHasOutput)
               : tile_lo + (xcd_order ? xcd_tile(blockIdx.x, ntiles) : (int64_t)blockIdx.x);
-  generate_tile<TW, NT, Src, dedup, true>(g, field, bits + g.word_off, nullptr, nullptr, tile * TW,
-                                          out, normals, 0, 0, s_dyn, cs, emit,
-                                          ordered && (ord & kOrderHasOutput) != 0u);
+  generate_tile<TW, NT, Src, dedup>(g, field, bits + g.word_off, tile * TW, out, normals, 0, 0,
+                                    s_dyn, cs, emit, ordered && (ord & kOrderHasOutput) != 0u);
 }
 
 // Slice classify: a thread per row word.  Along a row the plane value
@@ -338,13 +282,10 @@ __global__ __launch_bounds__(NT, 4) void k_generate(
 // halving steps, each evaluating one point with exactly the operations
 // FieldPlane uses, find the change.  Bound by the words' stores (512^3: 16.8
 // MB); a wave per 8 rows with a 64-way search per row took 37 us there, this
-// takes 11.  The same launch clears the count/scan state.
+// takes 11.
 __global__ __launch_bounds__(256) void k_classify_plane(VolGeom g, FieldPlane pl,
-                                                        uint64_t* __restrict__ bits,
-                                                        unsigned long long* __restrict__ zero_buf,
-                                                        int64_t zero_words) {
+                                                        uint64_t* __restrict__ bits) {
   const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (w < zero_words) zero_buf[w] = 0ull;
   if (w >= g.nwords) return;
   const uint32_t row = fast_div((uint32_t)w, g.div_wpr);
   const uint32_t k = fast_div(row, g.div_ny), j = row - k * (uint32_t)g.ny;
@@ -602,6 +543,7 @@ int make_geom(int64_t nx, int64_t ny, int64_t nz, const float* origin, const flo
   g.field_off = 0;
   g.word_off = 0;
   g.nwords = (int64_t)g.wpr * ny * nz;
+  g.tile_off = 0;
   set_geom_divs(g);
   return DAX_HIP_OK;
 }
@@ -639,41 +581,29 @@ int check_ws(const VolGeom& g, size_t ws_bytes, Workspace& L, void* ws) {
   return DAX_HIP_OK;
 }
 
-// Classify row words [w_lo, w_hi) (all when w_hi < 0); `zero` also clears
-// the count/scan state.
+// Classify the whole volume.
 int launch_bits(const VolGeom& g, const float* field, char* ws, const Workspace& L,
-                const Tuning& tu, hipStream_t s, int64_t w_lo = 0, int64_t w_hi = -1,
-                bool zero = true) {
-  if (w_hi < 0) w_hi = g.nwords;
+                const Tuning& tu, hipStream_t s) {
   uint64_t* bits = (uint64_t*)(ws + L.off_bits);
-  unsigned long long* status = (unsigned long long*)(ws + L.off_status);
-  const int64_t zero_words = zero ? L.ntiles + (int64_t)(sizeof(Ctrl) / 8) : 0;
-  const bool aligned = (g.nx % 64) == 0 && (g.field_off % 4) == 0 &&
-                       ((uintptr_t)field % 16) == 0 && (w_lo % 4) == 0;
+  const bool aligned = (g.nx % 64) == 0 && (g.field_off % 4) == 0 && ((uintptr_t)field % 16) == 0;
   if (!aligned) {
     // 8192 points, 8 float4 loads per thread, for rows of full or half words;
     // shorter rows hold fewer points per word, so four times the words
     const int tw = g.nx > 32 ? 128 : 512;
-    const int64_t blocks = std::max<int64_t>(
-        std::max(ceil_div(w_hi - w_lo, tw), ceil_div(zero_words, 256)), 1);
-    const dim3 grid((unsigned)blocks), block(256);
+    const dim3 grid((unsigned)ceil_div(g.nwords, tw)), block(256);
     if (tw == 128)
-      k_classify_flat<128><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi);
+      k_classify_flat<128><<<grid, block, 0, s>>>(g, field, bits, g.nwords);
     else
-      k_classify_flat<512><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi);
+      k_classify_flat<512><<<grid, block, 0, s>>>(g, field, bits, g.nwords);
     DAXHIP_LAUNCH_CHECK("k_classify_flat");
     return DAX_HIP_OK;
   }
   const int vec = tu.cls_vec, unroll = tu.cls_unroll;
-  const int64_t units = vec == 4 ? ceil_div(w_hi - w_lo, 4) : w_hi - w_lo;  // chunks or words
+  const int64_t units = vec == 4 ? ceil_div(g.nwords, 4) : g.nwords;  // chunks or words
   const int64_t waves = ceil_div(units, unroll);
-  int64_t blocks = std::max<int64_t>(ceil_div(waves * 64, 256), ceil_div(zero_words, 256));
-  blocks = std::max<int64_t>(blocks, 1);
-  const dim3 grid((unsigned)blocks), block(256);
-#define DAXHIP_CLS(U) \
-  k_classify<U><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi)
-#define DAXHIP_CLS4(U) \
-  k_classify_v4<U><<<grid, block, 0, s>>>(g, field, bits, status, zero_words, w_lo, w_hi)
+  const dim3 grid((unsigned)ceil_div(waves * 64, 256)), block(256);
+#define DAXHIP_CLS(U) k_classify<U><<<grid, block, 0, s>>>(g, field, bits, g.nwords)
+#define DAXHIP_CLS4(U) k_classify_v4<U><<<grid, block, 0, s>>>(g, field, bits, g.nwords)
   if (vec == 4) {
     if (unroll == 2) DAXHIP_CLS4(2);
     else if (unroll == 4) DAXHIP_CLS4(4);
@@ -708,7 +638,7 @@ CountSrc count_src(const char* ws, const Workspace& L) {
   char* wsm = const_cast<char*>(ws);
   return CountSrc{(const uint32_t*)(ws + L.off_counts),
                   (const unsigned long long*)(ws + L.off_tsum),
-                  (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0,
+                  (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0, 0,
                   (uint32_t*)(wsm + L.off_base_v), (uint32_t*)(wsm + L.off_base_t)};
 }
 
@@ -753,10 +683,10 @@ int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu
                     (uint32_t*)(ws + L.off_order), (uint32_t*)(ws + L.off_gorder)};
   if (ceil_div(ceil_div(g.nwords, (int64_t)tw), (int64_t)kTsumThreads) > kOrderRegTiles)
     k_scan_tsums<true><<<1, dim3(kTsumThreads), 0, s>>>(
-        bsum, bpre, nblocks, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
+        bsum, bpre, nblocks, tloc, n, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
   else
     k_scan_tsums<false><<<1, dim3(kTsumThreads), 0, s>>>(
-        bsum, bpre, nblocks, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
+        bsum, bpre, nblocks, tloc, n, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
   DAXHIP_LAUNCH_CHECK("k_scan_tsums");
   if (bases) {
     k_bases<<<dim3((unsigned)ceil_div(g.nwords + 1, 256)), dim3(256), 0, s>>>(
@@ -831,13 +761,11 @@ int launch_generate(const VolGeom& g, const float* field, const char* ws, const 
                              cap_tris, counts, tu, s, t_lo, t_hi);
 }
 
-// Slice classify over the whole volume (clears the count/scan state).
+// Slice classify over the whole volume.
 int launch_bits_plane(const VolGeom& g, const FieldPlane& pl, char* ws, const Workspace& L,
                       hipStream_t s) {
-  const int64_t zero_words = L.ntiles + (int64_t)(sizeof(Ctrl) / 8);
-  const int64_t blocks = std::max<int64_t>(ceil_div(std::max(g.nwords, zero_words), 256), 1);
-  k_classify_plane<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(
-      g, pl, (uint64_t*)(ws + L.off_bits), (unsigned long long*)(ws + L.off_status), zero_words);
+  k_classify_plane<<<dim3((unsigned)ceil_div(g.nwords, 256)), dim3(256), 0, s>>>(
+      g, pl, (uint64_t*)(ws + L.off_bits));
   DAXHIP_LAUNCH_CHECK("k_classify_plane");
   return DAX_HIP_OK;
 }
@@ -1010,9 +938,7 @@ int dax_hip_mc_forward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
 // callers that cannot allocate (code under graph capture, serving loops):
 // grids whose workspace fits kNoAllocScratchBytes (48 MiB: up to 512^3
 // points).  Every GPU the library runs on holds the array until the process
-// ends.  The forward clears what it needs cleared (its classify zeroes the
-// scan's status and control words); calls that overlap on one GPU share the
-// array and race.
+// ends.  Calls that overlap on one GPU share the array and race.
 constexpr size_t kNoAllocScratchBytes = (size_t)48 << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -3,8 +3,8 @@
 // (mc_batched.hip).
 //
 //   classify   : field -> inside-bits                         (one pass over f)
-//   count/scan : per-word edge and triangle counts, exclusive scan with
-//                decoupled look-back over scan tiles
+//   count/scan : per-word edge and triangle counts, prefixes within count
+//                tiles and blocks, one block scanning the blocks' sums
 //   generate   : per generate tile, maps of the tile's output vertices and
 //                triangles built in LDS, then one thread per vertex and per
 //                triangle with coalesced writes
@@ -113,15 +113,9 @@ __device__ __forceinline__ void classify_chunks_v4(const VolGeom& g, const float
 }
 
 // ---------------------------------------------------------------------------
-// count/scan.  A scan tile is NT threads x WPT consecutive row words.  Each
-// thread loads its words and their +x/+y/+z neighbour words straight from
-// global memory (L2), counts, and the block scans the per-thread sums; wave 0
-// then runs the decoupled look-back for the tile's global prefix.
-struct ScanShared {
-  uint32_t wave_v[16], wave_t[16];
-  uint32_t prefix[2];
-};
-
+// count/scan: every word's vertices and triangles, prefixes within tiles of
+// kCountTile words, the tiles' within count blocks, and one block scanning the
+// blocks' sums.
 // Active edges (vertices) and triangles of one row word from its eight
 // neighbour words (A = the word, 1 = the next word along x, B = +y row,
 // C = +z plane, D = +y+z).
@@ -135,22 +129,6 @@ __device__ __forceinline__ void word_counts_regs(const VolGeom& g, const WordPos
   CellPlanes cp;
   cell_planes(p, A, A1, B, B1, C, C1, D, D1, cp);
   nt = cp.active ? word_triangles(cp) : 0u;
-}
-
-// Loads the eight neighbour words of row word w (volume-local) and counts it.
-__device__ __forceinline__ void word_counts(const VolGeom& g, const uint64_t* __restrict__ b,
-                                            int64_t w, uint32_t& nv, uint32_t& nt) {
-  const int64_t plane = (int64_t)g.wpr * g.ny;
-  const int wpr = g.wpr;
-  const WordPos p = word_pos(g, w);
-  const bool nx1 = p.q + 1 < wpr;
-  const bool hy = w + wpr < g.nwords, hz = w + plane < g.nwords, hyz = w + plane + wpr < g.nwords;
-  const uint64_t A = b[w], A1 = nx1 ? b[w + 1] : 0ull;
-  const uint64_t B = hy ? b[w + wpr] : 0ull, B1 = (hy && nx1) ? b[w + wpr + 1] : 0ull;
-  const uint64_t C = hz ? b[w + plane] : 0ull, C1 = (hz && nx1) ? b[w + plane + 1] : 0ull;
-  const uint64_t D = hyz ? b[w + plane + wpr] : 0ull;
-  const uint64_t D1 = (hyz && nx1) ? b[w + plane + wpr + 1] : 0ull;
-  word_counts_regs(g, p, A, A1, B, B1, C, C1, D, D1, nv, nt);
 }
 
 // Two count tiles of kCountTile row words, one wave: lane l counts the four
@@ -217,164 +195,20 @@ __device__ __forceinline__ void count_tile_pair(const VolGeom& g, const uint64_t
   }
 }
 
-// Decoupled look-back by wave 0 over the tile states; returns the exclusive
-// prefix of `tile` (vertex, triangle) in sh.prefix.
-__device__ __forceinline__ void look_back(unsigned long long* __restrict__ status, int64_t tile,
-                                          uint32_t agg_v, uint32_t agg_t, Ctrl* __restrict__ ctrl,
-                                          uint32_t* prefix) {
-  const int lane = __lane_id();
-  uint32_t ex_v = 0, ex_t = 0;
-  if (tile == 0) {
-    if (lane == 0)
-      __hip_atomic_store(&status[0], pack_status(agg_v, agg_t, kStatusPrefix), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-  } else {
-    if (lane == 0)
-      __hip_atomic_store(&status[tile], pack_status(agg_v, agg_t, kStatusAgg), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    int64_t pos = tile - 1;
-    while (true) {
-      const int64_t idx = pos - lane;
-      unsigned long long s = pack_status(0, 0, kStatusPrefix);
-      if (idx >= 0) {
-        s = __hip_atomic_load(&status[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        while ((s >> 62) == 0ull) {
-          __builtin_amdgcn_s_sleep(1);
-          s = __hip_atomic_load(&status[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-      const uint64_t pm = __ballot((s >> 62) == kStatusPrefix);
-      uint32_t sv = (uint32_t)(s & 0x7fffffffull), st = (uint32_t)((s >> 31) & 0x7fffffffull);
-      if (pm) {
-        const int first = __builtin_ctzll(pm);
-        if (lane > first) {
-          sv = 0;
-          st = 0;
-        }
-      }
-      ex_v += wave_sum(sv);
-      ex_t += wave_sum(st);
-      if (pm) break;
-      pos -= 64;
-    }
-    if (lane == 0)
-      __hip_atomic_store(&status[tile], pack_status(ex_v + agg_v, ex_t + agg_t, kStatusPrefix),
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (lane == 0) {
-    prefix[0] = ex_v;
-    prefix[1] = ex_t;
-    atomicAdd(&ctrl->total_v, (unsigned long long)agg_v);
-    atomicAdd(&ctrl->total_t, (unsigned long long)agg_t);
-  }
-}
-
-// LDS words of a count/scan tile: one u32 per row word, one pad word per 32
-// so that both the coalesced (word u*NT + tid) and the per-thread
-// (word tid*WPT + u) access patterns are free of bank conflicts.
-template <int NT, int WPT>
-struct ScanTileLds {
-  static constexpr int kWords = NT * WPT;
-  static constexpr int kSize = kWords + kWords / 32;
-};
-__device__ __forceinline__ int pad32(int i) { return i + (i >> 5); }
-
-// One scan tile of a volume: words [w0, w0 + NT*WPT) (volume-local), status
-// slot `tile` in the global tile order.
-//   1. per-word vertex / triangle counts, consecutive threads on consecutive
-//      words (coalesced row loads), packed into LDS
-//   2. each thread sums WPT consecutive words; block scan; decoupled
-//      look-back for the tile's prefix
-//   3. the bases go back through LDS and out with coalesced stores
-template <int NT, int WPT>
-__device__ __forceinline__ void count_scan_tile(const VolGeom& g, const uint64_t* __restrict__ b,
-                                                uint32_t* __restrict__ base_v,
-                                                uint32_t* __restrict__ base_t,
-                                                unsigned long long* __restrict__ status,
-                                                Ctrl* __restrict__ ctrl, int64_t tile,
-                                                int64_t tile_w0, ScanShared& sh,
-                                                uint32_t* __restrict__ s_pk) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wv = tid >> 6;
-  const int64_t plane = (int64_t)g.wpr * g.ny;
-  const int wpr = g.wpr;
-#pragma unroll
-  for (int u = 0; u < WPT; ++u) {
-    const int i = u * NT + tid;
-    const int64_t w = tile_w0 + i;
-    uint32_t pk = 0;
-    if (w < g.nwords) {
-      const WordPos p = word_pos(g, w);
-      const bool nx1 = p.q + 1 < wpr;
-      const bool hy = w + wpr < g.nwords, hz = w + plane < g.nwords,
-                 hyz = w + plane + wpr < g.nwords;
-      const uint64_t A = b[w], A1 = nx1 ? b[w + 1] : 0ull;
-      const uint64_t B = hy ? b[w + wpr] : 0ull, B1 = (hy && nx1) ? b[w + wpr + 1] : 0ull;
-      const uint64_t C = hz ? b[w + plane] : 0ull, C1 = (hz && nx1) ? b[w + plane + 1] : 0ull;
-      const uint64_t D = hyz ? b[w + plane + wpr] : 0ull;
-      const uint64_t D1 = (hyz && nx1) ? b[w + plane + wpr + 1] : 0ull;
-      uint32_t nv, nt;
-      word_counts_regs(g, p, A, A1, B, B1, C, C1, D, D1, nv, nt);
-      pk = nv | (nt << 16);
-    }
-    s_pk[pad32(i)] = pk;
-  }
-  __syncthreads();
-  const int64_t w0 = tile_w0 + (int64_t)tid * WPT;
-  uint32_t packed[WPT];
-  uint32_t sum_v = 0, sum_t = 0;
-#pragma unroll
-  for (int u = 0; u < WPT; ++u) {
-    packed[u] = s_pk[pad32(tid * WPT + u)];
-    sum_v += packed[u] & 0xffffu;
-    sum_t += packed[u] >> 16;
-  }
-  const uint32_t inc_v = wave_incl_scan(sum_v), inc_t = wave_incl_scan(sum_t);
-  if (lane == 63) {
-    sh.wave_v[wv] = inc_v;
-    sh.wave_t[wv] = inc_t;
-  }
-  __syncthreads();
-  uint32_t off_v = 0, off_t = 0, agg_v = 0, agg_t = 0;
-#pragma unroll
-  for (int q = 0; q < NT / 64; ++q) {
-    if (q < wv) {
-      off_v += sh.wave_v[q];
-      off_t += sh.wave_t[q];
-    }
-    agg_v += sh.wave_v[q];
-    agg_t += sh.wave_t[q];
-  }
-  if (wv == 0) look_back(status, tile, agg_v, agg_t, ctrl, sh.prefix);
-  __syncthreads();
-  // vertex bases, then triangle bases, each through LDS
-#pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
-    uint32_t run = sh.prefix[pass] + (pass == 0 ? off_v + inc_v - sum_v : off_t + inc_t - sum_t);
-    uint32_t* base = pass == 0 ? base_v : base_t;
-#pragma unroll
-    for (int u = 0; u < WPT; ++u) {
-      s_pk[pad32(tid * WPT + u)] = run;
-      run += pass == 0 ? (packed[u] & 0xffffu) : (packed[u] >> 16);
-      if (w0 + u == g.nwords - 1) base[g.word_off + g.nwords] = run;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < WPT; ++u) {
-      const int i = u * NT + tid;
-      const int64_t w = tile_w0 + i;
-      if (w < g.nwords) base[g.word_off + w] = s_pk[pad32(i)];
-    }
-    __syncthreads();
-  }
-}
-
 // Blocks are dispatched round-robin over the 8 XCDs; give each XCD a
 // contiguous range of tiles so neighbouring tiles share its L2.
 __device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t n) {
   const int64_t per = n / 8, rem = n % 8;
   const int64_t x = b % 8, i = b / 8;
   return x * per + (x < rem ? x : rem) + i;
+}
+
+// The same within groups of 8 * kXcdRun tiles, so that no XCD is left with a
+// heavier part of the whole range.
+constexpr int64_t kXcdRun = 32;
+__device__ __forceinline__ int64_t xcd_tile_runs(int64_t b, int64_t n) {
+  const int64_t g0 = b / (8 * kXcdRun) * (8 * kXcdRun);
+  return g0 + xcd_tile(b - g0, min(8 * kXcdRun, n - g0));
 }
 
 // ---------------------------------------------------------------------------
@@ -793,11 +627,14 @@ __device__ __forceinline__ void write_order_units(uint64_t reg, uint32_t K, uint
 }
 
 // What one wave of a generate tile keeps of a round of up to 64 active cells:
-// the cells' table entries, the vertex ids of their 12 edges, their first
-// triangle within the round, and the round's triangle -> cell map.
+// the cells' table entries, the vertex ids of their 12 edges (the bases of
+// the four row words their lower endpoints lie in and each edge's rank there,
+// at most 194), their first triangle within the round, and the round's
+// triangle -> cell map.
 struct GenWave {
   uint64_t table[64];
-  uint32_t ids[12][64];
+  uint32_t base[4][64];
+  uint8_t rank[12][64];
   uint16_t first[64];
   uint16_t cell[64];           // word << 6 | bit
   uint8_t tri_cell[5 * 64];    // at most 5 triangles per cell
@@ -825,7 +662,7 @@ __device__ __forceinline__ uint32_t bit_window(uint64_t A, uint64_t A1, int b) {
   return __builtin_amdgcn_alignbit(up ? d2 : d1, up ? d1 : d0, (uint32_t)b & 31u);
 }
 
-// Case and edge ids of the active cell at bit b of a row word.  Rows of words
+// Case and edge ranks of the active cell at bit b of a row word.  Rows of words
 // r_yz: r00 the cell's own, r10 / r20 one and two rows up, r01 / r11 / r21
 // the same a plane up, r02 / r12 two planes up (each with its next word along
 // x, 0 past the row's end).  A row without a neighbour in y (z) is passed as
@@ -844,9 +681,7 @@ __device__ __forceinline__ uint32_t rank_below(uint64_t a, uint64_t y, uint64_t 
 __device__ __forceinline__ int cell_edges(const RowPair& r00, const RowPair& r10,
                                           const RowPair& r20, const RowPair& r01,
                                           const RowPair& r11, uint64_t r21, uint64_t r02,
-                                          uint64_t r12, int b, bool x2, uint32_t base00,
-                                          uint32_t base10,
-                                          uint32_t base01, uint32_t base11, uint32_t* id) {
+                                          uint64_t r12, int b, bool x2, uint32_t* id) {
   const uint64_t m = (1ull << b) - 1ull;
   const uint32_t w00 = bit_window(r00.a, r00.a1, b), w10 = bit_window(r10.a, r10.a1, b);
   const uint32_t w01 = bit_window(r01.a, r01.a1, b), w11 = bit_window(r11.a, r11.a1, b);
@@ -855,11 +690,11 @@ __device__ __forceinline__ int cell_edges(const RowPair& r00, const RowPair& r10
   const uint32_t x00 = w00 ^ (w00 >> 1), y00 = w00 ^ w10, z00 = w00 ^ w01;
   const uint32_t x10 = w10 ^ (w10 >> 1), y10 = w10 ^ w20, z10 = w10 ^ w11;
   const uint32_t x01 = w01 ^ (w01 >> 1), y01 = w01 ^ w11, z01 = w01 ^ w02;
-  const uint32_t e00 = base00 + rank_below(r00.a, r10.a, r01.a, m);
-  const uint32_t e10 = base10 + rank_below(r10.a, r20.a, r11.a, m);
-  const uint32_t e01 = base01 + rank_below(r01.a, r11.a, r02, m);
-  const uint32_t e11 = base11 + rank_below(r11.a, r21, r12, m);
-  const uint32_t n00 = e00 + (x00 & 1u) + (y00 & 1u) + (z00 & 1u);  // first id at b + 1
+  const uint32_t e00 = rank_below(r00.a, r10.a, r01.a, m);
+  const uint32_t e10 = rank_below(r10.a, r20.a, r11.a, m);
+  const uint32_t e01 = rank_below(r01.a, r11.a, r02, m);
+  const uint32_t e11 = rank_below(r11.a, r21, r12, m);
+  const uint32_t n00 = e00 + (x00 & 1u) + (y00 & 1u) + (z00 & 1u);  // first rank at b + 1
   const uint32_t n10 = e10 + (x10 & 1u) + (y10 & 1u) + (z10 & 1u);
   const uint32_t n01 = e01 + (x01 & 1u) + (y01 & 1u) + (z01 & 1u);
   const uint32_t one = x2 ? 1u : 0u;  // x-edges at b + 1 exist
@@ -880,6 +715,18 @@ __device__ __forceinline__ int cell_edges(const RowPair& r00, const RowPair& r10
                ((w11 & 2u) << 5) | ((w11 & 1u) << 7));
 }
 
+// The row (0: 00, 1: 10, 2: 01, 3: 11) of each edge's lower endpoint, 2 bits
+// per edge in the order cell_edges numbers them.
+constexpr uint32_t edge_rows_packed() {
+  uint32_t r = 0;
+  for (int e = 0; e < 12; ++e) {
+    const int c = edge_code(e);
+    r |= (uint32_t)(((c >> 1) & 1) | (((c >> 2) & 1) << 1)) << (2 * e);
+  }
+  return r;
+}
+constexpr uint32_t kEdgeRows = edge_rows_packed();
+
 // 12 contiguous bytes.
 template <class T>
 __device__ __forceinline__ void store3(T* p, T a, T b, T c) {
@@ -896,18 +743,19 @@ __device__ __forceinline__ void lds_flags(const VolGeom& g, const uint64_t* sA, 
   edge_flags(p, A, p.q + 1 < g.wpr ? A1n : 0ull, B, C, fx, fy, fz);
 }
 
-// Where the generate kernel of the single-volume forward takes its word
-// bases from: the count kernel's per-word prefixes within their count tiles
-// (lpre, v | t << 16), every count tile's prefix within its count block of
-// tpb tiles (tloc, v | t << 32) and the count blocks' exclusive prefixes
-// (bpre, the totals after the last); the tiles per block are a power of
-// two.  It writes the bases of its words to
+// Where the generate kernel takes its word bases from: the count kernel's
+// per-word prefixes within their count tiles (lpre, v | t << 16), every count
+// tile's prefix within its count block (tloc, v | t << 32; the entry after the
+// last tile completes the totals) and the count blocks' exclusive prefixes
+// (bpre, the totals after the last); the tiles per block are a power of two.
+// In a batch the volume's tiles are ct0, ct0 + 1, ..., and the one after its
+// last is the next volume's first.  Generate writes the bases of its words to
 // base_v / base_t, which the adjoint and the per-cell outputs read.
 struct CountSrc {
   const uint32_t* __restrict__ lpre;
   const unsigned long long* __restrict__ tloc;
   const unsigned long long* __restrict__ bpre;
-  int64_t n_ctiles;
+  int64_t n_ctiles, ct0;
   int tpb_shift;  // log2 of the count tiles per count block (from the control block)
   uint32_t* __restrict__ base_v;
   uint32_t* __restrict__ base_t;
@@ -918,37 +766,80 @@ __device__ __forceinline__ unsigned long long add_vt(unsigned long long a, unsig
          ((unsigned long long)((uint32_t)(a >> 32) + (uint32_t)(b >> 32)) << 32);
 }
 
-// Exclusive vertex / triangle prefix (v | t << 32) of count tile c; for c at
-// or past the last tile, the totals.
+// Exclusive vertex / triangle prefix (v | t << 32) of count tile c <= n_ctiles
+// of the volume.
 __device__ __forceinline__ unsigned long long ctile_prefix(const CountSrc& cs, int64_t c) {
-  if (c >= cs.n_ctiles)
-    return cs.bpre[(cs.n_ctiles + (1 << cs.tpb_shift) - 1) >> cs.tpb_shift];
-  return add_vt(cs.bpre[c >> cs.tpb_shift], cs.tloc[c]);
+  const int64_t g = cs.ct0 + c;
+  return add_vt(cs.bpre[g >> cs.tpb_shift], cs.tloc[g]);
 }
 
-// Vertex and triangle base of word w (v | t << 32); past the last count
-// tile the totals.
+// Vertex and triangle base of word w (v | t << 32); past the last count tile
+// the totals.  Every load is issued (clamped indices, results selected), so
+// that the loads of several words can be in flight together.
 __device__ __forceinline__ unsigned long long word_bases(const CountSrc& cs, int64_t w) {
   const int64_t ct = w / kCountTile;
-  const unsigned long long p = ctile_prefix(cs, ct);
-  if (ct >= cs.n_ctiles) return p;
-  const uint32_t l = cs.lpre[w];
+  const bool past = ct >= cs.n_ctiles;
+  const unsigned long long p = ctile_prefix(cs, past ? cs.n_ctiles : ct);
+  const uint32_t lw = cs.lpre[past ? 0 : w], l = past ? 0u : lw;
   return add_vt(p, (unsigned long long)(l & 0xffffu) | ((unsigned long long)(l >> 16) << 32));
 }
 
-// The same with every load issued (clamped indices, results selected), so
-// that the loads of several words can be in flight together.
-__device__ __forceinline__ unsigned long long word_bases_nb(const CountSrc& cs, int64_t w) {
-  const int64_t ct = w / kCountTile;
-  const bool past = ct >= cs.n_ctiles;
-  const int64_t bi = past ? (cs.n_ctiles + (1 << cs.tpb_shift) - 1) >> cs.tpb_shift
-                          : ct >> cs.tpb_shift;
-  const unsigned long long bp = cs.bpre[bi];
-  const unsigned long long tl = cs.tloc[past ? 0 : ct];
-  const uint32_t l = cs.lpre[past ? 0 : w];
-  const unsigned long long full =
-      add_vt(add_vt(bp, tl), (unsigned long long)(l & 0xffffu) | ((unsigned long long)(l >> 16) << 32));
-  return past ? bp : full;
+// Exclusive scan of the n count-block sums (v | t << 32, each half below
+// 2^32) by one block of kTsumThreads threads into bpre, the totals after the
+// last: four consecutive sums per thread and round, wave scans of the thread
+// totals' halves, the block's wave sums in 64 bits, 64-bit carries between
+// rounds.  s_v and s_t hold a word per wave.  Returns the totals in cv, ct.
+constexpr int kTsumThreads = 1024;
+constexpr int kTsumPerThread = 4;  // block sums per thread and round
+__device__ __forceinline__ void scan_block_sums(const unsigned long long* __restrict__ bsum,
+                                                unsigned long long* __restrict__ bpre, int64_t n,
+                                                uint32_t* s_v, uint32_t* s_t,
+                                                unsigned long long& cv, unsigned long long& ct) {
+  constexpr int kWaves = kTsumThreads / 64, kPer = kTsumPerThread;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  cv = ct = 0ull;
+  for (int64_t e0 = 0; e0 < n; e0 += kPer * kTsumThreads) {
+    const int64_t e = e0 + (int64_t)kPer * tid;  // the thread's kPer consecutive sums
+    uint32_t v[kPer], t[kPer], sv = 0u, st = 0u;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const unsigned long long x = e + i < n ? bsum[e + i] : 0ull;
+      v[i] = (uint32_t)x;
+      t[i] = (uint32_t)(x >> 32);
+      sv += v[i];
+      st += t[i];
+    }
+    // a round's sums stay below 2^32 only for the wave partials (a count
+    // block holds at most 3 * 2^18 vertices); the cross-wave totals are
+    // formed in 64 bits
+    const uint32_t iv = wave_incl_scan(sv), it = wave_incl_scan(st);
+    if (lane == 63) {
+      s_v[wv] = iv;
+      s_t[wv] = it;
+    }
+    __syncthreads();
+    unsigned long long ov = 0, ot = 0, rv = 0, rt = 0;
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) {
+      if (q < wv) {
+        ov += s_v[q];
+        ot += s_t[q];
+      }
+      rv += s_v[q];
+      rt += s_t[q];
+    }
+    __syncthreads();
+    unsigned long long pv = cv + ov + iv - sv, pt = ct + ot + it - st;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      if (e + i < n) bpre[e + i] = (pv & 0xffffffffull) | (pt << 32);
+      pv += v[i];
+      pt += t[i];
+    }
+    cv += rv;
+    ct += rt;
+  }
+  if (tid == 0) bpre[n] = (cv & 0xffffffffull) | (ct << 32);
 }
 
 // One generate tile: words [w_begin, w_begin + TW) of a volume, a block of NT
@@ -972,25 +863,22 @@ __device__ __forceinline__ unsigned long long word_bases_nb(const CountSrc& cs, 
 // at 256^3 (475 K vertices) and 88 at 512^3 (957 K); this one, with the tiles
 // gen_shape picks, 13, 36 and 62.
 //
-// FROM_COUNTS: the bases come from the count kernel's per-word prefixes and
-// count-tile prefixes (cs) instead of bv / bt; the tile writes the bases of
-// its words (and, for the last tile, entry nwords) to cs.base_v / base_t,
-// and with emit false only that.  has_output skips the check for a tile
-// without output (one round trip).
-template <int TW, int NT, class Src, bool dedup, bool FROM_COUNTS = false>
+// The bases come from the count kernel's prefixes (cs); the tile writes the
+// bases of its words (and, for the volume's last tile, entry nwords) to
+// cs.base_v / base_t, and with emit false only that.  has_output skips the
+// check for a tile without output (one round trip).
+template <int TW, int NT, class Src, bool dedup>
 __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
-                                              const uint64_t* __restrict__ b,
-                                              const uint32_t* __restrict__ bv,
-                                              const uint32_t* __restrict__ bt, int64_t w_begin,
+                                              const uint64_t* __restrict__ b, int64_t w_begin,
                                               const OutPtrs& out, bool normals,
                                               int64_t vol_base_v, int64_t vol_base_t,
-                                              uint64_t* s_dyn, const CountSrc& cs = CountSrc{},
-                                              bool emit = true, bool has_output = false) {
+                                              uint64_t* s_dyn, const CountSrc& cs, bool emit,
+                                              bool has_output) {
   const int tid = threadIdx.x, lane = tid & 63;
   static_assert(NT >= TW, "a thread per word");
   constexpr int nt = NT, nwaves = NT / 64;
   const int nw = (int)min((int64_t)TW, g.nwords - w_begin);
-  if constexpr (FROM_COUNTS) {
+  {
     // count tiles without output (has_output: known not to be the case):
     // constant bases, nothing else to do
     const int64_t c0 = w_begin / kCountTile;
@@ -1009,9 +897,6 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
       }
       return;
     }
-  } else {
-    if (bv[w_begin] == bv[w_begin + nw] && bt[w_begin] == bt[w_begin + nw])
-      return;  // uniform: no output in this tile
   }
 
   const GenLayout<TW, NT> L(g.wpr);
@@ -1049,60 +934,36 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
       }
     }
   }
-  if constexpr (FROM_COUNTS) {
-    for (int i0 = tid; i0 < L.segv; i0 += kStageU * nt) {
-      unsigned long long p0[kStageU], p1[kStageU];
+  for (int i0 = tid; i0 < L.segv; i0 += kStageU * nt) {
+    unsigned long long p0[kStageU], p1[kStageU];
 #pragma unroll
-      for (int u = 0; u < kStageU; ++u) {
-        const int i = i0 + u * nt;
-        p0[u] = word_bases_nb(cs, w_begin + i);
-        p1[u] = word_bases_nb(cs, w_begin + plane + i);
-      }
+    for (int u = 0; u < kStageU; ++u) {
+      const int i = i0 + u * nt;
+      p0[u] = word_bases(cs, w_begin + i);
+      p1[u] = word_bases(cs, w_begin + plane + i);
+    }
 #pragma unroll
-      for (int u = 0; u < kStageU; ++u) {
-        const int i = i0 + u * nt;
-        if (i < L.segv) {
-          s_v0[i] = (uint32_t)p0[u];
-          s_v1[i] = (uint32_t)p1[u];
-          if (i <= nw) s_t[i] = (uint32_t)(p0[u] >> 32);
-        }
+    for (int u = 0; u < kStageU; ++u) {
+      const int i = i0 + u * nt;
+      if (i < L.segv) {
+        s_v0[i] = (uint32_t)p0[u];
+        s_v1[i] = (uint32_t)p1[u];
+        if (i <= nw) s_t[i] = (uint32_t)(p0[u] >> 32);
       }
     }
-  } else {
-    for (int i0 = tid; i0 < L.segv; i0 += kStageU * nt) {
-      uint32_t a0[kStageU], a1[kStageU];
-#pragma unroll
-      for (int u = 0; u < kStageU; ++u) {
-        const int64_t w = w_begin + i0 + u * nt;
-        a0[u] = bv[w <= g.nwords ? w : 0];
-        a1[u] = bv[w + plane <= g.nwords ? w + plane : 0];
-      }
-#pragma unroll
-      for (int u = 0; u < kStageU; ++u) {
-        const int i = i0 + u * nt;
-        if (i < L.segv) {
-          const int64_t w = w_begin + i;
-          s_v0[i] = (w <= g.nwords) ? a0[u] : 0u;
-          s_v1[i] = (w + plane <= g.nwords) ? a1[u] : 0u;
-        }
-      }
-    }
-    for (int i = tid; i <= nw; i += nt) s_t[i] = bt[w_begin + i];
   }
   __syncthreads();
   const uint32_t tv0 = s_v0[0], tv1 = s_v0[nw];
   const uint32_t tt0 = s_t[0], tt1 = s_t[nw];
-  if constexpr (FROM_COUNTS) {
-    for (int i = tid; i < nw; i += nt) {
-      cs.base_v[w_begin + i] = s_v0[i];
-      cs.base_t[w_begin + i] = s_t[i];
-    }
-    if (tid == 0 && w_begin + nw == g.nwords) {
-      cs.base_v[g.nwords] = tv1;
-      cs.base_t[g.nwords] = tt1;
-    }
-    if (!emit || (tv0 == tv1 && tt0 == tt1)) return;  // bases only, or no output here
+  for (int i = tid; i < nw; i += nt) {
+    cs.base_v[w_begin + i] = s_v0[i];
+    cs.base_t[w_begin + i] = s_t[i];
   }
+  if (tid == 0 && w_begin + nw == g.nwords) {
+    cs.base_v[g.nwords] = tv1;
+    cs.base_t[g.nwords] = tt1;
+  }
+  if (!emit || (tv0 == tv1 && tt0 == tt1)) return;  // bases only, or no output here
 
   // 2. active cells of the thread's word
   if (tid < nw) {
@@ -1197,16 +1058,19 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
       uint32_t id[12];
       const int cs = cell_edges(pair(s_b0, li), pair(s_b0, l1), pair(s_b0, l2), pair(s_b1, li),
                                 pair(s_b1, l1), s_b1[l2], s_z2[li], s_z2[l1], bit,
-                                p.q * 64 + bit + 2 < g.nx, s_v0[li], s_v0[l1], s_v1[li], s_v1[l1],
-                                id);
+                                p.q * 64 + bit + 2 < g.nx, id);
       const uint64_t table = c_case_table[cs];
       const uint32_t nf = valid ? (uint32_t)(table >> 60) : 0u;
       const uint32_t finc = wave_incl_scan(nf), round_tris = wave_last(finc), ffirst = finc - nf;
       W.table[lane] = table;
       W.first[lane] = (uint16_t)ffirst;
       if (dedup) {
+        W.base[0][lane] = s_v0[li];
+        W.base[1][lane] = s_v0[l1];
+        W.base[2][lane] = s_v1[li];
+        W.base[3][lane] = s_v1[l1];
 #pragma unroll
-        for (int e = 0; e < 12; ++e) W.ids[e][lane] = id[e];
+        for (int e = 0; e < 12; ++e) W.rank[e][lane] = (uint8_t)id[e];
       } else {
         W.cell[lane] = (uint16_t)((li << 6) | bit);
       }
@@ -1222,8 +1086,11 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
         int32_t ids[3];
         if (dedup) {
 #pragma unroll
-          for (int v = 0; v < 3; ++v)
-            ids[v] = (int32_t)((int64_t)W.ids[(es >> (4 * v)) & 15u][cl] - vol_base_v);
+          for (int v = 0; v < 3; ++v) {
+            const uint32_t e = (es >> (4 * v)) & 15u;
+            ids[v] = (int32_t)((int64_t)W.base[(kEdgeRows >> (2u * e)) & 3u][cl] + W.rank[e][cl] -
+                               vol_base_v);
+          }
         } else {
           const int cw = (int)W.cell[cl] >> 6, cb = (int)W.cell[cl] & 63;
           const WordPos pc = word_pos(g, w_begin + cw);

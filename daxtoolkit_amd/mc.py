@@ -180,8 +180,7 @@ def forward_into(field: torch.Tensor, iso: float, buf: ForwardBuffers, origin=(0
 
 
 def classify_into(field: torch.Tensor, iso: float, buf: ForwardBuffers) -> None:
-    """The forward's first kernel alone: inside-bits into buf.workspace (and
-    the count/scan state cleared)."""
+    """The forward's first kernel alone: inside-bits into buf.workspace."""
     nx, ny, nz = _check_field(field)
     _check_buf(buf, (nx, ny, nz), field.device)
     _lib.call("dax_hip_mc_bits", field.data_ptr(), nx, ny, nz, float(iso), buf.workspace.data_ptr(),

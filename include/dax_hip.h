@@ -457,8 +457,7 @@ int dax_hip_mc_read_counts(const int64_t* d_counts, int64_t cap_points, int64_t 
 
 /* The three phases of dax_hip_mc_forward as separate calls on one
  * workspace, in this order:
- *   dax_hip_mc_bits      classify: field -> inside-bits (one kernel; also
- *                        resets the scan state of the workspace)
+ *   dax_hip_mc_bits      classify: field -> inside-bits (one kernel)
  *   dax_hip_mc_scan      per-word vertex / triangle counts, then the scan
  *                        of the 256-word count tiles' sums (two kernels)
  *   dax_hip_mc_generate  outputs, as dax_hip_mc_forward (d_counts written),
@@ -554,8 +553,8 @@ int dax_hip_mc_interpolate_scalar(const float* d_in, const int32_t* d_first,
  *                                     (synchronous); copies a header of
  *                                     dax_hip_mc_batch_header_bytes() bytes
  *                                     to h_header_out for the calls below
- *   dax_hip_mc_batch_forward          four persistent launches (classify,
- *                                     count/scan, generate, offsets)
+ *   dax_hip_mc_batch_forward          four launches (classify, count, scan,
+ *                                     generate)
  *   dax_hip_mc_batch_graph_create     the same, captured into a hipGraphExec
  *                                     on a non-null stream
  *   dax_hip_graph_launch / _destroy   replay / free a captured graph */
@@ -576,9 +575,10 @@ int dax_hip_mc_batch_graph_create(const float* d_fields, const void* h_header, v
                                   int64_t cap_points, int64_t cap_tris, int64_t* d_counts,
                                   int64_t* d_vol_offsets, void* stream, void** h_graph_exec);
 /* Launch shapes of the batch forward, held in the header:
- * {classify unroll 8|16|32, classify blocks per CU 2|4|8, scan threads per
- * 1024-word tile 256|512|1024, generate blocks per CU 2|4|8, generate
- * XCD-contiguous tile order 0|1}.  prepare starts from the shape cached for
+ * {classify unroll 8|16|32, classify blocks per CU 2|4|8, threads per count
+ * block 256|512|1024, generate blocks per CU 2|4|8 (no
+ * longer used: generate runs a block per tile), generate XCD-contiguous tile
+ * order 0|1}.  prepare starts from the shape cached for
  * the batch's class (volume count, ceil(log2(row words)), widest row) or the
  * default {16, 4, 256, 4, 1}.  Every shape gives the same outputs.
  *   dax_hip_mc_batch_set_tuning / _get_tuning  write / read the header's
