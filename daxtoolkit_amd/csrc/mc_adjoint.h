@@ -13,19 +13,20 @@
 //   dL/dgA  = (1-t) dL/dm,                dL/dgB  = t dL/dm
 // and each dL/dg_p[d] flows to the stencil points of g_p[d].
 //
-// Two kernels, deterministic (no atomics; every sum has a fixed order):
-//   k_vertex_adjoint : one thread per vertex, recomputes t, gA, gB from the
-//                      field and the compact edge list (the interpolants are
-//                      not stored by the forward), writes 8 floats per vertex
-//                      (sA, GA[3], sB, GB[3])
-//   k_point_gather   : tiles of 256 row words.  A thread per word forms the
-//                      mask of points within L1 distance 1 of an active-edge
-//                      endpoint (bit-parallel, from the inside-bits); the
-//                      other points get 0 with coalesced stores; the
-//                      receiving points are compacted and each gets one
-//                      thread, which sums over the active edges incident to
-//                      it and to its 6 neighbours.
+// Deterministic (no atomics; every sum has a fixed order), in four launches:
+//   records    one thread per vertex, recomputes t, gA, gB from the field and
+//              the compact edge list (the interpolants are not stored by the
+//              forward), writes 8 floats per vertex (sA, GA[3], sB, GB[3]);
+//              beside it a thread per row word writes the word's endpoints
+//              (the points of active edges) and their counts
+//   scan       the tiles' endpoint counts, so that every endpoint has a slot
+//   endpoints  each endpoint's sums (S, G) over its at most 6 edges, once
+//   gather     every point: 0, or within L1 distance 1 of an endpoint (the
+//              only points with a non-zero dL/df) the sum of its own S and the
+//              stencil terms of the G of its neighbours
 #pragma once
+
+#include <algorithm>
 
 #include "mc_kernels.h"
 
@@ -114,202 +115,338 @@ __device__ __forceinline__ void vertex_adjoint(const VolGeom& g, const float* __
   out[u] = r;
 }
 
-// ---- per-point gather ------------------------------------------------------
-// A point receives a non-zero dL/df only within L1 distance 1 of an endpoint
-// of an active edge (its own t-terms and the central-difference stencils of
-// the endpoint gradients).  A gather tile of up to kGatherTile consecutive row
-// words stages, for the planes k-2..k+1 around it, the active-edge flags
-// (fx, fy, fz: the same flags the forward numbers its vertices with) and the
-// vertex bases of the words within two rows (and one word) of the tile:
-// segment dz holds words [w0 + dz*plane - 2*wpr - 1, w_end + dz*plane +
-// 2*wpr + 1).  Every lower endpoint of an edge a tile point reads lies at
-// |dq| <= 1, -2 <= dy, dz <= 1 from its own word, inside its segment.
-constexpr int kGatherTile = kGatherTileWords;  // row words per tile
-constexpr int kGatherThreads = 512;  // threads per tile
-// Endpoint records a tile keeps (4 per thread, held in registers until the
-// flags are no longer needed, then written over them).
-constexpr int kRecPerThread = 4;
-constexpr int kMaxEndpoints = kRecPerThread * kGatherThreads;
+// ---- endpoints and gather ---------------------------------------------------
+// Endpoint words and prefixes by tiles of 256 row words, sums and gather a
+// wave per 32 words; nothing is shared between the waves of a block.  What the
+// steps hand on goes through global memory (the caches), so a wave needs
+// little LDS and no barrier, and no work is repeated at tile borders.  A block
+// per tile that staged edge flags with a halo, formed the sums of the tile's
+// and the halo's endpoints in LDS between six barriers and listed tiles too
+// dense for it for another pass took 56 + 28 us at 256^3 (447 K endpoints),
+// 490 + 14 on a noisy 640^3 surface (3.6 M) and 375 + 60 for 256 volumes of
+// 32..160 points an axis (1.4 M).  Sums and gather take 20 + 23, 99 + 305 and
+// 62 + 267, the words and the scan 5, 40 and 45 more.
+constexpr int kAdjTile = kGatherTileWords;  // row words per tile
+constexpr int kAdjThreads = kAdjTile;
+// Words per wave of the sums and the gather.  16 fill too few lanes of large
+// volumes, 64 leave small ones too few waves: a whole step took 125 / 126 /
+// 131 us at 256^3 with 16 / 32 / 64, 985 / 972 / 987 at 640^3, 781 / 757 / 768
+// for the batch.
+constexpr int kAdjWaveWords = 32;
+constexpr int kAdjBlockWords = kAdjThreads / 64 * kAdjWaveWords;
+constexpr int kAdjTileBlocks = kAdjTile / kAdjBlockWords;
 
-__host__ __device__ constexpr int gather_seg(int wpr) { return kGatherTile + 4 * wpr + 2; }
-// G-words: the tile's words with one row above and below in its plane, and
-// the tile's words in the planes below and above.
-__host__ __device__ constexpr int gather_gwords(int nw, int wpr) { return 3 * nw + 2 * wpr; }
-// Dynamic LDS of a gather tile: the staged flags and vertex bases (later the
-// endpoint records), the G-word endpoint masks and their exclusive scan, and
-// the G-word of each endpoint slot.
-__host__ __device__ constexpr size_t gather_flags_bytes(int wpr) {
-  const size_t flags = (size_t)4 * gather_seg(wpr) * (3 * sizeof(uint64_t) + sizeof(uint32_t));
-  const size_t recs = (size_t)kMaxEndpoints * 16;
-  return flags > recs ? flags : recs;
-}
-__host__ __device__ constexpr size_t gather_lds_bytes(int wpr) {
-  const size_t ng = (size_t)gather_gwords(kGatherTile, wpr);
-  return gather_flags_bytes(wpr) + ng * sizeof(uint64_t) + (ng + 1) * sizeof(uint32_t) +
-         (size_t)kMaxEndpoints * sizeof(uint16_t);
+// Endpoint words of a volume (or batch) and their prefixes: the endpoints of
+// word w before it are tile[w's tile] + pre[w].
+struct Endpoints {
+  uint64_t* words;
+  uint16_t* pre;
+  uint32_t* sums;  // per tile
+  uint32_t* tile;  // their exclusive prefixes
+  uint32_t* base;  // per count tile: vertex base
+};
+static_assert(kAdjTile * 64 < 65536, "prefixes within a tile fit 16 bits");
+static_assert(kAdjTile == 2 * kCountTile, "two count tiles per tile");
+
+// Vertex base of row word w of a volume (lpre: its count prefixes).
+__device__ __forceinline__ uint32_t vertex_base(const VolGeom& g, const Endpoints& ep,
+                                                const uint32_t* __restrict__ lpre, int64_t w) {
+  return ep.base[2 * g.tile_off + w / kCountTile] + (lpre[w] & 0xffffu);
 }
 
-// Part `part` (0..3) of the test whether the tile at word w0 stages any
-// active edge: segment dz = part - 2 holds one (the vertex bases count the
-// active edges of a word range).  A tile is quiet when no part holds one.
-__device__ __forceinline__ bool gather_segment_active(const VolGeom& g,
-                                                      const uint32_t* __restrict__ base_v,
-                                                      int64_t w0, int part) {
+// Edge flags of a row word, without the edges whose ids are not below n.
+struct WordEdges {
+  uint64_t fx, fy, fz;
+};
+__device__ __forceinline__ WordEdges word_edges_below(const VolGeom& g,
+                                                      const uint64_t* __restrict__ b,
+                                                      const CountSrc& cs, int64_t w, int64_t n) {
+  const WordPos p = word_pos(g, w);
+  const uint64_t A = b[w];
+  WordEdges m;
+  edge_flags(p, A, p.q + 1 < g.wpr ? b[w + 1] : 0ull, p.has_y ? b[w + g.wpr] : 0ull,
+             p.has_z ? b[w + (int64_t)g.wpr * g.ny] : 0ull, m.fx, m.fy, m.fz);
+  int64_t room = n - (int64_t)(uint32_t)word_bases(cs, w);
+  if (popc(m.fx) + popc(m.fy) + popc(m.fz) <= room) return m;
+  for (int bit = 0; bit < 64; ++bit) {
+    const uint64_t t = 1ull << bit;
+    if ((m.fx & t) && --room < 0) m.fx &= ~t;
+    if ((m.fy & t) && --room < 0) m.fy &= ~t;
+    if ((m.fz & t) && --room < 0) m.fz &= ~t;
+  }
+  return m;
+}
+
+// Endpoints of row word w: the points whose bit differs from one of their
+// neighbours' (grids without cells have none).  Of an edge list cut at n_adj
+// vertices only the endpoints of its edges, so that 2 n_adj slots hold them.
+__device__ __forceinline__ uint64_t endpoint_word(const VolGeom& g, const uint64_t* __restrict__ b,
+                                                  const CountSrc& cs, int64_t n_adj, int64_t w) {
   const int64_t plane = (int64_t)g.wpr * g.ny;
-  const int64_t ws0 = w0 + (part - 2) * plane - 2 * g.wpr - 1;
-  const int64_t ws = max(ws0, (int64_t)0);
-  const int64_t we = min(ws0 + gather_seg(g.wpr), g.nwords);
-  return we > ws && base_v[we] != base_v[ws];
-}
-
-struct Stage {
-  const uint64_t* fx;  // LDS [4][seg] each
-  const uint64_t* fy;
-  const uint64_t* fz;
-  const uint32_t* bv;
-  int seg;
-  int64_t w0;          // tile's first word
-};
-
-// A point's view of the staged words: its word at (q, j, k) lies dzp planes
-// from the tile's plane, at tile-plane word w (its own word minus dzp*plane).
-struct GatherCtx {
-  const VolGeom* g;
-  const Stage* st;
-  const VertexAdj* adj;
-  int64_t n_adj;  // records in adj
-  int64_t w;
-  int dzp;
-  int q, x, j, k;
-
-  // LDS index of word (q+dq, j+dy, k+dz); dzp + dz in -2..1
-  __device__ __forceinline__ int idx(int dq, int dy, int dz) const {
-    return (dzp + dz + 2) * st->seg + (int)(w - st->w0) + dq + dy * g->wpr + 2 * g->wpr + 1;
+  const WordPos p = word_pos(g, w);
+  const uint64_t A = b[w];
+  const uint64_t next = p.q + 1 < g.wpr ? b[w + 1] : 0ull;
+  const uint64_t yp = p.has_y ? b[w + g.wpr] : A, ym = p.j > 0 ? b[w - g.wpr] : A;
+  const uint64_t zp = p.has_z ? b[w + plane] : A, zm = p.k > 0 ? b[w - plane] : A;
+  const uint64_t prev = p.q > 0 ? b[w - 1] >> 63 : A & 1ull;
+  const uint32_t base = (uint32_t)word_bases(cs, w);
+  const uint64_t fx = (A ^ shr1(A, next)) & p.xmask;
+  uint64_t e = fx | (fx << 1) | ((prev ^ A) & 1ull) | (A ^ yp) | (A ^ ym) | (A ^ zp) | (A ^ zm);
+  e &= p.pmask;
+  if (e != 0ull && (int64_t)base + 192 > n_adj) {  // the last words, or a cut list
+    const WordEdges o = word_edges_below(g, b, cs, w, n_adj);
+    e = o.fx | (o.fx << 1) | o.fy | o.fz;
+    if (p.q > 0) e |= word_edges_below(g, b, cs, w - 1, n_adj).fx >> 63;
+    if (p.j > 0) e |= word_edges_below(g, b, cs, w - g.wpr, n_adj).fy;
+    if (p.k > 0) e |= word_edges_below(g, b, cs, w - plane, n_adj).fz;
   }
-};
-
-// Vertex id of the edge with lower endpoint (x,j,k) + (dx,dy,dz) along
-// `axis`, or -1 if that edge is not active (LDS only).
-__device__ __forceinline__ int64_t edge_vid(const GatherCtx& c, int dx, int dy, int dz, int axis) {
-  const VolGeom& g = *c.g;
-  const int xl = c.x + dx, jl = c.j + dy, kl = c.k + dz;
-  if (xl < 0 || xl >= g.nx || jl < 0 || jl >= g.ny || kl < 0 || kl >= g.nz) return -1;
-  const int qq = xl >> 6, bb = xl & 63;
-  const int i = c.idx(qq - c.q, dy, dz);
-  const uint64_t fa = (axis == 0 ? c.st->fx : (axis == 1 ? c.st->fy : c.st->fz))[i];
-  if (!((fa >> bb) & 1ull)) return -1;
-  const uint64_t fx = axis == 0 ? fa : c.st->fx[i];
-  const uint64_t fy = axis == 1 ? fa : c.st->fy[i];
-  const uint64_t fz = axis == 2 ? fa : c.st->fz[i];
-  const int64_t vid = (int64_t)c.st->bv[i] + edge_rank(fx, fy, fz, bb, axis);
-  return vid < c.n_adj ? vid : -1;
-}
-
-// (S_p, dL/dg_p) at p = (x,j,k) + (dx,dy,dz): over the 3 edges leaving p
-// (lower halves of their records) and the 3 edges entering p (upper halves),
-// summed in that order.
-__device__ __forceinline__ f32x4 point_sums(const GatherCtx& c, int dx, int dy, int dz) {
-  int64_t vid[6];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    vid[a] = edge_vid(c, dx, dy, dz, a);
-    vid[3 + a] = edge_vid(c, dx - (a == 0), dy - (a == 1), dz - (a == 2), a);
-  }
-  const f32x4* rec = reinterpret_cast<const f32x4*>(c.adj);
-  f32x4 r[6];
-  // unconditional loads (an inactive edge reads record 0 and is dropped
-  // below), so the six are in flight together instead of one conditional
-  // load and wait at a time; every record index is below n_adj
-  if (c.n_adj > 0) {
-#pragma unroll
-    for (int i = 0; i < 6; ++i) r[i] = rec[vid[i] >= 0 ? 2 * vid[i] + (i < 3 ? 0 : 1) : 0];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 6; ++i) r[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};  // S, G[0..2]
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    if (vid[i] >= 0) {
-      acc.x += r[i].x;
-      acc.y += r[i].y;
-      acc.z += r[i].z;
-      acc.w += r[i].w;
-    }
-  }
-  return acc;
-}
-
-// dL/df of the point q = (x, j, k) from (S, G) of q and of its 6 neighbours:
-// at(d, s) returns (S_p, G_p) of p = q + s e_d (s = 0: q itself).
-template <class At>
-__device__ __forceinline__ float combine_point(const VolGeom& g, int x, int j, int k, At at) {
-  const f32x4 own = at(0, 0);
-  const float G[3] = {own.y, own.z, own.w};
-  float acc = own.x;
-  const int co[3] = {x, j, k};
-  const int n[3] = {g.nx, g.ny, g.nz};
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const float h = g.spacing[d];
-    if (n[d] < 2) continue;
-    // f_q in g_q[d] (one-sided stencils on the first and last plane)
-    if (co[d] == 0)
-      acc += G[d] * (-1.0f / h);
-    else if (co[d] == n[d] - 1)
-      acc += G[d] * (1.0f / h);
-  }
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const float h = g.spacing[d];
-    if (n[d] < 2) continue;
-    if (co[d] >= 1) {  // p = q - e_d: f_q = f(p + e_d)
-      const f32x4 r = at(d, -1);
-      const float Gd = d == 0 ? r.y : (d == 1 ? r.z : r.w);
-      acc += (co[d] - 1 == 0) ? Gd / h : Gd / (2.0f * h);
-    }
-    if (co[d] <= n[d] - 2) {  // p = q + e_d: f_q = f(p - e_d)
-      const f32x4 r = at(d, 1);
-      const float Gd = d == 0 ? r.y : (d == 1 ? r.z : r.w);
-      acc += (co[d] + 1 == n[d] - 1) ? -(Gd / h) : -(Gd / (2.0f * h));
-    }
-  }
-  return acc;
-}
-
-// dL/df of the point (x, j, k), every sum from the staged flags.
-__device__ __forceinline__ float point_adjoint(const GatherCtx& c) {
-  return combine_point(*c.g, c.x, c.j, c.k, [&](int d, int s) {
-    return point_sums(c, d == 0 ? s : 0, d == 1 ? s : 0, d == 2 ? s : 0);
-  });
-}
-
-// Endpoint mask of row word (q+dq, j+dy, k+dz) of the context's word
-// (dzp + dz in -1..1): points with an active incident edge, from the staged
-// flags (0 outside the grid; the flags are 0 in grids without cells).
-__device__ __forceinline__ uint64_t endpoint_mask(const GatherCtx& c, int dq, int dy, int dz) {
-  const VolGeom& g = *c.g;
-  const int qq = c.q + dq, jj = c.j + dy, kk = c.k + dz;
-  if (qq < 0 || qq >= g.wpr || jj < 0 || jj >= g.ny || kk < 0 || kk >= g.nz) return 0ull;
-  const Stage& st = *c.st;
-  const int i = c.idx(dq, dy, dz);
-  const uint64_t fx = st.fx[i];
-  uint64_t e = fx | (fx << 1) | st.fy[i] | st.fz[i];
-  if (qq > 0) e |= st.fx[i - 1] >> 63;  // x-edge entering bit 0
-  if (jj > 0) e |= st.fy[i - g.wpr];     // y-edges entering the row
-  if (kk > 0) e |= st.fz[i - st.seg];    // z-edges entering the row
   return e;
 }
 
-// Points of the context's word within L1 distance 1 of an endpoint.
-__device__ __forceinline__ uint64_t receiving_mask(const GatherCtx& c) {
-  const uint64_t e = endpoint_mask(c, 0, 0, 0);
-  uint64_t r = e | (e << 1) | (e >> 1);
-  r |= endpoint_mask(c, -1, 0, 0) >> 63;
-  r |= endpoint_mask(c, 1, 0, 0) << 63;
-  r |= endpoint_mask(c, 0, -1, 0) | endpoint_mask(c, 0, 1, 0);
-  r |= endpoint_mask(c, 0, 0, -1) | endpoint_mask(c, 0, 0, 1);
-  return r & low_mask(c.g->nx - c.q * 64);
+// Endpoint words, counts and prefixes of a tile (block of kAdjThreads).
+__device__ __forceinline__ void endpoint_words_tile(const VolGeom& g,
+                                                    const uint64_t* __restrict__ b,
+                                                    const CountSrc& cs, int64_t n_adj,
+                                                    const Endpoints& ep, int64_t w0,
+                                                    uint32_t* s_scan) {
+  const int64_t w = w0 + threadIdx.x;
+  const uint64_t e = w < g.nwords ? endpoint_word(g, b, cs, n_adj, w) : 0ull;
+  uint32_t total;
+  const uint32_t pre = block_excl_scan((uint32_t)popc(e), total, s_scan);
+  if (w < g.nwords) {
+    ep.words[g.word_off + w] = e;
+    ep.pre[g.word_off + w] = (uint16_t)pre;
+  }
+  if (threadIdx.x == 0) ep.sums[g.tile_off + w0 / kAdjTile] = total;
+  if (threadIdx.x < 2) {
+    const int64_t c = w0 / kCountTile + threadIdx.x;
+    if (c < cs.n_ctiles) ep.base[2 * g.tile_off + c] = (uint32_t)ctile_prefix(cs, c);
+  }
+}
+
+// Exclusive scan of the tiles' counts by one block; it also clears slot 0 of the
+// endpoints' sums, which stands for the points that are no endpoints.
+constexpr int kAdjScanThreads = 1024;
+using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
+static __global__ __launch_bounds__(kAdjScanThreads) void k_scan_endpoints(
+    const uint32_t* __restrict__ sums, uint32_t* __restrict__ pre, int64_t n,
+    f32x4* __restrict__ endpoint_sums) {
+  if (threadIdx.x == 0) endpoint_sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  __shared__ uint32_t s_scan[kAdjScanThreads / 64];
+  constexpr int V = 16;
+  uint32_t carry = 0u;
+  for (int64_t c0 = 0; c0 < n; c0 += kAdjScanThreads * V) {
+    const int64_t i0 = c0 + (int64_t)threadIdx.x * V;
+    const bool whole = i0 + V <= n;
+    u32x4 v[V / 4];
+#pragma unroll
+    for (int q = 0; q < V / 4; ++q) {
+      if (whole) {
+        v[q] = *reinterpret_cast<const u32x4*>(sums + i0 + 4 * q);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[q][t] = i0 + 4 * q + t < n ? sums[i0 + 4 * q + t] : 0u;
+      }
+    }
+    uint32_t sum = 0u;
+#pragma unroll
+    for (int q = 0; q < V; ++q) sum += v[q / 4][q % 4];
+    uint32_t total, run = carry + block_excl_scan(sum, total, s_scan);
+    carry += total;
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const uint32_t x = v[q / 4][q % 4];
+      v[q / 4][q % 4] = run;
+      run += x;
+    }
+#pragma unroll
+    for (int q = 0; q < V / 4; ++q) {
+      if (whole) {
+        *reinterpret_cast<u32x4*>(pre + i0 + 4 * q) = v[q];
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (i0 + 4 * q + t < n) pre[i0 + 4 * q + t] = v[q][t];
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ uint64_t shfl64(uint64_t v, int l) {
+  return ((uint64_t)(uint32_t)__shfl((int)(uint32_t)(v >> 32), l, 64) << 32) |
+         (uint32_t)__shfl((int)(uint32_t)v, l, 64);
+}
+
+// The lane's word among lanes holding n items each (inclusive scan inc), for
+// the 64 items from e0 on: words mark their first item's lane, a prefix
+// maximum gives every lane its word.  Lanes past the last item get the last
+// word.
+__device__ __forceinline__ int item_word(uint32_t n, uint32_t inc, uint32_t e0, uint8_t* mark) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t start = inc - n;
+  mark[lane] = 0;
+  wave_lds_sync();
+  if (n != 0u && start < e0 + 64u && inc > e0) mark[max(start, e0) - e0] = (uint8_t)(lane + 1);
+  wave_lds_sync();
+  const int wl = (int)wave_incl_max((uint32_t)mark[lane]) - 1;
+  wave_lds_sync();  // the marks are reused
+  return wl;
+}
+
+// (S_p, dL/dg_p) of the endpoint p at `bit` of row word w: over the 3 edges
+// leaving p (lower halves of their records), then the 3 edges entering p
+// (upper halves), in axis order.  The edges leaving p follow each other in
+// the numbering, the x-edge entering it is counted back from them; the y- and
+// z-edges entering it are ranked in their own words.  Words are shifted up so
+// that p's bit is their sign and the bits above it are gone: a flag is then a
+// comparison, and the edges of the points up to p are popcounts.
+__device__ __forceinline__ f32x4 endpoint_sums(const VolGeom& g, const uint64_t* __restrict__ b,
+                                               const uint32_t* __restrict__ lpre,
+                                               const Endpoints& ep,
+                                               const VertexAdj* __restrict__ adj, int64_t n_adj,
+                                               int64_t w, int bit) {
+  const int64_t plane = (int64_t)g.wpr * g.ny;
+  const WordPos p = word_pos(g, w);
+  const bool hn = p.q + 1 < g.wpr;
+  const int up = 63 - bit;
+  // rows: own, +y, +z; the row before with +z; the plane before with +y (a row
+  // that is not there: one without edges to it)
+  const int64_t wy = p.j > 0 ? w - g.wpr : w, wz = p.k > 0 ? w - plane : w;
+  const int64_t sy = p.has_y ? g.wpr : 0, sz = p.has_z ? plane : 0;
+  const uint64_t A0 = b[w], Y0 = b[wy], Z0 = b[wz];
+  const uint64_t An = hn ? b[w + 1] : 0ull, Yn = hn ? b[wy + 1] : 0ull, Zn = hn ? b[wz + 1] : 0ull;
+  const uint64_t B = b[w + sy] << up, C = b[w + sz] << up;
+  const uint64_t YC = b[wy + sz] << up, ZB = b[wz + sy] << up;
+  const uint32_t ba = vertex_base(g, ep, lpre, w), by = vertex_base(g, ep, lpre, wy),
+                 bz = vertex_base(g, ep, lpre, wz);
+  const uint64_t A = A0 << up, Y = Y0 << up, Z = Z0 << up;
+  auto sign = [](uint64_t v) -> uint32_t { return (uint32_t)(v >> 32) >> 31; };
+  const uint32_t xin = p.q * 64 + bit + 1 < g.nx ? 1u : 0u;  // an x-edge leaves p
+  // x-edges among the points up to p, less the first point's own bit
+  auto count_x = [](uint64_t s, uint64_t s0) -> uint32_t {
+    return (uint32_t)popc(s ^ (s << 1)) - ((uint32_t)s0 & 1u);
+  };
+  auto next = [&](uint64_t s0, uint64_t sn) -> uint64_t {  // the point after p
+    return ((s0 >> 1) | (sn << 63)) << up;
+  };
+  // the edges leaving p
+  const uint64_t ab = A ^ B, ac = A ^ C;
+  const uint32_t x = sign(A ^ next(A0, An)) & xin, y = sign(ab), z = sign(ac);
+  const uint32_t first = ba + count_x(A, A0) + (uint32_t)popc(ab) + (uint32_t)popc(ac) - y - z;
+  // the point before p
+  uint64_t Pa = A << 1, Pb = B << 1, Pc = C << 1;
+  if (bit == 0) {
+    Pa = Pb = Pc = A;
+    if (p.q > 0) {
+      Pa = b[w - 1];
+      Pb = b[w - 1 + sy];
+      Pc = b[w - 1 + sz];
+    }
+  }
+  const uint32_t px = sign(Pa ^ A), py = sign(Pa ^ Pb), pz = sign(Pa ^ Pc);
+  const uint64_t ya = Y ^ A, yc = Y ^ YC, za = Z ^ A, zb = Z ^ ZB;
+  const uint32_t yin = sign(ya), zin = sign(za);  // Y is A in the first row
+  bool on[6] = {x != 0u, y != 0u, z != 0u, px != 0u, yin != 0u, zin != 0u};
+  const uint32_t id[6] = {
+      first, first + x, first + x + y, first - px - py - pz,
+      by + count_x(Y, Y0) + (uint32_t)popc(ya) + (uint32_t)popc(yc) - yin - sign(yc) +
+          (sign(Y ^ next(Y0, Yn)) & xin),
+      bz + count_x(Z, Z0) + (uint32_t)popc(zb) + (uint32_t)popc(za) - zin +
+          (sign(Z ^ next(Z0, Zn)) & xin)};
+  const f32x4* rec = reinterpret_cast<const f32x4*>(adj);
+  f32x4 v[6];
+  // unconditional loads (record 0 for an edge that is not there), in flight
+  // together
+#pragma unroll
+  for (int e = 0; e < 6; ++e) {
+    on[e] = on[e] && (int64_t)id[e] < n_adj;
+    v[e] = n_adj > 0 ? rec[on[e] ? 2 * (int64_t)id[e] + (e < 3 ? 0 : 1) : 0]
+                     : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};  // S, G[0..2]
+#pragma unroll
+  for (int e = 0; e < 6; ++e)
+    if (on[e]) acc += v[e];
+  return acc;
+}
+
+// The sums of a wave's words' endpoints, a lane per endpoint, at their
+// slots (1 + the endpoints before; at most cap).
+__device__ __forceinline__ void endpoint_sums_wave(const VolGeom& g,
+                                                   const uint64_t* __restrict__ b,
+                                                   const uint32_t* __restrict__ lpre,
+                                                   const Endpoints& ep,
+                                                   const VertexAdj* __restrict__ adj,
+                                                   int64_t n_adj, f32x4* __restrict__ sums,
+                                                   int64_t cap, int64_t ww, uint8_t* mark) {
+  const int lane = threadIdx.x & 63;
+  const int64_t w = ww + lane;
+  const uint64_t e = lane < kAdjWaveWords && w < g.nwords ? ep.words[g.word_off + w] : 0ull;
+  const uint32_t n = (uint32_t)popc(e);
+  if (!__ballot(n != 0u)) return;
+  const uint32_t inc = wave_incl_scan(n), total = wave_last(inc);
+  const int64_t slot0 = 1 + (int64_t)ep.tile[g.tile_off + ww / kAdjTile] + ep.pre[g.word_off + ww];
+  for (uint32_t e0 = 0; e0 < total; e0 += 64u) {  // wave-uniform
+    const int wl = item_word(n, inc, e0, mark);
+    const uint32_t i = e0 + (uint32_t)lane;
+    const uint32_t start = (uint32_t)__shfl((int)(inc - n), wl, 64);
+    const uint64_t word = shfl64(e, wl);
+    if (i < total && slot0 + i <= cap)
+      sums[slot0 + i] = endpoint_sums(g, b, lpre, ep, adj, n_adj, ww + wl,
+                                      select_bit(word, (int)(i - start)));
+  }
+}
+
+// v / h (one-sided) or v / (2 h) along axis d; a power of two divides exactly
+// by its reciprocal.
+__device__ __forceinline__ float over_step(const VolGeom& g, int d, float v, bool one_sided) {
+  if ((g.pow2_h >> d) & 1u) return v * (one_sided ? g.rcp_h[d] : 0.5f * g.rcp_h[d]);
+  return v / (one_sided ? g.spacing[d] : 2.0f * g.spacing[d]);
+}
+
+// What the point (x, j, k) receives: (S, G) of its own and, along each axis d,
+// G[d] of the points before and after it (zero where there is no endpoint).
+struct PointTerms {
+  f32x4 own;
+  float before[3], after[3];
+};
+
+// dL/df of the point: f_q in g_q[d] (one-sided stencils on the first and last
+// plane), then along each axis f_q = f(p + e_d) for p = q - e_d and
+// f_q = f(p - e_d) for p = q + e_d.  INTERIOR: the point is two points or more
+// from every border (no one-sided stencil takes part).
+template <bool INTERIOR>
+__device__ __forceinline__ float combine_point(const VolGeom& g, int x, int j, int k,
+                                               const PointTerms& t) {
+  float acc = t.own.x;
+  if constexpr (INTERIOR) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      acc += over_step(g, d, t.before[d], false);
+      acc += -over_step(g, d, t.after[d], false);
+    }
+    return acc;
+  }
+  const float G[3] = {t.own.y, t.own.z, t.own.w};
+  const int co[3] = {x, j, k};
+  const int n[3] = {g.nx, g.ny, g.nz};
+  float one = 1.0f;
+  asm volatile("" : "+v"(one));  // keeps the quotients in this rare path
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (n[d] < 2) continue;
+    if (co[d] == 0)
+      acc += G[d] * over_step(g, d, -one, true);
+    else if (co[d] == n[d] - 1)
+      acc += G[d] * over_step(g, d, one, true);
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (n[d] < 2) continue;
+    if (co[d] >= 1) acc += over_step(g, d, t.before[d], co[d] == 1);
+    if (co[d] <= n[d] - 2) acc += -over_step(g, d, t.after[d], co[d] == n[d] - 2);
+  }
+  return acc;
 }
 
 // Zeros over the points of row words [w0, w_end) of a volume: one
@@ -330,378 +467,143 @@ __device__ __forceinline__ void zero_run(const VolGeom& g, float* __restrict__ o
   for (int64_t t = head + 4 * n4 + tid; t < n; t += nt) o[t] = 0.0f;
 }
 
-struct GatherShared {
-  uint64_t recv[kGatherTile];
-  uint32_t first[kGatherTile + 1];  // exclusive scan of popcount(recv)
-  uint32_t scan[16];
+// What a wave of the gather keeps of its words: the endpoint words of the word
+// itself, the rows before and after it and the planes before and after it, the
+// slots before their first endpoints, the points that receive something and
+// the number of them before the word, the word's first point, and flags:
+// bit 0 / 1: the point before / after the word is an endpoint, bit 2: no
+// receiving point is within two points of a border.
+struct GatherWave {
+  uint64_t ends[5][kAdjWaveWords];
+  uint64_t recv[kAdjWaveWords];
+  uint32_t slot[5][kAdjWaveWords];
+  uint32_t start[kAdjWaveWords];
+  uint32_t base[kAdjWaveWords];
+  uint8_t flags[kAdjWaveWords];
+  uint8_t mark[64];
 };
 
-// Widest rows the gather stages (nx <= 15872): its LDS stays within a CU's
-// 160 KiB.
+// dL/df of the points of a wave's row words: zeros over all of
+// them, then, a lane per point, those that receive something (a wave's stores
+// to one address stay in order).  On a surface a row word has about 8 of them
+// in 64.  Bound by the lanes' instructions: one shift of an endpoint word puts
+// the point's flag in its sign and the endpoints up to the point under a
+// popcount, from the neighbours only the one component that the stencil takes
+// is read, and waves without points next to a border take a short sum.  Large
+// outputs are bound by their zeros (640^3: 162 us of 305 without a surface)
+// mixed with the reads.  A lane per point of a word (flags and ranks from
+// wave-uniform masks, whole words stored) took 44 us at 256^3 and 334 at
+// 640^3 where this takes 23 and 305..317; the points composed in LDS and stored
+// once 29 and 323.
+__device__ __forceinline__ void gather_wave(const VolGeom& g, const Endpoints& ep,
+                                            const f32x4* __restrict__ sums, uint32_t cap,
+                                            float* __restrict__ out, int64_t ww, GatherWave& W) {
+  const int lane = threadIdx.x & 63;
+  const int64_t plane = (int64_t)g.wpr * g.ny;
+  const int64_t w = ww + lane;
+  uint64_t e[5], r = 0ull;
+  int64_t at[5] = {w, w, w, w, w};
+  uint32_t flags = 0u, base = 0u;
+  if (lane < kAdjWaveWords && w < g.nwords && cap != 0u) {
+    const WordPos p = word_pos(g, w);
+    base = ((uint32_t)p.k * (uint32_t)g.ny + (uint32_t)p.j) * (uint32_t)g.nx + (uint32_t)p.q * 64u;
+    const uint64_t* ew = ep.words + g.word_off;
+    if (p.j > 0) at[1] = w - g.wpr;
+    if (p.has_y) at[2] = w + g.wpr;
+    if (p.k > 0) at[3] = w - plane;
+    if (p.has_z) at[4] = w + plane;
+#pragma unroll
+    for (int n = 0; n < 5; ++n) e[n] = ew[at[n]];
+    const uint64_t before = ew[p.q > 0 ? w - 1 : w] >> 63;
+    const uint64_t after = ew[p.q + 1 < g.wpr ? w + 1 : w];
+#pragma unroll
+    for (int n = 1; n < 5; ++n)
+      if (at[n] == w) e[n] = 0ull;
+    flags = (p.q > 0 ? (uint32_t)before : 0u) |
+            (p.q + 1 < g.wpr ? ((uint32_t)after & 1u) << 1 : 0u);
+    r = e[0] | (e[0] << 1) | (e[0] >> 1) | e[1] | e[2] | e[3] | e[4] | (flags & 1u) |
+        ((uint64_t)(flags >> 1) << 63);
+    r &= low_mask(g.nx - p.q * 64);
+    const uint64_t rim = (p.q == 0 ? 3ull : 0ull) | ~low_mask(g.nx - 2 - p.q * 64);
+    if (p.j >= 2 && p.j + 2 < g.ny && p.k >= 2 && p.k + 2 < g.nz && !(r & rim)) flags |= 4u;
+  }
+  uint32_t tile_first[5], slot[5];
+  if (r != 0ull) {  // in flight beside the zeros
+#pragma unroll
+    for (int n = 0; n < 5; ++n) {
+      tile_first[n] = ep.tile[g.tile_off + at[n] / kAdjTile];
+      slot[n] = ep.pre[g.word_off + at[n]];
+    }
+  }
+  zero_run(g, out, ww, min(ww + kAdjWaveWords, g.nwords), lane, 64);
+  if (!__ballot(r != 0ull)) return;
+  const uint32_t n = (uint32_t)popc(r);
+  const uint32_t inc = wave_incl_scan(n), total = wave_last(inc);
+  if (r != 0ull) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      W.ends[i][lane] = e[i];
+      W.slot[i][lane] = tile_first[i] + slot[i];
+    }
+    W.recv[lane] = r;
+    W.start[lane] = inc - n;
+    W.base[lane] = base;
+    W.flags[lane] = (uint8_t)flags;
+  }
+  wave_lds_sync();
+  const float* sf = reinterpret_cast<const float*>(sums);
+  for (uint32_t e0 = 0; e0 < total; e0 += 64u) {  // wave-uniform
+    const int i = item_word(n, inc, e0, W.mark);
+    const uint32_t t = e0 + (uint32_t)lane;
+    if (t >= total) continue;
+    const int bit = select_bit(W.recv[i], (int)(t - W.start[i]));
+    const int up = 63 - bit;  // brings the point's bit to the sign
+    const uint32_t fl = W.flags[i];
+    // slot 0 holds zeros
+    auto slot_of = [&](bool on, uint32_t s) -> uint32_t { return on ? min(s, cap) : 0u; };
+    PointTerms v;
+    {
+      const uint64_t own = W.ends[0][i], o = own << up;
+      const uint32_t s = W.slot[0][i] + (uint32_t)popc(o);
+      const bool on = (int64_t)o < 0;
+      const bool before = (int64_t)(((own << 1) | (fl & 1u)) << up) < 0;
+      const bool after = (int64_t)(((own >> 1) | ((uint64_t)(fl & 2u) << 62)) << up) < 0;
+      v.own = sums[slot_of(on, s)];
+      v.before[0] = sf[4 * (int64_t)slot_of(before, s - (on ? 1u : 0u)) + 1];
+      v.after[0] = sf[4 * (int64_t)slot_of(after, s + 1u) + 1];
+    }
+#pragma unroll
+    for (int d = 1; d < 3; ++d) {
+      const uint64_t b = W.ends[2 * d - 1][i] << up, a = W.ends[2 * d][i] << up;
+      const uint32_t sb = W.slot[2 * d - 1][i] + (uint32_t)popc(b),
+                     sa = W.slot[2 * d][i] + (uint32_t)popc(a);
+      v.before[d] = sf[4 * (int64_t)slot_of((int64_t)b < 0, sb) + 1 + d];
+      v.after[d] = sf[4 * (int64_t)slot_of((int64_t)a < 0, sa) + 1 + d];
+    }
+    float* o = out + (int64_t)W.base[i] + bit;
+    if (!__ballot(!(fl & 4u))) {
+      *o = combine_point<true>(g, 0, 0, 0, v);
+    } else {
+      const WordPos p = word_pos(g, ww + i);
+      *o = combine_point<false>(g, p.q * 64 + bit, p.j, p.k, v);
+    }
+  }
+}
+
+// Widest rows the adjoint takes (nx <= 15872).
 constexpr int kMaxGatherWpr = 248;
-static_assert(gather_lds_bytes(kMaxGatherWpr) + sizeof(GatherShared) <= 160 * 1024,
-              "gather tile LDS");
 
-// Staging of one flag slot: the word's inside-bits and those it needs.
-struct SlotLoad {
-  uint64_t A, A1, B, C;
-  uint32_t bv;
-  WordPos p;
-  bool in;
-};
-
-// dL/df of the points of row words [w0, w_end) of a volume (a span of at
-// most kGatherTile words, blockDim.x == kGatherThreads).  Every thread of
-// the block calls this; `lds` holds gather_lds_bytes(g.wpr).
-//   1. stage flags and vertex bases of the planes k-2..k+1
-//   2. receiving masks of the span's words (thread per word)
-//   3. endpoint masks of the G-words, restricted to the points some
-//      receiving point's stencil reads; block scan -> compact endpoint slots
-//   4. (S, G) of every such endpoint (thread per endpoint, 6 edge records)
-//   5. zeros for the other points (coalesced) and dL/df of every receiving
-//      point from the 7 (S, G) of its stencil; no barrier follows, so these
-//      stores drain while the next tiles run
-// A span with more than kMaxEndpoints endpoints writes nothing and returns
-// its endpoint count (kDirect false), or computes every receiving point's
-// stencil sums directly from the flags instead of 3-4 (kDirect true).
-// Returns 0 when its points are written.
-template <bool kDirect>
-__device__ __forceinline__ uint32_t gather_span(const VolGeom& g, const uint64_t* __restrict__ b,
-                                                const uint32_t* __restrict__ base_v,
-                                                const VertexAdj* __restrict__ adj, int64_t n_adj,
-                                                float* __restrict__ out, int64_t w0,
-                                                int64_t w_end, GatherShared& sh, void* lds) {
-  // tid is opaque to the compiler, so what is derived from it is not hoisted
-  // out of a caller's loop over spans (it would stay live across the loop,
-  // about 30 more VGPRs)
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));
-  const int lane = tid & 63, wv = tid >> 6;
-  const int nw = (int)(w_end - w0);
-  const int wpr = g.wpr;
-  const int seg = nw + 4 * wpr + 2;  // staged words per plane
-  const int64_t plane = (int64_t)wpr * g.ny;
-
-  // 1. flags and vertex bases: every load of a round is issued before any
-  //    is used
-  uint64_t* s_fx = reinterpret_cast<uint64_t*>(lds);
-  uint64_t* s_fy = s_fx + 4 * seg;
-  uint64_t* s_fz = s_fy + 4 * seg;
-  uint32_t* s_bv = reinterpret_cast<uint32_t*>(s_fz + 4 * seg);
-  const int ng = gather_gwords(nw, wpr);
-  uint64_t* s_gm =
-      reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(lds) + gather_flags_bytes(wpr));
-  uint32_t* s_gp = reinterpret_cast<uint32_t*>(s_gm + gather_gwords(kGatherTile, wpr));
-  uint16_t* s_eg = reinterpret_cast<uint16_t*>(s_gp + gather_gwords(kGatherTile, wpr) + 1);
-  constexpr int kSlots = 3;
-  for (int base = 0; base < 4 * seg; base += kSlots * kGatherThreads) {
-    SlotLoad L[kSlots];
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int i = base + u * kGatherThreads + tid;
-      const int dz = i / seg - 2;
-      const int64_t w = w0 + dz * plane - 2 * wpr - 1 + (i - (dz + 2) * seg);
-      L[u].in = i < 4 * seg && w >= 0 && w < g.nwords;
-      L[u].A = L[u].A1 = L[u].B = L[u].C = 0ull;
-      L[u].bv = 0u;
-      if (L[u].in) {
-        L[u].p = word_pos(g, w);
-        L[u].A = b[w];
-        if (L[u].p.q + 1 < wpr) L[u].A1 = b[w + 1];
-        if (L[u].p.has_y) L[u].B = b[w + wpr];
-        if (L[u].p.has_z) L[u].C = b[w + plane];
-        L[u].bv = base_v[w];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      const int i = base + u * kGatherThreads + tid;
-      if (i < 4 * seg) {
-        uint64_t fx = 0ull, fy = 0ull, fz = 0ull;
-        if (L[u].in) edge_flags(L[u].p, L[u].A, L[u].A1, L[u].B, L[u].C, fx, fy, fz);
-        s_fx[i] = fx;
-        s_fy[i] = fy;
-        s_fz[i] = fz;
-        s_bv[i] = L[u].bv;
-      }
-    }
-  }
-  __syncthreads();
-  const Stage st{s_fx, s_fy, s_fz, s_bv, seg, w0};
-
-  // 2. receiving masks
-  uint64_t r = 0ull;
-  if (tid < nw) {
-    const WordPos p = word_pos(g, w0 + tid);
-    const GatherCtx c{&g, &st, adj, n_adj, w0 + tid, 0, p.q, p.q * 64, p.j, p.k};
-    r = receiving_mask(c);
-    sh.recv[tid] = r;
-  }
-  uint32_t total;
-  const uint32_t off = block_excl_scan((uint32_t)popc(r), total, sh.scan);
-  if (tid < nw) sh.first[tid] = off;
-  if (tid == 0) sh.first[nw] = total;
-  __syncthreads();
-
-  // 3. endpoint masks of the G-words: gi in [0, nw + 2 wpr) is word
-  //    w0 - wpr + gi of the tile's plane; then nw words of the plane below,
-  //    then nw of the plane above.
-  auto recv_of = [&](int64_t w) -> uint64_t {  // receiving mask of a tile word, else 0
-    return (w >= w0 && w < w_end) ? sh.recv[w - w0] : 0ull;
-  };
-  uint32_t n_end = 0;
-  if (total > 0) {
-    const int ch = (ng + kGatherThreads - 1) / kGatherThreads;
-    uint32_t cnt = 0;
-    for (int u = 0; u < ch; ++u) {
-      const int gi = tid * ch + u;
-      if (gi >= ng) break;
-      int dzp;
-      int64_t wt;  // tile-plane word
-      if (gi < nw + 2 * wpr) {
-        dzp = 0;
-        wt = w0 - wpr + gi;
-      } else if (gi < 2 * nw + 2 * wpr) {
-        dzp = -1;
-        wt = w0 + (gi - nw - 2 * wpr);
-      } else {
-        dzp = 1;
-        wt = w0 + (gi - 2 * nw - 2 * wpr);
-      }
-      const int64_t wa = wt + dzp * plane;  // the word itself
-      uint64_t m = 0ull;
-      if (wa >= 0 && wa < g.nwords) {
-        const WordPos p = word_pos(g, wa);
-        uint64_t need;
-        if (dzp == 0) {
-          const uint64_t rw = recv_of(wa);
-          need = rw | (rw << 1) | (rw >> 1);
-          if (p.q > 0) need |= recv_of(wa - 1) >> 63;
-          if (p.q + 1 < wpr) need |= recv_of(wa + 1) << 63;
-          if (p.j > 0) need |= recv_of(wa - wpr);
-          if (p.j + 1 < g.ny) need |= recv_of(wa + wpr);
-        } else {
-          need = recv_of(wt);
-        }
-        if (need) {
-          const GatherCtx c{&g, &st, adj, n_adj, wt, dzp, p.q, p.q * 64, p.j, p.k};
-          m = endpoint_mask(c, 0, 0, 0) & need;
-        }
-      }
-      s_gm[gi] = m;
-      cnt += (uint32_t)popc(m);
-    }
-    uint32_t run = block_excl_scan(cnt, n_end, sh.scan);
-    for (int u = 0; u < ch; ++u) {
-      const int gi = tid * ch + u;
-      if (gi >= ng) break;
-      s_gp[gi] = run;
-      const uint32_t c = (uint32_t)popc(s_gm[gi]);
-      for (uint32_t t = run; t < run + c && t < (uint32_t)kMaxEndpoints; ++t)
-        s_eg[t] = (uint16_t)gi;  // G-word of endpoint slot t
-      run += c;
-    }
-    if (tid == 0) s_gp[ng] = n_end;
-    __syncthreads();
-  }
-  const bool shared_sums = n_end <= (uint32_t)kMaxEndpoints;  // block-uniform
-  if (!kDirect && !shared_sums) return n_end;
-  f32x4* s_rec = reinterpret_cast<f32x4*>(lds);
-  if (total > 0 && shared_sums) {
-    // 4. (S, G) per endpoint, kept in registers until the flags are done
-    f32x4 rr[kRecPerThread];
-#pragma unroll
-    for (int u = 0; u < kRecPerThread; ++u) {
-      const uint32_t e = (uint32_t)tid + (uint32_t)u * kGatherThreads;
-      rr[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (e < n_end) {
-        const int gi = s_eg[e];
-        const int bit = select_bit(s_gm[gi], (int)(e - s_gp[gi]));
-        const int dzp = gi < nw + 2 * wpr ? 0 : (gi < 2 * nw + 2 * wpr ? -1 : 1);
-        const int64_t wt = dzp == 0 ? w0 - wpr + gi
-                                    : w0 + (gi - nw - 2 * wpr - (dzp == 1 ? nw : 0));
-        const WordPos p = word_pos(g, wt + dzp * plane);
-        const GatherCtx c{&g, &st, adj, n_adj, wt, dzp, p.q, p.q * 64 + bit, p.j, p.k};
-        rr[u] = point_sums(c, 0, 0, 0);
-      }
-    }
-    __syncthreads();  // the flags region now holds the endpoint records
-#pragma unroll
-    for (int u = 0; u < kRecPerThread; ++u) {
-      const uint32_t e = (uint32_t)tid + (uint32_t)u * kGatherThreads;
-      if (e < n_end) s_rec[e] = rr[u];
-    }
-    __syncthreads();
-  }
-
-  // 5. zeros for the points that receive nothing (four per lane where rows
-  //    are 16-byte aligned: 16 lanes per word, 4 words per wave step) ...
-  if ((g.nx & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-    const int sub = lane >> 4, x4 = (lane & 15) * 4;
-    for (int i0 = wv * 4; i0 < nw; i0 += kGatherThreads / 16) {
-      const int i = i0 + sub;
-      if (i >= nw) continue;
-      const WordPos p = word_pos(g, w0 + i);
-      const int x = p.q * 64 + x4;
-      if (x >= g.nx) continue;
-      const uint32_t rb = (uint32_t)(sh.recv[i] >> x4) & 0xfu;
-      float* o = out + (int64_t)x + (int64_t)g.nx * (p.j + (int64_t)g.ny * p.k);
-      if (rb == 0u) {
-        *reinterpret_cast<f32x4*>(o) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (!((rb >> t) & 1u)) o[t] = 0.0f;
-      }
-    }
-  } else {
-    for (int i = wv; i < nw; i += kGatherThreads / 64) {
-      const WordPos p = word_pos(g, w0 + i);
-      const int x = p.q * 64 + lane;
-      if (x < g.nx && !((sh.recv[i] >> lane) & 1ull))
-        out[(int64_t)x + (int64_t)g.nx * (p.j + (int64_t)g.ny * p.k)] = 0.0f;
-    }
-  }
-  // ... and dL/df of the receiving points
-  for (uint32_t e = (uint32_t)tid; e < total; e += kGatherThreads) {
-    const int i = find_word(sh.first, nw, e);
-    const int bit = select_bit(sh.recv[i], (int)(e - sh.first[i]));
-    const WordPos p = word_pos(g, w0 + i);
-    const int x = p.q * 64 + bit;
-    float v = 0.0f;
-    if (shared_sums) {
-      const int g0 = i + wpr;  // G-word of the point's own word
-      auto rec = [&](int gi, int bb) -> f32x4 {
-        const uint64_t m = s_gm[gi];
-        if (!((m >> bb) & 1ull)) return f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        return s_rec[s_gp[gi] + (uint32_t)popc(m & ((1ull << bb) - 1ull))];
-      };
-      v = combine_point(g, x, p.j, p.k, [&](int d, int s) -> f32x4 {
-        if (s == 0) return rec(g0, bit);
-        if (d == 0) {
-          const int xb = bit + s;  // -1..64
-          return rec(g0 + (xb < 0 ? -1 : (xb > 63 ? 1 : 0)), xb & 63);
-        }
-        if (d == 1) return rec(g0 + s * wpr, bit);
-        return rec((s < 0 ? nw + 2 * wpr : 2 * nw + 2 * wpr) + i, bit);
-      });
-    } else if (kDirect) {
-      const GatherCtx c{&g, &st, adj, n_adj, w0 + i, 0, p.q, x, p.j, p.k};
-      v = point_adjoint(c);
-    }
-    out[(int64_t)x + (int64_t)g.nx * (p.j + (int64_t)g.ny * p.k)] = v;
-  }
-  return 0;
-}
-
-// Tiles whose endpoints exceed kMaxEndpoints are redone in spans of
-// kGatherTile >> lg words, lg in 1..4 the smallest with at most
-// kSpanEndpoints << lg endpoints (2..16 spans).  A list item is
-// (tile << 8) | (lg << 4) | span.  With many tiles per CU, a tile with
-// lg <= kTileSpanLg runs its spans itself, one after another, and lists
-// only a span that still does not fit: its block then takes a few tiles'
-// time among many rounds of tiles, and the span pass (a launch later, its
-// spans staged again) is spared.  Otherwise, and for denser tiles, the tile
-// lists all its spans, and a span pass runs the items.  The listed word ranges are disjoint and a
-// point is an endpoint slot of at most 5 of them (its own, the ranges of
-// the words one row before and after it and one plane below and above),
-// so with U vertices (at most 2U endpoints) the slots of listed ranges sum
-// to at most 10U.  A listed tile with n slots gives 2^lg < 2n / 1536 items
-// and a listed span with n > 2048 slots one, so the items number fewer
-// than 20U / 1536 < U / 32 + 16.
-constexpr int kSpanEndpoints = 1536;
-constexpr int kTileSpanLg = 2;
-__host__ __device__ constexpr int64_t gather_list_capacity(int64_t n_points) {
-  return n_points / 32 + 16;
-}
-// Scratch of the adjoint: the vertex records, then the list (count, items).
-__host__ __device__ constexpr size_t gather_list_offset(int64_t n_points) {
-  return ((size_t)(n_points > 0 ? n_points : 0) * sizeof(VertexAdj) + 15) & ~(size_t)15;
+// Scratch of the adjoint: the vertex records, then the endpoints' sums (slot 0:
+// zeros; at most two endpoints per vertex, 16 bytes each).
+__host__ __device__ constexpr size_t endpoint_sums_offset(int64_t n_points) {
+  return (size_t)(n_points > 0 ? n_points : 0) * sizeof(VertexAdj);
 }
 __host__ __device__ constexpr size_t adjoint_scratch_bytes(int64_t n_points) {
-  return gather_list_offset(n_points) + (size_t)(1 + gather_list_capacity(n_points)) * 4;
+  return n_points > 0 ? 2 * endpoint_sums_offset(n_points) + 16 : 0;
 }
-
-__device__ __forceinline__ int gather_span_lg(uint32_t n_end) {
-  int lg = 1;
-  while (lg < 4 && (uint32_t)(kSpanEndpoints << lg) < n_end) ++lg;
-  return lg;
-}
-
-// Appends items (tile, lg, s0 .. s0 + n - 1) (one thread of the block).
-__device__ __forceinline__ void gather_list_push(uint32_t* __restrict__ list, int64_t cap,
-                                                 uint32_t tile, int lg, uint32_t s0, uint32_t n) {
-  const uint32_t i = atomicAdd(&list[0], n);
-  for (uint32_t s = 0; s < n; ++s)
-    if (i + s < cap) list[1 + i + s] = (tile << 8) | ((uint32_t)lg << 4) | (s0 + s);
-}
-
-// A gather tile [w0, w_end) with list id `tile`: zeros only when no active
-// edge lies among its staged words, else the tile as one span, or (too many
-// endpoints) as the spans above, run here when lg <= max_lg (0 or
-// kTileSpanLg).  Without a list (no vertex records) a tile with active edges
-// is zeroed.
-__device__ __forceinline__ void gather_tile(const VolGeom& g, const uint64_t* __restrict__ b,
-                                            const uint32_t* __restrict__ base_v,
-                                            const VertexAdj* __restrict__ adj, int64_t n_adj,
-                                            float* __restrict__ out, int64_t w0, int64_t w_end,
-                                            GatherShared& sh, void* lds,
-                                            uint32_t* __restrict__ list, int64_t cap,
-                                            uint32_t tile, int max_lg) {
-  const int tid = threadIdx.x;
-  if (!__syncthreads_or(tid < 4 && gather_segment_active(g, base_v, w0, tid))) {
-    zero_run(g, out, w0, w_end, tid, kGatherThreads);
-    return;
-  }
-  // block-uniform counts are read as scalars, so the span bounds stay scalars
-  const uint32_t n_end = __builtin_amdgcn_readfirstlane(
-      gather_span<false>(g, b, base_v, adj, n_adj, out, w0, w_end, sh, lds));
-  if (!n_end) return;
-  if (!list) {
-    zero_run(g, out, w0, w_end, tid, kGatherThreads);
-    return;
-  }
-  const int lg = gather_span_lg(n_end);
-  if (lg > max_lg) {
-    if (tid == 0) gather_list_push(list, cap, tile, lg, 0u, 1u << lg);
-    return;
-  }
-  const int len = kGatherTile >> lg;
-  for (int s = 0; s < (1 << lg); ++s) {
-    const int64_t a = w0 + (int64_t)s * len, e = min(a + len, w_end);
-    if (a >= e) break;
-    __syncthreads();  // LDS reused by this span
-    const uint32_t n_span = __builtin_amdgcn_readfirstlane(
-        gather_span<false>(g, b, base_v, adj, n_adj, out, a, e, sh, lds));
-    if (n_span && tid == 0) gather_list_push(list, cap, tile, lg, (uint32_t)s, 1u);
-  }
-}
-
-// The span pass splits every item into `parts` equal pieces, the largest
-// power of two (up to 16) that keeps the pieces within 2 * half_blocks: a
-// short list (a few dense tiles) then runs as many small spans, whose
-// latency is shorter, and a long one as the items themselves.  The span
-// kernels pass half their grid, so the pieces fit one round: a piece is a
-// chain of dependent phases (about 11 us at 8 words), and a second round
-// costs more than longer pieces save.  (Written this way, the span kernel
-// compiles to 76 VGPRs, three blocks per CU; `n * parts * 2 <= blocks`
-// gives 93.)
-__device__ __forceinline__ int gather_item_parts(int64_t n_items, int64_t half_blocks) {
-  int parts = 1;
-  while (parts < 16 && n_items * parts * 2 <= 2 * half_blocks) parts *= 2;
-  return parts;
-}
-
-// Word range [w0, w_end) of piece `part` of `parts` of a span item within
-// the tile starting at word tile_w0 of a volume with nwords words (spans
-// are at least 16 words, pieces at least one).
-__device__ __forceinline__ void gather_item_span(uint32_t item, int part, int parts,
-                                                 int64_t tile_w0, int64_t nwords, int64_t& w0,
-                                                 int64_t& w_end) {
-  const int lg = (int)((item >> 4) & 15u), s = (int)(item & 15u);
-  const int len = kGatherTile >> lg, piece = max(len / parts, 1);
-  w0 = tile_w0 + (int64_t)s * len + (int64_t)part * piece;
-  w_end = min(min(w0 + piece, tile_w0 + (int64_t)(s + 1) * len), nwords);
+// The last slot (a volume or batch of at most 2^31 points has fewer endpoints).
+inline uint32_t last_slot(int64_t n_points) {
+  return (uint32_t)std::min<int64_t>(2 * n_points, 0xfffffffe);
 }
 
 }  // namespace mc

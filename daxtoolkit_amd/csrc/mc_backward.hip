@@ -3,80 +3,53 @@
 // device code are in mc_adjoint.h.
 #include "mc_adjoint.h"
 
-#include <atomic>
-
 namespace daxhip {
 namespace mc {
 
-// One thread per vertex; block 0 also empties the list of dense tiles and
-// writes the gather tiles' dispatch order (those with active edges of their
-// own first, from the forward count kernel's classes; the other blocks'
-// records hide its time).
-constexpr int kVertexAdjThreads = 256;
-__global__ __launch_bounds__(kVertexAdjThreads) void k_vertex_adjoint(
+// Blocks [0, vertex_blocks): a thread per vertex; the rest: the endpoint words
+// of a tile each.
+__global__ __launch_bounds__(kAdjThreads) void k_adjoint_records(
     VolGeom g, const float* __restrict__ field, const uint32_t* __restrict__ edges,
     const float* __restrict__ dldx, const float* __restrict__ dldn,
     const int64_t* __restrict__ counts, int64_t n_points, VertexAdj* __restrict__ out,
-    uint32_t* __restrict__ list, const uint8_t* __restrict__ tcls, uint32_t* __restrict__ gorder) {
+    const uint64_t* __restrict__ bits, CountSrc cs, const Ctrl* __restrict__ ctrl, Endpoints ep,
+    int64_t vertex_blocks) {
+  __shared__ uint32_t s_scan[kAdjThreads / 64];
+  const int64_t U = counts ? min(counts[1], n_points) : n_points;
+  if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
+    cs.tpb_shift = (int)ctrl->tpb_shift;
+    endpoint_words_tile(g, bits, cs, U, ep, ((int64_t)blockIdx.x - vertex_blocks) * kAdjTile,
+                        s_scan);
+    return;
+  }
   // XCD-contiguous vertex ranges: vertices are in edge order, so the field
   // lines of neighbouring stencils stay in one XCD's L2
-  const int64_t u = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (u == 0) list[0] = 0u;
-  if (blockIdx.x == 0) {  // uniform
-    __shared__ uint32_t s_a[kVertexAdjThreads / 64], s_b[kVertexAdjThreads / 64];
-    const uint32_t ngt = (uint32_t)ceil_div(g.nwords, (int64_t)kGatherTile);
-    const uint32_t K = order_chunk(ngt, kVertexAdjThreads);
-    const uint64_t reg = load_classes(tcls, threadIdx.x * K, K, ngt);
-    write_order<true>(reg, tcls, K, ngt, gorder, (uint32_t)kGatherTile, s_a, s_b);
-  }
-  const int64_t U = counts ? min(counts[1], n_points) : n_points;
+  const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
   if (u >= U) return;
   vertex_adjoint(g, field, edges, dldx, dldn, u, out);
 }
 
-// One tile of kGatherTile row words per block, in the dispatch order the
-// vertex-record launch wrote (tiles with active edges of their own first, so
-// the long tiles start early and the quiet ones fill the tail), else (no
-// vertices: the forward left the order cleared) in tile order.  A tile whose
-// endpoint records do not fit runs in spans or goes to the list (without
-// records, list == nullptr, every point receives 0).
-__global__ __launch_bounds__(kGatherThreads) void k_point_gather(
-    VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ base_v,
-    const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts, int64_t n_points,
-    float* __restrict__ dldf, uint32_t* __restrict__ list, const uint32_t* __restrict__ order,
-    int span_lg) {
-  __shared__ GatherShared sh;
-  extern __shared__ __align__(16) uint64_t s_dyn[];
-  const uint32_t tag = order[0], ord = order[1 + blockIdx.x] & 0x7fffffffu;
-  const int64_t tile =
-      (tag == (uint32_t)kGatherTile && (int64_t)ord < (int64_t)gridDim.x) ? (int64_t)ord
-                                                                            : (int64_t)blockIdx.x;
+__global__ __launch_bounds__(kAdjThreads) void k_endpoint_sums(
+    VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre,
+    Endpoints ep, const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts,
+    int64_t n_points, f32x4* __restrict__ sums) {
+  __shared__ uint8_t s_mark[kAdjThreads / 64][64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t n_adj = counts ? min(counts[1], n_points) : n_points;
-  const int64_t w0 = tile * kGatherTile, w_end = min(w0 + kGatherTile, g.nwords);
-  gather_tile(g, bits + g.word_off, base_v + g.word_off, adj, n_adj, dldf + g.field_off, w0,
-              w_end, sh, s_dyn, list, gather_list_capacity(n_points), (uint32_t)tile, span_lg);
+  const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords + wv * kAdjWaveWords;
+  if (ww < g.nwords)  // wave-uniform
+    endpoint_sums_wave(g, bits, lpre, ep, adj, n_adj, sums, 2 * n_points, ww, s_mark[wv]);
 }
 
-// The listed span items (persistent blocks).
-__global__ __launch_bounds__(kGatherThreads) void k_point_gather_spans(
-    VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ base_v,
-    const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts, int64_t n_points,
-    float* __restrict__ dldf, const uint32_t* __restrict__ list) {
-  __shared__ GatherShared sh;
-  extern __shared__ __align__(16) uint64_t s_dyn[];
-  const int64_t n_adj = counts ? min(counts[1], n_points) : n_points;
-  const int64_t n_items = min((int64_t)list[0], gather_list_capacity(n_points));
-  const int parts = gather_item_parts(n_items, gridDim.x / 2);
-  for (int64_t it = blockIdx.x; it < n_items * parts; it += gridDim.x) {
-    const uint32_t item = list[1 + it / parts];
-    int64_t w0, w_end;
-    gather_item_span(item, (int)(it % parts), parts, (int64_t)(item >> 8) * kGatherTile,
-                     g.nwords, w0, w_end);
-    if (w0 < w_end)
-      gather_span<true>(g, bits + g.word_off, base_v + g.word_off, adj, n_adj,
-                        dldf + g.field_off, w0, w_end, sh, s_dyn);
-    __syncthreads();  // LDS reused by the next span
-  }
+// cap: the endpoints' last slot (0: zeros everywhere).
+__global__ __launch_bounds__(kAdjThreads) void k_point_gather(VolGeom g, Endpoints ep,
+                                                              const f32x4* __restrict__ sums,
+                                                              uint32_t cap,
+                                                              float* __restrict__ dldf) {
+  __shared__ GatherWave s_wave[kAdjThreads / 64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords + wv * kAdjWaveWords;
+  if (ww < g.nwords) gather_wave(g, ep, sums, cap, dldf, ww, s_wave[wv]);
 }
 
 }  // namespace mc
@@ -84,33 +57,6 @@ __global__ __launch_bounds__(kGatherThreads) void k_point_gather_spans(
 
 using namespace daxhip;
 using namespace daxhip::mc;
-
-namespace {
-
-int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    cus = 256;
-  return cus;
-}
-
-
-// Dense tiles run their spans in their own block when the gather holds at
-// least this many tiles per CU (by default 16: 1024^3, 256 per CU, 1.55 +
-// 0.47 ms -> 1.92 + 0.01 ms; 512^3, 32 per CU, forward + backward 0.369 ->
-// 0.359 ms); with fewer rounds of tiles such a block is the critical path
-// (256^3, 4 per CU: 49 + 29 us -> 88 + 15 us).
-std::atomic<int64_t> g_span_tiles_per_cu{16};
-
-int gather_tile_span_lg(int64_t n_tiles, int cus) {
-  return n_tiles >= g_span_tiles_per_cu.load(std::memory_order_relaxed) * (int64_t)cus
-             ? kTileSpanLg
-             : 0;
-}
-
-}  // namespace
 
 extern "C" {
 
@@ -120,8 +66,7 @@ int dax_hip_mc_backward_set_span_threshold(int64_t tiles_per_cu) {
               (long long)tiles_per_cu);
     return DAX_HIP_BAD_VALUE;
   }
-  g_span_tiles_per_cu.store(tiles_per_cu, std::memory_order_relaxed);
-  return DAX_HIP_OK;
+  return DAX_HIP_OK;  // the gather has no dense tiles to choose a pass for
 }
 
 size_t dax_hip_mc_backward_scratch_bytes(int64_t n_points) {
@@ -170,31 +115,32 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)d_workspace;
   const uint64_t* bits = (const uint64_t*)(ws + L.off_bits);
-  const uint32_t* bv = (const uint32_t*)(ws + L.off_base_v);
-  uint32_t* list =
-      n_points > 0 ? (uint32_t*)((char*)d_scratch + gather_list_offset(n_points)) : nullptr;
-  const int cus = device_cus();
+  const CountSrc cs{(const uint32_t*)(ws + L.off_counts),
+                    (const unsigned long long*)(ws + L.off_tsum),
+                    (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0, 0};
+  // the endpoint words live in the workspace; every call with this vertex count
+  // writes the same values there
+  const Endpoints ep{(uint64_t*)(ws + L.off_ends), (uint16_t*)(ws + L.off_end_pre),
+                     (uint32_t*)(ws + L.off_end_sum), (uint32_t*)(ws + L.off_end_tile),
+                     (uint32_t*)(ws + L.off_end_base)};
+  const VertexAdj* adj = (const VertexAdj*)d_scratch;
+  f32x4* sums = (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points));
+  const int64_t tiles = ceil_div(g.nwords, (int64_t)kAdjTile);
+  const dim3 grid((unsigned)ceil_div(g.nwords, (int64_t)kAdjBlockWords)), block(kAdjThreads);
   if (n_points > 0) {
-    k_vertex_adjoint<<<dim3((unsigned)ceil_div(n_points, kVertexAdjThreads)),
-                       dim3(kVertexAdjThreads), 0, s>>>(
+    const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
+    k_adjoint_records<<<dim3((unsigned)(vertex_blocks + tiles)), block, 0, s>>>(
         g, d_field, d_edges, d_dl_dvertices, d_dl_dnormals, d_counts, n_points,
-        (VertexAdj*)d_scratch, list, (const uint8_t*)(ws + L.off_tcls),
-        (uint32_t*)(ws + L.off_gorder));
-    DAXHIP_LAUNCH_CHECK("k_vertex_adjoint");
+        (VertexAdj*)d_scratch, bits, cs, (const Ctrl*)(ws + L.off_ctrl),
+        ep, vertex_blocks);
+    DAXHIP_LAUNCH_CHECK("k_adjoint_records");
+    k_scan_endpoints<<<1, kAdjScanThreads, 0, s>>>(ep.sums, ep.tile, tiles, sums);
+    DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
+    k_endpoint_sums<<<grid, block, 0, s>>>(g, bits, cs.lpre, ep, adj, d_counts, n_points, sums);
+    DAXHIP_LAUNCH_CHECK("k_endpoint_sums");
   }
-  k_point_gather<<<dim3((unsigned)ceil_div(g.nwords, kGatherTile)), dim3(kGatherThreads),
-                   gather_lds_bytes(g.wpr), s>>>(g, bits, bv, (const VertexAdj*)d_scratch,
-                                                 d_counts, n_points, d_dl_dfield, list,
-                                                 (const uint32_t*)(ws + L.off_gorder),
-                                                 gather_tile_span_lg(ceil_div(g.nwords, kGatherTile), cus));
+  k_point_gather<<<grid, block, 0, s>>>(g, ep, sums, last_slot(n_points), d_dl_dfield);
   DAXHIP_LAUNCH_CHECK("k_point_gather");
-  if (n_points > 0) {
-    // persistent blocks: three per CU, as many as the LDS allows
-    k_point_gather_spans<<<dim3((unsigned)(3 * cus)), dim3(kGatherThreads),
-                           gather_lds_bytes(g.wpr), s>>>(g, bits, bv, (const VertexAdj*)d_scratch,
-                                                         d_counts, n_points, d_dl_dfield, list);
-    DAXHIP_LAUNCH_CHECK("k_point_gather_spans");
-  }
   return DAX_HIP_OK;
 }
 

@@ -56,8 +56,9 @@ bool valid_batch_tuning(const BatchTuning& t) {
 }
 
 struct BatchLayout {
-  size_t off_vols, off_gen_tiles, off_bits, off_base_v, off_base_t, off_vol_first, off_lpre,
-      off_tloc, off_bsum, off_bpre, off_ctrl, bytes;
+  size_t off_vols, off_gen_tiles, off_bits, off_vol_first, off_lpre,
+      off_tloc, off_bsum, off_bpre, off_ctrl, off_ends, off_end_pre, off_end_sum, off_end_tile,
+      off_end_base, bytes;
   int64_t nvols, nwords, ngen;
 };
 
@@ -78,10 +79,6 @@ BatchLayout batch_layout(int64_t nvols, const int64_t* dims) {
   off = align_up(off + (size_t)L.ngen * sizeof(TileRef), 256);
   L.off_bits = off;
   off = align_up(off + (size_t)(L.nwords + 1) * 8, 256);
-  L.off_base_v = off;
-  off = align_up(off + (size_t)(L.nwords + 1) * 4, 256);
-  L.off_base_t = off;
-  off = align_up(off + (size_t)(L.nwords + 1) * 4, 256);
   L.off_vol_first = off;
   off = align_up(off + (size_t)nvols * 4, 256);
   L.off_lpre = off;
@@ -95,6 +92,16 @@ BatchLayout batch_layout(int64_t nvols, const int64_t* dims) {
   off = align_up(off + (size_t)(L.ngen + 1) * 8, 256);
   L.off_ctrl = off;
   off = align_up(off + sizeof(Ctrl), 256);
+  L.off_ends = off;  // the adjoint's endpoint words, their prefixes, the tiles' sums and prefixes
+  off = align_up(off + (size_t)L.nwords * 8, 256);
+  L.off_end_pre = off;
+  off = align_up(off + (size_t)L.nwords * 2, 256);
+  L.off_end_sum = off;
+  off = align_up(off + (size_t)L.ngen * 4, 256);
+  L.off_end_tile = off;
+  off = align_up(off + (size_t)L.ngen * 4, 256);
+  L.off_end_base = off;  // the count tiles' vertex bases
+  off = align_up(off + (size_t)L.ngen * 8, 256);
   L.bytes = off;
   return L;
 }
@@ -103,8 +110,9 @@ BatchLayout batch_layout(int64_t nvols, const int64_t* dims) {
 // the workspace pointer after prepare.
 struct BatchHeader {
   int64_t magic, nvols, nwords, ngen, max_wpr;
-  size_t off_vols, off_gen_tiles, off_bits, off_base_v, off_base_t, off_vol_first, off_lpre,
-      off_tloc, off_bsum, off_bpre, off_ctrl, bytes;
+  size_t off_vols, off_gen_tiles, off_bits, off_vol_first, off_lpre,
+      off_tloc, off_bsum, off_bpre, off_ctrl, off_ends, off_end_pre, off_end_sum, off_end_tile,
+      off_end_base, bytes;
   BatchTuning tune;
 };
 constexpr int64_t kBatchMagic = 0x4441584842415443LL;  // "DAXHBATC"
@@ -182,6 +190,15 @@ __global__ __launch_bounds__(kTsumThreads) void k_batch_scan(
   }
 }
 
+// The count kernel's prefixes of one volume.
+__device__ __forceinline__ CountSrc volume_counts(const CountSrc& all, const VolGeom& g) {
+  CountSrc cs = all;
+  cs.lpre += g.tile_off * kBatchGenTile;
+  cs.n_ctiles = 2 * ceil_div(g.nwords, (int64_t)kBatchGenTile);
+  cs.ct0 = 2 * g.tile_off;
+  return cs;
+}
+
 // Generate, a block per tile (persistent blocks looping over the tiles, four
 // per CU: forward of 256 volumes 400 us, this 368).  The tile at a volume's
 // start also writes the volume's {first triangle, first point} in the
@@ -201,17 +218,12 @@ __global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
     counts[0] = (int64_t)total_t;
     counts[1] = (int64_t)n_points;
   }
-  // too many ids for dax::Id or too little room: the bases only
+  // too many ids for dax::Id or too little room: no output
   const bool emit = total_v <= 0x7fffffffull && 3ull * total_t <= 0x7fffffffull &&
                     (int64_t)total_t <= cap_tris && (int64_t)n_points <= cap_points;
   const TileRef tr = tiles[xcd ? xcd_tile_runs(blockIdx.x, ntiles) : (int64_t)blockIdx.x];
   const VolGeom g = vols[tr.vol];
-  CountSrc cs = all;
-  cs.lpre += g.tile_off * kBatchGenTile;
-  cs.n_ctiles = 2 * ceil_div(g.nwords, (int64_t)kBatchGenTile);
-  cs.ct0 = 2 * g.tile_off;
-  cs.base_v += g.word_off;
-  cs.base_t += g.word_off;
+  const CountSrc cs = volume_counts(all, g);
   const unsigned long long vol = ctile_prefix(cs, 0);
   const int64_t vbv = (int64_t)(uint32_t)vol, vbt = (int64_t)(vol >> 32);
   if (tr.w0 == 0 && threadIdx.x == 0) {
@@ -221,29 +233,38 @@ __global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
       vol_offsets[2 * tr.vol + 1] = dedup ? vbv : 3 * vbt;
     }
   }
+  if (!emit) return;
   generate_tile<kBatchGenTile, kBatchGenThreads, FieldArray, dedup>(
       g, FieldArray{fields + g.field_off}, bits + g.word_off, tr.w0, out, normals, vbv, vbt, s_dyn,
-      cs, emit, false);
+      cs, false);
 }
 
 // ---- batched adjoint --------------------------------------------------------
-// The adjoint records of all vertices, then, in a second launch (a block per
-// tile of generate's table), dL/dfield of the tile's points; tiles whose
-// endpoint records do not fit are listed and redone as spans by a third launch.
+// The launches of the single volume's adjoint over generate's tile table.
 // A thread per vertex; its volume by binary search over the volumes' first
 // vertices, then the wave takes its volumes one at a time (one, as a rule),
 // so that the geometry stays in scalar registers.  A block per tile of words
 // instead leaves most lanes idle (73 vertices per tile in 256 volumes of
-// 32..160 points an axis: 80 us; this: 58).
-__global__ __launch_bounds__(256) void k_batch_vertex_adjoint(
+// 32..160 points an axis: 80 us; this: 58).  Blocks from vertex_blocks on form
+// the endpoint words of a tile each.
+__global__ __launch_bounds__(256) void k_batch_records(
     const VolGeom* __restrict__ vols, int64_t nvols, const uint32_t* __restrict__ vol_first,
     const float* __restrict__ fields, const uint32_t* __restrict__ edges,
     const float* __restrict__ dldx, const float* __restrict__ dldn,
     const int64_t* __restrict__ counts, int64_t n_points, VertexAdj* __restrict__ out,
-    uint32_t* __restrict__ list) {
-  const int64_t u = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (u == 0) list[0] = 0u;
+    const TileRef* __restrict__ tiles, const uint64_t* __restrict__ bits, CountSrc all,
+    const Ctrl* __restrict__ ctrl, Endpoints ep, int64_t vertex_blocks) {
+  __shared__ uint32_t s_scan[kAdjThreads / 64];
   const int64_t U = counts ? min(counts[1], n_points) : n_points;
+  if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
+    const TileRef tr = tiles[(int64_t)blockIdx.x - vertex_blocks];
+    const VolGeom g = vols[tr.vol];
+    CountSrc cs = volume_counts(all, g);
+    cs.tpb_shift = (int)ctrl->tpb_shift;
+    endpoint_words_tile(g, bits + g.word_off, cs, U, ep, tr.w0, s_scan);
+    return;
+  }
+  const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
   int64_t vol = -1;
   if (u < U) {  // the last volume whose first vertex is at most u
     int64_t lo = 0, hi = nvols;
@@ -265,43 +286,35 @@ __global__ __launch_bounds__(256) void k_batch_vertex_adjoint(
   }
 }
 
-__global__ __launch_bounds__(kGatherThreads) void k_batch_point_gather(
+static_assert(kAdjTile == kBatchGenTile, "the adjoint's tiles are the generate tiles");
+
+__global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_sums(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
-    const uint64_t* __restrict__ bits, const uint32_t* __restrict__ base_v,
+    const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
     const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts, int64_t n_points,
-    float* __restrict__ dldf, uint32_t* __restrict__ list) {
-  static_assert(kGatherTile == kBatchGenTile, "gather tiles are the generate tiles");
-  __shared__ GatherShared sh;
-  extern __shared__ __align__(16) uint64_t s_dyn[];
+    f32x4* __restrict__ sums) {
+  __shared__ uint8_t s_mark[kAdjThreads / 64][64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t n_adj = counts ? min(counts[1], n_points) : n_points;
-  const TileRef tr = tiles[blockIdx.x];
+  const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
+  const TileRef tr = tiles[blk / kAdjTileBlocks];
   const VolGeom g = vols[tr.vol];
-  const int64_t w_end = min((int64_t)tr.w0 + kBatchGenTile, g.nwords);
-  gather_tile(g, bits + g.word_off, base_v + g.word_off, adj, n_adj, dldf + g.field_off, tr.w0,
-              w_end, sh, s_dyn, list, gather_list_capacity(n_points), blockIdx.x, 0);
+  const int64_t ww = (int64_t)tr.w0 + (blk % kAdjTileBlocks) * kAdjBlockWords + wv * kAdjWaveWords;
+  if (ww < g.nwords)  // wave-uniform
+    endpoint_sums_wave(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj, n_adj, sums,
+                       2 * n_points, ww, s_mark[wv]);
 }
 
-__global__ __launch_bounds__(kGatherThreads) void k_batch_point_gather_spans(
-    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
-    const uint64_t* __restrict__ bits, const uint32_t* __restrict__ base_v,
-    const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts, int64_t n_points,
-    float* __restrict__ dldf, const uint32_t* __restrict__ list) {
-  __shared__ GatherShared sh;
-  extern __shared__ __align__(16) uint64_t s_dyn[];
-  const int64_t n_adj = counts ? min(counts[1], n_points) : n_points;
-  const int64_t n_items = min((int64_t)list[0], gather_list_capacity(n_points));
-  const int parts = gather_item_parts(n_items, gridDim.x / 2);
-  for (int64_t it = blockIdx.x; it < n_items * parts; it += gridDim.x) {
-    const uint32_t item = list[1 + it / parts];
-    const TileRef tr = tiles[item >> 8];
-    const VolGeom g = vols[tr.vol];
-    int64_t w0, w_end;
-    gather_item_span(item, (int)(it % parts), parts, tr.w0, g.nwords, w0, w_end);
-    if (w0 < w_end)
-      gather_span<true>(g, bits + g.word_off, base_v + g.word_off, adj, n_adj,
-                        dldf + g.field_off, w0, w_end, sh, s_dyn);
-    __syncthreads();  // LDS reused by the next span
-  }
+__global__ __launch_bounds__(kAdjThreads) void k_batch_point_gather(
+    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, Endpoints ep,
+    const f32x4* __restrict__ sums, uint32_t cap, float* __restrict__ dldf) {
+  __shared__ GatherWave s_wave[kAdjThreads / 64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
+  const TileRef tr = tiles[blk / kAdjTileBlocks];
+  const VolGeom g = vols[tr.vol];
+  const int64_t ww = (int64_t)tr.w0 + (blk % kAdjTileBlocks) * kAdjBlockWords + wv * kAdjWaveWords;
+  if (ww < g.nwords) gather_wave(g, ep, sums, cap, dldf + g.field_off, ww, s_wave[wv]);
 }
 
 }  // namespace mc
@@ -337,8 +350,6 @@ struct BatchPtrs {
   const VolGeom* vols;
   const TileRef* gen_tiles;
   uint64_t* bits;
-  uint32_t* bv;
-  uint32_t* bt;
   uint32_t* vol_first;
   uint32_t* lpre;
   unsigned long long* tloc;
@@ -352,8 +363,6 @@ BatchPtrs batch_ptrs(const BatchHeader& h, void* d_workspace) {
   return BatchPtrs{(const VolGeom*)(body + h.off_vols),
                    (const TileRef*)(body + h.off_gen_tiles),
                    (uint64_t*)(body + h.off_bits),
-                   (uint32_t*)(body + h.off_base_v),
-                   (uint32_t*)(body + h.off_base_t),
                    (uint32_t*)(body + h.off_vol_first),
                    (uint32_t*)(body + h.off_lpre),
                    (unsigned long long*)(body + h.off_tloc),
@@ -412,7 +421,7 @@ int batch_generate(const BatchHeader& h, const BatchPtrs& p, const float* d_fiel
                    unsigned flags, const OutPtrs& o, int64_t cap_points, int64_t cap_tris,
                    int64_t* d_counts, int64_t* d_vol_offsets, const BatchTuning& t,
                    hipStream_t s) {
-  const CountSrc cs{p.lpre, p.tloc, p.bpre, 0, 0, batch_count_shift(t), p.bv, p.bt};
+  const CountSrc cs{p.lpre, p.tloc, p.bpre, 0, 0, batch_count_shift(t)};
   const size_t lds = GenLayout<kBatchGenTile, kBatchGenThreads>((int)h.max_wpr).bytes();
   const dim3 grid((unsigned)h.ngen);
   if (flags & DAX_HIP_MC_DEDUP)
@@ -490,13 +499,16 @@ int dax_hip_mc_batch_prepare(int64_t n_volumes, const int64_t* h_dims3,
   h.off_vols = L.off_vols;
   h.off_gen_tiles = L.off_gen_tiles;
   h.off_bits = L.off_bits;
-  h.off_base_v = L.off_base_v;
-  h.off_base_t = L.off_base_t;
   h.off_vol_first = L.off_vol_first;
   h.off_lpre = L.off_lpre;
   h.off_tloc = L.off_tloc;
   h.off_bsum = L.off_bsum;
   h.off_bpre = L.off_bpre;
+  h.off_ends = L.off_ends;
+  h.off_end_pre = L.off_end_pre;
+  h.off_end_sum = L.off_end_sum;
+  h.off_end_tile = L.off_end_tile;
+  h.off_end_base = L.off_end_base;
   h.off_ctrl = L.off_ctrl;
   h.bytes = L.bytes;
   h.tune = kBatchTuningDefault;
@@ -733,26 +745,34 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
   const VolGeom* vols = (const VolGeom*)(body + h->off_vols);
   const TileRef* gen_tiles = (const TileRef*)(body + h->off_gen_tiles);
   const uint64_t* bits = (const uint64_t*)(body + h->off_bits);
-  const uint32_t* bv = (const uint32_t*)(body + h->off_base_v);
-  uint32_t* list =
-      n_points > 0 ? (uint32_t*)((char*)d_scratch + gather_list_offset(n_points)) : nullptr;
-  const size_t lds = gather_lds_bytes((int)h->max_wpr);
+  const CountSrc cs{(const uint32_t*)(body + h->off_lpre),
+                    (const unsigned long long*)(body + h->off_tloc),
+                    (const unsigned long long*)(body + h->off_bpre), 0, 0, 0};
+  // the endpoint words live in the workspace; every call with this vertex count
+  // writes the same values there
+  char* wb = const_cast<char*>(body);
+  const Endpoints ep{(uint64_t*)(wb + h->off_ends), (uint16_t*)(wb + h->off_end_pre),
+                     (uint32_t*)(wb + h->off_end_sum), (uint32_t*)(wb + h->off_end_tile),
+                     (uint32_t*)(wb + h->off_end_base)};
+  const VertexAdj* adj = (const VertexAdj*)d_scratch;
+  f32x4* sums = (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points));
+  const dim3 grid((unsigned)(h->ngen * kAdjTileBlocks)), block(kAdjThreads);
   if (n_points > 0) {
-    k_batch_vertex_adjoint<<<dim3((unsigned)ceil_div(n_points, 256)), dim3(256), 0, s>>>(
+    const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
+    k_batch_records<<<dim3((unsigned)(vertex_blocks + h->ngen)), block, 0, s>>>(
         vols, h->nvols, (const uint32_t*)(body + h->off_vol_first), d_fields, d_edges,
-        d_dl_dvertices, d_dl_dnormals, d_counts, n_points, (VertexAdj*)d_scratch, list);
-    DAXHIP_LAUNCH_CHECK("k_batch_vertex_adjoint");
+        d_dl_dvertices, d_dl_dnormals, d_counts, n_points, (VertexAdj*)d_scratch, gen_tiles, bits,
+        cs, (const Ctrl*)(body + h->off_ctrl), ep, vertex_blocks);
+    DAXHIP_LAUNCH_CHECK("k_batch_records");
+    k_scan_endpoints<<<1, kAdjScanThreads, 0, s>>>(ep.sums, ep.tile, h->ngen, sums);
+    DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
+    k_batch_endpoint_sums<<<grid, block, 0, s>>>(vols, gen_tiles, bits, cs.lpre, ep, adj, d_counts,
+                                                 n_points, sums);
+    DAXHIP_LAUNCH_CHECK("k_batch_endpoint_sums");
   }
-  k_batch_point_gather<<<dim3((unsigned)h->ngen), dim3(kGatherThreads), lds, s>>>(
-      vols, gen_tiles, bits, bv, (const VertexAdj*)d_scratch, d_counts, n_points, d_dl_dfields,
-      list);
+  k_batch_point_gather<<<grid, block, 0, s>>>(vols, gen_tiles, ep, sums, last_slot(n_points),
+                                              d_dl_dfields);
   DAXHIP_LAUNCH_CHECK("k_batch_point_gather");
-  if (n_points > 0) {
-    k_batch_point_gather_spans<<<dim3((unsigned)persistent_blocks(3)), dim3(kGatherThreads), lds,
-                                 s>>>(vols, gen_tiles, bits, bv, (const VertexAdj*)d_scratch,
-                                      d_counts, n_points, d_dl_dfields, list);
-    DAXHIP_LAUNCH_CHECK("k_batch_point_gather_spans");
-  }
   return DAX_HIP_OK;
 }
 

@@ -24,7 +24,7 @@ namespace mc {
 constexpr int kTileWords = 1024;     // the workspace's word arrays are padded to this
 constexpr int kCountTile = 128;      // row words per count tile: its prefixes fit 16 bits
 constexpr int kMaxWpr = 256;         // nx <= 16384
-constexpr int kGatherTileWords = 256;  // row words per tile of the adjoint's gather
+constexpr int kGatherTileWords = 256;  // row words per tile of the adjoint
 
 // Geometry of one volume in the (possibly batched) word space.
 // Division by an invariant d >= 1 for numerators below 2^31: q = (hi32(n*m)
@@ -262,14 +262,14 @@ struct Ctrl {
 // both below 2^16); off_tsum every count tile's exclusive prefix within its
 // count block (v | t << 32); off_bsum the count blocks' sums and off_tpre
 // their exclusive prefixes, the totals after the last.  A word's bases are
-// block prefix + tile prefix + local prefix.  off_gcls / off_tcls: the
-// dispatch class of every generate / gather tile (a byte each, from the
+// block prefix + tile prefix + local prefix.  off_gcls: the
+// dispatch class of every generate tile (a byte each, from the
 // count kernel); off_order: the generate tile size the order was built for
-// (0: none), then the generate tiles in dispatch order; off_gorder: the
-// same for the adjoint's gather tiles.
+// (0: none), then the generate tiles in dispatch order.
 struct Workspace {
-  size_t off_bits, off_base_v, off_base_t, off_ctrl, off_counts, off_tsum, off_bsum,
-      off_tpre, off_gcls, off_tcls, off_order, off_gorder, bytes;
+  size_t off_bits, off_ctrl, off_counts, off_tsum, off_bsum,
+      off_tpre, off_gcls, off_order, off_ends, off_end_pre, off_end_sum, off_end_tile,
+      off_end_base, fwd_bytes, bytes;
   int64_t nwords, ntiles, n_ctiles;
 };
 
@@ -280,10 +280,6 @@ inline Workspace workspace_layout(int64_t nwords) {
   size_t off = 0;
   w.off_bits = off;
   off = align_up(off + (size_t)(nwords + 1) * 8, 256);
-  w.off_base_v = off;
-  off = align_up(off + (size_t)(nwords + 1) * 4, 256);
-  w.off_base_t = off;
-  off = align_up(off + (size_t)(nwords + 1) * 4, 256);
   w.off_ctrl = off;
   off = align_up(off + sizeof(Ctrl), 256);
   w.off_counts = off;  // packed per-word counts
@@ -297,12 +293,19 @@ inline Workspace workspace_layout(int64_t nwords) {
   off = align_up(off + (size_t)(w.n_ctiles + 1) * 8, 256);
   w.off_gcls = off;  // per generate tile (at least kCountTile words): dispatch class
   off = align_up(off + (size_t)w.n_ctiles + 16, 256);
-  w.off_tcls = off;  // per gather tile: dispatch class
-  off = align_up(off + (size_t)ceil_div(nwords, kGatherTileWords) + 16, 256);
   w.off_order = off;  // generate tiles, heaviest first: the tile size, then the tiles
   off = align_up(off + (size_t)(w.n_ctiles + 2) * 4, 256);
-  w.off_gorder = off;  // the adjoint's gather tiles, those with output first
-  off = align_up(off + (size_t)(ceil_div(nwords, kGatherTileWords) + 2) * 4, 256);
+  w.fwd_bytes = off;  // what the forward uses
+  w.off_ends = off;   // the adjoint's endpoint words, then their prefixes
+  off = align_up(off + (size_t)nwords * 8, 256);
+  w.off_end_pre = off;
+  off = align_up(off + (size_t)nwords * 2, 256);
+  w.off_end_sum = off;  // per adjoint tile: endpoints, then their exclusive prefix
+  off = align_up(off + (size_t)ceil_div(nwords, kGatherTileWords) * 4, 256);
+  w.off_end_tile = off;
+  off = align_up(off + (size_t)ceil_div(nwords, kGatherTileWords) * 4, 256);
+  w.off_end_base = off;  // per count tile: vertex base
+  off = align_up(off + (size_t)(w.n_ctiles + 1) * 4, 256);
   w.bytes = off;
   return w;
 }

@@ -69,17 +69,14 @@ __global__ __launch_bounds__(256) void k_classify_v4(VolGeom g, const float* __r
 //    No inter-block dependency.
 // 2. k_scan_tsums: one block scans the blocks' sums into exclusive prefixes
 //    (the totals after the last) and the 64-bit totals of the control block.
-// 3. the bases of every word (block + tile + local prefix): the generate
-//    kernel stores them for its words; k_bases stores them alone, for calls
-//    that classify without generating.
-// Dispatch classes of the generate and gather tiles (a byte per tile):
-// generate tiles 0 heavy (at least 5/4 outputs, vertices + triangles, per
-// word), 1 other with output, 2 none; gather tiles 0 with output of their
-// own, 2 none.  tw = 0: no generate classes (the count blocks do not cover
-// whole generate tiles).
+// A word's bases are block + tile + local prefix, formed where they are used
+// (stored for every word they were 8 bytes a word more to write, and a launch
+// of their own where nothing is generated).
+// Dispatch classes of the generate tiles (a byte per tile): 0 heavy (at least
+// 5/4 outputs, vertices + triangles, per word), 1 other with output, 2 none.
+// tw = 0: no classes (the count blocks do not cover whole generate tiles).
 struct TileClasses {
   uint8_t* gcls;
-  uint8_t* tcls;
   int tw;
 };
 
@@ -111,7 +108,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_count(VolGeom g, const uint64_t*
       run = add_vt(run, s_ts[i]);
     }
     bsum[blk] = run;
-  } else if (threadIdx.x < 64) {  // the block's generate and gather tiles
+  } else if (threadIdx.x < 64) {  // the block's generate tiles
     const int lane = threadIdx.x;
     auto weight = [&](int first, int n) -> uint32_t {  // outputs of count tiles [first, +n)
       uint32_t w = 0u;
@@ -120,15 +117,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_count(VolGeom g, const uint64_t*
           w += (uint32_t)s_ts[first + i] + (uint32_t)(s_ts[first + i] >> 32);
       return w;
     };
-    constexpr int gct = kGatherTileWords / kCountTile;
     const int l = lane - 1;
-    if (l >= 0 && l < (kBlockTiles + gct - 1) / gct) {
-      const int64_t c0 = blk * kBlockTiles + l * gct;
-      if (c0 < n_ctiles) {
-        const uint32_t w = weight(l * gct, gct);
-        tc.tcls[c0 / gct] = w == 0u ? 2 : (4u * w >= 8u * (uint32_t)kGatherTileWords ? 0 : 1);
-      }
-    }
     const int cpt = tc.tw / kCountTile;
     if (tc.tw > 0 && l >= 0 && l < kBlockTiles / cpt) {
       const int64_t c0 = blk * kBlockTiles + l * cpt;
@@ -148,8 +137,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_count(VolGeom g, const uint64_t*
 // longest-processing-time-first schedule).  Every tile writes at fixed
 // offsets, so an order changes no output.  Each thread of the scan block
 // takes a contiguous chunk of tiles; two block scans of its class counts
-// give its slots.  The adjoint orders its gather tiles the same way, from
-// the count kernel's gather classes.
+// give its slots.
 struct GenOrder {
   const uint8_t* __restrict__ gcls;  // classes of the generate tiles
   int64_t nwords;
@@ -157,7 +145,6 @@ struct GenOrder {
   bool gen_classes;  // gcls holds the classes
   uint32_t unit_sp;  // > 0: order units of kOrderUnitTiles tiles a plane (unit_sp tiles) apart
   uint32_t* order;   // [0]: tw (0: no order), [1 + i]: the i-th tile to dispatch
-  uint32_t* gorder;  // the gather tiles' order: entry 0 cleared (the adjoint writes it)
 };
 
 // Where the scan reports {T, U} besides the control block (each may be null):
@@ -170,7 +157,7 @@ struct ScanOut {
 constexpr uint32_t kOrderStage = 16384;  // 64 KiB of LDS
 
 // One block scans the count blocks' sums (scan_block_sums), completes the tile
-// prefixes and writes the two dispatch orders.
+// prefixes and writes the dispatch order.
 // LARGE: some thread's chunk exceeds kOrderRegTiles tiles (a separate
 // instance, so the common one stays small).
 template <bool LARGE>
@@ -224,19 +211,6 @@ __global__ __launch_bounds__(kTsumThreads) void k_scan_tsums(const unsigned long
                        kOrderStage);
   else if (tid == 0)
     go.order[0] = 0u;
-  // the adjoint builds the gather tiles' order itself; until then there is none
-  if (tid == 0) go.gorder[0] = 0u;
-}
-
-// Bases of every row word (and entry nwords): tile prefix + local prefix.
-__global__ __launch_bounds__(256) void k_bases(VolGeom g, CountSrc cs,
-                                               const Ctrl* __restrict__ ctrl) {
-  cs.tpb_shift = (int)ctrl->tpb_shift;
-  const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (w > g.nwords) return;
-  const unsigned long long p = word_bases(cs, w);
-  cs.base_v[g.word_off + w] = (uint32_t)p;
-  cs.base_t[g.word_off + w] = (uint32_t)(p >> 32);
 }
 
 template <int TW, int NT, class Src, bool dedup>
@@ -254,10 +228,10 @@ __global__ __launch_bounds__(NT, 4) void k_generate(
     counts[0] = (int64_t)total_t;
     counts[1] = (int64_t)n_points;
   }
-  // too many ids for dax::Id or too little room: the bases only (the adjoint
-  // and the per-cell outputs read them), no output
-  const bool emit = total_v <= 0x7fffffffull && 3ull * total_t <= 0x7fffffffull &&
-                    (int64_t)total_t <= cap_tris && (int64_t)n_points <= cap_points;
+  // too many ids for dax::Id or too little room: no output
+  if (total_v > 0x7fffffffull || 3ull * total_t > 0x7fffffffull ||
+      (int64_t)total_t > cap_tris || (int64_t)n_points > cap_points)
+    return;
   // the scan's dispatch order when it was built for this tile size (whole
   // volume launches only), else index order
   uint32_t tag = 0u, ord = 0u;
@@ -270,7 +244,7 @@ __global__ __launch_bounds__(NT, 4) void k_generate(
       ordered ? (int64_t)(ord & ~kOrderHasOutput)
               : tile_lo + (xcd_order ? xcd_tile(blockIdx.x, ntiles) : (int64_t)blockIdx.x);
   generate_tile<TW, NT, Src, dedup>(g, field, bits + g.word_off, tile * TW, out, normals, 0, 0,
-                                    s_dyn, cs, emit, ordered && (ord & kOrderHasOutput) != 0u);
+                                    s_dyn, cs, ordered && (ord & kOrderHasOutput) != 0u);
 }
 
 // Slice classify: a thread per row word.  Along a row the plane value
@@ -384,12 +358,13 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
 }
 
 __global__ __launch_bounds__(256) void k_cell_outputs(VolGeom g, const uint64_t* __restrict__ bits,
-                                                      const uint32_t* __restrict__ base_t,
+                                                      CountSrc src, const Ctrl* __restrict__ ctrl,
                                                       uint8_t* __restrict__ cases,
                                                       int32_t* __restrict__ count,
                                                       int32_t* __restrict__ offsets) {
   __shared__ uint8_t s_nf[256];  // NumFaces per case
   s_nf[threadIdx.x] = (uint8_t)(c_case_table[threadIdx.x] >> 60);
+  src.tpb_shift = (int)ctrl->tpb_shift;
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int64_t w0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kCellWords;
@@ -425,7 +400,7 @@ __global__ __launch_bounds__(256) void k_cell_outputs(VolGeom g, const uint64_t*
       const int64_t cell = (int64_t)p.q * 64 + lane + cx * (p.j + cy * (int64_t)p.k);
       if (cases) cases[cell] = (uint8_t)cs;
       if (count) count[cell] = (int32_t)nf;
-      if (offsets) offsets[cell] = (int32_t)(base_t[g.word_off + w] + incl - nf);
+      if (offsets) offsets[cell] = (int32_t)((uint32_t)(word_bases(src, w) >> 32) + incl - nf);
     }
   }
 }
@@ -632,22 +607,18 @@ int tiles_per_block_shift(const Tuning& tu) {
   return tu.scan_sub == 1 ? 1 : (tu.scan_sub == 2 ? 2 : (tu.scan_sub == 8 ? 4 : 3));
 }
 
-// Where the generate kernel reads the word bases (the tiles per count block
+// Where the word bases come from (the tiles per count block
 // come from the control block: the scan may have run under another tuning).
 CountSrc count_src(const char* ws, const Workspace& L) {
-  char* wsm = const_cast<char*>(ws);
   return CountSrc{(const uint32_t*)(ws + L.off_counts),
                   (const unsigned long long*)(ws + L.off_tsum),
-                  (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0, 0,
-                  (uint32_t*)(wsm + L.off_base_v), (uint32_t*)(wsm + L.off_base_t)};
+                  (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0, 0};
 }
 
 // Count + block-sum scan over the whole volume (scan_sub waves, i.e.
-// 2 * scan_sub count tiles, per count block); `bases` also stores every
-// word's bases (calls that stop before the generate kernel, which otherwise
-// stores them).
+// 2 * scan_sub count tiles, per count block).
 int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu, hipStream_t s,
-                bool bases = false, ScanOut so = ScanOut{nullptr, nullptr}) {
+                ScanOut so = ScanOut{nullptr, nullptr}) {
   const uint64_t* bits = (const uint64_t*)(ws + L.off_bits);
   uint32_t* lpre = (uint32_t*)(ws + L.off_counts);
   unsigned long long* tloc = (unsigned long long*)(ws + L.off_tsum);
@@ -658,7 +629,7 @@ int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu
   // generate classes when a count block covers whole generate tiles
   const int tw = gen_tile_words(tu);
   const int block_words = 2 * (waves == 1 || waves == 2 || waves == 8 ? waves : 4) * kCountTile;
-  const TileClasses tc{(uint8_t*)(ws + L.off_gcls), (uint8_t*)(ws + L.off_tcls),
+  const TileClasses tc{(uint8_t*)(ws + L.off_gcls),
                        tw >= kCountTile && tw <= block_words ? tw : 0};
   const int64_t nblocks = ceil_div(n, 2 * waves);
   if (nblocks > 0) {
@@ -680,7 +651,7 @@ int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu
   const bool units = tc.tw > 0 && sp > 0 && ng % (kUnitG * sp) == 0 && (ng / kUnitG) % 8 == 0 &&
                      ceil_div(ng / kUnitG, (int64_t)kTsumThreads) * kUnitG <= kOrderRegTiles;
   const GenOrder go{tc.gcls, g.nwords, tw, tc.tw > 0, units ? (uint32_t)sp : 0u,
-                    (uint32_t*)(ws + L.off_order), (uint32_t*)(ws + L.off_gorder)};
+                    (uint32_t*)(ws + L.off_order)};
   if (ceil_div(ceil_div(g.nwords, (int64_t)tw), (int64_t)kTsumThreads) > kOrderRegTiles)
     k_scan_tsums<true><<<1, dim3(kTsumThreads), 0, s>>>(
         bsum, bpre, nblocks, tloc, n, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
@@ -688,11 +659,6 @@ int launch_scan(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu
     k_scan_tsums<false><<<1, dim3(kTsumThreads), 0, s>>>(
         bsum, bpre, nblocks, tloc, n, (Ctrl*)(ws + L.off_ctrl), go, tiles_per_block_shift(tu), so);
   DAXHIP_LAUNCH_CHECK("k_scan_tsums");
-  if (bases) {
-    k_bases<<<dim3((unsigned)ceil_div(g.nwords + 1, 256)), dim3(256), 0, s>>>(
-        g, count_src(ws, L), (const Ctrl*)(ws + L.off_ctrl));
-    DAXHIP_LAUNCH_CHECK("k_bases");
-  }
   return DAX_HIP_OK;
 }
 
@@ -809,7 +775,7 @@ int count_sync(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu,
   int64_t c[2] = {0, 0};
   HostSlot slot;
   int rc;
-  if ((rc = launch_scan(g, ws, L, tu, s, false, ScanOut{nullptr, slot.p}))) return rc;
+  if ((rc = launch_scan(g, ws, L, tu, s, ScanOut{nullptr, slot.p}))) return rc;
   unsigned long long vt[2];
   if (!slot.p)
     DAXHIP_CHECK(hipMemcpyAsync(vt, ws + L.off_ctrl + offsetof(Ctrl, total_v), sizeof(vt),
@@ -891,7 +857,7 @@ int dax_hip_mc_classify(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   char* ws = (char*)d_workspace;
   const Tuning tu = tuning_for(nx, ny, nz);
   if ((rc = launch_bits(g, d_field, ws, L, tu, s))) return rc;
-  return launch_scan(g, ws, L, tu, s, true, ScanOut{d_counts, nullptr});
+  return launch_scan(g, ws, L, tu, s, ScanOut{d_counts, nullptr});
 }
 
 int dax_hip_mc_count(const float* d_field, int64_t nx, int64_t ny, int64_t nz, float iso,
@@ -936,10 +902,10 @@ int dax_hip_mc_forward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
 // ---- forward without allocation -------------------------------------------
 // dax_hip_mc_forward with its workspace in a file-scope device array, for
 // callers that cannot allocate (code under graph capture, serving loops):
-// grids whose workspace fits kNoAllocScratchBytes (48 MiB: up to 512^3
-// points).  Every GPU the library runs on holds the array until the process
+// grids of up to kNoAllocMaxWords row words (512^3 points have 2^21).  Every GPU the library runs on holds the array until the process
 // ends.  Calls that overlap on one GPU share the array and race.
-constexpr size_t kNoAllocScratchBytes = (size_t)48 << 20;
+constexpr int64_t kNoAllocMaxWords = 2484927;
+constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;  // 12.3 bytes a word
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -980,10 +946,11 @@ int dax_hip_mc_forward_noalloc(const float* d_field, int64_t nx, int64_t ny, int
   int rc = make_geom(nx, ny, nz, h_origin3, h_spacing3, iso, g);
   if (rc) return rc;
   const Workspace L = workspace_layout(g.nwords);
-  if (L.bytes > kNoAllocScratchBytes) {
-    set_error("dax_hip_mc_forward_noalloc: a %lld x %lld x %lld grid needs %zu bytes of scratch, "
-              "%zu are available",
-              (long long)nx, (long long)ny, (long long)nz, L.bytes, kNoAllocScratchBytes);
+  if (g.nwords > kNoAllocMaxWords || L.fwd_bytes > kNoAllocScratchBytes) {
+    set_error("dax_hip_mc_forward_noalloc: a %lld x %lld x %lld grid needs %zu bytes of scratch "
+              "(%lld row words), there is room for %lld row words",
+              (long long)nx, (long long)ny, (long long)nz, L.fwd_bytes, (long long)g.nwords,
+              (long long)kNoAllocMaxWords);
     return DAX_HIP_BAD_VALUE;
   }
   if ((rc = check_outputs(g, d_field, flags, d_vertices, d_conn, d_edges, d_counts))) return rc;
@@ -1011,7 +978,7 @@ int dax_hip_mc_slice_classify(int64_t nx, int64_t ny, int64_t nz, const float* h
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)d_workspace;
   if ((rc = launch_bits_plane(g, pl, ws, L, s))) return rc;
-  return launch_scan(g, ws, L, tuning_for(nx, ny, nz), s, true, ScanOut{d_counts, nullptr});
+  return launch_scan(g, ws, L, tuning_for(nx, ny, nz), s, ScanOut{d_counts, nullptr});
 }
 
 int dax_hip_mc_slice_count(int64_t nx, int64_t ny, int64_t nz, const float* h_origin3,
@@ -1109,8 +1076,8 @@ int dax_hip_mc_cell_outputs(int64_t nx, int64_t ny, int64_t nz, const void* d_wo
   const int64_t blocks = ceil_div(ceil_div(g.nwords, (int64_t)kCellWords) * 64, 256);
   if (blocks == 0) return DAX_HIP_OK;
   k_cell_outputs<<<dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream>>>(
-      g, (const uint64_t*)(ws + L.off_bits), (const uint32_t*)(ws + L.off_base_t), d_cases,
-      d_count, d_offsets);
+      g, (const uint64_t*)(ws + L.off_bits), count_src(ws, L),
+      (const Ctrl*)(ws + L.off_ctrl), d_cases, d_count, d_offsets);
   DAXHIP_LAUNCH_CHECK("k_cell_outputs");
   return DAX_HIP_OK;
 }

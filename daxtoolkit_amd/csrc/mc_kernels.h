@@ -388,9 +388,8 @@ __host__ __device__ constexpr uint64_t edge_codes_packed() {
 constexpr uint64_t kEdgeCodes = edge_codes_packed();
 
 // ---------------------------------------------------------------------------
-// Dispatch orders of tile grids (generate tiles, the adjoint's gather tiles):
-// tiles of class 0 first, then class 1, then class 2, each in index order,
-// from a class byte per tile.  The grid's blocks take order[1 + blockIdx].
+// Dispatch order of the generate tiles: tiles of class 0 first, then class 1,
+// then class 2, each in index order, from a class byte per tile.
 constexpr uint32_t kOrderHasOutput = 0x80000000u;  // order entry flag: class 0 or 1
 
 // A thread of the ordering block owns a chunk of K consecutive tiles.  Up to
@@ -749,16 +748,14 @@ __device__ __forceinline__ void lds_flags(const VolGeom& g, const uint64_t* sA, 
 // last tile completes the totals) and the count blocks' exclusive prefixes
 // (bpre, the totals after the last); the tiles per block are a power of two.
 // In a batch the volume's tiles are ct0, ct0 + 1, ..., and the one after its
-// last is the next volume's first.  Generate writes the bases of its words to
-// base_v / base_t, which the adjoint and the per-cell outputs read.
+// last is the next volume's first.  The adjoint and the per-cell outputs take
+// the bases from here too.
 struct CountSrc {
   const uint32_t* __restrict__ lpre;
   const unsigned long long* __restrict__ tloc;
   const unsigned long long* __restrict__ bpre;
   int64_t n_ctiles, ct0;
   int tpb_shift;  // log2 of the count tiles per count block (from the control block)
-  uint32_t* __restrict__ base_v;
-  uint32_t* __restrict__ base_t;
 };
 
 __device__ __forceinline__ unsigned long long add_vt(unsigned long long a, unsigned long long b) {
@@ -863,40 +860,23 @@ __device__ __forceinline__ void scan_block_sums(const unsigned long long* __rest
 // at 256^3 (475 K vertices) and 88 at 512^3 (957 K); this one, with the tiles
 // gen_shape picks, 13, 36 and 62.
 //
-// The bases come from the count kernel's prefixes (cs); the tile writes the
-// bases of its words (and, for the volume's last tile, entry nwords) to
-// cs.base_v / base_t, and with emit false only that.  has_output skips the
+// The bases come from the count kernel's prefixes (cs).  has_output skips the
 // check for a tile without output (one round trip).
 template <int TW, int NT, class Src, bool dedup>
 __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
                                               const uint64_t* __restrict__ b, int64_t w_begin,
                                               const OutPtrs& out, bool normals,
                                               int64_t vol_base_v, int64_t vol_base_t,
-                                              uint64_t* s_dyn, const CountSrc& cs, bool emit,
+                                              uint64_t* s_dyn, const CountSrc& cs,
                                               bool has_output) {
   const int tid = threadIdx.x, lane = tid & 63;
   static_assert(NT >= TW, "a thread per word");
   constexpr int nt = NT, nwaves = NT / 64;
   const int nw = (int)min((int64_t)TW, g.nwords - w_begin);
-  {
-    // count tiles without output (has_output: known not to be the case):
-    // constant bases, nothing else to do
+  if (!has_output) {  // count tiles without output
     const int64_t c0 = w_begin / kCountTile;
     const int64_t c1 = min((w_begin + nw + kCountTile - 1) / kCountTile, cs.n_ctiles);
-    const unsigned long long p0 = has_output ? 0ull : ctile_prefix(cs, c0);
-    const unsigned long long p1 = has_output ? 1ull : ctile_prefix(cs, c1);
-    if (p0 == p1) {
-      const uint32_t v0 = (uint32_t)p0, t0 = (uint32_t)(p0 >> 32);
-      for (int i = tid; i < nw; i += nt) {
-        cs.base_v[w_begin + i] = v0;
-        cs.base_t[w_begin + i] = t0;
-      }
-      if (tid == 0 && w_begin + nw == g.nwords) {
-        cs.base_v[g.nwords] = v0;
-        cs.base_t[g.nwords] = t0;
-      }
-      return;
-    }
+    if (ctile_prefix(cs, c0) == ctile_prefix(cs, c1)) return;
   }
 
   const GenLayout<TW, NT> L(g.wpr);
@@ -955,15 +935,7 @@ __device__ __forceinline__ void generate_tile(const VolGeom& g, const Src& f,
   __syncthreads();
   const uint32_t tv0 = s_v0[0], tv1 = s_v0[nw];
   const uint32_t tt0 = s_t[0], tt1 = s_t[nw];
-  for (int i = tid; i < nw; i += nt) {
-    cs.base_v[w_begin + i] = s_v0[i];
-    cs.base_t[w_begin + i] = s_t[i];
-  }
-  if (tid == 0 && w_begin + nw == g.nwords) {
-    cs.base_v[g.nwords] = tv1;
-    cs.base_t[g.nwords] = tt1;
-  }
-  if (!emit || (tv0 == tv1 && tt0 == tt1)) return;  // bases only, or no output here
+  if (tv0 == tv1 && tt0 == tt1) return;  // no output here
 
   // 2. active cells of the thread's word
   if (tid < nw) {

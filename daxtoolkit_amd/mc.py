@@ -86,7 +86,7 @@ class Contour:
     interp_first: Optional[torch.Tensor]
     interp_second: Optional[torch.Tensor]
     interp_weight: Optional[torch.Tensor]
-    workspace: Optional[torch.Tensor] = None   # inside-bits + vertex bases (for backward)
+    workspace: Optional[torch.Tensor] = None   # inside-bits + count prefixes (for backward)
     counts: Optional[torch.Tensor] = None      # device {T, U}
     grid_points: Optional[int] = None          # points of the input grid (interp ids index it)
 

@@ -201,7 +201,7 @@ int dax_hip_mc_forward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
                        void* stream);
 /* dax_hip_mc_forward that allocates nothing: no counterpart in the
  * reference; for callers that cannot allocate device memory (code under
- * graph capture, tight serving loops).  The workspace is a 48 MiB array the
+ * graph capture, tight serving loops).  The workspace is a 32 MiB array the
  * library holds on each GPU it runs on (grids up to 512^3 points; larger
  * ones return DAX_HIP_BAD_VALUE); every call on a GPU uses that GPU's array,
  * so calls that overlap on one GPU race.  Arguments as dax_hip_mc_forward
@@ -489,7 +489,7 @@ int dax_hip_mc_classify(const float* d_field, int64_t nx, int64_t ny, int64_t nz
 /* The same two steps for a caller that sizes its outputs next (synchronous):
  * *h_tris = T, *h_points = U with duplicate removal; DAX_HIP_EXEC_ERROR if
  * either leaves the int32 dax::Id range.  Follow with dax_hip_mc_generate on
- * the same workspace, which also stores the words' bases. */
+ * the same workspace. */
 int dax_hip_mc_count(const float* d_field, int64_t nx, int64_t ny, int64_t nz, float iso,
                      void* d_workspace, size_t workspace_bytes, int64_t* h_tris,
                      int64_t* h_points, void* stream);
@@ -633,17 +633,15 @@ int dax_hip_graph_destroy(void* graph_exec);
 /* ---- adjoint (no reference counterpart) ---------------------------------
  * dL/dfield of L(vertices, normals) given dL/dvertices [U][3] and
  * dL/dnormals [U][3], with the topology of the forward held fixed.  Uses the
- * forward's workspace (inside-bits and vertex bases must still hold the
- * forward of this field and iso; the backward writes only the dispatch order
- * of its gather tiles there) and its compact edge list d_edges; the
+ * forward's workspace (inside-bits and count prefixes must still hold the
+ * forward of this field and iso; the backward writes only its endpoint words
+ * there, in a part of their own) and its compact edge list d_edges; the
  * interpolants (t, endpoint gradients) are recomputed from the field.
  * U = min(d_counts[1], n_points) if d_counts is given (device {T, U} of the
  * forward), else n_points.  d_scratch needs
  * dax_hip_mc_backward_scratch_bytes(n_points) bytes (a 32-byte record per
- * vertex and a list of the tiles dense enough to be redone in spans).
- * Deterministic: every sum has a fixed order (an atomic counter only fills
- * the tile list, whose order does not change any value), so the result is
- * bitwise reproducible.  Rows of at most 15872 points (nx).  d_dl_dfield [P]
+ * vertex and the sums of its two endpoints).  Deterministic: every sum has a
+ * fixed order, so the result is bitwise reproducible.  Rows of at most 15872 points (nx).  d_dl_dfield [P]
  * f32 is fully written. */
 size_t dax_hip_mc_backward_scratch_bytes(int64_t n_points);
 int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
@@ -653,12 +651,9 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
                         const float* d_dl_dnormals, void* d_scratch, size_t scratch_bytes,
                         float* d_dl_dfield, void* stream);
 
-/* No reference counterpart.  Gather tiles too dense for their block's
- * endpoint records are redone in spans: by their own block, one span after
- * another, when the volume has at least `tiles_per_cu` gather tiles per CU
- * (many rounds of tiles hide such a block), else in a separate span pass
- * over many blocks.  Default 16; 0 keeps the spans in their tile's block at
- * any size.  Process-wide; the result does not depend on it (bit for bit). */
+/* No reference counterpart.  Once chose the pass for gather tiles too dense
+ * for their block; the gather has no such tiles any more, and the call only
+ * checks its argument. */
 int dax_hip_mc_backward_set_span_threshold(int64_t tiles_per_cu);
 
 /* The same for a Vector3 point field ([n][3] f32, e.g. coordinates). */

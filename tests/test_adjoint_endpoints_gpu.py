@@ -1,0 +1,67 @@
+"""GPU adjoint over row words: sizes at the edges of words, waves (64 words)
+and tiles (256 words), from no surface to a point in two an endpoint, bit for
+bit against the oracle's FP32 restatement; an edge list cut below the
+surface's vertices against the whole list with zero gradients from there on
+(equal values: the vertices left out add exact zeros)."""
+import numpy as np
+import pytest
+import torch
+
+from daxtoolkit_amd import mc
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _field(dims, seed, noise):
+    nx, ny, nz = dims
+    r = np.random.default_rng(seed)
+    z, y, x = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    smooth = np.sin(x / 7.3) * np.cos(y / 5.1 + 0.3) + np.sin(z / 4.7 + 0.2)
+    return (smooth + noise * r.standard_normal((nz, ny, nx))).astype(np.float32)
+
+
+def _grads(U, seed):
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn((U, 3), generator=gen, dtype=torch.float32),
+            torch.randn((U, 3), generator=gen, dtype=torch.float32))
+
+
+@pytest.mark.parametrize("noise", [0.0, 2.0])
+@pytest.mark.parametrize("dims", [(2, 2, 2), (1, 9, 9), (63, 3, 5), (64, 17, 17), (65, 16, 8),
+                                  (128, 8, 16), (130, 21, 19), (1000, 5, 3), (4, 64, 65)])
+def test_endpoints_and_gather(dims, noise):
+    print(f"[case] adjoint words {dims} noise {noise}", flush=True)
+    f = _field(dims, 5, noise)
+    sp = (0.5, 1.0, 1.5)
+    field = torch.from_numpy(f).cuda()
+    out = mc.forward(field, 0.1, edges=True, spacing=sp)
+    U = out.num_points
+    dx, dn = _grads(U, 7)
+    got = mc.backward(field, 0.1, out, dx.cuda(), dn.cuda(), spacing=sp).cpu().numpy().reshape(-1)
+    r = orc.generate(f, 0.1, spacing=sp)
+    assert r["n_pts"] == U
+    want = (orc.backward_f32(f, 0.1, r["first"], r["second"], dx.numpy(), dn.numpy(), spacing=sp)
+            if U else np.zeros(f.size, np.float32))
+    assert np.array_equal(got.view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("cut", [0, 1, 2, 7, 100, 1000, -1])
+def test_cut_edge_list(cut):
+    dims = (70, 13, 11)
+    print(f"[case] adjoint cut {cut}", flush=True)
+    f = _field(dims, 3, 1.0)
+    field = torch.from_numpy(f).cuda()
+    out = mc.forward(field, 0.1, edges=True)
+    U = out.num_points
+    n = cut if cut >= 0 else U - 1
+    assert n < U
+    dx, dn = _grads(U, 9)
+    dx[n:] = 0.0
+    dn[n:] = 0.0
+    whole = mc.backward(field, 0.1, out, dx.cuda(), dn.cuda())
+    cut_out = mc.Contour(**{**out.__dict__, "vertices": out.vertices[:n]})
+    assert cut_out.num_points == n
+    got = mc.backward(field, 0.1, cut_out, dx[:n].contiguous().cuda(),
+                      dn[:n].contiguous().cuda())
+    assert torch.equal(got, whole)
