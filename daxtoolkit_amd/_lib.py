@@ -143,6 +143,8 @@ _SIGNATURES = {
     "dax_hip_topology_plan_uniform": (C.c_int, [i64, i64, i64, vp, C.c_uint, vp, sz, vp, vp, vp]),
     "dax_hip_topology_fill_uniform": (C.c_int, [i64, i64, i64, vp, vp, vp, C.c_uint, vp, sz, vp,
                                                 vp, vp, vp, vp]),
+    "dax_hip_threshold_plan_cells": (C.c_int, [vp, C.c_int, i64, vp, i64, f32, f32, C.c_uint, vp,
+                                               vp, sz, vp, vp, vp]),
     "dax_hip_topology_plan_cells": (C.c_int, [vp, C.c_int, i64, i64, vp, C.c_uint, vp, sz, vp, vp,
                                               vp]),
     "dax_hip_topology_fill_cells": (C.c_int, [vp, C.c_int, i64, vp, i64, vp, C.c_uint, vp, sz, vp,

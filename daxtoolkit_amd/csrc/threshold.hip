@@ -30,10 +30,11 @@ constexpr int kTX = 64, kTY = 4;  // uniform-grid blocks: 64 x-cells by 4 rows
 constexpr int kZRun = 16;         // planes one thread marches through
 
 // How prepare laid out the workspace (its first int): per-cell offsets and
-// per-point ranks (any counts, any grid), or bit words (counts 0/1 on a
-// uniform grid: a bit per cell and per point, 64 to a word along x, with
-// exclusive popcount prefixes).
-constexpr int kModeCells = 0, kModeBits = 1;
+// per-point ranks (any counts, any grid), or bit words with exclusive popcount
+// prefixes for counts 0/1: on a uniform grid a bit per cell and per point, 64
+// to a word along x (kModeBits), on an unstructured one 64 to a word in index
+// order (kModeLinear).
+constexpr int kModeCells = 0, kModeBits = 1, kModeLinear = 2;
 
 __device__ __forceinline__ bool in_range(float v, float lo, float hi) {
   return v >= lo && v <= hi;
@@ -412,6 +413,30 @@ __host__ __device__ __forceinline__ FlatRows point_rows(const BitGeom& g) {
   return FlatRows{g.nx, g.wpx, g.nx * g.ny * g.nz, g.div_wpx};
 }
 
+// Header of the workspace: [0] layout mode, [1] flag of counts outside
+// {0, 1}, [2..4] the uniform grid's nx, ny, nz, [5] 1 when prepare computed
+// the point ranks (duplicate removal), [6] output cells, [7] used points, [8]
+// flag of a cell with a point id out of range.
+constexpr int kHeaderInts = 9, kHeaderBadId = 8;
+
+// The words of an unstructured grid: one row of cells, one of points.
+inline BitGeom bit_linear(int64_t n_cells, int64_t n_points) {
+  BitGeom b;
+  b.nx = (int)n_points;
+  b.cx = (int)n_cells;
+  b.ny = b.nz = b.cy = b.cz = 1;
+  b.wcx = (int)((n_cells + 63) / 64);
+  b.wpx = (int)((n_points + 63) / 64);
+  b.n_cwords = b.wcx;
+  b.n_pwords = b.wpx;
+  b.div_wcx = mc::make_fast_div((uint32_t)b.wcx);
+  b.div_cx = mc::make_fast_div((uint32_t)b.cx);
+  b.div_wpx = mc::make_fast_div((uint32_t)b.wpx);
+  b.div_nx = mc::make_fast_div((uint32_t)b.nx);
+  b.div_cy = b.div_ny = mc::make_fast_div(1u);
+  return b;
+}
+
 // Words, exclusive popcount prefixes within the tiles and the tiles' (sums,
 // then exclusive prefixes) of the cells or the points.
 struct WordSet {
@@ -494,8 +519,13 @@ __global__ __launch_bounds__(kWordTile) void k_cell_words(BitGeom g,
                   (uint32_t)min((int64_t)w0 + kWordTile, g.n_cwords), counts);
 }
 
-// Popcount prefixes of words already there.
-__global__ __launch_bounds__(kWordTile) void k_word_prefix(WordSet ws, int64_t nwords) {
+// Popcount prefixes of words already there (with a second row of blocks, of
+// two sets).
+__global__ __launch_bounds__(kWordTile) void k_word_prefix(WordSet w0, int64_t n0, WordSet w1,
+                                                           int64_t n1) {
+  const WordSet ws = blockIdx.y == 0 ? w0 : w1;
+  const int64_t nwords = blockIdx.y == 0 ? n0 : n1;
+  if ((int64_t)blockIdx.x * kWordTile >= nwords) return;  // uniform
   __shared__ uint64_t s_w[kWordTile + 1];
   __shared__ uint32_t s_scan[kWordTile / 64];
   const int64_t w = (int64_t)blockIdx.x * kWordTile + threadIdx.x;
@@ -672,9 +702,153 @@ __global__ __launch_bounds__(256) void k_compact_words(BitGeom g, WordSet pts, i
   }
 }
 
+// ---- unstructured grids, counts 0/1 ----
+// The cells' vertex ids: 16-byte loads for 4 and 8 vertices where the cells
+// are 16-byte aligned (NV; 0: any number of vertices, single loads).
+template <int NV>
+__device__ __forceinline__ void load_ids(const int32_t* __restrict__ cells, int nv, int64_t c,
+                                         int32_t* ids) {
+  if constexpr (NV != 0) {
+#pragma unroll
+    for (int q = 0; q < NV / 4; ++q) {
+      const i32x4 v = reinterpret_cast<const i32x4*>(cells)[c * (NV / 4) + q];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ids[4 * q + t] = v[t];
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+      if (v < nv) ids[v] = cells[c * nv + v];
+  }
+}
+
+// Zeroes the mask and the header's flags.
+__global__ __launch_bounds__(256) void k_clear_linear(int32_t* __restrict__ hdr, int ranked,
+                                                      int32_t* __restrict__ mask, int64_t n) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i == 0) {
+    hdr[0] = kModeLinear;
+    hdr[1] = hdr[2] = hdr[3] = hdr[4] = 0;
+    hdr[5] = ranked;
+    hdr[kHeaderBadId] = 0;
+  }
+  if (i + 4 <= n && ((uintptr_t)mask & 15u) == 0) {
+    *reinterpret_cast<i32x4*>(mask + i) = i32x4{0, 0, 0, 0};
+  } else {
+    for (int64_t t = i; t < min(i + 4, n); ++t) mask[t] = 0;
+  }
+}
+
+// A thread per cell, a wave per cell word: from the points' values whether the
+// cell is kept (writing the counts and the word), or (f null) from the word;
+// kept cells store 1 in the mask at their vertices.  Bound by the ids (129 MB
+// for 4.0 M hexahedra: 29 us, 4.4 TB/s), which are read once: counting (a load
+// per id), checking the counts' sum, scanning and marking in passes of their
+// own took 67 + 90 + 17 + 15 us.
+template <int NV>
+__global__ __launch_bounds__(256) void k_cell_range(const int32_t* __restrict__ cells, int nv,
+                                                    int64_t n_cells, const float* __restrict__ f,
+                                                    int64_t n_points, float lo, float hi,
+                                                    int32_t* __restrict__ counts,
+                                                    uint64_t* __restrict__ cbits,
+                                                    int32_t* __restrict__ mask,
+                                                    int32_t* __restrict__ hdr) {
+  const int n = NV ? NV : nv;
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const bool there = c < n_cells;
+  bool keep = false, ok = true;
+  int32_t ids[8];
+  if (f) {
+    if (there) {
+      load_ids<NV>(cells, nv, c, ids);
+#pragma unroll
+      for (int v = 0; v < (NV ? NV : 8); ++v)
+        if (v < n) ok = ok && ids[v] >= 0 && ids[v] < n_points;
+      keep = ok;
+      float x[8];
+#pragma unroll
+      for (int v = 0; v < (NV ? NV : 8); ++v)
+        if (v < n) x[v] = f[ok ? ids[v] : 0];
+#pragma unroll
+      for (int v = 0; v < (NV ? NV : 8); ++v)
+        if (v < n) keep = keep && in_range(x[v], lo, hi);
+      counts[c] = keep ? 1 : 0;
+    }
+    const uint64_t word = __ballot(keep);
+    if ((threadIdx.x & 63) == 0 && there) cbits[c >> 6] = word;
+  } else if (there && ((cbits[c >> 6] >> (c & 63)) & 1ull)) {
+    load_ids<NV>(cells, nv, c, ids);
+#pragma unroll
+    for (int v = 0; v < (NV ? NV : 8); ++v)
+      if (v < n) ok = ok && ids[v] >= 0 && ids[v] < n_points;
+    keep = ok;
+  }
+  if (!ok) hdr[kHeaderBadId] = 1;
+  if (keep && mask) {
+#pragma unroll
+    for (int v = 0; v < (NV ? NV : 8); ++v)
+      if (v < n) mask[ids[v]] = 1;
+  }
+}
+
+// Words of the non-zero mask entries.
+__global__ __launch_bounds__(256) void k_mask_bits(FlatRows rows, int64_t nwords,
+                                                   const int32_t* __restrict__ mask,
+                                                   uint64_t* __restrict__ bits) {
+  __shared__ FlatLds<128> sh;
+  const int64_t w0 = (int64_t)blockIdx.x * 128;
+  classify_flat<128, kFlatLoads>(rows, reinterpret_cast<const float*>(mask), bits, (uint32_t)w0,
+                                 (uint32_t)min(w0 + 128, nwords), sh,
+                                 [](float v) { return __builtin_bit_cast(int32_t, v) != 0; });
+}
+
+// The kept cells' vertex ids, a thread per cell (waves whose word is empty
+// leave at once); with `dedup` the used points' ranks, from the point words.
+// With a scanned rank per point and an offset per cell, four cells a thread,
+// it took 44 us for 4.0 M hexahedra, this 14 (and the scans of 4 bytes a cell
+// and a point, 35 us, are of a word per 64).
+template <int NV>
+__global__ __launch_bounds__(256) void k_emit_linear(const int32_t* __restrict__ cells, int nv,
+                                                     int64_t n_cells, int64_t n_points,
+                                                     WordSet cs, WordSet ps, bool dedup,
+                                                     int64_t n_out, bool vec,
+                                                     int32_t* __restrict__ conn) {
+  const int n = NV ? NV : nv;
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= n_cells) return;
+  const int64_t w = c >> 6;
+  const uint64_t word = cs.bits[w];
+  if (!((word >> (c & 63)) & 1ull)) return;
+  const int64_t t = (int64_t)cs.tile[w / kWordTile] + cs.pre[w] +
+                    __popcll(word & ((1ull << (c & 63)) - 1ull));
+  if (t >= n_out) return;
+  int32_t ids[8];
+  load_ids<NV>(cells, nv, c, ids);
+  if (dedup) {
+#pragma unroll
+    for (int v = 0; v < (NV ? NV : 8); ++v) {
+      if (v >= n || ids[v] < 0 || ids[v] >= n_points) continue;
+      const int32_t pw = ids[v] >> 6;
+      ids[v] = ps.tile[pw / kWordTile] + ps.pre[pw] +
+               __popcll(ps.bits[pw] & ((1ull << (ids[v] & 63)) - 1ull));
+    }
+  }
+  int32_t* dst = conn + t * n;
+  if (NV && vec) {
+#pragma unroll
+    for (int q = 0; q < NV / 4; ++q)
+      reinterpret_cast<i32x4*>(dst)[q] =
+          i32x4{ids[4 * q], ids[4 * q + 1], ids[4 * q + 2], ids[4 * q + 3]};
+  } else {
+#pragma unroll
+    for (int v = 0; v < (NV ? NV : 8); ++v)
+      if (v < n) dst[v] = ids[v];
+  }
+}
+
 // Exclusive scans of the tiles' sums, block 0 the cells', block 1 the
 // points'; the totals go to the header and, with `host`, to pinned memory
-// with the flag of counts outside {0, 1}.
+// with the header's flags.
 constexpr int kSumThreads = 1024;
 __global__ __launch_bounds__(kSumThreads) void k_scan_word_tiles(int32_t* __restrict__ ctile,
                                                                  int64_t nc,
@@ -708,16 +882,14 @@ __global__ __launch_bounds__(kSumThreads) void k_scan_word_tiles(int32_t* __rest
     if (host) {
       __hip_atomic_store(host + blockIdx.x, (int64_t)carry, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
-      if (blockIdx.x == 0)
+      if (blockIdx.x == 0) {
         __hip_atomic_store(host + 2, (int64_t)hdr[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(host + 3, (int64_t)hdr[kHeaderBadId], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
   }
 }
-
-// Header of the workspace: [0] layout mode, [1] flag of counts outside
-// {0, 1}, [2..4] the uniform grid's nx, ny, nz, [5] 1 when prepare computed
-// the point ranks (duplicate removal), [6] output cells, [7] used points.
-constexpr int kHeaderInts = 8;
 
 // Sum of the caller's per-cell counts in 64 bits (out[0]) and a flag for
 // negative counts (out[1]).  The int32 scan of the counts wraps past 2^31-1
@@ -844,6 +1016,28 @@ int count_uniform(const float* d_field, int64_t nx, int64_t ny, int64_t nz, floa
   return DAX_HIP_OK;
 }
 
+// ThresholdCount of an unstructured grid (checked arguments, n_cells > 0).
+int count_cells(const Geometry& g, const float* d_field, float min_value, float max_value,
+                int32_t* d_counts, hipStream_t s) {
+  TempBuf flag(s);
+  int rc = flag.alloc(sizeof(int32_t));
+  if (rc) return rc;
+  DAXHIP_CHECK(hipMemsetAsync(flag.p, 0, sizeof(int32_t), s));
+  k_count_cells<<<dim3((unsigned)ceil_div(g.n_cells, 256)), dim3(256), 0, s>>>(
+      g.cells, g.nv, g.n_cells, d_field, g.n_points, min_value, max_value, d_counts,
+      (int32_t*)flag.p);
+  DAXHIP_LAUNCH_CHECK("k_count_cells");
+  int32_t bad = 0;
+  DAXHIP_CHECK(hipMemcpyAsync(&bad, flag.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  DAXHIP_CHECK(hipStreamSynchronize(s));
+  if (bad) {
+    set_error("dax_hip_threshold_count_cells: a cell references a point outside [0, %lld)",
+              (long long)g.n_points);
+    return DAX_HIP_BAD_VALUE;
+  }
+  return DAX_HIP_OK;
+}
+
 // Cell words of a uniform grid from its in-range points or from its counts,
 // the point words and the totals, read back together.  *general: a count
 // outside {0, 1} was found, and nothing else holds.
@@ -867,7 +1061,7 @@ int prepare_bits(const BitGeom& bg, const BitWs& bw, char* ws, const float* d_fi
     k_count_bits<<<dim3((unsigned)ceil_div(bg.n_cwords, 128)), dim3(256), 0, s>>>(
         cell_rows(bg), bg.n_cwords, d_counts, cs.bits, hdr + 1);
     DAXHIP_LAUNCH_CHECK("k_count_bits");
-    k_word_prefix<<<gc, b, 0, s>>>(cs, bg.n_cwords);
+    k_word_prefix<<<gc, b, 0, s>>>(cs, bg.n_cwords, cs, 0);
     DAXHIP_LAUNCH_CHECK("k_word_prefix");
   }
   if (dedup) {
@@ -890,8 +1084,57 @@ int prepare_bits(const BitGeom& bg, const BitWs& bw, char* ws, const float* d_fi
   return DAX_HIP_OK;
 }
 
+// The same for an unstructured grid, whose kept cells mark their points in
+// the mask.  *bad: a kept cell (from a field: any cell) has a point id out of
+// range, and nothing else holds.
+int prepare_linear(const Geometry& g, const BitGeom& bg, const BitWs& bw, char* ws,
+                   const float* d_field, float lo, float hi, int32_t* d_counts, bool dedup,
+                   int32_t* d_mask, int64_t* cells, int64_t* points, bool* general, bool* bad,
+                   hipStream_t s) {
+  int32_t* hdr = (int32_t*)ws;
+  const WordSet cs = cell_set(ws, bw), ps = point_set(ws, bw);
+  const dim3 b(256), grid((unsigned)ceil_div(g.n_cells, 256));
+  int32_t* mask = dedup ? d_mask : nullptr;
+  k_clear_linear<<<dim3((unsigned)ceil_div(dedup ? g.n_points : 1, (int64_t)1024)), b, 0, s>>>(
+      hdr, dedup ? 1 : 0, mask, dedup ? g.n_points : 0);
+  DAXHIP_LAUNCH_CHECK("k_clear_linear");
+  if (!d_field) {
+    k_count_bits<<<dim3((unsigned)ceil_div(bg.n_cwords, 128)), b, 0, s>>>(
+        cell_rows(bg), bg.n_cwords, d_counts, cs.bits, hdr + 1);
+    DAXHIP_LAUNCH_CHECK("k_count_bits");
+  }
+  if (d_field || dedup) {
+    const bool vec = aligned16(g.cells);
+    auto k = vec && g.nv == 8 ? k_cell_range<8> : (vec && g.nv == 4 ? k_cell_range<4> : k_cell_range<0>);
+    k<<<grid, b, 0, s>>>(g.cells, g.nv, g.n_cells, d_field, g.n_points, lo, hi, d_counts, cs.bits,
+                         mask, hdr);
+    DAXHIP_LAUNCH_CHECK("k_cell_range");
+  }
+  if (dedup) {
+    k_mask_bits<<<dim3((unsigned)ceil_div(bg.n_pwords, 128)), b, 0, s>>>(
+        point_rows(bg), bg.n_pwords, d_mask, ps.bits);
+    DAXHIP_LAUNCH_CHECK("k_mask_bits");
+  }
+  k_word_prefix<<<dim3((unsigned)std::max(bw.nct, dedup ? bw.nmt : 0), dedup ? 2 : 1),
+                  dim3(kWordTile), 0, s>>>(cs, bg.n_cwords, ps, bg.n_pwords);
+  DAXHIP_LAUNCH_CHECK("k_word_prefix");
+  HostSlot slot;
+  k_scan_word_tiles<<<dedup ? 2 : 1, kSumThreads, 0, s>>>(cs.tile, bw.nct, ps.tile, bw.nmt, hdr,
+                                                          slot.p);
+  DAXHIP_LAUNCH_CHECK("k_scan_word_tiles");
+  int32_t h[kHeaderInts] = {};
+  if (!slot.p) DAXHIP_CHECK(hipMemcpyAsync(h, hdr, sizeof(h), hipMemcpyDeviceToHost, s));
+  DAXHIP_CHECK(hipStreamSynchronize(s));
+  const volatile int64_t* v = slot.p;
+  *cells = v ? v[0] : h[6];
+  *points = !dedup ? 0 : (v ? v[1] : h[7]);
+  *general = (v ? v[2] : h[1]) != 0;
+  *bad = (v ? v[3] : h[kHeaderBadId]) != 0;
+  return DAX_HIP_OK;
+}
+
 // Prepare from the caller's counts, or (d_field) from a field's range with
-// the counts written.  The bit-word layout where it holds, else per-cell
+// the counts written.  The bit-word layouts where they hold, else per-cell
 // offsets and per-point ranks.
 int prepare(const Geometry& g, const float* d_field, float lo, float hi, int32_t* d_counts,
             unsigned flags, void* d_ws, size_t ws_bytes, int32_t* d_mask, Plan* plan,
@@ -929,6 +1172,36 @@ int prepare(const Geometry& g, const float* d_field, float lo, float hi, int32_t
       }
     } else if (d_field) {
       if ((rc = count_uniform(d_field, g.nx, g.ny, g.nz, lo, hi, d_counts, s))) return rc;
+    }
+  }
+  if (g.cells) {
+    const BitGeom bg = bit_linear(g.n_cells, g.n_points);
+    const BitWs bw = bit_ws(w, bg);
+    // (one row: the end of its last word has to stay an int32)
+    if (bw.fits && std::max(g.n_cells, g.n_points) <= 0x7fff0000LL) {
+      int64_t cells = 0, points = 0;
+      bool general = false, bad = false;
+      if ((rc = prepare_linear(g, bg, bw, ws, d_field, lo, hi, d_counts, dedup, d_mask, &cells,
+                               &points, &general, &bad, s)))
+        return rc;
+      if (bad && d_field) {
+        set_error("dax_hip_threshold_count_cells: a cell references a point outside [0, %lld)",
+                  (long long)g.n_points);
+        return DAX_HIP_BAD_VALUE;
+      }
+      if (bad && !general) {
+        set_error("topology prepare: a kept cell references a point outside [0, %lld)",
+                  (long long)g.n_points);
+        return DAX_HIP_BAD_VALUE;
+      }
+      if (!general) {
+        plan->mode = kModeLinear;
+        plan->cells = cells;
+        plan->points = points;
+        return DAX_HIP_OK;
+      }
+    } else if (d_field) {
+      if ((rc = count_cells(g, d_field, lo, hi, d_counts, s))) return rc;
     }
   }
   k_set_header<<<1, 64, 0, s>>>(hdr, kModeCells, g.nx, g.ny, g.nz, dedup ? 1 : 0);
@@ -1050,6 +1323,28 @@ int generate(const Geometry& g, const float* d_points, const float* origin, cons
           aligned16(d_mask), rank, hdr, d_coords);
       DAXHIP_LAUNCH_CHECK("k_compact_points");
     }
+  } else if (plan.mode == kModeLinear && g.cells) {
+    const BitGeom bg = bit_linear(g.n_cells, g.n_points);
+    const BitWs bw = bit_ws(w, bg);
+    if (!bw.fits) {
+      set_error("topology generate: workspace of another grid");
+      return DAX_HIP_BAD_VALUE;
+    }
+    const WordSet cs = cell_set(ws, bw), ps = point_set(ws, bw);
+    if (plan.cells > 0) {
+      const bool vec = aligned16(g.cells);
+      auto k = vec && g.nv == 8 ? k_emit_linear<8> : (vec && g.nv == 4 ? k_emit_linear<4> : k_emit_linear<0>);
+      k<<<dim3((unsigned)ceil_div(g.n_cells, 256)), b, 0, s>>>(g.cells, g.nv, g.n_cells, g.n_points,
+                                                              cs, ps, dedup, plan.cells,
+                                                              aligned16(d_conn), d_conn);
+      DAXHIP_LAUNCH_CHECK("k_emit_linear");
+    }
+    if (dedup && plan.points > 0) {
+      k_compact_words<<<dim3((unsigned)ceil_div(bg.n_pwords, 4 * kCompactWords)), b, 0, s>>>(
+          bg, ps, plan.points, 0, 0, 0, 0, 0, 0, nullptr, (const uint32_t*)d_points, 3,
+          (uint32_t*)d_coords);
+      DAXHIP_LAUNCH_CHECK("k_compact_words");
+    }
   } else if (!g.cells) {
     const BitGeom bg = bit_geom(g.nx, g.ny, g.nz);
     const BitWs bw = bit_ws(w, bg);
@@ -1073,16 +1368,19 @@ int generate(const Geometry& g, const float* d_points, const float* origin, cons
 }
 
 // CompactPointField (checked arguments).
-int compact_field(const void* d_in, int words, int64_t n_points, const TopoWs& w, const char* ws,
+int compact_field(const void* d_in, int words, int64_t n_cells, int64_t n_points, const TopoWs& w,
+                  const char* ws,
                   const int32_t* d_mask, const Plan& plan, void* d_out, hipStream_t s) {
   if (!plan.ranked) {
     set_error("dax_hip_topology_compact_point_field: the prepare step did not remove duplicates");
     return DAX_HIP_BAD_VALUE;
   }
-  if (plan.mode == kModeBits) {
-    const BitGeom bg = bit_geom((int)plan.nx, (int)plan.ny, (int)plan.nz);
+  if (plan.mode == kModeBits || plan.mode == kModeLinear) {
+    const bool linear = plan.mode == kModeLinear;
+    const BitGeom bg = linear ? bit_linear(std::max<int64_t>(n_cells, 1), n_points)
+                              : bit_geom((int)plan.nx, (int)plan.ny, (int)plan.nz);
     const BitWs bw = bit_ws(w, bg);
-    if (plan.nx * plan.ny * plan.nz != n_points || !bw.fits) {
+    if ((!linear && plan.nx * plan.ny * plan.nz != n_points) || !bw.fits) {
       set_error("dax_hip_topology_compact_point_field: workspace of another grid");
       return DAX_HIP_BAD_VALUE;
     }
@@ -1133,23 +1431,8 @@ int dax_hip_threshold_count_cells(const int32_t* d_cells, int nv, int64_t n_cell
     return DAX_HIP_BAD_VALUE;
   }
   if (n_cells == 0) return DAX_HIP_OK;
-  hipStream_t s = (hipStream_t)stream;
-  TempBuf flag(s);
-  int rc = flag.alloc(sizeof(int32_t));
-  if (rc) return rc;
-  DAXHIP_CHECK(hipMemsetAsync(flag.p, 0, sizeof(int32_t), s));
-  k_count_cells<<<dim3((unsigned)ceil_div(n_cells, 256)), dim3(256), 0, s>>>(
-      d_cells, nv, n_cells, d_field, n_points, min_value, max_value, d_counts, (int32_t*)flag.p);
-  DAXHIP_LAUNCH_CHECK("k_count_cells");
-  int32_t bad = 0;
-  DAXHIP_CHECK(hipMemcpyAsync(&bad, flag.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
-  if (bad) {
-    set_error("dax_hip_threshold_count_cells: a cell references a point outside [0, %lld)",
-              (long long)n_points);
-    return DAX_HIP_BAD_VALUE;
-  }
-  return DAX_HIP_OK;
+  return count_cells(Geometry{d_cells, nv, n_cells, n_points, 0, 0, 0}, d_field, min_value,
+                     max_value, d_counts, (hipStream_t)stream);
 }
 
 // Geometry of a uniform grid the entry points accept.
@@ -1246,6 +1529,21 @@ int dax_hip_topology_generate_uniform(int64_t nx, int64_t ny, int64_t nz, const 
                                        d_coords, stream);
 }
 
+int dax_hip_threshold_plan_cells(const int32_t* d_cells, int nv, int64_t n_cells,
+                                 const float* d_field, int64_t n_points, float min_value,
+                                 float max_value, unsigned flags, int32_t* d_counts,
+                                 void* d_workspace, size_t workspace_bytes, int32_t* d_point_mask,
+                                 int64_t* h_plan8, void* stream) {
+  if (nv < 1 || nv > 8 || n_cells < 1 || n_points < 1 || n_points > 0x7fffffffLL ||
+      n_cells > 0x7fffffffLL / nv || !d_cells || !d_field) {
+    set_error("dax_hip_threshold_plan_cells: bad arguments");
+    return DAX_HIP_BAD_VALUE;
+  }
+  const Geometry g{d_cells, nv, n_cells, n_points, 0, 0, 0};
+  return prepare(g, d_field, min_value, max_value, d_counts, flags, d_workspace, workspace_bytes,
+                 d_point_mask, (Plan*)h_plan8, (hipStream_t)stream);
+}
+
 int dax_hip_topology_plan_cells(const int32_t* d_cells, int nv, int64_t n_cells, int64_t n_points,
                                 const int32_t* d_counts, unsigned flags, void* d_workspace,
                                 size_t workspace_bytes, int32_t* d_point_mask, int64_t* h_plan8,
@@ -1327,7 +1625,7 @@ int dax_hip_topology_fill_point_field(const void* d_in, size_t value_bytes, int6
   } else if (const int rc = read_plan(d_workspace, &plan, s)) {
     return rc;
   }
-  return compact_field(d_in, (int)(value_bytes / 4), n_points, w, (const char*)d_workspace,
+  return compact_field(d_in, (int)(value_bytes / 4), n_cells, n_points, w, (const char*)d_workspace,
                        d_point_mask, plan, d_out, s);
 }
 

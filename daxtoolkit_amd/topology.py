@@ -168,6 +168,23 @@ def generate_topology(counts: torch.Tensor, dims=None, cells: Optional[torch.Ten
     return _generate(counts, dims, cells, points, origin, spacing, dedup, ws, mask, plan)
 
 
+def _threshold_cells(field, lo, hi, cells, points, dedup) -> Topology:
+    """threshold_count and generate_topology of an unstructured grid in one
+    call (checked arguments)."""
+    C, V = cells.shape
+    P = field.numel()
+    dev = field.device
+    counts = torch.empty(C, dtype=torch.int32, device=dev)
+    ws = torch.empty(int(_lib.load().dax_hip_topology_workspace_bytes(C, P)), dtype=torch.uint8,
+                     device=dev)
+    mask = torch.empty(P, dtype=torch.int32, device=dev) if dedup else None
+    plan = (ctypes.c_int64 * 8)()
+    _lib.call("dax_hip_threshold_plan_cells", cells.data_ptr(), V, C, field.data_ptr(), P,
+              float(lo), float(hi), MC_DEDUP if dedup else 0, counts.data_ptr(), ws.data_ptr(),
+              ws.numel(), mask.data_ptr() if dedup else None, plan, _stream())
+    return _generate(counts, None, cells, points, None, None, dedup, ws, mask, plan)
+
+
 def threshold(field: torch.Tensor, lo: float, hi: float, cells: Optional[torch.Tensor] = None,
               points: Optional[torch.Tensor] = None, origin=(0, 0, 0), spacing=(1, 1, 1),
               dedup: bool = True, point_mask: bool = True) -> Topology:
@@ -177,6 +194,12 @@ def threshold(field: torch.Tensor, lo: float, hi: float, cells: Optional[torch.T
     point_mask=False the int32 point mask is not kept (CompactPointField
     does not need it)."""
     if cells is not None or field.dim() != 3:
+        if (points is not None and cells is not None and field.dtype == torch.float32 and
+                field.is_contiguous() and points.dtype == torch.float32 and
+                points.is_contiguous() and points.shape == (field.numel(), 3)):
+            _check_cells(cells, field.numel())
+            if cells.shape[0] > 0:
+                return _threshold_cells(field, lo, hi, cells, points, dedup)
         counts = threshold_count(field, lo, hi, cells)
         return generate_topology(counts, cells=cells, points=points, origin=origin,
                                  spacing=spacing, dedup=dedup)

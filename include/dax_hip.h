@@ -421,6 +421,13 @@ int dax_hip_topology_fill_uniform(int64_t nx, int64_t ny, int64_t nz, const floa
                                   unsigned flags, const void* d_workspace, size_t workspace_bytes,
                                   const int32_t* d_point_mask, const int64_t* h_plan8,
                                   int32_t* d_conn, float* d_coords, void* stream);
+/* ThresholdCount of an unstructured grid (the counts are written) and its
+ * plan in one, as dax_hip_threshold_plan_uniform; n_cells >= 1. */
+int dax_hip_threshold_plan_cells(const int32_t* d_cells, int nv, int64_t n_cells,
+                                 const float* d_field, int64_t n_points, float min_value,
+                                 float max_value, unsigned flags, int32_t* d_counts,
+                                 void* d_workspace, size_t workspace_bytes, int32_t* d_point_mask,
+                                 int64_t* h_plan8, void* stream);
 int dax_hip_topology_plan_cells(const int32_t* d_cells, int nv, int64_t n_cells, int64_t n_points,
                                 const int32_t* d_counts, unsigned flags, void* d_workspace,
                                 size_t workspace_bytes, int32_t* d_point_mask, int64_t* h_plan8,
