@@ -348,8 +348,11 @@ bool valid_tuning(const Tuning& t) {
 // Per-cell outputs of the count step: case byte, NumFaces[case] and the
 // exclusive triangle offset.  A wavefront takes kCellWords (8) consecutive
 // row words: one load instruction brings all their neighbour words (lane
-// 8u+v holds neighbour v of word u), each word then reads its eight from
-// the lanes and writes its 64 cells (lane = cell).
+// 8u+v holds neighbour v of word u) and their bases, each word then reads its
+// eight from the lanes and writes its 64 cells (lane = cell).  Words without
+// a mixed cell need no case lookup.  Bound by the stores (9 bytes a cell):
+// 253x241x230 (125 MB) took 48 us with a lookup, a scan and a dependent base
+// load in every word, this 42; with scalar loads of the neighbours 78.
 constexpr int kCellWords = 8;
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
@@ -367,18 +370,20 @@ __global__ __launch_bounds__(256) void k_cell_outputs(VolGeom g, const uint64_t*
   src.tpb_shift = (int)ctrl->tpb_shift;
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  const int64_t w0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kCellWords;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t w0 = ((int64_t)blockIdx.x * (256 / 64) + wv) * kCellWords;
   if (w0 >= g.nwords) return;  // wave-uniform
-  const uint64_t* b = bits + g.word_off;
   const int64_t plane = (int64_t)g.wpr * g.ny;
   uint64_t mine = 0ull;  // neighbour (lane & 7) of word w0 + (lane >> 3)
+  uint32_t base = 0u;    // triangle base of that word
   {
     const int64_t w = w0 + (lane >> 3);
     const int v = lane & 7;
     if (w < g.nwords) {
       const WordPos p = word_pos(g, w);
       if (p.has_y && p.has_z && (!(v & 1) || p.q + 1 < g.wpr))
-        mine = b[w + (v & 1) + ((v >> 1) & 1) * g.wpr + (v >> 2) * plane];
+        mine = bits[w + (v & 1) + ((v >> 1) & 1) * g.wpr + (v >> 2) * plane];
+      if (offsets) base = (uint32_t)(word_bases(src, w) >> 32);
     }
   }
   const int64_t cx = g.nx - 1, cy = g.ny - 1;
@@ -393,14 +398,19 @@ __global__ __launch_bounds__(256) void k_cell_outputs(VolGeom g, const uint64_t*
     CellPlanes cp;
     cell_planes(p, nb[0], nb[1], nb[2], nb[3], nb[4], nb[5], nb[6], nb[7], cp);
     const bool valid = ((p.xmask >> lane) & 1ull) != 0;
-    const int cs = cell_case(cp, lane);
-    const uint32_t nf = valid ? (uint32_t)s_nf[cs] : 0u;
-    const uint32_t incl = offsets ? wave_incl_scan(nf) : 0u;
+    int cs = (nb[0] >> lane) & 1ull ? 255 : 0;  // no mixed corners: no faces
+    uint32_t nf = 0u, incl = 0u;
+    if (cp.active != 0ull) {  // wave-uniform
+      cs = cell_case(cp, lane);
+      nf = valid ? (uint32_t)s_nf[cs] : 0u;
+      incl = offsets ? wave_incl_scan(nf) : 0u;
+    }
     if (valid) {
-      const int64_t cell = (int64_t)p.q * 64 + lane + cx * (p.j + cy * (int64_t)p.k);
-      if (cases) cases[cell] = (uint8_t)cs;
-      if (count) count[cell] = (int32_t)nf;
-      if (offsets) offsets[cell] = (int32_t)((uint32_t)(word_bases(src, w) >> 32) + incl - nf);
+      const int64_t cell = (int64_t)p.q * 64 + cx * (p.j + cy * (int64_t)p.k);
+      const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)base, 8 * u);
+      if (cases) (cases + cell)[lane] = (uint8_t)cs;
+      if (count) (count + cell)[lane] = (int32_t)nf;
+      if (offsets) (offsets + cell)[lane] = (int32_t)(first + incl - nf);
     }
   }
 }
@@ -427,56 +437,118 @@ __global__ void k_interpolate_vec3(const float* __restrict__ in, const int32_t* 
   for (int d = 0; d < 3; ++d) out[3 * u + d] = in[a + d] + w * (in[b + d] - in[a + d]);
 }
 
-__global__ void k_point_gradient(VolGeom g, const float* __restrict__ f, float* __restrict__ grad) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t P = (int64_t)g.nx * g.ny * g.nz;
-  if (p >= P) return;
-  const uint32_t row = fast_div((uint32_t)p, g.div_nx), zz = fast_div(row, g.div_ny);
-  const int x = (int)((uint32_t)p - row * (uint32_t)g.nx), y = (int)(row - zz * (uint32_t)g.ny),
-            z = (int)zz;
-  float gr[3];
-  point_gradient(g, FieldArray{f}, x, y, z, gr);
-  grad[3 * p + 0] = gr[0];
-  grad[3 * p + 1] = gr[1];
-  grad[3 * p + 2] = gr[2];
+// A block's 256 vectors of three, from entry `first` of n on, through LDS: 192
+// 16-byte stores instead of three 4-byte ones a thread at a stride of 12
+// (s: 768 floats).
+__device__ __forceinline__ void store_block3(float* __restrict__ out, int64_t first, int64_t n,
+                                             const float v[3], f32x4* s) {
+  const int tid = threadIdx.x;
+  float* sf = reinterpret_cast<float*>(s);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) sf[3 * tid + d] = v[d];
+  __syncthreads();
+  float* o = out + 3 * first;
+  const int m = 3 * (int)min((int64_t)256, n - first);
+  if ((reinterpret_cast<uintptr_t>(o) & 15u) == 0) {
+    if (4 * tid + 4 <= m)
+      reinterpret_cast<f32x4*>(o)[tid] = s[tid];
+    else
+      for (int i = 4 * tid; i < m; ++i) o[i] = sf[i];
+  } else {
+    for (int i = tid; i < m; i += 256) o[i] = sf[i];
+  }
+}
+
+// Planes a block of the gradient kernels marches through: neighbours in z stay
+// in registers and indexes are formed once, up to 8 where that leaves enough
+// blocks.
+inline int gradient_planes(int64_t plane_blocks, int64_t nz) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(8, plane_blocks * nz / 4096));
+}
+
+// A block takes 256 points of a plane and the points above them in `planes`
+// planes.  Blocks of one XCD are next to each other, so that the rows around a
+// point are in its L2.  Bound by the stores (12 of the 16 bytes a point moves).
+// Again and again on one field, 253x241x230: 66 us with one plane a block, 55
+// with eight, 39 in XCD order; 512^3: 746, 521, 506 (4.2 TB/s).
+__global__ __launch_bounds__(256) void k_point_gradient(VolGeom g, int planes, FastDiv div_pb,
+                                                        const float* __restrict__ f,
+                                                        float* __restrict__ grad) {
+  __shared__ f32x4 s[2][192];
+  const int32_t plane = g.nx * g.ny;
+  const uint32_t id = (uint32_t)xcd_tile_runs(blockIdx.x, gridDim.x), zc = fast_div(id, div_pb);
+  const int32_t first = (int32_t)(id - zc * (uint32_t)ceil_div((int64_t)plane, 256)) * 256;
+  const int z0 = (int)zc * planes, z1 = min(z0 + planes, g.nz);
+  const uint32_t p = (uint32_t)min(first + (int32_t)threadIdx.x, plane - 1);
+  const int y = (int)fast_div(p, g.div_nx), x = (int)(p - (uint32_t)y * (uint32_t)g.nx);
+  const int xm = x > 0 ? -1 : 0, xp = x + 1 < g.nx ? 1 : 0;
+  const int ym = y > 0 ? -g.nx : 0, yp = y + 1 < g.ny ? g.nx : 0;
+  const float* q = f + (int64_t)z0 * plane + p;
+  float c = q[0], before = z0 > 0 ? q[-(int64_t)plane] : c;
+  for (int z = z0; z < z1; ++z, q += plane) {
+    const float after = z + 1 < g.nz ? q[plane] : c;
+    const float lo[3] = {q[xm], q[ym], before}, hi[3] = {q[xp], q[yp], after};
+    float gr[3];
+    gradient_finish(g, x, y, z, lo, hi, gr);
+    store_block3(grad + 3 * (int64_t)z * plane, first, plane, gr, s[(z - z0) & 1]);
+    before = c;
+    c = after;
+  }
 }
 
 // CellGradient (dax/worklet/CellGradient.h:28-48): weights of
 // DerivativeWeights(Voxel) at the centre are +-0.25 in the corner order of
 // TopologyUniform.h:139-159; sum in vertex order, divided by the voxel width
 // coords[6]-coords[0] (Derivative.h:37-75).
-__global__ void k_cell_gradient(VolGeom g, const float* __restrict__ f, float* __restrict__ out) {
-  const int64_t cx = g.nx - 1, cy = g.ny - 1, cz = g.nz - 1;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cx * cy * cz) return;
-  const int i = (int)(c % cx), j = (int)((c / cx) % cy), k = (int)(c / (cx * cy));
-  const int64_t sy = g.nx, sz = (int64_t)g.nx * g.ny;
-  const int64_t p0 = i + sy * j + sz * k;
-  const int64_t pv[8] = {p0, p0 + 1, p0 + sy + 1, p0 + sy, p0 + sz, p0 + sz + 1, p0 + sz + sy + 1,
-                         p0 + sz + sy};
-  // sign of the x/y/z weight per corner (all magnitudes 0.25)
-  const float sx[8] = {-1, 1, 1, -1, -1, 1, 1, -1};
-  const float syy[8] = {-1, -1, 1, 1, -1, -1, 1, 1};
-  const float szz[8] = {-1, -1, -1, -1, 1, 1, 1, 1};
-  float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
+// Blocks as k_point_gradient's; 253x241x230: 64, 47, 41 us, 512^3: 829, 523,
+// 493 (a thread per cell with 64-bit divisions and stores at a stride of 12
+// bytes, among other work: 85 us where this takes 57..66).
+__global__ __launch_bounds__(256) void k_cell_gradient(VolGeom g, int planes, FastDiv div_pb,
+                                                       FastDiv div_cx,
+                                                       const float* __restrict__ f,
+                                                       float* __restrict__ out) {
+  __shared__ f32x4 s[2][192];
+  const int32_t cx = g.nx - 1, cy = g.ny - 1, cz = g.nz - 1, cells = cx * cy;  // of a plane
+  const int32_t plane = g.nx * g.ny;
+  const uint32_t id = (uint32_t)xcd_tile_runs(blockIdx.x, gridDim.x), zc = fast_div(id, div_pb);
+  const int32_t first = (int32_t)(id - zc * (uint32_t)ceil_div((int64_t)cells, 256)) * 256;
+  const int z0 = (int)zc * planes, z1 = min(z0 + planes, cz);
+  const uint32_t c = (uint32_t)min(first + (int32_t)threadIdx.x, cells - 1);
+  const int j = (int)fast_div(c, div_cx), i = (int)(c - (uint32_t)j * (uint32_t)cx);
+  auto width = [&](int d, int n) -> float {
+    const float a = g.origin[d] + g.spacing[d] * (float)n;
+    const float b = g.origin[d] + g.spacing[d] * (float)(n + 1);
+    return b - a;
+  };
+  // s / w; a power of two divides exactly by its reciprocal
+  auto quotient = [](float v, float w) -> float {
+    const uint32_t u = __float_as_uint(w);
+    const bool pow2 = (u & 0x7fffffu) == 0u && (u >> 23) - 1u < 253u;
+    if (!__ballot(!pow2)) return v * __uint_as_float(0x7f000000u - u);
+    return v / w;
+  };
+  const float wx = width(0, i), wy = width(1, j);
+  const float* q = f + (int64_t)z0 * plane + i + (int64_t)j * g.nx;
+  // the weights are +-0.25: a quarter of the value (the product with either
+  // sign rounds alike) with the sign of the corner
+  float lo[4] = {0.25f * q[0], 0.25f * q[1], 0.25f * q[g.nx + 1], 0.25f * q[g.nx]};
+  for (int z = z0; z < z1; ++z) {
+    q += plane;
+    const float hi[4] = {0.25f * q[0], 0.25f * q[1], 0.25f * q[g.nx + 1], 0.25f * q[g.nx]};
+    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
-  for (int v = 0; v < 8; ++v) {
-    const float fv = f[pv[v]];
-    s0 = s0 + fv * (0.25f * sx[v]);
-    s1 = s1 + fv * (0.25f * syy[v]);
-    s2 = s2 + fv * (0.25f * szz[v]);
-  }
-  const int ijk[3] = {i, j, k};
-  float wd[3];
+    for (int v = 0; v < 8; ++v) {
+      const float t = v < 4 ? lo[v & 3] : hi[v & 3];
+      const bool px = (v & 3) == 1 || (v & 3) == 2, py = (v & 2) != 0, pz = v >= 4;
+      s0 = px ? s0 + t : s0 - t;
+      s1 = py ? s1 + t : s1 - t;
+      s2 = pz ? s2 + t : s2 - t;
+    }
+    const float gr[3] = {quotient(s0, wx), quotient(s1, wy), quotient(s2, width(2, z))};
+    store_block3(out + 3 * (int64_t)z * cells, first, cells, gr, s[(z - z0) & 1]);
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const float a = g.origin[d] + g.spacing[d] * (float)ijk[d];
-    const float b = g.origin[d] + g.spacing[d] * (float)(ijk[d] + 1);
-    wd[d] = b - a;
+    for (int v = 0; v < 4; ++v) lo[v] = hi[v];
   }
-  out[3 * c + 0] = s0 / wd[0];
-  out[3 * c + 1] = s1 / wd[1];
-  out[3 * c + 2] = s2 / wd[2];
 }
 
 }  // namespace mc
@@ -1106,9 +1178,11 @@ int dax_hip_point_gradient(const float* d_field, int64_t nx, int64_t ny, int64_t
   VolGeom g;
   int rc = make_geom(nx, ny, nz, nullptr, h_spacing3, 0.0f, g);
   if (rc) return rc;
-  const int64_t P = nx * ny * nz;
-  k_point_gradient<<<dim3((unsigned)ceil_div(P, 256)), dim3(256), 0, (hipStream_t)stream>>>(
-      g, d_field, d_grad);
+  const int64_t pb = ceil_div(nx * ny, (int64_t)256);
+  const int planes = gradient_planes(pb, nz);
+  k_point_gradient<<<dim3((unsigned)(pb * ceil_div(nz, (int64_t)planes))), dim3(256), 0,
+                     (hipStream_t)stream>>>(g, planes, make_fast_div((uint32_t)pb), d_field,
+                                            d_grad);
   DAXHIP_LAUNCH_CHECK("k_point_gradient");
   return DAX_HIP_OK;
 }
@@ -1119,10 +1193,12 @@ int dax_hip_cell_gradient(const float* d_field, int64_t nx, int64_t ny, int64_t 
   VolGeom g;
   int rc = make_geom(nx, ny, nz, h_origin3, h_spacing3, 0.0f, g);
   if (rc) return rc;
-  const int64_t C = (nx - 1) * (ny - 1) * (nz - 1);
-  if (C <= 0) return DAX_HIP_OK;
-  k_cell_gradient<<<dim3((unsigned)ceil_div(C, 256)), dim3(256), 0, (hipStream_t)stream>>>(
-      g, d_field, d_grad);
+  if (nx < 2 || ny < 2 || nz < 2) return DAX_HIP_OK;
+  const int64_t pb = ceil_div((nx - 1) * (ny - 1), (int64_t)256);
+  const int planes = gradient_planes(pb, nz - 1);
+  k_cell_gradient<<<dim3((unsigned)(pb * ceil_div(nz - 1, (int64_t)planes))), dim3(256), 0,
+                    (hipStream_t)stream>>>(g, planes, make_fast_div((uint32_t)pb),
+                                           make_fast_div((uint32_t)nx - 1u), d_field, d_grad);
   DAXHIP_LAUNCH_CHECK("k_cell_gradient");
   return DAX_HIP_OK;
 }

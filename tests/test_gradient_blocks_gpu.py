@@ -1,0 +1,70 @@
+"""Point and cell gradients at the edges of their blocks of 256 (below, at and
+above one and several), with outputs on and off 16-byte boundaries, and the
+cells' cases, counts and offsets (words with and without mixed cells), bit
+for bit against the oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from daxtoolkit_amd import _lib, mc
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (255, 1, 1), (257, 2, 2), (16, 16, 1),
+                                  (17, 17, 17), (65, 5, 33), (64, 64, 9), (129, 3, 7)])
+def test_gradients(dims, offset):
+    print(f"[case] gradients {dims} offset {offset}", flush=True)
+    nx, ny, nz = dims
+    f = np.random.default_rng(sum(dims)).standard_normal((nz, ny, nx)).astype(np.float32)
+    field = torch.from_numpy(f).cuda()
+    sp, org = (0.7, 1.5, 2.0), (1.0, -2.0, 3.0)
+    C = (nx - 1) * (ny - 1) * (nz - 1)
+    args = (ctypes.c_float * 3)(*sp)
+    o3 = (ctypes.c_float * 3)(*org)
+    stream = torch.cuda.current_stream().cuda_stream
+    for n, ref, call in (
+            (f.size, orc.point_gradient(f, spacing=sp),
+             lambda o: _lib.call("dax_hip_point_gradient", field.data_ptr(), nx, ny, nz, args, o,
+                                 stream)),
+            (C, orc.cell_gradient(f, origin=org, spacing=sp) if C else None,
+             lambda o: _lib.call("dax_hip_cell_gradient", field.data_ptr(), nx, ny, nz, o3, args,
+                                 o, stream))):
+        if n == 0:
+            continue
+        buf = torch.full((3 * n + offset + 4,), 7.0, device="cuda")
+        call(buf[offset:].data_ptr())
+        got = buf.cpu().numpy()
+        assert np.array_equal(got[offset:offset + 3 * n].view(np.uint32),
+                              np.asarray(ref, np.float32).reshape(-1).view(np.uint32))
+        assert np.all(got[:offset] == 7.0) and np.all(got[offset + 3 * n:] == 7.0)
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (66, 9, 7), (200, 12, 5)])
+def test_cell_outputs_quiet_and_mixed_words(dims):
+    nx, ny, nz = dims
+    f = np.zeros((nz, ny, nx), np.float32)
+    f[:, :, nx // 2:] = 1.0          # whole words in and out
+    f[nz // 2, ny // 2, 0] = 1.0     # and mixed ones
+    field = torch.from_numpy(f).cuda()
+    ws, _ = mc.classify(field, 0.5)
+    C = (nx - 1) * (ny - 1) * (nz - 1)
+    cases = torch.empty(C, dtype=torch.uint8, device="cuda")
+    count = torch.empty(C, dtype=torch.int32, device="cuda")
+    offs = torch.empty(C, dtype=torch.int32, device="cuda")
+    _lib.call("dax_hip_mc_cell_outputs", nx, ny, nz, ws.data_ptr(), ws.numel(), cases.data_ptr(),
+              count.data_ptr(), offs.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    m = (f > 0.5).astype(np.int64)
+    c = np.zeros((nz - 1, ny - 1, nx - 1), np.int64)
+    for v, (dx, dy, dz) in enumerate([(0, 0, 0), (1, 0, 0), (1, 1, 0), (0, 1, 0), (0, 0, 1),
+                                      (1, 0, 1), (1, 1, 1), (0, 1, 1)]):
+        c |= m[dz:nz - 1 + dz, dy:ny - 1 + dy, dx:nx - 1 + dx] << v
+    assert np.array_equal(cases.cpu().numpy(), c.reshape(-1).astype(np.uint8))
+    n = count.cpu().numpy()
+    mixed = (c.reshape(-1) != 0) & (c.reshape(-1) != 255)
+    assert np.array_equal(n > 0, mixed)
+    assert np.array_equal(offs.cpu().numpy(), np.cumsum(n) - n)
