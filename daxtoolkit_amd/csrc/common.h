@@ -149,6 +149,46 @@ __device__ __forceinline__ int select_bit(uint64_t m, int k) {
   return pos;
 }
 
+// The thread's kScanChunk values [i0, i0 + kScanChunk) of n (zeros past the
+// end) and their exclusive prefixes back, in 16-byte pieces where the array is
+// aligned: a block that scans many values is bound by its round trips, and
+// with single accesses at a stride a round of 8 values a thread took 5 us.
+constexpr int kScanChunk = 16;
+using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void load_chunk(const uint32_t* __restrict__ v, int64_t i0, int64_t n,
+                                           u32x4 (&x)[kScanChunk / 4]) {
+  const bool whole = i0 + kScanChunk <= n && (reinterpret_cast<uintptr_t>(v) & 15u) == 0;
+#pragma unroll
+  for (int q = 0; q < kScanChunk / 4; ++q) {
+    if (whole) {
+      x[q] = *reinterpret_cast<const u32x4*>(v + i0 + 4 * q);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[q][t] = i0 + 4 * q + t < n ? v[i0 + 4 * q + t] : 0u;
+    }
+  }
+}
+__device__ __forceinline__ void store_prefixes(uint32_t* __restrict__ v, int64_t i0, int64_t n,
+                                               u32x4 (&x)[kScanChunk / 4], uint32_t run) {
+#pragma unroll
+  for (int q = 0; q < kScanChunk; ++q) {
+    const uint32_t t = x[q / 4][q % 4];
+    x[q / 4][q % 4] = run;
+    run += t;
+  }
+  const bool whole = i0 + kScanChunk <= n && (reinterpret_cast<uintptr_t>(v) & 15u) == 0;
+#pragma unroll
+  for (int q = 0; q < kScanChunk / 4; ++q) {
+    if (whole) {
+      *reinterpret_cast<u32x4*>(v + i0 + 4 * q) = x[q];
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (i0 + 4 * q + t < n) v[i0 + 4 * q + t] = x[q][t];
+    }
+  }
+}
+
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

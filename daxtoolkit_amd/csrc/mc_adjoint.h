@@ -227,48 +227,23 @@ __device__ __forceinline__ void endpoint_words_tile(const VolGeom& g,
 // Exclusive scan of the tiles' counts by one block; it also clears slot 0 of the
 // endpoints' sums, which stands for the points that are no endpoints.
 constexpr int kAdjScanThreads = 1024;
-using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 static __global__ __launch_bounds__(kAdjScanThreads) void k_scan_endpoints(
     const uint32_t* __restrict__ sums, uint32_t* __restrict__ pre, int64_t n,
     f32x4* __restrict__ endpoint_sums) {
   if (threadIdx.x == 0) endpoint_sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   __shared__ uint32_t s_scan[kAdjScanThreads / 64];
-  constexpr int V = 16;
+  constexpr int64_t kRound = (int64_t)kAdjScanThreads * kScanChunk;
   uint32_t carry = 0u;
-  for (int64_t c0 = 0; c0 < n; c0 += kAdjScanThreads * V) {
-    const int64_t i0 = c0 + (int64_t)threadIdx.x * V;
-    const bool whole = i0 + V <= n;
-    u32x4 v[V / 4];
+  for (int64_t c0 = 0; c0 < n; c0 += kRound) {
+    const int64_t i0 = c0 + (int64_t)threadIdx.x * kScanChunk;
+    u32x4 x[kScanChunk / 4];
+    load_chunk(sums, i0, n, x);
+    uint32_t sum = 0u, total;
 #pragma unroll
-    for (int q = 0; q < V / 4; ++q) {
-      if (whole) {
-        v[q] = *reinterpret_cast<const u32x4*>(sums + i0 + 4 * q);
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) v[q][t] = i0 + 4 * q + t < n ? sums[i0 + 4 * q + t] : 0u;
-      }
-    }
-    uint32_t sum = 0u;
-#pragma unroll
-    for (int q = 0; q < V; ++q) sum += v[q / 4][q % 4];
-    uint32_t total, run = carry + block_excl_scan(sum, total, s_scan);
+    for (int q = 0; q < kScanChunk; ++q) sum += x[q / 4][q % 4];
+    const uint32_t run = carry + block_excl_scan(sum, total, s_scan);
     carry += total;
-#pragma unroll
-    for (int q = 0; q < V; ++q) {
-      const uint32_t x = v[q / 4][q % 4];
-      v[q / 4][q % 4] = run;
-      run += x;
-    }
-#pragma unroll
-    for (int q = 0; q < V / 4; ++q) {
-      if (whole) {
-        *reinterpret_cast<u32x4*>(pre + i0 + 4 * q) = v[q];
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (i0 + 4 * q + t < n) pre[i0 + 4 * q + t] = v[q][t];
-      }
-    }
+    store_prefixes(pre, i0, n, x, run);
   }
 }
 

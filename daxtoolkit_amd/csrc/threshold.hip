@@ -857,25 +857,19 @@ __global__ __launch_bounds__(kSumThreads) void k_scan_word_tiles(int32_t* __rest
                                                                  int32_t* __restrict__ hdr,
                                                                  int64_t* __restrict__ host) {
   __shared__ uint32_t s_scan[kSumThreads / 64];
-  int32_t* t = blockIdx.x == 0 ? ctile : ptile;
+  uint32_t* t = reinterpret_cast<uint32_t*>(blockIdx.x == 0 ? ctile : ptile);
   const int64_t n = blockIdx.x == 0 ? nc : np;
-  constexpr int V = 8;
   uint32_t carry = 0u;
-  for (int64_t c0 = 0; c0 < n; c0 += kSumThreads * V) {
-    const int64_t b = c0 + (int64_t)threadIdx.x * V;
-    uint32_t v[V], sum = 0u;
+  for (int64_t c0 = 0; c0 < n; c0 += kSumThreads * kScanChunk) {
+    const int64_t i0 = c0 + (int64_t)threadIdx.x * kScanChunk;
+    u32x4 x[kScanChunk / 4];
+    load_chunk(t, i0, n, x);
+    uint32_t sum = 0u, total;
 #pragma unroll
-    for (int q = 0; q < V; ++q) {
-      v[q] = b + q < n ? (uint32_t)t[b + q] : 0u;
-      sum += v[q];
-    }
-    uint32_t total, run = carry + block_excl_scan(sum, total, s_scan);
+    for (int q = 0; q < kScanChunk; ++q) sum += x[q / 4][q % 4];
+    const uint32_t run = carry + block_excl_scan(sum, total, s_scan);
     carry += total;
-#pragma unroll
-    for (int q = 0; q < V; ++q) {
-      if (b + q < n) t[b + q] = (int32_t)run;
-      run += v[q];
-    }
+    store_prefixes(t, i0, n, x, run);
   }
   if (threadIdx.x == 0) {
     hdr[6 + blockIdx.x] = (int32_t)carry;

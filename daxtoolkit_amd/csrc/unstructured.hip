@@ -362,27 +362,24 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_block(uint32_t* __restrict_
                                                            const uint32_t* __restrict__ flag,
                                                            int64_t* __restrict__ host) {
   __shared__ uint32_t s_scan[kScanBlock / 64];
-  constexpr int V = 8;
   if (n_dev) n = min(n, ceil_div((int64_t)*n_dev, (int64_t)kRowTile));
   unsigned long long carry = 0ull;
   bool top = false;
-  for (int64_t c0 = 0; c0 < n; c0 += kScanBlock * V) {
-    const int64_t b = c0 + (int64_t)threadIdx.x * V;
-    uint32_t x[V], sum = 0u;
+  for (int64_t c0 = 0; c0 < n; c0 += kScanBlock * kScanChunk) {
+    const int64_t i0 = c0 + (int64_t)threadIdx.x * kScanChunk;
+    u32x4 x[kScanChunk / 4];
+    load_chunk(v, i0, n, x);
+    uint32_t sum = 0u, bits = 0u, total;
 #pragma unroll
-    for (int q = 0; q < V; ++q) {
-      x[q] = b + q < n ? v[b + q] : 0u;
-      top = top || (x[q] & kBadCells);
-      x[q] &= ~kBadCells;
-      sum += x[q];
+    for (int q = 0; q < kScanChunk; ++q) {
+      bits |= x[q / 4][q % 4];
+      x[q / 4][q % 4] &= ~kBadCells;
+      sum += x[q / 4][q % 4];
     }
-    uint32_t total, run = (uint32_t)carry + block_excl_scan(sum, total, s_scan);
+    top = top || (bits & kBadCells);
+    const uint32_t run = (uint32_t)carry + block_excl_scan(sum, total, s_scan);
     carry += total;
-#pragma unroll
-    for (int q = 0; q < V; ++q) {
-      if (b + q < n) v[b + q] = run;
-      run += x[q];
-    }
+    store_prefixes(v, i0, n, x, run);
   }
   const bool any_top = __syncthreads_or(top);
   if (threadIdx.x == 0) {
