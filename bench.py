@@ -67,8 +67,7 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, GB/s
 def _kernel_variants(n, tuned):
     """Template names of the three forward kernels a tuning launches."""
     unroll, vec, sub, tile = tuned[0], tuned[1], tuned[2], tuned[3]
-    cls = (f"k_classify_v4<{unroll}>" if vec == 4 else
-           f"k_classify<{unroll}, {'true' if n % 64 == 0 else 'false'}>")
+    cls = f"k_classify_v4<{unroll}>" if vec == 4 else f"k_classify<{unroll}>"
     return cls, f"k_count<{sub}>", f"k_generate<{tile}, FieldArray>"
 
 
