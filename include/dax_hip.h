@@ -604,7 +604,9 @@ int dax_hip_mc_batch_autotune(const float* d_fields, void* h_header, void* d_wor
 /* Batched adjoint: dL/dfield of every volume (written at the fields'
  * offsets) from dL/dvertex and dL/dnormal [U][3] of the concatenated outputs
  * of the last dax_hip_mc_batch_forward on this workspace (run with the edge
- * list).  d_scratch holds dax_hip_mc_backward_scratch_bytes(n_points).
+ * list).  d_scratch holds dax_hip_mc_backward_scratch_bytes(n_points).  Writes
+ * its endpoint words into a part of the workspace of their own, the same ones
+ * whenever n_points covers the forward's vertices.
  * No reference counterpart. */
 int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
                               const void* d_workspace, size_t workspace_bytes,
