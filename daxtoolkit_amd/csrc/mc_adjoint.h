@@ -136,6 +136,21 @@ constexpr int kAdjWaveWords = 32;
 constexpr int kAdjBlockWords = kAdjThreads / 64 * kAdjWaveWords;
 constexpr int kAdjTileBlocks = kAdjTile / kAdjBlockWords;
 
+// How many edges of the list a call takes: n_points, and not more than counts[1]
+// where the forward's counts are given.  The list is cut if that leaves out a
+// vertex of the surface (ctrl: the forward's totals).
+struct EdgeList {
+  const int64_t* counts;
+  int64_t n_points;
+  const Ctrl* ctrl;
+};
+__device__ __forceinline__ int64_t edge_count(const EdgeList& l) {
+  return l.counts ? min(l.counts[1], l.n_points) : l.n_points;
+}
+__device__ __forceinline__ bool is_cut(const EdgeList& l, int64_t n) {
+  return n > 0 && (unsigned long long)n < l.ctrl->total_v;
+}
+
 // Endpoint words of a volume (or batch) and their prefixes: the endpoints of
 // word w before it are tile[w's tile] + pre[w].
 struct Endpoints {
@@ -154,34 +169,12 @@ __device__ __forceinline__ uint32_t vertex_base(const VolGeom& g, const Endpoint
   return ep.base[2 * g.tile_off + w / kCountTile] + (lpre[w] & 0xffffu);
 }
 
-// Edge flags of a row word, without the edges whose ids are not below n.
-struct WordEdges {
-  uint64_t fx, fy, fz;
-};
-__device__ __forceinline__ WordEdges word_edges_below(const VolGeom& g,
-                                                      const uint64_t* __restrict__ b,
-                                                      const CountSrc& cs, int64_t w, int64_t n) {
-  const WordPos p = word_pos(g, w);
-  const uint64_t A = b[w];
-  WordEdges m;
-  edge_flags(p, A, p.q + 1 < g.wpr ? b[w + 1] : 0ull, p.has_y ? b[w + g.wpr] : 0ull,
-             p.has_z ? b[w + (int64_t)g.wpr * g.ny] : 0ull, m.fx, m.fy, m.fz);
-  int64_t room = n - (int64_t)(uint32_t)word_bases(cs, w);
-  if (popc(m.fx) + popc(m.fy) + popc(m.fz) <= room) return m;
-  for (int bit = 0; bit < 64; ++bit) {
-    const uint64_t t = 1ull << bit;
-    if ((m.fx & t) && --room < 0) m.fx &= ~t;
-    if ((m.fy & t) && --room < 0) m.fy &= ~t;
-    if ((m.fz & t) && --room < 0) m.fz &= ~t;
-  }
-  return m;
-}
-
 // Endpoints of row word w: the points whose bit differs from one of their
-// neighbours' (grids without cells have none).  Of an edge list cut at n_adj
-// vertices only the endpoints of its edges, so that 2 n_adj slots hold them.
+// neighbours' (grids without cells have none).  They depend on the bits alone,
+// not on how many of the edges a call takes, so that calls that share a
+// workspace write the same words there.
 __device__ __forceinline__ uint64_t endpoint_word(const VolGeom& g, const uint64_t* __restrict__ b,
-                                                  const CountSrc& cs, int64_t n_adj, int64_t w) {
+                                                  int64_t w) {
   const int64_t plane = (int64_t)g.wpr * g.ny;
   const WordPos p = word_pos(g, w);
   const uint64_t A = b[w];
@@ -189,28 +182,19 @@ __device__ __forceinline__ uint64_t endpoint_word(const VolGeom& g, const uint64
   const uint64_t yp = p.has_y ? b[w + g.wpr] : A, ym = p.j > 0 ? b[w - g.wpr] : A;
   const uint64_t zp = p.has_z ? b[w + plane] : A, zm = p.k > 0 ? b[w - plane] : A;
   const uint64_t prev = p.q > 0 ? b[w - 1] >> 63 : A & 1ull;
-  const uint32_t base = (uint32_t)word_bases(cs, w);
   const uint64_t fx = (A ^ shr1(A, next)) & p.xmask;
-  uint64_t e = fx | (fx << 1) | ((prev ^ A) & 1ull) | (A ^ yp) | (A ^ ym) | (A ^ zp) | (A ^ zm);
-  e &= p.pmask;
-  if (e != 0ull && (int64_t)base + 192 > n_adj) {  // the last words, or a cut list
-    const WordEdges o = word_edges_below(g, b, cs, w, n_adj);
-    e = o.fx | (o.fx << 1) | o.fy | o.fz;
-    if (p.q > 0) e |= word_edges_below(g, b, cs, w - 1, n_adj).fx >> 63;
-    if (p.j > 0) e |= word_edges_below(g, b, cs, w - g.wpr, n_adj).fy;
-    if (p.k > 0) e |= word_edges_below(g, b, cs, w - plane, n_adj).fz;
-  }
-  return e;
+  const uint64_t e =
+      fx | (fx << 1) | ((prev ^ A) & 1ull) | (A ^ yp) | (A ^ ym) | (A ^ zp) | (A ^ zm);
+  return e & p.pmask;
 }
 
 // Endpoint words, counts and prefixes of a tile (block of kAdjThreads).
 __device__ __forceinline__ void endpoint_words_tile(const VolGeom& g,
                                                     const uint64_t* __restrict__ b,
-                                                    const CountSrc& cs, int64_t n_adj,
-                                                    const Endpoints& ep, int64_t w0,
-                                                    uint32_t* s_scan) {
+                                                    const CountSrc& cs, const Endpoints& ep,
+                                                    int64_t w0, uint32_t* s_scan) {
   const int64_t w = w0 + threadIdx.x;
-  const uint64_t e = w < g.nwords ? endpoint_word(g, b, cs, n_adj, w) : 0ull;
+  const uint64_t e = w < g.nwords ? endpoint_word(g, b, w) : 0ull;
   uint32_t total;
   const uint32_t pre = block_excl_scan((uint32_t)popc(e), total, s_scan);
   if (w < g.nwords) {
@@ -440,6 +424,73 @@ __device__ __forceinline__ void zero_run(const VolGeom& g, float* __restrict__ o
   const int64_t n4 = (n - head) >> 2;
   for (int64_t t = tid; t < n4; t += nt) o4[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   for (int64_t t = head + 4 * n4 + tid; t < n; t += nt) o[t] = 0.0f;
+}
+
+// dL/df of the point (x, j, k) of row word w from the records of its and its
+// neighbours' edges, in combine_point's order: for an edge list cut below the
+// surface's vertices, whose endpoints' sums have no slots.
+__device__ float cut_point(const VolGeom& g, const uint64_t* __restrict__ b,
+                           const uint32_t* __restrict__ lpre, const Endpoints& ep,
+                           const VertexAdj* __restrict__ adj, int64_t n_adj, int64_t w, int x, int j,
+                           int k) {
+  const int64_t plane = (int64_t)g.wpr * g.ny;
+  float acc = 0.0f;
+#pragma unroll 1
+  for (int n = 0; n < 7; ++n) {  // the point, then before and after it along each axis
+    const int d = (n - 1) >> 1, step = n == 0 ? 0 : ((n & 1) ? -1 : 1);
+    const int c = d == 0 ? x : (d == 1 ? j : k), size = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
+    if (n > 0 && (c + step < 0 || c + step >= size)) continue;
+    const int xs = n > 0 && d == 0 ? x + step : x;
+    const int64_t ws = w + (xs >> 6) - (x >> 6) +
+                       (n > 0 && d > 0 ? step * (d == 1 ? (int64_t)g.wpr : plane) : 0);
+    const f32x4 v = endpoint_sums(g, b, lpre, ep, adj, n_adj, ws, xs & 63);
+    if (n == 0) {
+      acc = v.x;
+      const float G[3] = {v.y, v.z, v.w};
+      const int co[3] = {x, j, k}, nn[3] = {g.nx, g.ny, g.nz};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        if (co[a] == 0)
+          acc += G[a] * over_step(g, a, -1.0f, true);
+        else if (co[a] == nn[a] - 1)
+          acc += G[a] * over_step(g, a, 1.0f, true);
+      }
+      continue;
+    }
+    const float q = d == 0 ? over_step(g, 0, v.y, step < 0 ? x == 1 : x == g.nx - 2)
+                           : (d == 1 ? over_step(g, 1, v.z, step < 0 ? j == 1 : j == g.ny - 2)
+                                     : over_step(g, 2, v.w, step < 0 ? k == 1 : k == g.nz - 2));
+    acc += step < 0 ? q : -q;
+  }
+  return acc;
+}
+
+// dL/df of the points of a wave's row words for a cut edge list, a lane per
+// point of a word.
+__device__ __forceinline__ void gather_cut_wave(const VolGeom& g, const uint64_t* __restrict__ b,
+                                                const uint32_t* __restrict__ lpre,
+                                                const Endpoints& ep,
+                                                const VertexAdj* __restrict__ adj, int64_t n_adj,
+                                                float* __restrict__ out, int64_t ww) {
+  const int lane = threadIdx.x & 63;
+  const int64_t plane = (int64_t)g.wpr * g.ny;
+  const uint64_t* ew = ep.words + g.word_off;
+  for (int64_t w = ww; w < min(ww + kAdjWaveWords, g.nwords); ++w) {  // wave-uniform
+    const WordPos p = word_pos(g, w);
+    const uint64_t e = ew[w];
+    uint64_t r = e | (e << 1) | (e >> 1);
+    if (p.q > 0) r |= ew[w - 1] >> 63;
+    if (p.q + 1 < g.wpr) r |= ew[w + 1] << 63;
+    if (p.j > 0) r |= ew[w - g.wpr];
+    if (p.has_y) r |= ew[w + g.wpr];
+    if (p.k > 0) r |= ew[w - plane];
+    if (p.has_z) r |= ew[w + plane];
+    const int x = p.q * 64 + lane;
+    if (x >= g.nx) continue;
+    const float v = (r >> lane) & 1ull
+                        ? cut_point(g, b, lpre, ep, adj, n_adj, w, x, p.j, p.k) : 0.0f;
+    out[x + (int64_t)g.nx * (p.j + (int64_t)g.ny * p.k)] = v;
+  }
 }
 
 // What a wave of the gather keeps of its words: the endpoint words of the word

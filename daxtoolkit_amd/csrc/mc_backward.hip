@@ -11,45 +11,46 @@ namespace mc {
 __global__ __launch_bounds__(kAdjThreads) void k_adjoint_records(
     VolGeom g, const float* __restrict__ field, const uint32_t* __restrict__ edges,
     const float* __restrict__ dldx, const float* __restrict__ dldn,
-    const int64_t* __restrict__ counts, int64_t n_points, VertexAdj* __restrict__ out,
-    const uint64_t* __restrict__ bits, CountSrc cs, const Ctrl* __restrict__ ctrl, Endpoints ep,
-    int64_t vertex_blocks) {
+    EdgeList list, VertexAdj* __restrict__ out, const uint64_t* __restrict__ bits, CountSrc cs,
+    Endpoints ep, int64_t vertex_blocks) {
   __shared__ uint32_t s_scan[kAdjThreads / 64];
-  const int64_t U = counts ? min(counts[1], n_points) : n_points;
   if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
-    cs.tpb_shift = (int)ctrl->tpb_shift;
-    endpoint_words_tile(g, bits, cs, U, ep, ((int64_t)blockIdx.x - vertex_blocks) * kAdjTile,
-                        s_scan);
+    cs.tpb_shift = (int)list.ctrl->tpb_shift;
+    endpoint_words_tile(g, bits, cs, ep, ((int64_t)blockIdx.x - vertex_blocks) * kAdjTile, s_scan);
     return;
   }
   // XCD-contiguous vertex ranges: vertices are in edge order, so the field
   // lines of neighbouring stencils stay in one XCD's L2
   const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
-  if (u >= U) return;
+  if (u >= edge_count(list)) return;
   vertex_adjoint(g, field, edges, dldx, dldn, u, out);
 }
 
 __global__ __launch_bounds__(kAdjThreads) void k_endpoint_sums(
     VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre,
-    Endpoints ep, const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts,
-    int64_t n_points, f32x4* __restrict__ sums) {
+    Endpoints ep, const VertexAdj* __restrict__ adj, EdgeList list, f32x4* __restrict__ sums) {
   __shared__ uint8_t s_mark[kAdjThreads / 64][64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t n_adj = counts ? min(counts[1], n_points) : n_points;
   const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords + wv * kAdjWaveWords;
   if (ww < g.nwords)  // wave-uniform
-    endpoint_sums_wave(g, bits, lpre, ep, adj, n_adj, sums, 2 * n_points, ww, s_mark[wv]);
+    endpoint_sums_wave(g, bits, lpre, ep, adj, edge_count(list), sums, 2 * list.n_points, ww,
+                       s_mark[wv]);
 }
 
-// cap: the endpoints' last slot (0: zeros everywhere).
-__global__ __launch_bounds__(kAdjThreads) void k_point_gather(VolGeom g, Endpoints ep,
-                                                              const f32x4* __restrict__ sums,
-                                                              uint32_t cap,
-                                                              float* __restrict__ dldf) {
+// From the endpoints' sums, or (a cut list) from the records.
+__global__ __launch_bounds__(kAdjThreads) void k_point_gather(
+    VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
+    const VertexAdj* __restrict__ adj, EdgeList list, const f32x4* __restrict__ sums,
+    uint32_t last, float* __restrict__ dldf) {
   __shared__ GatherWave s_wave[kAdjThreads / 64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords + wv * kAdjWaveWords;
-  if (ww < g.nwords) gather_wave(g, ep, sums, cap, dldf, ww, s_wave[wv]);
+  if (ww >= g.nwords) return;  // wave-uniform
+  const int64_t n_adj = edge_count(list);
+  if (is_cut(list, n_adj))
+    gather_cut_wave(g, bits, lpre, ep, adj, n_adj, dldf, ww);
+  else
+    gather_wave(g, ep, sums, n_adj > 0 ? last : 0u, dldf, ww, s_wave[wv]);
 }
 
 }  // namespace mc
@@ -118,8 +119,8 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   const CountSrc cs{(const uint32_t*)(ws + L.off_counts),
                     (const unsigned long long*)(ws + L.off_tsum),
                     (const unsigned long long*)(ws + L.off_tpre), L.n_ctiles, 0, 0};
-  // the endpoint words live in the workspace; every call with this vertex count
-  // writes the same values there
+  // the endpoint words live in the workspace; every call on it writes the same
+  // values there
   const Endpoints ep{(uint64_t*)(ws + L.off_ends), (uint16_t*)(ws + L.off_end_pre),
                      (uint32_t*)(ws + L.off_end_sum), (uint32_t*)(ws + L.off_end_tile),
                      (uint32_t*)(ws + L.off_end_base)};
@@ -127,19 +128,20 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   f32x4* sums = (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points));
   const int64_t tiles = ceil_div(g.nwords, (int64_t)kAdjTile);
   const dim3 grid((unsigned)ceil_div(g.nwords, (int64_t)kAdjBlockWords)), block(kAdjThreads);
+  const EdgeList list{d_counts, n_points, (const Ctrl*)(ws + L.off_ctrl)};
   if (n_points > 0) {
     const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
     k_adjoint_records<<<dim3((unsigned)(vertex_blocks + tiles)), block, 0, s>>>(
-        g, d_field, d_edges, d_dl_dvertices, d_dl_dnormals, d_counts, n_points,
-        (VertexAdj*)d_scratch, bits, cs, (const Ctrl*)(ws + L.off_ctrl),
+        g, d_field, d_edges, d_dl_dvertices, d_dl_dnormals, list, (VertexAdj*)d_scratch, bits, cs,
         ep, vertex_blocks);
     DAXHIP_LAUNCH_CHECK("k_adjoint_records");
     k_scan_endpoints<<<1, kAdjScanThreads, 0, s>>>(ep.sums, ep.tile, tiles, sums);
     DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
-    k_endpoint_sums<<<grid, block, 0, s>>>(g, bits, cs.lpre, ep, adj, d_counts, n_points, sums);
+    k_endpoint_sums<<<grid, block, 0, s>>>(g, bits, cs.lpre, ep, adj, list, sums);
     DAXHIP_LAUNCH_CHECK("k_endpoint_sums");
   }
-  k_point_gather<<<grid, block, 0, s>>>(g, ep, sums, last_slot(n_points), d_dl_dfield);
+  k_point_gather<<<grid, block, 0, s>>>(g, bits, cs.lpre, ep, adj, list, sums, last_slot(n_points),
+                                        d_dl_dfield);
   DAXHIP_LAUNCH_CHECK("k_point_gather");
   return DAX_HIP_OK;
 }

@@ -251,17 +251,16 @@ __global__ __launch_bounds__(256) void k_batch_records(
     const VolGeom* __restrict__ vols, int64_t nvols, const uint32_t* __restrict__ vol_first,
     const float* __restrict__ fields, const uint32_t* __restrict__ edges,
     const float* __restrict__ dldx, const float* __restrict__ dldn,
-    const int64_t* __restrict__ counts, int64_t n_points, VertexAdj* __restrict__ out,
-    const TileRef* __restrict__ tiles, const uint64_t* __restrict__ bits, CountSrc all,
-    const Ctrl* __restrict__ ctrl, Endpoints ep, int64_t vertex_blocks) {
+    EdgeList list, VertexAdj* __restrict__ out, const TileRef* __restrict__ tiles,
+    const uint64_t* __restrict__ bits, CountSrc all, Endpoints ep, int64_t vertex_blocks) {
   __shared__ uint32_t s_scan[kAdjThreads / 64];
-  const int64_t U = counts ? min(counts[1], n_points) : n_points;
+  const int64_t U = edge_count(list);
   if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
     const TileRef tr = tiles[(int64_t)blockIdx.x - vertex_blocks];
     const VolGeom g = vols[tr.vol];
     CountSrc cs = volume_counts(all, g);
-    cs.tpb_shift = (int)ctrl->tpb_shift;
-    endpoint_words_tile(g, bits + g.word_off, cs, U, ep, tr.w0, s_scan);
+    cs.tpb_shift = (int)list.ctrl->tpb_shift;
+    endpoint_words_tile(g, bits + g.word_off, cs, ep, tr.w0, s_scan);
     return;
   }
   const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
@@ -291,30 +290,36 @@ static_assert(kAdjTile == kBatchGenTile, "the adjoint's tiles are the generate t
 __global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_sums(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
     const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
-    const VertexAdj* __restrict__ adj, const int64_t* __restrict__ counts, int64_t n_points,
-    f32x4* __restrict__ sums) {
+    const VertexAdj* __restrict__ adj, EdgeList list, f32x4* __restrict__ sums) {
   __shared__ uint8_t s_mark[kAdjThreads / 64][64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t n_adj = counts ? min(counts[1], n_points) : n_points;
   const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
   const TileRef tr = tiles[blk / kAdjTileBlocks];
   const VolGeom g = vols[tr.vol];
   const int64_t ww = (int64_t)tr.w0 + (blk % kAdjTileBlocks) * kAdjBlockWords + wv * kAdjWaveWords;
   if (ww < g.nwords)  // wave-uniform
-    endpoint_sums_wave(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj, n_adj, sums,
-                       2 * n_points, ww, s_mark[wv]);
+    endpoint_sums_wave(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj,
+                       edge_count(list), sums, 2 * list.n_points, ww, s_mark[wv]);
 }
 
 __global__ __launch_bounds__(kAdjThreads) void k_batch_point_gather(
-    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, Endpoints ep,
-    const f32x4* __restrict__ sums, uint32_t cap, float* __restrict__ dldf) {
+    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
+    const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
+    const VertexAdj* __restrict__ adj, EdgeList list, const f32x4* __restrict__ sums,
+    uint32_t last, float* __restrict__ dldf) {
   __shared__ GatherWave s_wave[kAdjThreads / 64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
   const TileRef tr = tiles[blk / kAdjTileBlocks];
   const VolGeom g = vols[tr.vol];
   const int64_t ww = (int64_t)tr.w0 + (blk % kAdjTileBlocks) * kAdjBlockWords + wv * kAdjWaveWords;
-  if (ww < g.nwords) gather_wave(g, ep, sums, cap, dldf + g.field_off, ww, s_wave[wv]);
+  if (ww >= g.nwords) return;  // wave-uniform
+  const int64_t n_adj = edge_count(list);
+  if (is_cut(list, n_adj))
+    gather_cut_wave(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj, n_adj,
+                    dldf + g.field_off, ww);
+  else
+    gather_wave(g, ep, sums, n_adj > 0 ? last : 0u, dldf + g.field_off, ww, s_wave[wv]);
 }
 
 }  // namespace mc
@@ -748,8 +753,8 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
   const CountSrc cs{(const uint32_t*)(body + h->off_lpre),
                     (const unsigned long long*)(body + h->off_tloc),
                     (const unsigned long long*)(body + h->off_bpre), 0, 0, 0};
-  // the endpoint words live in the workspace; every call with this vertex count
-  // writes the same values there
+  // the endpoint words live in the workspace; every call on it writes the same
+  // values there
   char* wb = const_cast<char*>(body);
   const Endpoints ep{(uint64_t*)(wb + h->off_ends), (uint16_t*)(wb + h->off_end_pre),
                      (uint32_t*)(wb + h->off_end_sum), (uint32_t*)(wb + h->off_end_tile),
@@ -757,21 +762,22 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
   const VertexAdj* adj = (const VertexAdj*)d_scratch;
   f32x4* sums = (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points));
   const dim3 grid((unsigned)(h->ngen * kAdjTileBlocks)), block(kAdjThreads);
+  const EdgeList list{d_counts, n_points, (const Ctrl*)(body + h->off_ctrl)};
   if (n_points > 0) {
     const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
     k_batch_records<<<dim3((unsigned)(vertex_blocks + h->ngen)), block, 0, s>>>(
         vols, h->nvols, (const uint32_t*)(body + h->off_vol_first), d_fields, d_edges,
-        d_dl_dvertices, d_dl_dnormals, d_counts, n_points, (VertexAdj*)d_scratch, gen_tiles, bits,
-        cs, (const Ctrl*)(body + h->off_ctrl), ep, vertex_blocks);
+        d_dl_dvertices, d_dl_dnormals, list, (VertexAdj*)d_scratch, gen_tiles, bits, cs, ep,
+        vertex_blocks);
     DAXHIP_LAUNCH_CHECK("k_batch_records");
     k_scan_endpoints<<<1, kAdjScanThreads, 0, s>>>(ep.sums, ep.tile, h->ngen, sums);
     DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
-    k_batch_endpoint_sums<<<grid, block, 0, s>>>(vols, gen_tiles, bits, cs.lpre, ep, adj, d_counts,
-                                                 n_points, sums);
+    k_batch_endpoint_sums<<<grid, block, 0, s>>>(vols, gen_tiles, bits, cs.lpre, ep, adj, list,
+                                                 sums);
     DAXHIP_LAUNCH_CHECK("k_batch_endpoint_sums");
   }
-  k_batch_point_gather<<<grid, block, 0, s>>>(vols, gen_tiles, ep, sums, last_slot(n_points),
-                                              d_dl_dfields);
+  k_batch_point_gather<<<grid, block, 0, s>>>(vols, gen_tiles, bits, cs.lpre, ep, adj, list, sums,
+                                              last_slot(n_points), d_dl_dfields);
   DAXHIP_LAUNCH_CHECK("k_batch_point_gather");
   return DAX_HIP_OK;
 }

@@ -605,8 +605,9 @@ int dax_hip_mc_batch_autotune(const float* d_fields, void* h_header, void* d_wor
  * offsets) from dL/dvertex and dL/dnormal [U][3] of the concatenated outputs
  * of the last dax_hip_mc_batch_forward on this workspace (run with the edge
  * list).  d_scratch holds dax_hip_mc_backward_scratch_bytes(n_points).  Writes
- * its endpoint words into a part of the workspace of their own, the same ones
- * whenever n_points covers the forward's vertices.
+ * its endpoint words into a part of the workspace of their own, the same values
+ * from every call after one forward, so that calls with scratches of their own
+ * may overlap.
  * No reference counterpart. */
 int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
                               const void* d_workspace, size_t workspace_bytes,
@@ -644,7 +645,8 @@ int dax_hip_graph_destroy(void* graph_exec);
  * dL/dnormals [U][3], with the topology of the forward held fixed.  Uses the
  * forward's workspace (inside-bits and count prefixes must still hold the
  * forward of this field and iso; the backward writes only its endpoint words
- * there, in a part of their own) and its compact edge list d_edges; the
+ * there, in a part of their own, the same values from every call after one
+ * forward) and its compact edge list d_edges; the
  * interpolants (t, endpoint gradients) are recomputed from the field.
  * U = min(d_counts[1], n_points) if d_counts is given (device {T, U} of the
  * forward), else n_points.  d_scratch needs

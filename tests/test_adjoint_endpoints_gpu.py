@@ -65,3 +65,56 @@ def test_cut_edge_list(cut):
     got = mc.backward(field, 0.1, cut_out, dx[:n].contiguous().cuda(),
                       dn[:n].contiguous().cuda())
     assert torch.equal(got, whole)
+
+
+def _batch(n_volumes):
+    dims = [(70, 13, 11), (9, 8, 7), (64, 5, 6), (130, 9, 4)][:n_volumes]
+    fs = [_field(d, 3 + i, 1.0).reshape(-1) for i, d in enumerate(dims)]
+    flat = torch.from_numpy(np.concatenate(fs)).cuda()
+    b = mc.Batch(dims, [0.1] * len(dims))
+    T, U = b.sizes(flat)
+    bufs = b.alloc(U, T)
+    b.forward_into(flat, bufs)
+    return b, flat, bufs, U
+
+
+@pytest.mark.parametrize("cut", [1, 40, 2000, -1])
+def test_batch_cut_edge_list(cut):
+    print(f"[case] batch adjoint cut {cut}", flush=True)
+    b, flat, bufs, U = _batch(4)
+    n = cut if cut >= 0 else U - 1
+    assert 0 < n < U
+    dx, dn = (t.cuda() for t in _grads(U, 9))
+    dx[n:] = 0.0
+    dn[n:] = 0.0
+    scratch = torch.empty(b.scratch_bytes(U), dtype=torch.uint8, device="cuda")
+    whole, got = torch.empty_like(flat), torch.empty_like(flat)
+    b.backward(flat, bufs, dx, dn, scratch, whole)
+    b.backward(flat, dict(bufs, cap_points=n), dx, dn, scratch, got)
+    assert torch.equal(got, whole)
+
+
+def test_calls_write_the_same_workspace():
+    """What a backward leaves in the workspace does not depend on how many of
+    the edges it takes, so that calls that share one may overlap."""
+    print("[case] adjoint workspace of whole and cut lists", flush=True)
+    field = torch.from_numpy(_field((70, 13, 11), 3, 1.0)).cuda()
+    out = mc.forward(field, 0.1, edges=True)
+    U = out.num_points
+    dx, dn = (t.cuda() for t in _grads(U, 9))
+    mc.backward(field, 0.1, out, dx, dn)
+    before = out.workspace.clone()
+    for n in (1, 100, U // 2, U - 1):
+        cut = mc.Contour(**{**out.__dict__, "vertices": out.vertices[:n]})
+        mc.backward(field, 0.1, cut, dx[:n].contiguous(), dn[:n].contiguous())
+        assert torch.equal(out.workspace, before), n
+
+    b, flat, bufs, U = _batch(4)
+    dx, dn = (t.cuda() for t in _grads(U, 9))
+    scratch = torch.empty(b.scratch_bytes(U), dtype=torch.uint8, device="cuda")
+    g = torch.empty_like(flat)
+    b.backward(flat, bufs, dx, dn, scratch, g)
+    before = b.workspace.clone()
+    for n in (1, 100, U // 2, U - 1):
+        b.backward(flat, dict(bufs, cap_points=n), dx, dn, scratch, g)
+        assert torch.equal(b.workspace, before), n
