@@ -17,8 +17,8 @@
 //   records    one thread per vertex, recomputes t, gA, gB from the field and
 //              the compact edge list (the interpolants are not stored by the
 //              forward), writes 8 floats per vertex (sA, GA[3], sB, GB[3]);
-//              beside it a thread per row word writes the word's endpoints
-//              (the points of active edges) and their counts
+//              beside it the row words' endpoints are written
+//              (the points of active edges) and their counts, a wave per tile
 //   scan       the tiles' endpoint counts, so that every endpoint has a slot
 //   endpoints  each endpoint's sums (S, G) over its at most 6 edges, once
 //   gather     every point: 0, or within L1 distance 1 of an endpoint (the
@@ -116,39 +116,38 @@ __device__ __forceinline__ void vertex_adjoint(const VolGeom& g, const float* __
 }
 
 // ---- endpoints and gather ---------------------------------------------------
-// Endpoint words and prefixes by tiles of 256 row words, sums and gather a
-// wave per 32 words; nothing is shared between the waves of a block.  What the
+// Endpoint words and prefixes a wave per tile of 256 row words, sums and gather
+// a wave per WW words; nothing is shared between the waves of a block.  What the
 // steps hand on goes through global memory (the caches), so a wave needs
 // little LDS and no barrier, and no work is repeated at tile borders.  A block
 // per tile that staged edge flags with a halo, formed the sums of the tile's
 // and the halo's endpoints in LDS between six barriers and listed tiles too
 // dense for it for another pass took 56 + 28 us at 256^3 (447 K endpoints),
-// 490 + 14 on a noisy 640^3 surface (3.6 M) and 375 + 60 for 256 volumes of
-// 32..160 points an axis (1.4 M).  Sums and gather take 20 + 23, 99 + 305 and
-// 62 + 267, the words and the scan 5, 40 and 45 more.
+// 490 + 14 on a noisy 640^3 surface (3.6 M), 375 + 60 for 256 volumes of
+// 32..160 points an axis (1.4 M) and 1674 + 4 on the 1024^3 Mandelbulb.  Sums and
+// gather take 20 + 24, 100 + 311, 57 + 264 and 252 + 1216; the words, beside the
+// records, and their scan 4, 30, 28 and 105 more.
 constexpr int kAdjTile = kGatherTileWords;  // row words per tile
 constexpr int kAdjThreads = kAdjTile;
-// Words per wave of the sums and the gather.  16 fill too few lanes of large
-// volumes, 64 leave small ones too few waves: a whole step took 125 / 126 /
-// 131 us at 256^3 with 16 / 32 / 64, 985 / 972 / 987 at 640^3, 781 / 757 / 768
-// for the batch.
-constexpr int kAdjWaveWords = 32;
-constexpr int kAdjBlockWords = kAdjThreads / 64 * kAdjWaveWords;
-constexpr int kAdjTileBlocks = kAdjTile / kAdjBlockWords;
+// Words per wave of the sums and the gather (adjoint_wave_words).
+template <int WW>
+constexpr int kAdjBlockWords = kAdjThreads / 64 * WW;
+template <int WW>
+constexpr int kAdjTileBlocks = kAdjTile / kAdjBlockWords<WW>;
+// Waves per SIMD the gather is compiled for: as many as there are, except on
+// large volumes, where fewer waves keep what they share in the caches (1024^3
+// 1258 us with 8, 1216 with the 6 it takes by itself; 256 volumes 279, 264).
+template <int WW>
+constexpr int kGatherWaves = WW == 64 ? 1 : 8;
 
 // How many edges of the list a call takes: n_points, and not more than counts[1]
-// where the forward's counts are given.  The list is cut if that leaves out a
-// vertex of the surface (ctrl: the forward's totals).
+// where the forward's counts are given.
 struct EdgeList {
   const int64_t* counts;
   int64_t n_points;
-  const Ctrl* ctrl;
 };
 __device__ __forceinline__ int64_t edge_count(const EdgeList& l) {
   return l.counts ? min(l.counts[1], l.n_points) : l.n_points;
-}
-__device__ __forceinline__ bool is_cut(const EdgeList& l, int64_t n) {
-  return n > 0 && (unsigned long long)n < l.ctrl->total_v;
 }
 
 // Endpoint words of a volume (or batch) and their prefixes: the endpoints of
@@ -169,56 +168,103 @@ __device__ __forceinline__ uint32_t vertex_base(const VolGeom& g, const Endpoint
   return ep.base[2 * g.tile_off + w / kCountTile] + (lpre[w] & 0xffffu);
 }
 
-// Endpoints of row word w: the points whose bit differs from one of their
-// neighbours' (grids without cells have none).  They depend on the bits alone,
-// not on how many of the edges a call takes, so that calls that share a
-// workspace write the same words there.
-__device__ __forceinline__ uint64_t endpoint_word(const VolGeom& g, const uint64_t* __restrict__ b,
-                                                  int64_t w) {
-  const int64_t plane = (int64_t)g.wpr * g.ny;
-  const WordPos p = word_pos(g, w);
-  const uint64_t A = b[w];
-  const uint64_t next = p.q + 1 < g.wpr ? b[w + 1] : 0ull;
-  const uint64_t yp = p.has_y ? b[w + g.wpr] : A, ym = p.j > 0 ? b[w - g.wpr] : A;
-  const uint64_t zp = p.has_z ? b[w + plane] : A, zm = p.k > 0 ? b[w - plane] : A;
-  const uint64_t prev = p.q > 0 ? b[w - 1] >> 63 : A & 1ull;
-  const uint64_t fx = (A ^ shr1(A, next)) & p.xmask;
-  const uint64_t e =
-      fx | (fx << 1) | ((prev ^ A) & 1ull) | (A ^ yp) | (A ^ ym) | (A ^ zp) | (A ^ zm);
-  return e & p.pmask;
-}
-
-// Endpoint words, counts and prefixes of a tile (block of kAdjThreads).
+// Endpoint words, counts and prefixes of a tile by one wave, four consecutive
+// words a lane.  Endpoints of a word: the points whose bit differs from one of
+// their neighbours' (grids without cells have none).  They depend on the bits
+// alone, not on how many of the edges a call takes, so that calls that share a
+// workspace write the same values there.
 __device__ __forceinline__ void endpoint_words_tile(const VolGeom& g,
                                                     const uint64_t* __restrict__ b,
                                                     const CountSrc& cs, const Endpoints& ep,
-                                                    int64_t w0, uint32_t* s_scan) {
-  const int64_t w = w0 + threadIdx.x;
-  const uint64_t e = w < g.nwords ? endpoint_word(g, b, w) : 0ull;
-  uint32_t total;
-  const uint32_t pre = block_excl_scan((uint32_t)popc(e), total, s_scan);
+                                                    int64_t w0) {
+  const int lane = threadIdx.x & 63;
+  const int64_t w = w0 + 4 * lane, plane = (int64_t)g.wpr * g.ny;
+  const int64_t tile = g.tile_off + w0 / kAdjTile;
+  uint64_t e[4] = {0ull, 0ull, 0ull, 0ull};
+  uint32_t n = 0u;
   if (w < g.nwords) {
-    ep.words[g.word_off + w] = e;
-    ep.pre[g.word_off + w] = (uint16_t)pre;
+    auto load4 = [&](int64_t at, uint64_t (&v)[4]) {
+      if (at >= 0 && at + 4 <= g.nwords) {
+        __builtin_memcpy(v, b + at, 32);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = at + i >= 0 && at + i < g.nwords ? b[at + i] : 0ull;
+      }
+    };
+    uint64_t A[4], yp[4], ym[4], zp[4], zm[4];
+    load4(w, A);
+    load4(w + g.wpr, yp);
+    load4(w - g.wpr, ym);
+    load4(w + plane, zp);
+    load4(w - plane, zm);
+    uint64_t prev = w > 0 ? b[w - 1] : 0ull;
+    const uint64_t last = w + 4 < g.nwords ? b[w + 4] : 0ull;
+    WordIter wi;
+    wi.init(g, (int)w);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const WordPos p = wi.pos(g);
+      const uint64_t a = A[i], next = p.q + 1 < g.wpr ? (i < 3 ? A[(i + 1) % 4] : last) : 0ull;
+      const uint64_t fx = (a ^ shr1(a, next)) & p.xmask;
+      uint64_t m = fx | (fx << 1);
+      if (p.q > 0) m |= ((prev >> 63) ^ a) & 1ull;
+      if (p.has_y) m |= a ^ yp[i];
+      if (p.j > 0) m |= a ^ ym[i];
+      if (p.has_z) m |= a ^ zp[i];
+      if (p.k > 0) m |= a ^ zm[i];
+      e[i] = w + i < g.nwords ? m & p.pmask : 0ull;
+      n += (uint32_t)popc(e[i]);
+      prev = a;
+      wi.next(g);
+    }
   }
-  if (threadIdx.x == 0) ep.sums[g.tile_off + w0 / kAdjTile] = total;
-  if (threadIdx.x < 2) {
-    const int64_t c = w0 / kCountTile + threadIdx.x;
+  const uint32_t inc = wave_incl_scan(n);
+  uint32_t run = inc - n;
+  uint16_t pre[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    pre[i] = (uint16_t)run;
+    run += (uint32_t)popc(e[i]);
+  }
+  if (w + 4 <= g.nwords) {
+    __builtin_memcpy(ep.words + g.word_off + w, e, 32);
+    __builtin_memcpy(ep.pre + g.word_off + w, pre, 8);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (w + i < g.nwords) {
+        ep.words[g.word_off + w + i] = e[i];
+        ep.pre[g.word_off + w + i] = pre[i];
+      }
+  }
+  if (lane == 63) ep.sums[tile] = inc;
+  if (lane < 2) {
+    const int64_t c = w0 / kCountTile + lane;
     if (c < cs.n_ctiles) ep.base[2 * g.tile_off + c] = (uint32_t)ctile_prefix(cs, c);
   }
 }
 
-// Exclusive scan of the tiles' counts by one block; it also clears slot 0 of the
-// endpoints' sums, which stands for the points that are no endpoints.
+// Exclusive scan of the tiles' counts, a block per kScanTiles of them (at most
+// kScanBlocks blocks, so more each for more tiles): a block sums up what lies
+// before its part by itself.  It also clears slot 0 of the endpoints' sums,
+// which stands for the points that are no endpoints.
 constexpr int kAdjScanThreads = 1024;
+constexpr int64_t kScanTiles = (int64_t)kAdjScanThreads * kScanChunk;
+constexpr int kScanBlocks = 16;
 static __global__ __launch_bounds__(kAdjScanThreads) void k_scan_endpoints(
-    const uint32_t* __restrict__ sums, uint32_t* __restrict__ pre, int64_t n,
+    const uint32_t* __restrict__ sums, uint32_t* __restrict__ pre, int64_t n, int64_t part,
     f32x4* __restrict__ endpoint_sums) {
-  if (threadIdx.x == 0) endpoint_sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   __shared__ uint32_t s_scan[kAdjScanThreads / 64];
-  constexpr int64_t kRound = (int64_t)kAdjScanThreads * kScanChunk;
-  uint32_t carry = 0u;
-  for (int64_t c0 = 0; c0 < n; c0 += kRound) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) endpoint_sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int64_t first = (int64_t)blockIdx.x * part, end = min(first + part, n);
+  uint32_t before = 0u, carry;
+  for (int64_t i = 4 * (int64_t)threadIdx.x; i < first; i += 4 * kAdjScanThreads) {
+    uint32_t v[4];  // first is a multiple of 4
+    __builtin_memcpy(v, sums + i, 16);
+    before += v[0] + v[1] + v[2] + v[3];
+  }
+  (void)block_excl_scan(before, carry, s_scan);
+  for (int64_t c0 = first; c0 < end; c0 += kScanTiles) {
     const int64_t i0 = c0 + (int64_t)threadIdx.x * kScanChunk;
     u32x4 x[kScanChunk / 4];
     load_chunk(sums, i0, n, x);
@@ -229,6 +275,14 @@ static __global__ __launch_bounds__(kAdjScanThreads) void k_scan_endpoints(
     carry += total;
     store_prefixes(pre, i0, n, x, run);
   }
+}
+inline int launch_scan_endpoints(const Endpoints& ep, int64_t tiles, f32x4* sums, hipStream_t s) {
+  const int64_t part = align_up(
+      (size_t)std::max(kScanTiles, ceil_div(tiles, (int64_t)kScanBlocks)), (size_t)kScanTiles);
+  k_scan_endpoints<<<dim3((unsigned)ceil_div(tiles, part)), kAdjScanThreads, 0, s>>>(
+      ep.sums, ep.tile, tiles, part, sums);
+  DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
+  return DAX_HIP_OK;
 }
 
 __device__ __forceinline__ uint64_t shfl64(uint64_t v, int l) {
@@ -330,21 +384,25 @@ __device__ __forceinline__ f32x4 endpoint_sums(const VolGeom& g, const uint64_t*
 }
 
 // The sums of a wave's words' endpoints, a lane per endpoint, at their
-// slots (1 + the endpoints before; at most cap).
+// slots (1 + the endpoints before; at most two per point).  before: those
+// before the words' tile.
+template <int WW>
 __device__ __forceinline__ void endpoint_sums_wave(const VolGeom& g,
                                                    const uint64_t* __restrict__ b,
                                                    const uint32_t* __restrict__ lpre,
                                                    const Endpoints& ep,
                                                    const VertexAdj* __restrict__ adj,
-                                                   int64_t n_adj, f32x4* __restrict__ sums,
-                                                   int64_t cap, int64_t ww, uint8_t* mark) {
+                                                   const EdgeList& list, f32x4* __restrict__ sums,
+                                                   int64_t ww, uint32_t before, uint8_t* mark) {
   const int lane = threadIdx.x & 63;
   const int64_t w = ww + lane;
-  const uint64_t e = lane < kAdjWaveWords && w < g.nwords ? ep.words[g.word_off + w] : 0ull;
+  const uint64_t e = lane < WW && w < g.nwords ? ep.words[g.word_off + w] : 0ull;
   const uint32_t n = (uint32_t)popc(e);
   if (!__ballot(n != 0u)) return;
+  // read when it is needed: most waves of a large volume have left by now
+  const int64_t n_adj = edge_count(list), cap = 2 * list.n_points;
   const uint32_t inc = wave_incl_scan(n), total = wave_last(inc);
-  const int64_t slot0 = 1 + (int64_t)ep.tile[g.tile_off + ww / kAdjTile] + ep.pre[g.word_off + ww];
+  const int64_t slot0 = 1 + (int64_t)before + ep.pre[g.word_off + ww];
   for (uint32_t e0 = 0; e0 < total; e0 += 64u) {  // wave-uniform
     const int wl = item_word(n, inc, e0, mark);
     const uint32_t i = e0 + (uint32_t)lane;
@@ -427,12 +485,13 @@ __device__ __forceinline__ void zero_run(const VolGeom& g, float* __restrict__ o
 }
 
 // dL/df of the point (x, j, k) of row word w from the records of its and its
-// neighbours' edges, in combine_point's order: for an edge list cut below the
-// surface's vertices, whose endpoints' sums have no slots.
-__device__ float cut_point(const VolGeom& g, const uint64_t* __restrict__ b,
-                           const uint32_t* __restrict__ lpre, const Endpoints& ep,
-                           const VertexAdj* __restrict__ adj, int64_t n_adj, int64_t w, int x, int j,
-                           int k) {
+// neighbours' edges, in combine_point's order: an edge list cut below the
+// surface's vertices has slots for two endpoints per edge it holds, so that the
+// sums of later endpoints have none.
+__device__ __forceinline__ float cut_point(const VolGeom& g, const uint64_t* __restrict__ b,
+                                           const uint32_t* __restrict__ lpre, const Endpoints& ep,
+                                           const VertexAdj* __restrict__ adj, int64_t n_adj,
+                                           int64_t w, int x, int j, int k) {
   const int64_t plane = (int64_t)g.wpr * g.ny;
   float acc = 0.0f;
 #pragma unroll 1
@@ -465,47 +524,20 @@ __device__ float cut_point(const VolGeom& g, const uint64_t* __restrict__ b,
   return acc;
 }
 
-// dL/df of the points of a wave's row words for a cut edge list, a lane per
-// point of a word.
-__device__ __forceinline__ void gather_cut_wave(const VolGeom& g, const uint64_t* __restrict__ b,
-                                                const uint32_t* __restrict__ lpre,
-                                                const Endpoints& ep,
-                                                const VertexAdj* __restrict__ adj, int64_t n_adj,
-                                                float* __restrict__ out, int64_t ww) {
-  const int lane = threadIdx.x & 63;
-  const int64_t plane = (int64_t)g.wpr * g.ny;
-  const uint64_t* ew = ep.words + g.word_off;
-  for (int64_t w = ww; w < min(ww + kAdjWaveWords, g.nwords); ++w) {  // wave-uniform
-    const WordPos p = word_pos(g, w);
-    const uint64_t e = ew[w];
-    uint64_t r = e | (e << 1) | (e >> 1);
-    if (p.q > 0) r |= ew[w - 1] >> 63;
-    if (p.q + 1 < g.wpr) r |= ew[w + 1] << 63;
-    if (p.j > 0) r |= ew[w - g.wpr];
-    if (p.has_y) r |= ew[w + g.wpr];
-    if (p.k > 0) r |= ew[w - plane];
-    if (p.has_z) r |= ew[w + plane];
-    const int x = p.q * 64 + lane;
-    if (x >= g.nx) continue;
-    const float v = (r >> lane) & 1ull
-                        ? cut_point(g, b, lpre, ep, adj, n_adj, w, x, p.j, p.k) : 0.0f;
-    out[x + (int64_t)g.nx * (p.j + (int64_t)g.ny * p.k)] = v;
-  }
-}
-
 // What a wave of the gather keeps of its words: the endpoint words of the word
 // itself, the rows before and after it and the planes before and after it, the
 // slots before their first endpoints, the points that receive something and
 // the number of them before the word, the word's first point, and flags:
 // bit 0 / 1: the point before / after the word is an endpoint, bit 2: no
 // receiving point is within two points of a border.
+template <int WW>
 struct GatherWave {
-  uint64_t ends[5][kAdjWaveWords];
-  uint64_t recv[kAdjWaveWords];
-  uint32_t slot[5][kAdjWaveWords];
-  uint32_t start[kAdjWaveWords];
-  uint32_t base[kAdjWaveWords];
-  uint8_t flags[kAdjWaveWords];
+  uint64_t ends[5][WW];
+  uint64_t recv[WW];
+  uint32_t slot[5][WW];
+  uint32_t start[WW];
+  uint32_t base[WW];
+  uint8_t flags[WW];
   uint8_t mark[64];
 };
 
@@ -521,16 +553,20 @@ struct GatherWave {
 // wave-uniform masks, whole words stored) took 44 us at 256^3 and 334 at
 // 640^3 where this takes 23 and 305..317; the points composed in LDS and stored
 // once 29 and 323.
-__device__ __forceinline__ void gather_wave(const VolGeom& g, const Endpoints& ep,
+template <int WW>
+__device__ __forceinline__ void gather_wave(const VolGeom& g, const uint64_t* __restrict__ b,
+                                            const uint32_t* __restrict__ lpre, const Endpoints& ep,
+                                            const VertexAdj* __restrict__ adj, const EdgeList& list,
                                             const f32x4* __restrict__ sums, uint32_t cap,
-                                            float* __restrict__ out, int64_t ww, GatherWave& W) {
+                                            float* __restrict__ out, int64_t ww,
+                                            GatherWave<WW>& W) {
   const int lane = threadIdx.x & 63;
   const int64_t plane = (int64_t)g.wpr * g.ny;
   const int64_t w = ww + lane;
   uint64_t e[5], r = 0ull;
   int64_t at[5] = {w, w, w, w, w};
   uint32_t flags = 0u, base = 0u;
-  if (lane < kAdjWaveWords && w < g.nwords && cap != 0u) {
+  if (lane < WW && w < g.nwords && cap != 0u) {
     const WordPos p = word_pos(g, w);
     base = ((uint32_t)p.k * (uint32_t)g.ny + (uint32_t)p.j) * (uint32_t)g.nx + (uint32_t)p.q * 64u;
     const uint64_t* ew = ep.words + g.word_off;
@@ -561,8 +597,9 @@ __device__ __forceinline__ void gather_wave(const VolGeom& g, const Endpoints& e
       slot[n] = ep.pre[g.word_off + at[n]];
     }
   }
-  zero_run(g, out, ww, min(ww + kAdjWaveWords, g.nwords), lane, 64);
+  zero_run(g, out, ww, min(ww + WW, g.nwords), lane, 64);
   if (!__ballot(r != 0ull)) return;
+  const int64_t n_adj = edge_count(list);
   const uint32_t n = (uint32_t)popc(r);
   const uint32_t inc = wave_incl_scan(n), total = wave_last(inc);
   if (r != 0ull) {
@@ -578,6 +615,7 @@ __device__ __forceinline__ void gather_wave(const VolGeom& g, const Endpoints& e
   }
   wave_lds_sync();
   const float* sf = reinterpret_cast<const float*>(sums);
+  bool cut = false;
   for (uint32_t e0 = 0; e0 < total; e0 += 64u) {  // wave-uniform
     const int i = item_word(n, inc, e0, W.mark);
     const uint32_t t = e0 + (uint32_t)lane;
@@ -585,34 +623,53 @@ __device__ __forceinline__ void gather_wave(const VolGeom& g, const Endpoints& e
     const int bit = select_bit(W.recv[i], (int)(t - W.start[i]));
     const int up = 63 - bit;  // brings the point's bit to the sign
     const uint32_t fl = W.flags[i];
-    // slot 0 holds zeros
-    auto slot_of = [&](bool on, uint32_t s) -> uint32_t { return on ? min(s, cap) : 0u; };
-    PointTerms v;
+    uint32_t slot[7];  // own, then before and after along each axis; slot 0 holds zeros
     {
       const uint64_t own = W.ends[0][i], o = own << up;
       const uint32_t s = W.slot[0][i] + (uint32_t)popc(o);
       const bool on = (int64_t)o < 0;
       const bool before = (int64_t)(((own << 1) | (fl & 1u)) << up) < 0;
       const bool after = (int64_t)(((own >> 1) | ((uint64_t)(fl & 2u) << 62)) << up) < 0;
-      v.own = sums[slot_of(on, s)];
-      v.before[0] = sf[4 * (int64_t)slot_of(before, s - (on ? 1u : 0u)) + 1];
-      v.after[0] = sf[4 * (int64_t)slot_of(after, s + 1u) + 1];
+      slot[0] = on ? s : 0u;
+      slot[1] = before ? s - (on ? 1u : 0u) : 0u;
+      slot[2] = after ? s + 1u : 0u;
     }
 #pragma unroll
     for (int d = 1; d < 3; ++d) {
-      const uint64_t b = W.ends[2 * d - 1][i] << up, a = W.ends[2 * d][i] << up;
-      const uint32_t sb = W.slot[2 * d - 1][i] + (uint32_t)popc(b),
-                     sa = W.slot[2 * d][i] + (uint32_t)popc(a);
-      v.before[d] = sf[4 * (int64_t)slot_of((int64_t)b < 0, sb) + 1 + d];
-      v.after[d] = sf[4 * (int64_t)slot_of((int64_t)a < 0, sa) + 1 + d];
+      const uint64_t b4 = W.ends[2 * d - 1][i] << up, af = W.ends[2 * d][i] << up;
+      slot[2 * d + 1] = (int64_t)b4 < 0 ? W.slot[2 * d - 1][i] + (uint32_t)popc(b4) : 0u;
+      slot[2 * d + 2] = (int64_t)af < 0 ? W.slot[2 * d][i] + (uint32_t)popc(af) : 0u;
     }
+    uint32_t far = slot[0];
+#pragma unroll
+    for (int q = 1; q < 7; ++q) far = max(far, slot[q]);
     float* o = out + (int64_t)W.base[i] + bit;
+    cut = cut || far > cap;  // a cut list: some sums have no slot
+#pragma unroll
+    for (int q = 0; q < 7; ++q) slot[q] = min(slot[q], cap);
+    PointTerms v;
+    v.own = sums[slot[0]];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      v.before[d] = sf[4 * (int64_t)slot[2 * d + 1] + 1 + d];
+      v.after[d] = sf[4 * (int64_t)slot[2 * d + 2] + 1 + d];
+    }
     if (!__ballot(!(fl & 4u))) {
       *o = combine_point<true>(g, 0, 0, 0, v);
     } else {
       const WordPos p = word_pos(g, ww + i);
       *o = combine_point<false>(g, p.q * 64 + bit, p.j, p.k, v);
     }
+  }
+  if (__builtin_expect(!__ballot(cut), 1)) return;
+  for (uint32_t e0 = 0; e0 < total; e0 += 64u) {  // wave-uniform
+    const int i = item_word(n, inc, e0, W.mark);
+    const uint32_t t = e0 + (uint32_t)lane;
+    if (t >= total) continue;
+    const int bit = select_bit(W.recv[i], (int)(t - W.start[i]));
+    const WordPos p = word_pos(g, ww + i);
+    out[(int64_t)W.base[i] + bit] =
+        cut_point(g, b, lpre, ep, adj, n_adj, ww + i, p.q * 64 + bit, p.j, p.k);
   }
 }
 
@@ -626,6 +683,18 @@ __host__ __device__ constexpr size_t endpoint_sums_offset(int64_t n_points) {
 }
 __host__ __device__ constexpr size_t adjoint_scratch_bytes(int64_t n_points) {
   return n_points > 0 ? 2 * endpoint_sums_offset(n_points) + 16 : 0;
+}
+// Words per wave of the sums and the gather of `nwords` row words in `tiles`
+// tiles.  Large volumes have mostly words without points, where a wave of few
+// words is spent on finding that out, and fewer lanes have something to do.
+// Backward in us with 32 / 64 words, Gaussian mixtures of n^3 points: 256
+// 59 / 65, 512 219 / 221; 256 volumes of 32..160 points an axis 439 / 428;
+// sums + gather of the 1024^3 Mandelbulb 1754 / 1460.  Volumes of a batch that
+// leave their tiles mostly empty take one wave each (20000 of 6 x 7 x 5 points
+// 83 / 42).
+inline int adjoint_wave_words(int64_t nwords, int64_t tiles) {
+  if (nwords < 64 * tiles && tiles > 1) return 64;
+  return nwords < (1 << 22) ? 32 : 64;
 }
 // The last slot (a volume or batch of at most 2^31 points has fewer endpoints).
 inline uint32_t last_slot(int64_t n_points) {

@@ -7,50 +7,52 @@ namespace daxhip {
 namespace mc {
 
 // Blocks [0, vertex_blocks): a thread per vertex; the rest: the endpoint words
-// of a tile each.
+// of a tile per wave (in a launch of their own they took as long: 1024^3 110 +
+// 337 us against 451).
 __global__ __launch_bounds__(kAdjThreads) void k_adjoint_records(
     VolGeom g, const float* __restrict__ field, const uint32_t* __restrict__ edges,
-    const float* __restrict__ dldx, const float* __restrict__ dldn,
-    EdgeList list, VertexAdj* __restrict__ out, const uint64_t* __restrict__ bits, CountSrc cs,
-    Endpoints ep, int64_t vertex_blocks) {
-  __shared__ uint32_t s_scan[kAdjThreads / 64];
+    const float* __restrict__ dldx, const float* __restrict__ dldn, EdgeList list,
+    VertexAdj* __restrict__ out, const uint64_t* __restrict__ bits, CountSrc cs,
+    const Ctrl* __restrict__ ctrl, Endpoints ep, int64_t vertex_blocks) {
+  const int64_t U = edge_count(list);
   if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
-    cs.tpb_shift = (int)list.ctrl->tpb_shift;
-    endpoint_words_tile(g, bits, cs, ep, ((int64_t)blockIdx.x - vertex_blocks) * kAdjTile, s_scan);
+    const int64_t w0 = (((int64_t)blockIdx.x - vertex_blocks) * (kAdjThreads / 64) +
+                        __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kAdjTile;
+    if (w0 >= g.nwords) return;  // wave-uniform
+    cs.tpb_shift = (int)ctrl->tpb_shift;
+    endpoint_words_tile(g, bits, cs, ep, w0);
     return;
   }
   // XCD-contiguous vertex ranges: vertices are in edge order, so the field
   // lines of neighbouring stencils stay in one XCD's L2
   const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
-  if (u >= edge_count(list)) return;
+  if (u >= U) return;
   vertex_adjoint(g, field, edges, dldx, dldn, u, out);
 }
 
+template <int WW>
 __global__ __launch_bounds__(kAdjThreads) void k_endpoint_sums(
     VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre,
     Endpoints ep, const VertexAdj* __restrict__ adj, EdgeList list, f32x4* __restrict__ sums) {
   __shared__ uint8_t s_mark[kAdjThreads / 64][64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords + wv * kAdjWaveWords;
+  const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
+  const int64_t ww = blk * kAdjBlockWords<WW> + wv * WW;
+  const uint32_t before = ep.tile[blk / kAdjTileBlocks<WW>];
   if (ww < g.nwords)  // wave-uniform
-    endpoint_sums_wave(g, bits, lpre, ep, adj, edge_count(list), sums, 2 * list.n_points, ww,
-                       s_mark[wv]);
+    endpoint_sums_wave<WW>(g, bits, lpre, ep, adj, list, sums, ww, before, s_mark[wv]);
 }
 
-// From the endpoints' sums, or (a cut list) from the records.
-__global__ __launch_bounds__(kAdjThreads) void k_point_gather(
+template <int WW>
+__global__ __launch_bounds__(kAdjThreads, kGatherWaves<WW>) void k_point_gather(
     VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
     const VertexAdj* __restrict__ adj, EdgeList list, const f32x4* __restrict__ sums,
     uint32_t last, float* __restrict__ dldf) {
-  __shared__ GatherWave s_wave[kAdjThreads / 64];
+  __shared__ GatherWave<WW> s_wave[kAdjThreads / 64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords + wv * kAdjWaveWords;
-  if (ww >= g.nwords) return;  // wave-uniform
-  const int64_t n_adj = edge_count(list);
-  if (is_cut(list, n_adj))
-    gather_cut_wave(g, bits, lpre, ep, adj, n_adj, dldf, ww);
-  else
-    gather_wave(g, ep, sums, n_adj > 0 ? last : 0u, dldf, ww, s_wave[wv]);
+  const int64_t ww = xcd_tile_runs(blockIdx.x, gridDim.x) * kAdjBlockWords<WW> + wv * WW;
+  if (ww < g.nwords)  // wave-uniform
+    gather_wave<WW>(g, bits, lpre, ep, adj, list, sums, last, dldf, ww, s_wave[wv]);
 }
 
 }  // namespace mc
@@ -58,6 +60,34 @@ __global__ __launch_bounds__(kAdjThreads) void k_point_gather(
 
 using namespace daxhip;
 using namespace daxhip::mc;
+
+namespace {
+
+// What the last two launches of a backward take besides the geometry.
+struct AdjointCall {
+  const uint64_t* bits;
+  CountSrc cs;
+  Endpoints ep;
+  EdgeList list;
+  VertexAdj* adj;
+  f32x4* sums;
+  float* dldf;
+};
+
+template <int WW>
+int launch_sums_gather(const VolGeom& g, const AdjointCall& c, hipStream_t s) {
+  const dim3 grid((unsigned)ceil_div(g.nwords, (int64_t)kAdjBlockWords<WW>)), block(kAdjThreads);
+  if (c.list.n_points > 0) {
+    k_endpoint_sums<WW><<<grid, block, 0, s>>>(g, c.bits, c.cs.lpre, c.ep, c.adj, c.list, c.sums);
+    DAXHIP_LAUNCH_CHECK("k_endpoint_sums");
+  }
+  k_point_gather<WW><<<grid, block, 0, s>>>(g, c.bits, c.cs.lpre, c.ep, c.adj, c.list, c.sums,
+                                            last_slot(c.list.n_points), c.dldf);
+  DAXHIP_LAUNCH_CHECK("k_point_gather");
+  return DAX_HIP_OK;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -124,26 +154,22 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
   const Endpoints ep{(uint64_t*)(ws + L.off_ends), (uint16_t*)(ws + L.off_end_pre),
                      (uint32_t*)(ws + L.off_end_sum), (uint32_t*)(ws + L.off_end_tile),
                      (uint32_t*)(ws + L.off_end_base)};
-  const VertexAdj* adj = (const VertexAdj*)d_scratch;
-  f32x4* sums = (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points));
+  const AdjointCall call{bits, cs, ep, EdgeList{d_counts, n_points}, (VertexAdj*)d_scratch,
+                         (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points)), d_dl_dfield};
   const int64_t tiles = ceil_div(g.nwords, (int64_t)kAdjTile);
-  const dim3 grid((unsigned)ceil_div(g.nwords, (int64_t)kAdjBlockWords)), block(kAdjThreads);
-  const EdgeList list{d_counts, n_points, (const Ctrl*)(ws + L.off_ctrl)};
   if (n_points > 0) {
     const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
-    k_adjoint_records<<<dim3((unsigned)(vertex_blocks + tiles)), block, 0, s>>>(
-        g, d_field, d_edges, d_dl_dvertices, d_dl_dnormals, list, (VertexAdj*)d_scratch, bits, cs,
-        ep, vertex_blocks);
+    const int64_t word_blocks = ceil_div(tiles, (int64_t)(kAdjThreads / 64));
+    k_adjoint_records<<<dim3((unsigned)(vertex_blocks + word_blocks)), kAdjThreads, 0, s>>>(
+        g, d_field, d_edges, d_dl_dvertices, d_dl_dnormals, call.list, call.adj, bits, cs,
+        (const Ctrl*)(ws + L.off_ctrl), ep, vertex_blocks);
     DAXHIP_LAUNCH_CHECK("k_adjoint_records");
-    k_scan_endpoints<<<1, kAdjScanThreads, 0, s>>>(ep.sums, ep.tile, tiles, sums);
-    DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
-    k_endpoint_sums<<<grid, block, 0, s>>>(g, bits, cs.lpre, ep, adj, list, sums);
-    DAXHIP_LAUNCH_CHECK("k_endpoint_sums");
+    if (const int rc = launch_scan_endpoints(ep, tiles, call.sums, s)) return rc;
   }
-  k_point_gather<<<grid, block, 0, s>>>(g, bits, cs.lpre, ep, adj, list, sums, last_slot(n_points),
-                                        d_dl_dfield);
-  DAXHIP_LAUNCH_CHECK("k_point_gather");
-  return DAX_HIP_OK;
+  switch (adjoint_wave_words(g.nwords, tiles)) {
+    case 32: return launch_sums_gather<32>(g, call, s);
+    default: return launch_sums_gather<64>(g, call, s);
+  }
 }
 
 }  // extern "C"

@@ -246,21 +246,24 @@ __global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
 // so that the geometry stays in scalar registers.  A block per tile of words
 // instead leaves most lanes idle (73 vertices per tile in 256 volumes of
 // 32..160 points an axis: 80 us; this: 58).  Blocks from vertex_blocks on form
-// the endpoint words of a tile each.
+// the endpoint words, a wave per tile.
 __global__ __launch_bounds__(256) void k_batch_records(
     const VolGeom* __restrict__ vols, int64_t nvols, const uint32_t* __restrict__ vol_first,
     const float* __restrict__ fields, const uint32_t* __restrict__ edges,
     const float* __restrict__ dldx, const float* __restrict__ dldn,
     EdgeList list, VertexAdj* __restrict__ out, const TileRef* __restrict__ tiles,
-    const uint64_t* __restrict__ bits, CountSrc all, Endpoints ep, int64_t vertex_blocks) {
-  __shared__ uint32_t s_scan[kAdjThreads / 64];
+    int64_t ntiles, const uint64_t* __restrict__ bits, CountSrc all,
+    const Ctrl* __restrict__ ctrl, Endpoints ep, int64_t vertex_blocks) {
   const int64_t U = edge_count(list);
   if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
-    const TileRef tr = tiles[(int64_t)blockIdx.x - vertex_blocks];
+    const int64_t t = ((int64_t)blockIdx.x - vertex_blocks) * (kAdjThreads / 64) +
+                      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (t >= ntiles) return;  // wave-uniform
+    const TileRef tr = tiles[t];
     const VolGeom g = vols[tr.vol];
     CountSrc cs = volume_counts(all, g);
-    cs.tpb_shift = (int)list.ctrl->tpb_shift;
-    endpoint_words_tile(g, bits + g.word_off, cs, ep, tr.w0, s_scan);
+    cs.tpb_shift = (int)ctrl->tpb_shift;
+    endpoint_words_tile(g, bits + g.word_off, cs, ep, tr.w0);
     return;
   }
   const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
@@ -287,6 +290,7 @@ __global__ __launch_bounds__(256) void k_batch_records(
 
 static_assert(kAdjTile == kBatchGenTile, "the adjoint's tiles are the generate tiles");
 
+template <int WW>
 __global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_sums(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
     const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
@@ -294,32 +298,32 @@ __global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_sums(
   __shared__ uint8_t s_mark[kAdjThreads / 64][64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
-  const TileRef tr = tiles[blk / kAdjTileBlocks];
+  const int64_t t = blk / kAdjTileBlocks<WW>, part = blk % kAdjTileBlocks<WW>;
+  const uint32_t before = ep.tile[t];
+  const TileRef tr = tiles[t];
   const VolGeom g = vols[tr.vol];
-  const int64_t ww = (int64_t)tr.w0 + (blk % kAdjTileBlocks) * kAdjBlockWords + wv * kAdjWaveWords;
+  const int64_t ww = (int64_t)tr.w0 + part * kAdjBlockWords<WW> + wv * WW;
   if (ww < g.nwords)  // wave-uniform
-    endpoint_sums_wave(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj,
-                       edge_count(list), sums, 2 * list.n_points, ww, s_mark[wv]);
+    endpoint_sums_wave<WW>(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj, list,
+                           sums, ww, before, s_mark[wv]);
 }
 
-__global__ __launch_bounds__(kAdjThreads) void k_batch_point_gather(
+template <int WW>
+__global__ __launch_bounds__(kAdjThreads, kGatherWaves<WW>) void k_batch_point_gather(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
     const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
     const VertexAdj* __restrict__ adj, EdgeList list, const f32x4* __restrict__ sums,
     uint32_t last, float* __restrict__ dldf) {
-  __shared__ GatherWave s_wave[kAdjThreads / 64];
+  __shared__ GatherWave<WW> s_wave[kAdjThreads / 64];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
-  const TileRef tr = tiles[blk / kAdjTileBlocks];
+  const TileRef tr = tiles[blk / kAdjTileBlocks<WW>];
   const VolGeom g = vols[tr.vol];
-  const int64_t ww = (int64_t)tr.w0 + (blk % kAdjTileBlocks) * kAdjBlockWords + wv * kAdjWaveWords;
-  if (ww >= g.nwords) return;  // wave-uniform
-  const int64_t n_adj = edge_count(list);
-  if (is_cut(list, n_adj))
-    gather_cut_wave(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj, n_adj,
-                    dldf + g.field_off, ww);
-  else
-    gather_wave(g, ep, sums, n_adj > 0 ? last : 0u, dldf + g.field_off, ww, s_wave[wv]);
+  const int64_t ww =
+      (int64_t)tr.w0 + blk % kAdjTileBlocks<WW> * kAdjBlockWords<WW> + wv * WW;
+  if (ww < g.nwords)  // wave-uniform
+    gather_wave<WW>(g, bits + g.word_off, lpre + g.tile_off * kBatchGenTile, ep, adj, list, sums,
+                    last, dldf + g.field_off, ww, s_wave[wv]);
 }
 
 }  // namespace mc
@@ -438,6 +442,35 @@ int batch_generate(const BatchHeader& h, const BatchPtrs& p, const float* d_fiel
         p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points, cap_tris,
         d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
   DAXHIP_LAUNCH_CHECK("k_batch_generate");
+  return DAX_HIP_OK;
+}
+
+// What the last two launches of a batch backward take.
+struct BatchAdjoint {
+  const VolGeom* vols;
+  const TileRef* tiles;
+  int64_t ntiles;
+  const uint64_t* bits;
+  const uint32_t* lpre;
+  Endpoints ep;
+  VertexAdj* adj;
+  EdgeList list;
+  f32x4* sums;
+  float* dldf;
+};
+
+template <int WW>
+int launch_batch_sums_gather(const BatchAdjoint& c, hipStream_t s) {
+  const dim3 grid((unsigned)(c.ntiles * kAdjTileBlocks<WW>)), block(kAdjThreads);
+  if (c.list.n_points > 0) {
+    k_batch_endpoint_sums<WW><<<grid, block, 0, s>>>(c.vols, c.tiles, c.bits, c.lpre, c.ep, c.adj,
+                                                     c.list, c.sums);
+    DAXHIP_LAUNCH_CHECK("k_batch_endpoint_sums");
+  }
+  k_batch_point_gather<WW><<<grid, block, 0, s>>>(c.vols, c.tiles, c.bits, c.lpre, c.ep, c.adj,
+                                                  c.list, c.sums, last_slot(c.list.n_points),
+                                                  c.dldf);
+  DAXHIP_LAUNCH_CHECK("k_batch_point_gather");
   return DAX_HIP_OK;
 }
 
@@ -728,7 +761,7 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
     return DAX_HIP_BAD_VALUE;
   }
   if (h->ngen >= (1 << 24)) {
-    set_error("dax_hip_mc_batch_backward: %lld tiles exceed the 2^24 the adjoint lists",
+    set_error("dax_hip_mc_batch_backward: %lld tiles, fewer than 2^24 fit a launch",
               (long long)h->ngen);
     return DAX_HIP_BAD_VALUE;
   }
@@ -759,27 +792,25 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
   const Endpoints ep{(uint64_t*)(wb + h->off_ends), (uint16_t*)(wb + h->off_end_pre),
                      (uint32_t*)(wb + h->off_end_sum), (uint32_t*)(wb + h->off_end_tile),
                      (uint32_t*)(wb + h->off_end_base)};
-  const VertexAdj* adj = (const VertexAdj*)d_scratch;
-  f32x4* sums = (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points));
-  const dim3 grid((unsigned)(h->ngen * kAdjTileBlocks)), block(kAdjThreads);
-  const EdgeList list{d_counts, n_points, (const Ctrl*)(body + h->off_ctrl)};
+  const BatchAdjoint call{vols, gen_tiles, h->ngen, bits, cs.lpre, ep,
+                          (VertexAdj*)d_scratch,
+                          EdgeList{d_counts, n_points},
+                          (f32x4*)((char*)d_scratch + endpoint_sums_offset(n_points)),
+                          d_dl_dfields};
   if (n_points > 0) {
     const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
-    k_batch_records<<<dim3((unsigned)(vertex_blocks + h->ngen)), block, 0, s>>>(
+    const int64_t word_blocks = ceil_div(h->ngen, (int64_t)(kAdjThreads / 64));
+    k_batch_records<<<dim3((unsigned)(vertex_blocks + word_blocks)), kAdjThreads, 0, s>>>(
         vols, h->nvols, (const uint32_t*)(body + h->off_vol_first), d_fields, d_edges,
-        d_dl_dvertices, d_dl_dnormals, list, (VertexAdj*)d_scratch, gen_tiles, bits, cs, ep,
-        vertex_blocks);
+        d_dl_dvertices, d_dl_dnormals, call.list, call.adj, gen_tiles, h->ngen, bits, cs,
+        (const Ctrl*)(body + h->off_ctrl), ep, vertex_blocks);
     DAXHIP_LAUNCH_CHECK("k_batch_records");
-    k_scan_endpoints<<<1, kAdjScanThreads, 0, s>>>(ep.sums, ep.tile, h->ngen, sums);
-    DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
-    k_batch_endpoint_sums<<<grid, block, 0, s>>>(vols, gen_tiles, bits, cs.lpre, ep, adj, list,
-                                                 sums);
-    DAXHIP_LAUNCH_CHECK("k_batch_endpoint_sums");
+    if (const int rc = launch_scan_endpoints(ep, h->ngen, call.sums, s)) return rc;
   }
-  k_batch_point_gather<<<grid, block, 0, s>>>(vols, gen_tiles, bits, cs.lpre, ep, adj, list, sums,
-                                              last_slot(n_points), d_dl_dfields);
-  DAXHIP_LAUNCH_CHECK("k_batch_point_gather");
-  return DAX_HIP_OK;
+  switch (adjoint_wave_words(h->nwords, h->ngen)) {
+    case 32: return launch_batch_sums_gather<32>(call, s);
+    default: return launch_batch_sums_gather<64>(call, s);
+  }
 }
 
 // Capture of any sequence of this library's launches on `stream` (e.g. a

@@ -1,6 +1,6 @@
-"""GPU adjoint over row words: sizes at the edges of words, waves (64 words)
-and tiles (256 words), from no surface to a point in two an endpoint, bit for
-bit against the oracle's FP32 restatement; an edge list cut below the
+"""GPU adjoint over row words: sizes at the edges of words, waves (8, 32 or 64
+words) and tiles (256 words), from no surface to a point in two an endpoint, bit
+for bit against the oracle's FP32 restatement; an edge list cut below the
 surface's vertices against the whole list with zero gradients from there on
 (equal values: the vertices left out add exact zeros)."""
 import numpy as np
@@ -46,6 +46,58 @@ def test_endpoints_and_gather(dims, noise):
     assert np.array_equal(got.view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
 
 
+@pytest.mark.parametrize("dims", [(2, 256, 256), (2, 257, 256), (3, 512, 512), (2, 513, 512),
+                                  (2, 2048, 2047), (2, 2049, 2048), (64, 2053, 2052)])
+def test_many_row_words(dims):
+    """Row words around 2^16, 2^18 (1024 tiles) and 2^22, where the words per
+    wave and the way to the tiles' prefixes change, and more tiles than one
+    block scans."""
+    print(f"[case] adjoint words {dims}", flush=True)
+    f = np.zeros((dims[2], dims[1], dims[0]), np.float32)
+    r = np.random.default_rng(11)
+    for k in (0, dims[2] // 2, dims[2] - 3):  # noise in three slabs
+        f[k:k + 3, :, :] = r.random((3, dims[1], dims[0]), dtype=np.float32)
+    field = torch.from_numpy(f).cuda()
+    out = mc.forward(field, 0.4, edges=True)
+    U = out.num_points
+    dx, dn = _grads(U, 7)
+    got = mc.backward(field, 0.4, out, dx.cuda(), dn.cuda()).cpu().numpy().reshape(-1)
+    r = orc.generate(f, 0.4)
+    assert r["n_pts"] == U
+    want = orc.backward_f32(f, 0.4, r["first"], r["second"], dx.numpy(), dn.numpy())
+    assert np.array_equal(got.view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 40, 1025, 3000])
+def test_batch_of_small_volumes(n):
+    """Volumes that leave their tiles mostly empty, up to more of them than
+    blocks add up the tiles before themselves; against each on its own."""
+    print(f"[case] adjoint of {n} small volumes", flush=True)
+    dims = [(5 + i % 3, 4 + i % 5, 3 + i % 4) for i in range(n)]
+    r = np.random.default_rng(n)
+    fs = [r.random((d[2], d[1], d[0]), dtype=np.float32) for d in dims]
+    flat = torch.from_numpy(np.concatenate([f.reshape(-1) for f in fs])).cuda()
+    b = mc.Batch(dims, [0.4] * n)
+    T, U = b.sizes(flat)
+    bufs = b.alloc(U, T)
+    b.forward_into(flat, bufs)
+    dx, dn = _grads(U, 3)
+    scratch = torch.empty(b.scratch_bytes(U), dtype=torch.uint8, device="cuda")
+    got = torch.empty_like(flat)
+    b.backward(flat, bufs, dx.cuda(), dn.cuda(), scratch, got)
+    got, at, u = got.cpu().numpy(), 0, 0
+    for f in fs:
+        ref = orc.generate(f, 0.4)
+        m = ref["n_pts"]
+        want = (orc.backward_f32(f, 0.4, ref["first"], ref["second"], dx[u:u + m].numpy(),
+                                 dn[u:u + m].numpy()) if m else np.zeros(f.size, np.float32))
+        assert np.array_equal(got[at:at + f.size].view(np.uint32),
+                              np.asarray(want, np.float32).view(np.uint32))
+        at += f.size
+        u += m
+    assert u == U
+
+
 @pytest.mark.parametrize("cut", [0, 1, 2, 7, 100, 1000, -1])
 def test_cut_edge_list(cut):
     dims = (70, 13, 11)
@@ -68,7 +120,7 @@ def test_cut_edge_list(cut):
 
 
 def _batch(n_volumes):
-    dims = [(70, 13, 11), (9, 8, 7), (64, 5, 6), (130, 9, 4)][:n_volumes]
+    dims = [(9, 3, 5), (70, 13, 11), (64, 5, 6), (130, 9, 4)][:n_volumes]  # odd word offsets
     fs = [_field(d, 3 + i, 1.0).reshape(-1) for i, d in enumerate(dims)]
     flat = torch.from_numpy(np.concatenate(fs)).cuda()
     b = mc.Batch(dims, [0.1] * len(dims))
