@@ -685,16 +685,19 @@ __host__ __device__ constexpr size_t adjoint_scratch_bytes(int64_t n_points) {
   return n_points > 0 ? 2 * endpoint_sums_offset(n_points) + 16 : 0;
 }
 // Words per wave of the sums and the gather of `nwords` row words in `tiles`
-// tiles.  Large volumes have mostly words without points, where a wave of few
-// words is spent on finding that out, and fewer lanes have something to do.
-// Backward in us with 32 / 64 words, Gaussian mixtures of n^3 points: 256
-// 59 / 65, 512 219 / 221; 256 volumes of 32..160 points an axis 439 / 428;
-// sums + gather of the 1024^3 Mandelbulb 1754 / 1460.  Volumes of a batch that
-// leave their tiles mostly empty take one wave each (20000 of 6 x 7 x 5 points
-// 83 / 42).
+// tiles.  Small volumes have too few waves with many words each, and a wave
+// goes through its words' points 64 at a time, one round after another; large
+// ones have mostly words without points, where a wave of few words is spent on
+// finding that out, and fewer lanes have something to do.  Backward in us with
+// 8 / 32 / 64 words, Gaussian mixtures of n^3 points: 96 22 / 30 / 41,
+// 128 26 / 39 / 53, 160 32 / 32 / 40, 256 73 / 59 / 65, 512 382 / 219 / 221;
+// 256 volumes of 32..160 points an axis 668 / 439 / 428; sums + gather of the
+// 1024^3 Mandelbulb 2972 / 1754 / 1460, of 64^3 noise 30 / 93 / 177.  Volumes
+// of a batch that leave their tiles mostly empty take one wave each (20000 of
+// 6 x 7 x 5 points 242 / 83 / 42).
 inline int adjoint_wave_words(int64_t nwords, int64_t tiles) {
   if (nwords < 64 * tiles && tiles > 1) return 64;
-  return nwords < (1 << 22) ? 32 : 64;
+  return nwords <= (1 << 16) ? 8 : (nwords < (1 << 22) ? 32 : 64);
 }
 // The last slot (a volume or batch of at most 2^31 points has fewer endpoints).
 inline uint32_t last_slot(int64_t n_points) {

@@ -167,6 +167,7 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
     if (const int rc = launch_scan_endpoints(ep, tiles, call.sums, s)) return rc;
   }
   switch (adjoint_wave_words(g.nwords, tiles)) {
+    case 8: return launch_sums_gather<8>(g, call, s);
     case 32: return launch_sums_gather<32>(g, call, s);
     default: return launch_sums_gather<64>(g, call, s);
   }

@@ -808,6 +808,7 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
     if (const int rc = launch_scan_endpoints(ep, h->ngen, call.sums, s)) return rc;
   }
   switch (adjoint_wave_words(h->nwords, h->ngen)) {
+    case 8: return launch_batch_sums_gather<8>(call, s);
     case 32: return launch_batch_sums_gather<32>(call, s);
     default: return launch_batch_sums_gather<64>(call, s);
   }
