@@ -13,7 +13,8 @@
 //   dL/dgA  = (1-t) dL/dm,                dL/dgB  = t dL/dm
 // and each dL/dg_p[d] flows to the stencil points of g_p[d].
 //
-// Deterministic (no atomics; every sum has a fixed order), in four launches:
+// Deterministic (no atomics; every sum has a fixed order), in four launches
+// (three where the endpoints add up the few tiles' counts themselves):
 //   records    one thread per vertex, recomputes t, gA, gB from the field and
 //              the compact edge list (the interpolants are not stored by the
 //              forward), writes 8 floats per vertex (sA, GA[3], sB, GB[3]);
@@ -253,9 +254,10 @@ constexpr int64_t kScanTiles = (int64_t)kAdjScanThreads * kScanChunk;
 constexpr int kScanBlocks = 16;
 static __global__ __launch_bounds__(kAdjScanThreads) void k_scan_endpoints(
     const uint32_t* __restrict__ sums, uint32_t* __restrict__ pre, int64_t n, int64_t part,
-    f32x4* __restrict__ endpoint_sums) {
+    EdgeList list, f32x4* __restrict__ endpoint_sums) {
   __shared__ uint32_t s_scan[kAdjScanThreads / 64];
   if (blockIdx.x == 0 && threadIdx.x == 0) endpoint_sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (edge_count(list) == 0) return;
   const int64_t first = (int64_t)blockIdx.x * part, end = min(first + part, n);
   uint32_t before = 0u, carry;
   for (int64_t i = 4 * (int64_t)threadIdx.x; i < first; i += 4 * kAdjScanThreads) {
@@ -276,13 +278,41 @@ static __global__ __launch_bounds__(kAdjScanThreads) void k_scan_endpoints(
     store_prefixes(pre, i0, n, x, run);
   }
 }
-inline int launch_scan_endpoints(const Endpoints& ep, int64_t tiles, f32x4* sums, hipStream_t s) {
+inline int launch_scan_endpoints(const Endpoints& ep, int64_t tiles, const EdgeList& list,
+                                 f32x4* sums, hipStream_t s) {
   const int64_t part = align_up(
       (size_t)std::max(kScanTiles, ceil_div(tiles, (int64_t)kScanBlocks)), (size_t)kScanTiles);
   k_scan_endpoints<<<dim3((unsigned)ceil_div(tiles, part)), kAdjScanThreads, 0, s>>>(
-      ep.sums, ep.tile, tiles, part, sums);
+      ep.sums, ep.tile, tiles, part, list, sums);
   DAXHIP_LAUNCH_CHECK("k_scan_endpoints");
   return DAX_HIP_OK;
+}
+
+// Up to this many tiles the sums' blocks add up the counts before their tile
+// themselves and leave them for the gather, which saves the scan's launch.
+constexpr int64_t kFoldTiles = 1024;
+
+// Endpoints before `tile`: from the scan, or (fold) the counts' sum (all threads
+// of the block, whose first one notes it for the gather).
+template <bool FOLD>
+__device__ __forceinline__ uint32_t endpoints_before(const Endpoints& ep, int64_t tile, bool note,
+                                                     const EdgeList& list) {
+  if constexpr (!FOLD) return ep.tile[tile];
+  __shared__ uint32_t s_sum[kAdjThreads / 64];
+  uint32_t v = 0u;
+#pragma unroll
+  for (int u = 0; u < (int)(kFoldTiles / kAdjThreads); ++u) {
+    const int i = u * kAdjThreads + (int)threadIdx.x;
+    v += i < tile ? ep.sums[i] : 0u;
+  }
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = 0u;
+#pragma unroll
+  for (int q = 0; q < kAdjThreads / 64; ++q) v += s_sum[q];
+  if (note && threadIdx.x == 0 && edge_count(list) != 0) ep.tile[tile] = v;
+  return v;
 }
 
 __device__ __forceinline__ uint64_t shfl64(uint64_t v, int l) {
@@ -401,6 +431,7 @@ __device__ __forceinline__ void endpoint_sums_wave(const VolGeom& g,
   if (!__ballot(n != 0u)) return;
   // read when it is needed: most waves of a large volume have left by now
   const int64_t n_adj = edge_count(list), cap = 2 * list.n_points;
+  if (n_adj == 0) return;  // the words were not formed
   const uint32_t inc = wave_incl_scan(n), total = wave_last(inc);
   const int64_t slot0 = 1 + (int64_t)before + ep.pre[g.word_off + ww];
   for (uint32_t e0 = 0; e0 < total; e0 += 64u) {  // wave-uniform
@@ -600,6 +631,7 @@ __device__ __forceinline__ void gather_wave(const VolGeom& g, const uint64_t* __
   zero_run(g, out, ww, min(ww + WW, g.nwords), lane, 64);
   if (!__ballot(r != 0ull)) return;
   const int64_t n_adj = edge_count(list);
+  if (n_adj == 0) return;  // the words were not formed
   const uint32_t n = (uint32_t)popc(r);
   const uint32_t inc = wave_incl_scan(n), total = wave_last(inc);
   if (r != 0ull) {

@@ -18,7 +18,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_adjoint_records(
   if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
     const int64_t w0 = (((int64_t)blockIdx.x - vertex_blocks) * (kAdjThreads / 64) +
                         __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kAdjTile;
-    if (w0 >= g.nwords) return;  // wave-uniform
+    if (U == 0 || w0 >= g.nwords) return;  // wave-uniform
     cs.tpb_shift = (int)ctrl->tpb_shift;
     endpoint_words_tile(g, bits, cs, ep, w0);
     return;
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_adjoint_records(
   vertex_adjoint(g, field, edges, dldx, dldn, u, out);
 }
 
-template <int WW>
+template <int WW, bool FOLD>
 __global__ __launch_bounds__(kAdjThreads) void k_endpoint_sums(
     VolGeom g, const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre,
     Endpoints ep, const VertexAdj* __restrict__ adj, EdgeList list, f32x4* __restrict__ sums) {
@@ -38,7 +38,9 @@ __global__ __launch_bounds__(kAdjThreads) void k_endpoint_sums(
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
   const int64_t ww = blk * kAdjBlockWords<WW> + wv * WW;
-  const uint32_t before = ep.tile[blk / kAdjTileBlocks<WW>];
+  if (FOLD && blockIdx.x == 0 && threadIdx.x == 0) sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const uint32_t before = endpoints_before<FOLD>(ep, blk / kAdjTileBlocks<WW>,
+                                                 blk % kAdjTileBlocks<WW> == 0, list);
   if (ww < g.nwords)  // wave-uniform
     endpoint_sums_wave<WW>(g, bits, lpre, ep, adj, list, sums, ww, before, s_mark[wv]);
 }
@@ -75,10 +77,15 @@ struct AdjointCall {
 };
 
 template <int WW>
-int launch_sums_gather(const VolGeom& g, const AdjointCall& c, hipStream_t s) {
+int launch_sums_gather(const VolGeom& g, const AdjointCall& c, int64_t tiles, hipStream_t s) {
   const dim3 grid((unsigned)ceil_div(g.nwords, (int64_t)kAdjBlockWords<WW>)), block(kAdjThreads);
   if (c.list.n_points > 0) {
-    k_endpoint_sums<WW><<<grid, block, 0, s>>>(g, c.bits, c.cs.lpre, c.ep, c.adj, c.list, c.sums);
+    if (tiles > kFoldTiles)
+      k_endpoint_sums<WW, false><<<grid, block, 0, s>>>(g, c.bits, c.cs.lpre, c.ep, c.adj, c.list,
+                                                        c.sums);
+    else
+      k_endpoint_sums<WW, true><<<grid, block, 0, s>>>(g, c.bits, c.cs.lpre, c.ep, c.adj, c.list,
+                                                       c.sums);
     DAXHIP_LAUNCH_CHECK("k_endpoint_sums");
   }
   k_point_gather<WW><<<grid, block, 0, s>>>(g, c.bits, c.cs.lpre, c.ep, c.adj, c.list, c.sums,
@@ -164,12 +171,13 @@ int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz
         g, d_field, d_edges, d_dl_dvertices, d_dl_dnormals, call.list, call.adj, bits, cs,
         (const Ctrl*)(ws + L.off_ctrl), ep, vertex_blocks);
     DAXHIP_LAUNCH_CHECK("k_adjoint_records");
-    if (const int rc = launch_scan_endpoints(ep, tiles, call.sums, s)) return rc;
+    if (tiles > kFoldTiles)
+      if (const int rc = launch_scan_endpoints(ep, tiles, call.list, call.sums, s)) return rc;
   }
   switch (adjoint_wave_words(g.nwords, tiles)) {
-    case 8: return launch_sums_gather<8>(g, call, s);
-    case 32: return launch_sums_gather<32>(g, call, s);
-    default: return launch_sums_gather<64>(g, call, s);
+    case 8: return launch_sums_gather<8>(g, call, tiles, s);
+    case 32: return launch_sums_gather<32>(g, call, tiles, s);
+    default: return launch_sums_gather<64>(g, call, tiles, s);
   }
 }
 

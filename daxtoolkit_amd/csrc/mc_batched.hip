@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void k_batch_records(
   if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
     const int64_t t = ((int64_t)blockIdx.x - vertex_blocks) * (kAdjThreads / 64) +
                       __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (t >= ntiles) return;  // wave-uniform
+    if (U == 0 || t >= ntiles) return;  // wave-uniform
     const TileRef tr = tiles[t];
     const VolGeom g = vols[tr.vol];
     CountSrc cs = volume_counts(all, g);
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(256) void k_batch_records(
 
 static_assert(kAdjTile == kBatchGenTile, "the adjoint's tiles are the generate tiles");
 
-template <int WW>
+template <int WW, bool FOLD>
 __global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_sums(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles,
     const uint64_t* __restrict__ bits, const uint32_t* __restrict__ lpre, Endpoints ep,
@@ -299,7 +299,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_sums(
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t blk = xcd_tile_runs(blockIdx.x, gridDim.x);
   const int64_t t = blk / kAdjTileBlocks<WW>, part = blk % kAdjTileBlocks<WW>;
-  const uint32_t before = ep.tile[t];
+  if (FOLD && blockIdx.x == 0 && threadIdx.x == 0) sums[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const uint32_t before = endpoints_before<FOLD>(ep, t, part == 0, list);
   const TileRef tr = tiles[t];
   const VolGeom g = vols[tr.vol];
   const int64_t ww = (int64_t)tr.w0 + part * kAdjBlockWords<WW> + wv * WW;
@@ -463,8 +464,12 @@ template <int WW>
 int launch_batch_sums_gather(const BatchAdjoint& c, hipStream_t s) {
   const dim3 grid((unsigned)(c.ntiles * kAdjTileBlocks<WW>)), block(kAdjThreads);
   if (c.list.n_points > 0) {
-    k_batch_endpoint_sums<WW><<<grid, block, 0, s>>>(c.vols, c.tiles, c.bits, c.lpre, c.ep, c.adj,
-                                                     c.list, c.sums);
+    if (c.ntiles > kFoldTiles)
+      k_batch_endpoint_sums<WW, false><<<grid, block, 0, s>>>(c.vols, c.tiles, c.bits, c.lpre, c.ep,
+                                                              c.adj, c.list, c.sums);
+    else
+      k_batch_endpoint_sums<WW, true><<<grid, block, 0, s>>>(c.vols, c.tiles, c.bits, c.lpre, c.ep,
+                                                             c.adj, c.list, c.sums);
     DAXHIP_LAUNCH_CHECK("k_batch_endpoint_sums");
   }
   k_batch_point_gather<WW><<<grid, block, 0, s>>>(c.vols, c.tiles, c.bits, c.lpre, c.ep, c.adj,
@@ -805,7 +810,8 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
         d_dl_dvertices, d_dl_dnormals, call.list, call.adj, gen_tiles, h->ngen, bits, cs,
         (const Ctrl*)(body + h->off_ctrl), ep, vertex_blocks);
     DAXHIP_LAUNCH_CHECK("k_batch_records");
-    if (const int rc = launch_scan_endpoints(ep, h->ngen, call.sums, s)) return rc;
+    if (h->ngen > kFoldTiles)
+      if (const int rc = launch_scan_endpoints(ep, h->ngen, call.list, call.sums, s)) return rc;
   }
   switch (adjoint_wave_words(h->nwords, h->ngen)) {
     case 8: return launch_batch_sums_gather<8>(call, s);
