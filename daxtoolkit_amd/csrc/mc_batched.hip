@@ -241,12 +241,38 @@ __global__ __launch_bounds__(kBatchGenThreads, 4) void k_batch_generate(
 
 // ---- batched adjoint --------------------------------------------------------
 // The launches of the single volume's adjoint over generate's tile table.
+__device__ __forceinline__ void batch_endpoint_words(
+    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
+    const uint64_t* __restrict__ bits, const CountSrc& all, const Ctrl* __restrict__ ctrl,
+    const Endpoints& ep, const EdgeList& list, int64_t blk) {  // a wave per tile
+  const int64_t t =
+      blk * (kAdjThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (edge_count(list) == 0 || t >= ntiles) return;  // wave-uniform
+  const TileRef tr = tiles[t];
+  const VolGeom g = vols[tr.vol];
+  CountSrc cs = volume_counts(all, g);
+  cs.tpb_shift = (int)ctrl->tpb_shift;
+  endpoint_words_tile(g, bits + g.word_off, cs, ep, tr.w0);
+}
+
+__global__ __launch_bounds__(kAdjThreads) void k_batch_endpoint_words(
+    const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
+    const uint64_t* __restrict__ bits, CountSrc all, const Ctrl* __restrict__ ctrl, Endpoints ep,
+    EdgeList list) {
+  batch_endpoint_words(vols, tiles, ntiles, bits, all, ctrl, ep, list, blockIdx.x);
+}
+
 // A thread per vertex; its volume by binary search over the volumes' first
 // vertices, then the wave takes its volumes one at a time (one, as a rule),
 // so that the geometry stays in scalar registers.  A block per tile of words
 // instead leaves most lanes idle (73 vertices per tile in 256 volumes of
 // 32..160 points an axis: 80 us; this: 58).  Blocks from vertex_blocks on form
-// the endpoint words, a wave per tile.
+// the endpoint words (WORDS).  Their registers leave the records six waves of
+// eight, which costs many vertices more than a launch beside them saves: 1024
+// volumes with 20 a word 8100 us against 59 + 7156, 256 volumes with one in
+// three words 82 against 27 + 63.
+constexpr int64_t kDenseWords = 4;  // vertices per row word from which they go apart
+template <bool WORDS>
 __global__ __launch_bounds__(256) void k_batch_records(
     const VolGeom* __restrict__ vols, int64_t nvols, const uint32_t* __restrict__ vol_first,
     const float* __restrict__ fields, const uint32_t* __restrict__ edges,
@@ -254,18 +280,10 @@ __global__ __launch_bounds__(256) void k_batch_records(
     EdgeList list, VertexAdj* __restrict__ out, const TileRef* __restrict__ tiles,
     int64_t ntiles, const uint64_t* __restrict__ bits, CountSrc all,
     const Ctrl* __restrict__ ctrl, Endpoints ep, int64_t vertex_blocks) {
+  if (WORDS && (int64_t)blockIdx.x >= vertex_blocks)  // uniform
+    return batch_endpoint_words(vols, tiles, ntiles, bits, all, ctrl, ep, list,
+                                (int64_t)blockIdx.x - vertex_blocks);
   const int64_t U = edge_count(list);
-  if ((int64_t)blockIdx.x >= vertex_blocks) {  // uniform
-    const int64_t t = ((int64_t)blockIdx.x - vertex_blocks) * (kAdjThreads / 64) +
-                      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (U == 0 || t >= ntiles) return;  // wave-uniform
-    const TileRef tr = tiles[t];
-    const VolGeom g = vols[tr.vol];
-    CountSrc cs = volume_counts(all, g);
-    cs.tpb_shift = (int)ctrl->tpb_shift;
-    endpoint_words_tile(g, bits + g.word_off, cs, ep, tr.w0);
-    return;
-  }
   const int64_t u = xcd_tile(blockIdx.x, vertex_blocks) * blockDim.x + threadIdx.x;
   int64_t vol = -1;
   if (u < U) {  // the last volume whose first vertex is at most u
@@ -805,10 +823,20 @@ int dax_hip_mc_batch_backward(const float* d_fields, const void* h_header,
   if (n_points > 0) {
     const int64_t vertex_blocks = ceil_div(n_points, (int64_t)kAdjThreads);
     const int64_t word_blocks = ceil_div(h->ngen, (int64_t)(kAdjThreads / 64));
-    k_batch_records<<<dim3((unsigned)(vertex_blocks + word_blocks)), kAdjThreads, 0, s>>>(
-        vols, h->nvols, (const uint32_t*)(body + h->off_vol_first), d_fields, d_edges,
-        d_dl_dvertices, d_dl_dnormals, call.list, call.adj, gen_tiles, h->ngen, bits, cs,
-        (const Ctrl*)(body + h->off_ctrl), ep, vertex_blocks);
+    const uint32_t* vol_first = (const uint32_t*)(body + h->off_vol_first);
+    const Ctrl* ctrl = (const Ctrl*)(body + h->off_ctrl);
+    if (n_points > kDenseWords * h->nwords) {
+      k_batch_endpoint_words<<<dim3((unsigned)word_blocks), kAdjThreads, 0, s>>>(
+          vols, gen_tiles, h->ngen, bits, cs, ctrl, ep, call.list);
+      DAXHIP_LAUNCH_CHECK("k_batch_endpoint_words");
+      k_batch_records<false><<<dim3((unsigned)vertex_blocks), kAdjThreads, 0, s>>>(
+          vols, h->nvols, vol_first, d_fields, d_edges, d_dl_dvertices, d_dl_dnormals, call.list,
+          call.adj, gen_tiles, h->ngen, bits, cs, ctrl, ep, vertex_blocks);
+    } else {
+      k_batch_records<true><<<dim3((unsigned)(vertex_blocks + word_blocks)), kAdjThreads, 0, s>>>(
+          vols, h->nvols, vol_first, d_fields, d_edges, d_dl_dvertices, d_dl_dnormals, call.list,
+          call.adj, gen_tiles, h->ngen, bits, cs, ctrl, ep, vertex_blocks);
+    }
     DAXHIP_LAUNCH_CHECK("k_batch_records");
     if (h->ngen > kFoldTiles)
       if (const int rc = launch_scan_endpoints(ep, h->ngen, call.list, call.sums, s)) return rc;
