@@ -459,6 +459,14 @@ __device__ __forceinline__ void store_block3(float* __restrict__ out, int64_t fi
   }
 }
 
+// A plane of the gradient kernels fills its blocks of 256 to three quarters or
+// more: blocks march over planes.  Below that a thread takes one point (cell)
+// of the flat index, so that small planes leave no lanes idle and no grid more
+// blocks than a launch takes (point gradient, flat / marching: 8 x 8 x 500000
+// 131 / 282 us, 4 x 4 x 1000000 44 / 417, 300 x 1 x 100000 123 / 166, 17 x 13 x
+// 50000 39 / 35, 16 x 16 x 100000 104 / 99).
+inline bool march_planes(int64_t plane) { return 4 * plane >= 3 * 256 * ceil_div(plane, 256); }
+
 // Planes a block of the gradient kernels marches through: neighbours in z stay
 // in registers and indexes are formed once, up to 8 where that leaves enough
 // blocks.
@@ -496,10 +504,52 @@ __global__ __launch_bounds__(256) void k_point_gradient(VolGeom g, int planes, F
   }
 }
 
-// CellGradient (dax/worklet/CellGradient.h:28-48): weights of
-// DerivativeWeights(Voxel) at the centre are +-0.25 in the corner order of
+// The same for planes that would leave a marching block idle, a thread per point
+// of the flat index (its stores through LDS took as long).
+__global__ __launch_bounds__(256) void k_point_gradient_flat(VolGeom g, int64_t n,
+                                                             const float* __restrict__ f,
+                                                             float* __restrict__ grad) {
+  const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (at >= n) return;
+  const uint32_t p = (uint32_t)at;
+  const uint32_t row = fast_div(p, g.div_nx), z = fast_div(row, g.div_ny);
+  float gr[3];
+  point_gradient(g, FieldArray{f}, (int)(p - row * (uint32_t)g.nx),
+                 (int)(row - z * (uint32_t)g.ny), (int)z, gr);
+  store3(grad + 3 * at, gr[0], gr[1], gr[2]);
+}
+
+// Gradient of the cell (i, j, z) from a quarter of its corners' values, lower
+// and upper plane (the weights are +-0.25; the product with either sign rounds
+// alike): CellGradient (dax/worklet/CellGradient.h:28-48), weights of
+// DerivativeWeights(Voxel) at the centre in the corner order of
 // TopologyUniform.h:139-159; sum in vertex order, divided by the voxel width
 // coords[6]-coords[0] (Derivative.h:37-75).
+__device__ __forceinline__ float cell_width(const VolGeom& g, int d, int n) {
+  const float a = g.origin[d] + g.spacing[d] * (float)n;
+  const float b = g.origin[d] + g.spacing[d] * (float)(n + 1);
+  return b - a;
+}
+__device__ __forceinline__ void cell_gradient(const float lo[4], const float hi[4],
+                                              const float width[3], float gr[3]) {
+  float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int v = 0; v < 8; ++v) {
+    const float t = v < 4 ? lo[v & 3] : hi[v & 3];
+    const bool px = (v & 3) == 1 || (v & 3) == 2, py = (v & 2) != 0, pz = v >= 4;
+    s[0] = px ? s[0] + t : s[0] - t;
+    s[1] = py ? s[1] + t : s[1] - t;
+    s[2] = pz ? s[2] + t : s[2] - t;
+  }
+  // s / w; a power of two divides exactly by its reciprocal
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const uint32_t u = __float_as_uint(width[d]);
+    const bool pow2 = (u & 0x7fffffu) == 0u && (u >> 23) - 1u < 253u;
+    gr[d] = !__ballot(!pow2) ? s[d] * __uint_as_float(0x7f000000u - u) : s[d] / width[d];
+  }
+}
+
 // Blocks as k_point_gradient's; 253x241x230: 64, 47, 41 us, 512^3: 829, 523,
 // 493 (a thread per cell with 64-bit divisions and stores at a stride of 12
 // bytes, among other work: 85 us where this takes 57..66).
@@ -515,40 +565,38 @@ __global__ __launch_bounds__(256) void k_cell_gradient(VolGeom g, int planes, Fa
   const int z0 = (int)zc * planes, z1 = min(z0 + planes, cz);
   const uint32_t c = (uint32_t)min(first + (int32_t)threadIdx.x, cells - 1);
   const int j = (int)fast_div(c, div_cx), i = (int)(c - (uint32_t)j * (uint32_t)cx);
-  auto width = [&](int d, int n) -> float {
-    const float a = g.origin[d] + g.spacing[d] * (float)n;
-    const float b = g.origin[d] + g.spacing[d] * (float)(n + 1);
-    return b - a;
-  };
-  // s / w; a power of two divides exactly by its reciprocal
-  auto quotient = [](float v, float w) -> float {
-    const uint32_t u = __float_as_uint(w);
-    const bool pow2 = (u & 0x7fffffu) == 0u && (u >> 23) - 1u < 253u;
-    if (!__ballot(!pow2)) return v * __uint_as_float(0x7f000000u - u);
-    return v / w;
-  };
-  const float wx = width(0, i), wy = width(1, j);
+  float width[3] = {cell_width(g, 0, i), cell_width(g, 1, j), 0.0f};
   const float* q = f + (int64_t)z0 * plane + i + (int64_t)j * g.nx;
-  // the weights are +-0.25: a quarter of the value (the product with either
-  // sign rounds alike) with the sign of the corner
   float lo[4] = {0.25f * q[0], 0.25f * q[1], 0.25f * q[g.nx + 1], 0.25f * q[g.nx]};
   for (int z = z0; z < z1; ++z) {
     q += plane;
     const float hi[4] = {0.25f * q[0], 0.25f * q[1], 0.25f * q[g.nx + 1], 0.25f * q[g.nx]};
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const float t = v < 4 ? lo[v & 3] : hi[v & 3];
-      const bool px = (v & 3) == 1 || (v & 3) == 2, py = (v & 2) != 0, pz = v >= 4;
-      s0 = px ? s0 + t : s0 - t;
-      s1 = py ? s1 + t : s1 - t;
-      s2 = pz ? s2 + t : s2 - t;
-    }
-    const float gr[3] = {quotient(s0, wx), quotient(s1, wy), quotient(s2, width(2, z))};
+    width[2] = cell_width(g, 2, z);
+    float gr[3];
+    cell_gradient(lo, hi, width, gr);
     store_block3(out + 3 * (int64_t)z * cells, first, cells, gr, s[(z - z0) & 1]);
 #pragma unroll
     for (int v = 0; v < 4; ++v) lo[v] = hi[v];
   }
+}
+
+__global__ __launch_bounds__(256) void k_cell_gradient_flat(VolGeom g, int64_t n, FastDiv div_cx,
+                                                            FastDiv div_cy,
+                                                            const float* __restrict__ f,
+                                                            float* __restrict__ out) {
+  const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (at >= n) return;
+  const uint32_t c = (uint32_t)at;
+  const uint32_t row = fast_div(c, div_cx), z = fast_div(row, div_cy);
+  const int i = (int)(c - row * (uint32_t)(g.nx - 1)), j = (int)(row - z * (uint32_t)(g.ny - 1));
+  const float* q = f + i + (int64_t)g.nx * (j + (int64_t)g.ny * z);
+  const float* u = q + (int64_t)g.nx * g.ny;
+  const float lo[4] = {0.25f * q[0], 0.25f * q[1], 0.25f * q[g.nx + 1], 0.25f * q[g.nx]};
+  const float hi[4] = {0.25f * u[0], 0.25f * u[1], 0.25f * u[g.nx + 1], 0.25f * u[g.nx]};
+  const float width[3] = {cell_width(g, 0, i), cell_width(g, 1, j), cell_width(g, 2, (int)z)};
+  float gr[3];
+  cell_gradient(lo, hi, width, gr);
+  store3(out + 3 * at, gr[0], gr[1], gr[2]);
 }
 
 }  // namespace mc
@@ -1178,6 +1226,13 @@ int dax_hip_point_gradient(const float* d_field, int64_t nx, int64_t ny, int64_t
   VolGeom g;
   int rc = make_geom(nx, ny, nz, nullptr, h_spacing3, 0.0f, g);
   if (rc) return rc;
+  if (!march_planes(nx * ny)) {
+    const int64_t n = nx * ny * nz;
+    k_point_gradient_flat<<<dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, (hipStream_t)stream>>>(
+        g, n, d_field, d_grad);
+    DAXHIP_LAUNCH_CHECK("k_point_gradient_flat");
+    return DAX_HIP_OK;
+  }
   const int64_t pb = ceil_div(nx * ny, (int64_t)256);
   const int planes = gradient_planes(pb, nz);
   k_point_gradient<<<dim3((unsigned)(pb * ceil_div(nz, (int64_t)planes))), dim3(256), 0,
@@ -1194,11 +1249,19 @@ int dax_hip_cell_gradient(const float* d_field, int64_t nx, int64_t ny, int64_t 
   int rc = make_geom(nx, ny, nz, h_origin3, h_spacing3, 0.0f, g);
   if (rc) return rc;
   if (nx < 2 || ny < 2 || nz < 2) return DAX_HIP_OK;
+  const FastDiv div_cx = make_fast_div((uint32_t)nx - 1u);
+  if (!march_planes((nx - 1) * (ny - 1))) {
+    const int64_t n = (nx - 1) * (ny - 1) * (nz - 1);
+    k_cell_gradient_flat<<<dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, (hipStream_t)stream>>>(
+        g, n, div_cx, make_fast_div((uint32_t)ny - 1u), d_field, d_grad);
+    DAXHIP_LAUNCH_CHECK("k_cell_gradient_flat");
+    return DAX_HIP_OK;
+  }
   const int64_t pb = ceil_div((nx - 1) * (ny - 1), (int64_t)256);
   const int planes = gradient_planes(pb, nz - 1);
   k_cell_gradient<<<dim3((unsigned)(pb * ceil_div(nz - 1, (int64_t)planes))), dim3(256), 0,
-                    (hipStream_t)stream>>>(g, planes, make_fast_div((uint32_t)pb),
-                                           make_fast_div((uint32_t)nx - 1u), d_field, d_grad);
+                    (hipStream_t)stream>>>(g, planes, make_fast_div((uint32_t)pb), div_cx, d_field,
+                                           d_grad);
   DAXHIP_LAUNCH_CHECK("k_cell_gradient");
   return DAX_HIP_OK;
 }

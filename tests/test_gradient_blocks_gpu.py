@@ -1,7 +1,9 @@
 """Point and cell gradients at the edges of their blocks of 256 (below, at and
-above one and several), with outputs on and off 16-byte boundaries, and the
-cells' cases, counts and offsets (words with and without mixed cells), bit
-for bit against the oracle."""
+above one and several; planes that fill their blocks and planes that do not),
+with outputs on and off 16-byte boundaries, and the cells' cases, counts and
+offsets (words with and without mixed cells), bit for bit against the oracle.
+Grids of many small planes in the time of a cube of as many points, and with
+more planes than a launch has room for at a block each."""
 import ctypes
 
 import numpy as np
@@ -16,7 +18,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (255, 1, 1), (257, 2, 2), (16, 16, 1),
-                                  (17, 17, 17), (65, 5, 33), (64, 64, 9), (129, 3, 7)])
+                                  (17, 17, 17), (65, 5, 33), (64, 64, 9), (129, 3, 7), (1, 1, 700),
+                                  (1, 5, 300), (7, 1, 90), (3, 4, 200), (13, 14, 30), (12, 16, 40),
+                                  (14, 14, 21), (20, 15, 9), (33, 17, 5)])
 def test_gradients(dims, offset):
     print(f"[case] gradients {dims} offset {offset}", flush=True)
     nx, ny, nz = dims
@@ -42,6 +46,54 @@ def test_gradients(dims, offset):
         assert np.array_equal(got[offset:offset + 3 * n].view(np.uint32),
                               np.asarray(ref, np.float32).reshape(-1).view(np.uint32))
         assert np.all(got[:offset] == 7.0) and np.all(got[offset + 3 * n:] == 7.0)
+
+
+def _best_of(fn, n=5):
+    start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    fn()
+    best = float("inf")
+    for _ in range(n):
+        start.record()
+        fn()
+        stop.record()
+        stop.synchronize()
+        best = min(best, start.elapsed_time(stop))
+    return best
+
+
+@pytest.mark.parametrize("gradient", [mc.point_gradient, mc.cell_gradient])
+@pytest.mark.parametrize("dims", [(2, 2, 4_000_000), (4, 4, 1_000_000), (8, 8, 250_000)])
+def test_small_planes_take_no_longer(dims, gradient):
+    """Lanes left idle by planes of a few points took 10 to 100 times as long."""
+    print(f"[case] gradients of small planes {dims}", flush=True)
+    nx, ny, nz = dims
+    cube = torch.rand((252, 252, 252), device="cuda")
+    thin = torch.rand((nz, ny, nx), device="cuda")
+    assert thin.numel() <= cube.numel()
+    assert _best_of(lambda: gradient(thin)) < 3.0 * _best_of(lambda: gradient(cube))
+
+
+def test_more_planes_than_blocks_of_a_launch():
+    n = (1 << 27) + 9  # eight planes a block of 256 threads would pass 2^32 threads
+    print(f"[case] gradients of {n} planes", flush=True)
+    f = (torch.arange(n, device="cuda", dtype=torch.int32) % 8191).float().view(n, 1, 1)
+    g = mc.point_gradient(f)
+    v = f.view(-1)
+    assert torch.equal(g[1:-1, 2], (v[2:] - v[:-2]) * 0.5)
+    assert float(g[0, 2]) == float(v[1] - v[0]) and float(g[-1, 2]) == float(v[-1] - v[-2])
+    assert not bool(g[:, :2].any())
+    del g, v, f
+    m = (1 << 27) + 5
+    f = (torch.arange(4 * m, device="cuda", dtype=torch.int32) % 8191).float().view(m, 2, 2)
+    g = mc.cell_gradient(f)
+    assert g.shape == (m - 1, 3)
+    # exact in float32: sums of four whole numbers below 2^13, times a quarter; the
+    # voxel's width is the difference of its float32 coordinates (0 or 2 from 2^24 on)
+    q = f.view(m, 4)
+    z = torch.arange(m, device="cuda", dtype=torch.int32).float()
+    want = (q[1:].sum(1) - q[:-1].sum(1)) * 0.25 / (z[1:] - z[:-1])
+    assert torch.equal(g[:, 2].nan_to_num(nan=-7.0, posinf=7e9, neginf=-7e9),
+                       want.nan_to_num(nan=-7.0, posinf=7e9, neginf=-7e9))
 
 
 @pytest.mark.parametrize("dims", [(2, 2, 2), (66, 9, 7), (200, 12, 5)])
