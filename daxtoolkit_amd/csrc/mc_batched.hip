@@ -38,6 +38,10 @@ constexpr int kBatchGenTile = 256;
 // threads, 1250 with 1024).
 constexpr int kBatchGenThreads = 256;
 
+// Tiles of one launch: a launch takes fewer than 2^32 threads, and the tiles of
+// more volumes than that go over several.
+constexpr int64_t kLaunchTiles = 1 << 23;
+
 // Launch shapes of the batch forward, picked by dax_hip_mc_batch_autotune
 // and cached per batch shape class: classify unroll (row words per wave
 // step, a float4 load in flight per thread for two of them) and persistent blocks per CU, threads per count block (a wave per
@@ -145,11 +149,11 @@ template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void k_batch_count(
     const VolGeom* __restrict__ vols, const TileRef* __restrict__ tiles, int64_t ntiles,
     const uint64_t* __restrict__ bits, uint32_t* __restrict__ lpre,
-    unsigned long long* __restrict__ tloc, unsigned long long* __restrict__ bsum) {
+    unsigned long long* __restrict__ tloc, unsigned long long* __restrict__ bsum, int64_t blk0) {
   constexpr int kBlockTiles = 2 * WAVES;
   __shared__ unsigned long long s_ts[kBlockTiles];
   const int wv = threadIdx.x >> 6;
-  const int64_t blk = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t blk = blk0 + xcd_tile(blockIdx.x, gridDim.x);
   const int64_t t = blk * WAVES + wv;
   unsigned long long s0 = 0ull, s1 = 0ull;
   if (t < ntiles) {
@@ -423,22 +427,25 @@ int batch_count_shift(const BatchTuning& t) {
 
 int batch_scan(const BatchHeader& h, const BatchPtrs& p, const BatchTuning& t, hipStream_t s) {
   const int waves = t.scan_threads / 64;
-  const int64_t blocks = ceil_div(h.ngen, (int64_t)waves);
-  const dim3 grid((unsigned)blocks), blk((unsigned)t.scan_threads);
-  switch (waves) {
-    case 8:
-      k_batch_count<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
-                                            p.bsum);
-      break;
-    case 16:
-      k_batch_count<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
-                                             p.bsum);
-      break;
-    default:
-      k_batch_count<4><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
-                                            p.bsum);
+  const int64_t blocks = ceil_div(h.ngen, (int64_t)waves), most = kLaunchTiles / waves;
+  const dim3 blk((unsigned)t.scan_threads);
+  for (int64_t b0 = 0; b0 < blocks; b0 += most) {
+    const dim3 grid((unsigned)std::min(most, blocks - b0));
+    switch (waves) {
+      case 8:
+        k_batch_count<8><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
+                                              p.bsum, b0);
+        break;
+      case 16:
+        k_batch_count<16><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
+                                               p.bsum, b0);
+        break;
+      default:
+        k_batch_count<4><<<grid, blk, 0, s>>>(p.vols, p.gen_tiles, h.ngen, p.bits, p.lpre, p.tloc,
+                                              p.bsum, b0);
+    }
+    DAXHIP_LAUNCH_CHECK("k_batch_count");
   }
-  DAXHIP_LAUNCH_CHECK("k_batch_count");
   k_batch_scan<<<1, dim3(kTsumThreads), 0, s>>>(p.bsum, p.bpre, blocks, p.tloc, 2 * h.ngen, p.ctrl,
                                                 batch_count_shift(t));
   DAXHIP_LAUNCH_CHECK("k_batch_scan");
@@ -451,16 +458,19 @@ int batch_generate(const BatchHeader& h, const BatchPtrs& p, const float* d_fiel
                    hipStream_t s) {
   const CountSrc cs{p.lpre, p.tloc, p.bpre, 0, 0, batch_count_shift(t)};
   const size_t lds = GenLayout<kBatchGenTile, kBatchGenThreads>((int)h.max_wpr).bytes();
-  const dim3 grid((unsigned)h.ngen);
-  if (flags & DAX_HIP_MC_DEDUP)
-    k_batch_generate<true><<<grid, dim3(kBatchGenThreads), lds, s>>>(
-        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points, cap_tris,
-        d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
-  else
-    k_batch_generate<false><<<grid, dim3(kBatchGenThreads), lds, s>>>(
-        p.vols, p.gen_tiles, h.ngen, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points, cap_tris,
-        d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
-  DAXHIP_LAUNCH_CHECK("k_batch_generate");
+  for (int64_t t0 = 0; t0 < h.ngen; t0 += kLaunchTiles) {
+    const int64_t n = std::min(kLaunchTiles, h.ngen - t0);
+    const dim3 grid((unsigned)n);
+    if (flags & DAX_HIP_MC_DEDUP)
+      k_batch_generate<true><<<grid, dim3(kBatchGenThreads), lds, s>>>(
+          p.vols, p.gen_tiles + t0, n, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points,
+          cap_tris, d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
+    else
+      k_batch_generate<false><<<grid, dim3(kBatchGenThreads), lds, s>>>(
+          p.vols, p.gen_tiles + t0, n, d_fields, p.bits, cs, p.ctrl, o, flags, cap_points,
+          cap_tris, d_counts, d_vol_offsets, p.vol_first, t.gen_xcd);
+    DAXHIP_LAUNCH_CHECK("k_batch_generate");
+  }
   return DAX_HIP_OK;
 }
 
