@@ -299,18 +299,15 @@ struct Tuning {
   int scan_sub = 8;     // count tiles (waves) per count block
   int gen_tile = 512;   // generate tile words
   int gen_xcd = 0;      // 1: each XCD takes a contiguous range of generate tiles
-  bool operator==(const Tuning& o) const {
-    return cls_unroll == o.cls_unroll && cls_vec == o.cls_vec && scan_sub == o.scan_sub &&
-           gen_tile == o.gen_tile && gen_xcd == o.gen_xcd;
-  }
 };
 
 std::mutex g_tune_mu;
 Tuning g_tune_default;
+bool g_tune_default_set = false;  // by a caller: it then holds for every size
 std::map<std::tuple<int64_t, int64_t, int64_t>, Tuning> g_tune_cache;
 
-// The launch shape of a volume without a choice of its own, while the default
-// is the built-in one.  Generate tiles: 64 words (spread over the waves
+// The launch shape of a volume without a choice of its own, while no caller has
+// set the default.  Generate tiles: 64 words (spread over the waves
 // launch_generate_src gives them) up to 2^20 words, 256 beyond, where the
 // dispatch order of tiles of at least a count tile pays (forward, 64 / 256
 // words: 256^3 points 59 / 65 us, 384^3 105 / 109, 512^3 194 / 176; dense
@@ -331,7 +328,7 @@ Tuning tuning_for(int64_t nx, int64_t ny, int64_t nz) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune_cache.find(std::make_tuple(nx, ny, nz));
   if (it != g_tune_cache.end()) return it->second;
-  return g_tune_default == Tuning{} ? shape_tuning(nx, ny, nz) : g_tune_default;
+  return g_tune_default_set ? g_tune_default : shape_tuning(nx, ny, nz);
 }
 
 bool valid_tuning(const Tuning& t) {
@@ -1311,10 +1308,12 @@ int dax_hip_mc_set_tuning(int64_t nx, int64_t ny, int64_t nz, const int* h_param
     return DAX_HIP_BAD_VALUE;
   }
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  if (nx == 0 && ny == 0 && nz == 0)
+  if (nx == 0 && ny == 0 && nz == 0) {
     g_tune_default = t;
-  else
+    g_tune_default_set = true;
+  } else {
     g_tune_cache[std::make_tuple(nx, ny, nz)] = t;
+  }
   return DAX_HIP_OK;
 }
 

@@ -520,7 +520,8 @@ int dax_hip_mc_cell_outputs(int64_t nx, int64_t ny, int64_t nz, const void* d_wo
  *   kernel, two count tiles of 128 row words per wave); gen_tile
  *   64/128/256/512/1024 (row words per generate block); gen_xcd 1 gives each
  *   XCD a contiguous range of generate tiles, 0 keeps the plain block order.
- * A shape of (0,0,0) sets or gets the default for shapes not tuned. */
+ * A shape of (0,0,0) sets or gets the default for shapes not tuned; until it
+ * is set, theirs follow from their size, and (0,0,0) gets {4, 4, 8, 512, 0}. */
 int dax_hip_mc_set_tuning(int64_t nx, int64_t ny, int64_t nz, const int* h_params5);
 int dax_hip_mc_get_tuning(int64_t nx, int64_t ny, int64_t nz, int* h_params5);
 /* Times the classify variants with HIP events (reps launches each), then

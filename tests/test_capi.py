@@ -52,3 +52,25 @@ def test_span_threshold_setter_is_host_only():
     assert b"negative" in lib.dax_hip_last_error()
     assert lib.dax_hip_mc_backward_set_span_threshold(0) == 0
     assert lib.dax_hip_mc_backward_set_span_threshold(16) == 0
+
+
+def test_default_tuning_as_set():
+    """Sizes without a tuning of their own take the default that a caller sets,
+    whatever it is; before that they follow from the size (a process of its
+    own: the default holds for the process)."""
+    import subprocess
+    import sys
+    code = """
+from daxtoolkit_amd import mc
+shapes = [(300, 300, 300), (20, 20, 20), (700, 700, 700)]
+built_in = mc.get_tuning((0, 0, 0))
+by_size = [mc.get_tuning(s) for s in shapes]
+assert any(t != built_in for t in by_size)
+mc.set_tuning((20, 20, 20), [8, 1, 2, 128, 1])
+for default in (built_in, [2, 4, 1, 256, 0], built_in):
+    mc.set_tuning((0, 0, 0), default)
+    assert mc.get_tuning((0, 0, 0)) == default
+    assert mc.get_tuning(shapes[0]) == mc.get_tuning(shapes[2]) == default
+    assert mc.get_tuning(shapes[1]) == [8, 1, 2, 128, 1]
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT, timeout=300)
