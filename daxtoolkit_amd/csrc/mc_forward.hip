@@ -235,7 +235,7 @@ __global__ __launch_bounds__(NT, 4) void k_generate(
   // the scan's dispatch order when it was built for this tile size (whole
   // volume launches only), else index order
   uint32_t tag = 0u, ord = 0u;
-  if (order != nullptr) {
+  if (TW >= kCountTile && order != nullptr) {
     tag = order[0];
     ord = order[1 + blockIdx.x];
   }
@@ -791,8 +791,9 @@ int launch_generate_tw(const VolGeom& g, const Src& field, const char* ws, const
   if (t_hi < 0) t_hi = all;
   const int64_t ntiles = std::max<int64_t>(t_hi - t_lo, 1);
   const CountSrc cs = count_src(ws, L);
-  const uint32_t* order =
-      (t_lo == 0 && t_hi == all) ? (const uint32_t*)(ws + L.off_order) : nullptr;
+  // the order lists tiles of at least a count tile: it has no entries for more
+  const uint32_t* order = TW >= kCountTile && t_lo == 0 && t_hi == all
+                              ? (const uint32_t*)(ws + L.off_order) : nullptr;
 #define DAXHIP_GEN(DEDUP)                                                                        \
   k_generate<TW, NT, Src, DEDUP><<<dim3((unsigned)ntiles), dim3(NT), lds, s>>>(                  \
       g, field, (const uint64_t*)(ws + L.off_bits), cs, (const Ctrl*)(ws + L.off_ctrl), o, flags, \
