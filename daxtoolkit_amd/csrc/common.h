@@ -37,16 +37,22 @@ struct TempBuf {
 // copy launch and no staging buffer between.  From a fixed table of slots
 // (one page, kept until the process ends), held by one call at a time; `p` is
 // null when every slot is taken or there is no pinned memory, and the caller
-// then copies.  A slot is reused only after its holder has synchronised.
+// then copies.  A slot goes to another call only when the kernels of its
+// holder's stream have ended: the holder waits for them with wait(), or (where
+// it returns early with an error) its destructor does; a slot whose stream
+// cannot be waited for is not given out again.
 struct HostSlot {
   int64_t* p = nullptr;
-  HostSlot();
+  explicit HostSlot(hipStream_t stream);
   ~HostSlot();
   HostSlot(const HostSlot&) = delete;
   HostSlot& operator=(const HostSlot&) = delete;
+  hipError_t wait();
 
  private:
+  hipStream_t s_;
   int index_ = -1;
+  bool waited_ = false;
 };
 
 #define DAXHIP_CHECK(expr)                                  \

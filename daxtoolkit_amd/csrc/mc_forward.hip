@@ -891,14 +891,14 @@ int check_totals(int64_t t, int64_t u) {
 int count_sync(const VolGeom& g, char* ws, const Workspace& L, const Tuning& tu, int64_t* h_tris,
                int64_t* h_points, hipStream_t s) {
   int64_t c[2] = {0, 0};
-  HostSlot slot;
+  HostSlot slot(s);
   int rc;
   if ((rc = launch_scan(g, ws, L, tu, s, ScanOut{nullptr, slot.p}))) return rc;
   unsigned long long vt[2];
   if (!slot.p)
     DAXHIP_CHECK(hipMemcpyAsync(vt, ws + L.off_ctrl + offsetof(Ctrl, total_v), sizeof(vt),
                                 hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
+  DAXHIP_CHECK(slot.wait());
   c[0] = slot.p ? ((volatile int64_t*)slot.p)[0] : (int64_t)vt[1];
   c[1] = slot.p ? ((volatile int64_t*)slot.p)[1] : (int64_t)vt[0];
   *h_tris = c[0];

@@ -93,16 +93,20 @@ uint64_t g_slots_used = 0;        // bit i: slot i is held
 static_assert(kHostSlots == 64, "one bit per slot");
 }  // namespace
 
-HostSlot::HostSlot() {
+HostSlot::HostSlot(hipStream_t stream) : s_(stream) {
   std::lock_guard<std::mutex> lock(g_slot_mu);
   if (!g_slots_tried) {
     g_slots_tried = true;
     void* m = nullptr;
+    // (not an error to a capture that another thread has under way)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
     if (hipHostMalloc(&m, (size_t)kHostSlots * 64, hipHostMallocPortable | hipHostMallocMapped) ==
         hipSuccess)
       g_slots = (int64_t*)m;
     else
       (void)hipGetLastError();
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
   }
   if (!g_slots || ~g_slots_used == 0ull) return;
   index_ = __builtin_ctzll(~g_slots_used);
@@ -110,8 +114,14 @@ HostSlot::HostSlot() {
   p = g_slots + 8 * index_;
 }
 
+hipError_t HostSlot::wait() {
+  const hipError_t e = hipStreamSynchronize(s_);
+  waited_ = e == hipSuccess;
+  return e;
+}
+
 HostSlot::~HostSlot() {
-  if (index_ < 0) return;
+  if (index_ < 0 || (!waited_ && wait() != hipSuccess)) return;
   std::lock_guard<std::mutex> lock(g_slot_mu);
   g_slots_used &= ~(1ull << index_);
 }

@@ -1063,14 +1063,14 @@ int prepare_bits(const BitGeom& bg, const BitWs& bw, char* ws, const float* d_fi
         bg, cs.bits, ps, (flags & DAX_HIP_TOPOLOGY_MASK_OPTIONAL) ? nullptr : d_mask);
     DAXHIP_LAUNCH_CHECK("k_mask_words");
   }
-  HostSlot slot;
+  HostSlot slot(s);
   k_scan_word_tiles<<<dedup ? 2 : 1, kSumThreads, 0, s>>>(cs.tile, bw.nct, ps.tile, bw.nmt, hdr,
                                                           slot.p);
   DAXHIP_LAUNCH_CHECK("k_scan_word_tiles");
   int32_t h[kHeaderInts] = {};
   if (!slot.p)
     DAXHIP_CHECK(hipMemcpyAsync(h, hdr, sizeof(h), hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
+  DAXHIP_CHECK(slot.wait());
   const volatile int64_t* v = slot.p;
   *cells = v ? v[0] : h[6];
   *points = !dedup ? 0 : (v ? v[1] : h[7]);
@@ -1112,13 +1112,13 @@ int prepare_linear(const Geometry& g, const BitGeom& bg, const BitWs& bw, char* 
   k_word_prefix<<<dim3((unsigned)std::max(bw.nct, dedup ? bw.nmt : 0), dedup ? 2 : 1),
                   dim3(kWordTile), 0, s>>>(cs, bg.n_cwords, ps, bg.n_pwords);
   DAXHIP_LAUNCH_CHECK("k_word_prefix");
-  HostSlot slot;
+  HostSlot slot(s);
   k_scan_word_tiles<<<dedup ? 2 : 1, kSumThreads, 0, s>>>(cs.tile, bw.nct, ps.tile, bw.nmt, hdr,
                                                           slot.p);
   DAXHIP_LAUNCH_CHECK("k_scan_word_tiles");
   int32_t h[kHeaderInts] = {};
   if (!slot.p) DAXHIP_CHECK(hipMemcpyAsync(h, hdr, sizeof(h), hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
+  DAXHIP_CHECK(slot.wait());
   const volatile int64_t* v = slot.p;
   *cells = v ? v[0] : h[6];
   *points = !dedup ? 0 : (v ? v[1] : h[7]);

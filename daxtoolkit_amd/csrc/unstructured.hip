@@ -973,7 +973,7 @@ int dedup_corners(Dedup& d, void* d_scratch, int64_t n_tris, const float* d_fiel
   // grids over the rows loop: how many there are is known on the device only
   const dim3 gr((unsigned)std::min<int64_t>(d.n_tiles, 4096));
   const dim3 gl((unsigned)ceil_div(n, kListCorners));
-  HostSlot slot;
+  HostSlot slot(s);
   k_point_prefix<<<dim3((unsigned)d.npt), dim3(kPointTile), 0, s>>>(d.used, d.pw, d.nw, d.ptile);
   DAXHIP_LAUNCH_CHECK("k_point_prefix");
   k_scan_block<<<1, kScanBlock, 0, s>>>(d.ptile, d.npt, nullptr, &d.state->rows, nullptr, nullptr);
@@ -1005,7 +1005,7 @@ int dedup_corners(Dedup& d, void* d_scratch, int64_t n_tris, const float* d_fiel
     DAXHIP_CHECK(hipMemcpyAsync(&u, res.p, 4, hipMemcpyDeviceToHost, s));
     DAXHIP_CHECK(hipMemcpyAsync(&over, &d.state->overflow, 4, hipMemcpyDeviceToHost, s));
   }
-  DAXHIP_CHECK(hipStreamSynchronize(s));
+  DAXHIP_CHECK(slot.wait());
   if (slot.p) {
     u = (uint32_t)((volatile int64_t*)slot.p)[0];
     over = (uint32_t)((volatile int64_t*)slot.p)[1];
@@ -1088,7 +1088,7 @@ int count_blocks(const char* name, const int32_t* d_cells, int64_t n_cells, cons
   else
     k_count_blocks<NV, false><<<g, b, 0, s>>>(d_cells, n_cells, d_field, n_points, iso, bits, sums);
   DAXHIP_LAUNCH_CHECK("k_count_blocks");
-  HostSlot slot;
+  HostSlot slot(s);
   TempBuf res(s);
   if (!slot.p)
     if (const int rc = res.alloc(16)) return rc;
@@ -1096,7 +1096,7 @@ int count_blocks(const char* name, const int32_t* d_cells, int64_t n_cells, cons
   DAXHIP_LAUNCH_CHECK("k_scan_block");
   uint32_t h[2] = {0, 0};
   if (!slot.p) DAXHIP_CHECK(hipMemcpyAsync(h, res.p, sizeof(h), hipMemcpyDeviceToHost, s));
-  DAXHIP_CHECK(hipStreamSynchronize(s));
+  DAXHIP_CHECK(slot.wait());
   const volatile int64_t* v = slot.p;
   if (v ? v[1] != 0 : h[1] != 0) {
     set_error("%s: a cell references a point outside [0, %lld)", name, (long long)n_points);

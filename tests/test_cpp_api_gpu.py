@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 BIN = Path(__file__).resolve().parent / "cpp" / "bin"
 TESTS = ["UnitTestDeviceAdapterHip", "UnitTestWorkletMarchingCubesHip",
          "UnitTestWorkletCellGradientHip", "UnitTestWorkletSliceHip",
-         "UnitTestWorkletMarchingTetrahedraHip", "UnitTestWorkletThresholdHip"]
+         "UnitTestWorkletMarchingTetrahedraHip", "UnitTestWorkletThresholdHip",
+         "UnitTestHostSlotHip"]
 
 
 @pytest.mark.parametrize("name", TESTS)
