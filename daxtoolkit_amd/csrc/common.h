@@ -30,6 +30,10 @@ struct TempBuf {
   TempBuf(const TempBuf&) = delete;
   TempBuf& operator=(const TempBuf&) = delete;
   int alloc(size_t bytes) { return temp_alloc(&p, bytes, s); }
+  void release() {  // early, in stream order as well
+    temp_free(p, s);
+    p = nullptr;
+  }
 };
 
 // Eight 64-bit words of pinned host memory that kernels write results into, so

@@ -131,7 +131,7 @@ __device__ __forceinline__ void lerp3(const float* __restrict__ pts, int64_t a, 
 __device__ __forceinline__ void note_edge(int2* __restrict__ pairs, uint8_t* __restrict__ used,
                                           int64_t i, int a, int b) {
   pairs[i] = make_int2(a, b);
-  used[a] = 1;
+  if (used) used[a] = 1;  // null: the edges are sorted
 }
 
 // Corners of every triangle: with pairs, each corner's edge (dedup); without,
@@ -498,21 +498,22 @@ __global__ __launch_bounds__(256) void k_generate_blocks(
 
 // ---- dedup -------------------------------------------------------------------
 // The corners' edges (A, B) numbered in the order of their pairs without
-// sorting them: the lower endpoints A are ranked by the words of their bits;
-// each rank has a row of kRowSlots upper endpoints B, each distinct B once.
-// The corners are listed by tile of kRowTile ranks (a wave reserves room for
-// the few tiles its corners fall into), and a block per tile fills its rows in
-// LDS with compare-and-swap, sizes them, and numbers its corners within the
-// tile; a scan of the tiles' sizes makes the numbers final.  Any order of
-// insertion gives the same numbers.  More than kRowSlots active edges up from
-// one point, or more rows than there is room for, set a flag and the general
-// sort is run instead.
+// sorting them all: the lower endpoints A are ranked by the words of their bits;
+// the corners are listed by tile of kRowTile ranks (a block reserves room for
+// the few tiles its corners fall into), and a block per tile finds its distinct
+// pairs in an LDS table, places them by rank and upper endpoint, and numbers its
+// corners within the tile; a scan of the tiles' sizes makes the numbers final.
+// Any order of insertion gives the same numbers.  A tile of more pairs than the
+// table takes goes through its ranks in parts.  A lower endpoint with more
+// active edges up from it than that, or a tile of very many corners, sets a flag
+// and the general sort is run instead.
 //
 // The sort's six radix passes and the scans around them took 220 us for 540 K
 // corners and 370 for 2.06 M; rows in global memory 62 and 133 us for the
-// insertion alone (atomics across the XCDs' L2s); this chain takes
-// 58 and 130 in all.
-constexpr int kRowSlots = 16;
+// insertion alone (atomics across the XCDs' L2s); this chain takes 42 and 99 us,
+// besides three scans of 4.  Rows of at most 16 edges in LDS instead of the table
+// took 18 us for what now takes 17 (42 and 38), but sent every mesh with a longer
+// row to the sort: three million unshared tetrahedra 1681 us, now 793.
 constexpr int kPointTile = 256;
 
 // 64 points' bits and their exclusive popcount prefix within a tile of
@@ -522,14 +523,10 @@ struct alignas(16) PointWord {
   uint32_t pre, pad;
 };
 
-struct alignas(16) EdgeRow {
-  uint32_t b[kRowSlots];  // upper endpoint + 1, filled from slot 0; 0: free
-};
-
 struct DedupState {
   uint32_t rows;      // lower endpoints
   uint32_t rows_top;  // (k_scan_block's second word)
-  uint32_t overflow;
+  uint32_t overflow;  // to be sorted
   uint32_t pad;
 };
 
@@ -593,12 +590,15 @@ constexpr uint32_t kNoRow = 0xffffffffu;
 // atomic per block and tile reserves their places: with one per wave and tile
 // the launch took 52 us for 540 K corners and 94 for 2.06 M (neighbouring
 // waves wait for the same counters), now 10 and 25.
+// A tile has some 700 corners (2.06 M in 2900 tiles); beyond kMaxTileCorners
+// going through its ranks in parts costs more than the sort.
 constexpr int kListCorners = 1024;
+constexpr uint32_t kMaxTileCorners = 1 << 14;
 __global__ __launch_bounds__(256) void k_corner_rows(const int2* __restrict__ pairs, int64_t n,
                                                      int64_t n_points,
                                                      const PointWord* __restrict__ pw,
                                                      const uint32_t* __restrict__ ptile,
-                                                     int64_t cap, uint32_t* __restrict__ count,
+                                                     uint32_t* __restrict__ count,
                                                      uint2* __restrict__ row_place,
                                                      DedupState* __restrict__ st) {
   constexpr int kPer = kListCorners / 256;
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(256) void k_corner_rows(const int2* __restrict__ pa
     s_key[h] = kNoRow;
     s_cnt[h] = 0u;
   }
-  const int64_t rows = min((int64_t)st->rows, cap);
+  const uint32_t rows = st->rows;
   uint32_t r[kPer], slot[kPer], place[kPer];
   const int64_t i0 = (int64_t)blockIdx.x * kListCorners + threadIdx.x;
 #pragma unroll
@@ -618,10 +618,7 @@ __global__ __launch_bounds__(256) void k_corner_rows(const int2* __restrict__ pa
     if (i < n) {
       const int2 e = pairs[i];
       if (is_edge(e, n_points)) r[u] = point_rank(pw, ptile, e.x);
-      if (r[u] != kNoRow && (int64_t)r[u] >= rows) {
-        if ((int64_t)r[u] >= cap) st->overflow = 1u;
-        r[u] = kNoRow;
-      }
+      if (r[u] >= rows) r[u] = kNoRow;
     }
   }
   __syncthreads();
@@ -641,7 +638,11 @@ __global__ __launch_bounds__(256) void k_corner_rows(const int2* __restrict__ pa
   }
   __syncthreads();
   for (uint32_t h = threadIdx.x; h < kTable; h += 256u)
-    if (s_cnt[h]) s_cnt[h] = atomicAdd(&count[s_key[h]], s_cnt[h]);  // now the first place
+    if (s_cnt[h]) {
+      const uint32_t first = atomicAdd(&count[s_key[h]], s_cnt[h]);
+      if (first + s_cnt[h] > kMaxTileCorners) st->overflow = 1u;
+      s_cnt[h] = first;  // the first place
+    }
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
@@ -654,136 +655,174 @@ __global__ __launch_bounds__(256) void k_corner_rows(const int2* __restrict__ pa
 __global__ __launch_bounds__(256) void k_list_corners(const int2* __restrict__ pairs, int64_t n,
                                                       const uint2* __restrict__ row_place,
                                                       const uint32_t* __restrict__ start,
-                                                      TileCorner* __restrict__ list,
-                                                      int32_t* __restrict__ conn) {
+                                                      const DedupState* __restrict__ st,
+                                                      TileCorner* __restrict__ list) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || st->overflow) return;
   const uint2 rp = row_place[i];
-  if (rp.x == kNoRow) {
-    conn[i] = -1;
-    return;
-  }
+  if (rp.x == kNoRow) return;
   const int64_t at = (int64_t)start[rp.x / kRowTile] + rp.y;
   if (at >= n) return;  // always below: the places are the counts'
   const TileCorner c{(int32_t)i, pairs[i].y, rp.x % kRowTile};
   __builtin_memcpy(&list[at], &c, sizeof(c));
 }
 
-__device__ __forceinline__ void load_row(const EdgeRow* row, uint32_t* b) {
-  const uint4* p = reinterpret_cast<const uint4*>(row);
-#pragma unroll
-  for (int q = 0; q < kRowSlots / 4; ++q) {
-    const uint4 v = p[q];
-    b[4 * q + 0] = v.x;
-    b[4 * q + 1] = v.y;
-    b[4 * q + 2] = v.z;
-    b[4 * q + 3] = v.w;
-  }
-}
-
-__device__ __forceinline__ uint32_t smaller_in_row(const uint32_t* b, uint32_t want) {
-  uint32_t k = 0u;
-#pragma unroll
-  for (int s = 0; s < kRowSlots; ++s) k += b[s] != 0u && b[s] < want;
-  return k;
-}
-
 // A block per tile of rows (the grid loops: their number is the device's).
-// Leaves every corner's tile and number within it in conn (tile << 10 |
-// number: a tile holds at most 1024).  64 rows per tile: with 256 the 120
-// tiles of the 128^3 tetrahedra's surface left half the CUs idle (27 us, now 14).
-constexpr int kNumberBits = 10;
-static_assert(kRowTile * kRowSlots == 1 << kNumberBits, "a tile's numbers");
-__global__ __launch_bounds__(256) void k_fill_rows(
+// Leaves every corner's number within its tile in place[corner].y and the tile's
+// distinct edges, in the order of their numbers, from its first corner's place in
+// the list on (it has no more edges than corners).  64 rows per tile: with 256
+// the 120 tiles of the 128^3 tetrahedra's surface left half the CUs idle (27 us,
+// now 12.4).  Bound by the chain of loads and barriers of a tile: a thread has its
+// four corners' loads in flight together, and what follows the table runs over the
+// distinct edges.  512 of them: at 1024 fewer tiles are taken in two passes, but
+// fewer blocks fit a CU (256^3 hexahedra 28.4 us, now 24.1; three million unshared
+// tetrahedra 887 us in all, now 793; 40 fans of 5000 271, now 313).
+constexpr uint32_t kTileEdges = 512;  // distinct edges of a pass over the tile, at most
+constexpr uint32_t kTileTable = 2 * kTileEdges;
+constexpr int kTilePer = 4;           // corners per thread and turn
+__global__ __launch_bounds__(256) void k_tile_edges(
     const int2* __restrict__ pairs, const TileCorner* __restrict__ list,
-    const uint32_t* __restrict__ start, const uint32_t* __restrict__ n_list, int64_t cap,
-    EdgeRow* __restrict__ rows, int32_t* __restrict__ row_a, uint32_t* __restrict__ pre,
-    uint32_t* __restrict__ sizes, DedupState* __restrict__ st, int32_t* __restrict__ conn) {
-  __shared__ EdgeRow s_rows[kRowTile];
-  __shared__ int32_t s_a[kRowTile];
-  __shared__ uint32_t s_pre[kRowTile];
-  const int tid = threadIdx.x;
-  const int64_t n_rows = min((int64_t)st->rows, cap);
-  const int64_t n_tiles = ceil_div(n_rows, (int64_t)kRowTile);
+    const uint32_t* __restrict__ start, const uint32_t* __restrict__ n_list,
+    int2* __restrict__ edges, uint32_t* __restrict__ sizes, DedupState* __restrict__ st,
+    uint2* __restrict__ place) {
+  __shared__ unsigned long long s_key[kTileTable];  // (row + 1) << 32 | upper endpoint; 0: free
+  __shared__ uint32_t s_at[kTileTable];        // an entry's corner, then its number
+  __shared__ uint16_t s_entry[kTileEdges + 256], s_pos[kTileEdges + 256];  // by order of arrival
+  __shared__ uint32_t s_b[kTileEdges];         // upper endpoints by row
+  __shared__ uint32_t s_cnt[kRowTile], s_first[kRowTile];
+  __shared__ uint32_t s_edges, s_stop;
+  const uint32_t tid = threadIdx.x;
+  const int64_t n_tiles = ceil_div((int64_t)st->rows, (int64_t)kRowTile);
   for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    static_assert(kRowTile * sizeof(EdgeRow) == 256 * 16, "16 bytes per thread");
-    reinterpret_cast<uint4*>(s_rows)[tid] = make_uint4(0u, 0u, 0u, 0u);
-    __syncthreads();
+    if (tid == 0) s_stop = __hip_atomic_load(&st->overflow, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t c0 = start[t], c1 = t + 1 < n_tiles ? start[t + 1] : *n_list;
-    for (uint32_t c = c0 + (uint32_t)tid; c < c1; c += 256u) {
-      TileCorner e;
-      __builtin_memcpy(&e, &list[c], sizeof(e));
-      const uint32_t want = (uint32_t)e.b + 1u;
-      uint32_t* b = s_rows[e.row].b;
-      int s = 0;
-      for (; s < kRowSlots; ++s) {
-        const uint32_t have = atomicCAS(b + s, 0u, want);
-        if (have == 0u && s == 0) s_a[e.row] = e.corner;  // one winner
-        if (have == 0u || have == want) break;
-      }
-      if (s == kRowSlots) st->overflow = 1u;
-    }
-    __syncthreads();
-    if (tid < kRowTile) {  // wave 0: the rows' sizes and first numbers
-      uint32_t b[kRowSlots], cnt = 0u;
-      load_row(&s_rows[tid], b);
+    uint32_t total = 0u, r0 = 0u, span = kRowTile;
+    TileCorner e[kTilePer];
+    uint32_t at[kTilePer];
+    auto key_of = [](const TileCorner& c) -> unsigned long long {
+      return ((unsigned long long)(c.row + 1u) << 32) | (uint32_t)c.b;
+    };
+    auto load = [&](uint32_t base) {  // rows outside the pass: none
 #pragma unroll
-      for (int s = 0; s < kRowSlots; ++s) cnt += b[s] != 0u;
-      const uint32_t inc = wave_incl_scan(cnt), p = inc - cnt;
-      const int64_t r = t * kRowTile + tid;
-      s_pre[tid] = p;
-      if (r < n_rows) {
-        pre[r] = p;
-        row_a[r] = cnt ? pairs[s_a[tid]].x : 0;
+      for (int u = 0; u < kTilePer; ++u) {
+        const uint32_t c = base + 256u * u + tid;
+        e[u].row = kNoRow;
+        if (c < c1) __builtin_memcpy(&e[u], &list[c], sizeof(e[u]));
       }
-      if (tid == kRowTile - 1) sizes[t] = inc;
+    };
+    // the key's entry, or the free one that ends its chain (never more than
+    // kTileEdges + 256 keys in the table)
+    auto find = [&](const TileCorner& c) -> uint32_t {
+      uint32_t h = ((uint32_t)c.b * 2654435761u + c.row * 0x9e3779b9u) >> 12;
+      while (true) {
+        h &= kTileTable - 1u;
+        const unsigned long long have =
+            __hip_atomic_load(&s_key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (have == 0ull || have == key_of(c)) return h;
+        ++h;
+      }
+    };
+    while (r0 < (uint32_t)kRowTile) {
+      for (uint32_t h = tid; h < kTileTable; h += 256u) s_key[h] = 0ull;
+      if (tid < kRowTile) s_cnt[tid] = 0u;
+      if (tid == 0) s_edges = 0u;
+      __syncthreads();
+      if (s_stop) return;  // uniform: written before the first pass
+      for (uint32_t base = c0; base < c1; base += 256u * kTilePer) {
+        load(base);
+#pragma unroll
+        for (int u = 0; u < kTilePer; ++u) {
+          at[u] = 0u;
+          if (e[u].row - r0 >= span) continue;
+          if (__hip_atomic_load(&s_edges, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >
+              kTileEdges)
+            continue;
+          while (true) {
+            const uint32_t h = find(e[u]);
+            const unsigned long long have = atomicCAS(&s_key[h], 0ull, key_of(e[u]));
+            if (have == 0ull) {  // one winner
+              const uint32_t i = atomicAdd(&s_edges, 1u);
+              s_entry[i] = (uint16_t)h;
+              s_at[h] = (uint32_t)e[u].corner;
+              s_pos[i] = (uint16_t)atomicAdd(&s_cnt[e[u].row], 1u);
+            }
+            at[u] = h;
+            if (have == 0ull || have == key_of(e[u])) break;
+          }
+        }
+      }
+      __syncthreads();
+      const uint32_t n = s_edges;
+      if (n > kTileEdges) {  // uniform
+        __syncthreads();
+        if (span == 1u) {
+          if (tid == 0) st->overflow = 1u;
+          return;
+        }
+        span /= 2u;
+        continue;
+      }
+      if (tid < kRowTile) {  // wave 0: the rows' first numbers
+        const uint32_t cnt = s_cnt[tid];
+        s_first[tid] = wave_incl_scan(cnt) - cnt;
+      }
+      __syncthreads();
+      for (uint32_t i = tid; i < n; i += 256u) {
+        const unsigned long long key = s_key[s_entry[i]];
+        s_b[s_first[(uint32_t)(key >> 32) - 1u] + s_pos[i]] = (uint32_t)key;
+      }
+      __syncthreads();
+      for (uint32_t i = tid; i < n; i += 256u) {
+        const uint32_t h = s_entry[i];
+        const uint32_t row = (uint32_t)(s_key[h] >> 32) - 1u, b = (uint32_t)s_key[h];
+        const int a = pairs[s_at[h]].x;
+        uint32_t k = s_first[row];
+        for (uint32_t q = 0; q < s_cnt[row]; ++q) k += s_b[s_first[row] + q] < b;
+        edges[c0 + total + k] = make_int2(a, (int)b);
+        s_at[h] = k;
+      }
+      __syncthreads();
+      const bool kept = c1 - c0 <= 256u * kTilePer;  // the corners are still in registers
+      for (uint32_t base = c0; base < c1; base += 256u * kTilePer) {
+        if (!kept) load(base);
+#pragma unroll
+        for (int u = 0; u < kTilePer; ++u)
+          if (e[u].row - r0 < span)
+            place[e[u].corner].y = total + s_at[kept ? at[u] : find(e[u])];
+      }
+      total += n;
+      r0 += span;
+      __syncthreads();  // LDS reused
     }
-    if (t * kRowTile + tid / 4 < n_rows)
-      reinterpret_cast<uint4*>(rows + t * kRowTile)[tid] = reinterpret_cast<uint4*>(s_rows)[tid];
-    __syncthreads();
-    for (uint32_t c = c0 + (uint32_t)tid; c < c1; c += 256u) {
-      TileCorner e;
-      __builtin_memcpy(&e, &list[c], sizeof(e));
-      uint32_t w[kRowSlots];
-      load_row(&s_rows[e.row], w);
-      conn[e.corner] = (int32_t)(((uint32_t)t << kNumberBits) |
-                                 (s_pre[e.row] + smaller_in_row(w, (uint32_t)e.b + 1u)));
-    }
-    __syncthreads();  // LDS reused by the next tile
+    if (tid == 0) sizes[t] = total;
   }
 }
 
-// The unique points, four lanes per row: records, weights and coordinates.
-__global__ __launch_bounds__(256) void k_row_points(
-    const EdgeRow* __restrict__ rows, int64_t cap, const DedupState* __restrict__ st,
-    const int32_t* __restrict__ row_a, const uint32_t* __restrict__ pre,
-    const uint32_t* __restrict__ tile, int64_t max_points, const float* __restrict__ field,
-    const float* __restrict__ pts, float iso, int32_t* __restrict__ first,
-    int32_t* __restrict__ second, float* __restrict__ weight, float* __restrict__ verts) {
+// The unique points, a block per tile: records, weights and coordinates.
+__global__ __launch_bounds__(256) void k_tile_points(
+    const int2* __restrict__ edges, const uint32_t* __restrict__ start,
+    const uint32_t* __restrict__ n_list, const DedupState* __restrict__ st,
+    const uint32_t* __restrict__ tile, const uint32_t* __restrict__ n_edges, int64_t max_points,
+    const float* __restrict__ field, const float* __restrict__ pts, float iso,
+    int32_t* __restrict__ first, int32_t* __restrict__ second, float* __restrict__ weight,
+    float* __restrict__ verts) {
   if (st->overflow) return;
-  const int64_t n = min((int64_t)st->rows, cap);
-  const int64_t step = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 4 * n; i += step) {
-    const int64_t r = i >> 2;
-    uint32_t b[kRowSlots];
-    load_row(rows + r, b);
-    const int32_t ia = row_a[r];
-    const float fa = field[ia];
-    const uint32_t base = tile[r / kRowTile] + pre[r];
-#pragma unroll
-    for (int q = 0; q < kRowSlots / 4; ++q) {
-      const int sub = (int)(i & 3);
-      const uint32_t want = sub == 0 ? b[4 * q] : (sub == 1 ? b[4 * q + 1]
-                                                            : (sub == 2 ? b[4 * q + 2] : b[4 * q + 3]));
-      const int64_t u = (int64_t)base + smaller_in_row(b, want);
-      if (want == 0u || u >= max_points) continue;
-      const int32_t ib = (int32_t)(want - 1u);
-      const float w = (iso - fa) / (field[ib] - fa);
-      if (first) first[u] = ia;
-      if (second) second[u] = ib;
+  const int lane = threadIdx.x;
+  const int64_t n_tiles = ceil_div((int64_t)st->rows, (int64_t)kRowTile);
+  const int64_t step = gridDim.x;
+  for (int64_t t = blockIdx.x; t < n_tiles; t += step) {
+    const uint32_t u0 = tile[t], u1 = t + 1 < n_tiles ? tile[t + 1] : *n_edges;
+    const int2* e0 = edges + start[t];
+    for (int64_t u = (int64_t)u0 + lane; u < u1 && u < max_points; u += 256) {
+      const int2 e = e0[u - u0];
+      const float fa = field[e.x];
+      const float w = (iso - fa) / (field[e.y] - fa);
+      if (first) first[u] = e.x;
+      if (second) second[u] = e.y;
       if (weight) weight[u] = w;
       float xyz[3];
-      lerp3(pts, ia, ib, w, xyz);
+      lerp3(pts, e.x, e.y, w, xyz);
       __builtin_memcpy(verts + 3 * u, xyz, 12);
     }
   }
@@ -793,12 +832,12 @@ __global__ __launch_bounds__(256) void k_row_points(
 __global__ __launch_bounds__(256) void k_number_corners(int64_t n,
                                                         const DedupState* __restrict__ st,
                                                         const uint32_t* __restrict__ tile,
+                                                        const uint2* __restrict__ place,
                                                         int32_t* __restrict__ conn) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n || st->overflow) return;
-  const int32_t v = conn[i];
-  conn[i] = v < 0 ? 0
-                  : (int32_t)(tile[v >> kNumberBits] + (uint32_t)(v & ((1 << kNumberBits) - 1)));
+  const uint2 p = place[i];
+  conn[i] = p.x == kNoRow ? 0 : (int32_t)(tile[p.x / kRowTile] + p.y);
 }
 
 // The general path's sort keys A * P + B and their corner indices, from the
@@ -907,27 +946,22 @@ int sort_corners(void* d_scratch, int64_t n_tris, const float* d_field, const fl
 // corners are noted.
 struct Dedup {
   TempBuf buf;
-  uint8_t* used = nullptr;
+  uint8_t* used = nullptr;  // bytes that note points
   DedupState* state = nullptr;
-  uint32_t *count = nullptr, *sizes = nullptr, *pre = nullptr, *ptile = nullptr, *n_list = nullptr;
+  uint32_t *count = nullptr, *sizes = nullptr, *ptile = nullptr, *n_list = nullptr,
+           *n_edges = nullptr;
   PointWord* pw = nullptr;
-  EdgeRow* rows = nullptr;
-  int32_t* row_a = nullptr;
   uint2* row_place = nullptr;
   TileCorner* list = nullptr;
-  int64_t nw = 0, npt = 0, cap = 0, n_tiles = 0;
+  int64_t nw = 0, npt = 0, n_tiles = 0;
   explicit Dedup(hipStream_t s) : buf(s) {}
 
-  // Rows for every corner of a small surface, for one edge per triangle of a
-  // large one (closed surfaces have about half as many points as triangles);
-  // at most 2^27, whose tiles fit the 21 bits beside a number.
+  // 60 bytes a triangle and a byte and a quarter a point.
   int begin(int64_t n_tris, int64_t n_points, hipStream_t s) {
     const int64_t n = 3 * n_tris;
     nw = ceil_div(n_points, 64);
     npt = ceil_div(nw, (int64_t)kPointTile);
-    cap = std::min(std::min(n_points, n), std::max(n_tris, (int64_t)1 << 18));
-    cap = std::min(cap, (int64_t)1 << 27);
-    n_tiles = ceil_div(cap, (int64_t)kRowTile);
+    n_tiles = ceil_div(std::min(n_points, n), (int64_t)kRowTile);
     size_t at = 0;
     auto take = [&](size_t bytes) {
       const size_t o = at;
@@ -938,11 +972,11 @@ struct Dedup {
     const size_t count_at = take((size_t)n_tiles * 4);
     const size_t clear = at;
     const size_t pw_at = take((size_t)nw * sizeof(PointWord)), pt_at = take((size_t)npt * 4);
-    const size_t nl_at = take(8), sizes_at = take((size_t)n_tiles * 4);
-    const size_t rows_at = take((size_t)cap * sizeof(EdgeRow)), a_at = take((size_t)cap * 4);
-    const size_t pre_at = take((size_t)cap * 4), rp_at = take((size_t)n * sizeof(uint2));
+    const size_t nl_at = take(8), ne_at = take(8), sizes_at = take((size_t)n_tiles * 4);
+    const size_t rp_at = take((size_t)n * sizeof(uint2));
     const size_t list_at = take((size_t)n * sizeof(TileCorner));
-    if (const int rc = buf.alloc(at)) return rc;
+    const int rc = buf.alloc(at);
+    if (rc) return rc;
     char* p = (char*)buf.p;
     used = (uint8_t*)(p + used_at);
     state = (DedupState*)(p + state_at);
@@ -950,10 +984,8 @@ struct Dedup {
     pw = (PointWord*)(p + pw_at);
     ptile = (uint32_t*)(p + pt_at);
     n_list = (uint32_t*)(p + nl_at);
+    n_edges = (uint32_t*)(p + ne_at);
     sizes = (uint32_t*)(p + sizes_at);
-    rows = (EdgeRow*)(p + rows_at);
-    row_a = (int32_t*)(p + a_at);
-    pre = (uint32_t*)(p + pre_at);
     row_place = (uint2*)(p + rp_at);
     list = (TileCorner*)(p + list_at);
     const int64_t n16 = (int64_t)(clear / 16);
@@ -963,55 +995,60 @@ struct Dedup {
   }
 };
 
+// The scratch holds the corners' pairs and, in its second half, the tiles'
+// distinct edges.
 int dedup_corners(Dedup& d, void* d_scratch, int64_t n_tris, const float* d_field,
                   const float* d_points, int64_t n_points, float iso, float* d_vertices,
                   int32_t* d_conn, int32_t* d_first, int32_t* d_second, float* d_weight,
                   int64_t* h_points, hipStream_t s) {
   const int64_t n = 3 * n_tris;
   const int2* pairs = (const int2*)d_scratch;
+  int2* edges = (int2*)d_scratch + n;
   const dim3 b(256), gn((unsigned)ceil_div(n, 256));
-  // grids over the rows loop: how many there are is known on the device only
-  const dim3 gr((unsigned)std::min<int64_t>(d.n_tiles, 4096));
+  // grids over the tiles loop: how many there are is known on the device only
+  const dim3 gt((unsigned)std::min<int64_t>(d.n_tiles, 4096));
   const dim3 gl((unsigned)ceil_div(n, kListCorners));
-  HostSlot slot(s);
-  k_point_prefix<<<dim3((unsigned)d.npt), dim3(kPointTile), 0, s>>>(d.used, d.pw, d.nw, d.ptile);
-  DAXHIP_LAUNCH_CHECK("k_point_prefix");
-  k_scan_block<<<1, kScanBlock, 0, s>>>(d.ptile, d.npt, nullptr, &d.state->rows, nullptr, nullptr);
-  DAXHIP_LAUNCH_CHECK("k_scan_block");
-  k_corner_rows<<<gl, b, 0, s>>>(pairs, n, n_points, d.pw, d.ptile, d.cap, d.count, d.row_place,
-                                 d.state);
-  DAXHIP_LAUNCH_CHECK("k_corner_rows");
-  k_scan_block<<<1, kScanBlock, 0, s>>>(d.count, d.n_tiles, &d.state->rows, d.n_list, nullptr,
-                                        nullptr);
-  DAXHIP_LAUNCH_CHECK("k_scan_block");
-  k_list_corners<<<gn, b, 0, s>>>(pairs, n, d.row_place, d.count, d.list, d_conn);
-  DAXHIP_LAUNCH_CHECK("k_list_corners");
-  k_fill_rows<<<gr, b, 0, s>>>(pairs, d.list, d.count, d.n_list, d.cap, d.rows, d.row_a, d.pre,
-                               d.sizes, d.state, d_conn);
-  DAXHIP_LAUNCH_CHECK("k_fill_rows");
-  TempBuf res(s);  // {points, -} when there is no pinned slot
-  if (!slot.p)
-    if (const int rc = res.alloc(16)) return rc;
-  k_scan_block<<<1, kScanBlock, 0, s>>>(d.sizes, d.n_tiles, &d.state->rows, (uint32_t*)res.p,
-                                        &d.state->overflow, slot.p);
-  DAXHIP_LAUNCH_CHECK("k_scan_block");
-  k_row_points<<<gr, b, 0, s>>>(d.rows, d.cap, d.state, d.row_a, d.pre, d.sizes, n, d_field,
-                                d_points, iso, d_first, d_second, d_weight, d_vertices);
-  DAXHIP_LAUNCH_CHECK("k_row_points");
-  k_number_corners<<<gn, b, 0, s>>>(n, d.state, d.sizes, d_conn);
-  DAXHIP_LAUNCH_CHECK("k_number_corners");
-  uint32_t u = 0, over = 0;
-  if (!slot.p) {
-    DAXHIP_CHECK(hipMemcpyAsync(&u, res.p, 4, hipMemcpyDeviceToHost, s));
-    DAXHIP_CHECK(hipMemcpyAsync(&over, &d.state->overflow, 4, hipMemcpyDeviceToHost, s));
+  bool sort = !d.used;
+  if (!sort) {
+    HostSlot slot(s);
+    k_point_prefix<<<dim3((unsigned)d.npt), dim3(kPointTile), 0, s>>>(d.used, d.pw, d.nw, d.ptile);
+    DAXHIP_LAUNCH_CHECK("k_point_prefix");
+    k_scan_block<<<1, kScanBlock, 0, s>>>(d.ptile, d.npt, nullptr, &d.state->rows, nullptr, nullptr);
+    DAXHIP_LAUNCH_CHECK("k_scan_block");
+    k_corner_rows<<<gl, b, 0, s>>>(pairs, n, n_points, d.pw, d.ptile, d.count, d.row_place,
+                                   d.state);
+    DAXHIP_LAUNCH_CHECK("k_corner_rows");
+    k_scan_block<<<1, kScanBlock, 0, s>>>(d.count, d.n_tiles, &d.state->rows, d.n_list, nullptr,
+                                          nullptr);
+    DAXHIP_LAUNCH_CHECK("k_scan_block");
+    k_list_corners<<<gn, b, 0, s>>>(pairs, n, d.row_place, d.count, d.state, d.list);
+    DAXHIP_LAUNCH_CHECK("k_list_corners");
+    k_tile_edges<<<gt, b, 0, s>>>(pairs, d.list, d.count, d.n_list, edges, d.sizes, d.state,
+                                  d.row_place);
+    DAXHIP_LAUNCH_CHECK("k_tile_edges");
+    k_scan_block<<<1, kScanBlock, 0, s>>>(d.sizes, d.n_tiles, &d.state->rows, d.n_edges,
+                                          &d.state->overflow, slot.p);
+    DAXHIP_LAUNCH_CHECK("k_scan_block");
+    k_tile_points<<<gt, b, 0, s>>>(edges, d.count, d.n_list, d.state, d.sizes, d.n_edges, n,
+                                   d_field, d_points, iso, d_first, d_second, d_weight, d_vertices);
+    DAXHIP_LAUNCH_CHECK("k_tile_points");
+    k_number_corners<<<gn, b, 0, s>>>(n, d.state, d.sizes, d.row_place, d_conn);
+    DAXHIP_LAUNCH_CHECK("k_number_corners");
+    uint32_t u = 0, over = 0;
+    if (!slot.p) {
+      DAXHIP_CHECK(hipMemcpyAsync(&u, d.n_edges, 4, hipMemcpyDeviceToHost, s));
+      DAXHIP_CHECK(hipMemcpyAsync(&over, &d.state->overflow, 4, hipMemcpyDeviceToHost, s));
+    }
+    DAXHIP_CHECK(slot.wait());
+    if (slot.p) {
+      u = (uint32_t)((volatile int64_t*)slot.p)[0];
+      over = (uint32_t)((volatile int64_t*)slot.p)[1];
+    }
+    *h_points = u;
+    sort = over != 0u;
+    if (sort) d.buf.release();
   }
-  DAXHIP_CHECK(slot.wait());
-  if (slot.p) {
-    u = (uint32_t)((volatile int64_t*)slot.p)[0];
-    over = (uint32_t)((volatile int64_t*)slot.p)[1];
-  }
-  *h_points = u;
-  if (!over) return DAX_HIP_OK;
+  if (!sort) return DAX_HIP_OK;
   return sort_corners(d_scratch, n_tris, d_field, d_points, n_points, iso, d_vertices, d_conn,
                       d_first, d_second, d_weight, h_points, s);
 }

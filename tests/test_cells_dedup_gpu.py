@@ -1,7 +1,8 @@
-"""Edges numbered through rows of upper endpoints, and the sort taken when they
-do not fit: more than 16 active edges up from one point, more lower endpoints
-than rows.  Both give the oracle's (or torch.unique's) numbering.  Cells at the
-edges of the 1024-cell blocks, and connectivity off a 16-byte boundary."""
+"""Edges numbered by tiles of 64 lower endpoints: tiles that hold up to 512
+distinct edges, tiles of more that go through their endpoints in parts, and the
+sort taken for more edges up from one point or very many corners of a tile.  All
+give the oracle's numbering.  Cells at the edges of the 1024-cell blocks, and
+connectivity off a 16-byte boundary."""
 import numpy as np
 import pytest
 import torch
@@ -24,7 +25,8 @@ def _fan(n):
     return cells, f, pts
 
 
-@pytest.mark.parametrize("n", [3, 14, 15, 16, 40, 700])
+@pytest.mark.parametrize("n", [3, 14, 15, 16, 40, 509, 510, 511, 700, 1021, 1022, 1023, 1500,
+                               9000])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_fan_matches_oracle(n, offset):
     cells, f, pts = _fan(n)
@@ -40,10 +42,59 @@ def test_fan_matches_oracle(n, offset):
         assert np.array_equal(c.vertices.cpu().numpy(), r["coords"])
 
 
+@pytest.mark.parametrize("fans,n", [(16, 29), (16, 30), (16, 31), (25, 38), (25, 39), (26, 38),
+                                    (63, 40), (65, 40), (200, 100), (5, 700), (66, 300),
+                                    (300, 60)])
+def test_many_fans_match_oracle(fans, n):
+    """Tiles of up to 64 points with n + 2 edges up from each: around 512 edges,
+    in halves, quarters and fewer points, and beyond 16384 corners."""
+    parts = [_fan(n) for _ in range(fans)]
+    step = n + 3
+    # the inside points first, so that they are neighbours
+    cells = np.concatenate([np.where(c == 0, i, fans + i * (step - 1) + c - 1)
+                            for i, (c, _, _) in enumerate(parts)]).astype(np.int32)
+    rng = np.random.default_rng(fans * n)
+    f = np.concatenate([np.full(fans, 1.0), rng.random(fans * (step - 1)) * 0.4]).astype(np.float32)
+    pts = rng.random((len(f), 3)).astype(np.float32)
+    cells = np.ascontiguousarray(cells[rng.permutation(len(cells))])
+    ct, ft, pt = (torch.from_numpy(a).cuda() for a in (cells, f, pts))
+    c = mc.tetrahedra(ct, ft, pt, 0.5)
+    r = orc.mt_generate(cells, f, pts, 0.5, dedup=True)
+    assert np.array_equal(c.connectivity.cpu().numpy().reshape(-1), r["conn"])
+    assert np.array_equal(c.interp_first.cpu().numpy(), r["first"])
+    assert np.array_equal(c.interp_second.cpu().numpy(), r["second"])
+    assert np.array_equal(c.vertices.cpu().numpy(), r["coords"])
+
+
+def test_sorted_edges_take_no_longer():
+    """200 000 cells around one point: finding out that its edges have to be
+    sorted took 20 times as long as the cells' own work."""
+    def best_of(cells, f, pts, n=5):
+        args = [torch.from_numpy(a).cuda() for a in (cells, f, pts)]
+        start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        mc.tetrahedra(*args, 0.5)
+        best = float("inf")
+        for _ in range(n):
+            start.record()
+            mc.tetrahedra(*args, 0.5)
+            stop.record()
+            stop.synchronize()
+            best = min(best, start.elapsed_time(stop))
+        return best
+
+    n = 200_000
+    cells, f, pts = _fan(n)
+    apart = np.arange(4 * n, dtype=np.int32).reshape(n, 4)
+    fa = np.zeros((n, 4), np.float32)
+    fa[:, 0] = 1.0
+    rng = np.random.default_rng(1)
+    other = best_of(apart, fa.reshape(-1), rng.random((4 * n, 3)).astype(np.float32))
+    assert best_of(cells, f, pts) < 4.0 * other
+
+
 @pytest.mark.parametrize("tets", [1, 63, 64, 65, 1023, 1024, 1025, 4097, 300_000])
 def test_disjoint_tetrahedra(tets):
-    """Every tetrahedron its own four points, three of them lower endpoints: at
-    300 000 more lower endpoints than rows."""
+    """Every tetrahedron its own four points, three of them lower endpoints."""
     cells = torch.arange(4 * tets, dtype=torch.int32, device="cuda").view(tets, 4)
     g = torch.Generator(device="cuda")
     g.manual_seed(tets)
