@@ -946,7 +946,7 @@ int sort_corners(void* d_scratch, int64_t n_tris, const float* d_field, const fl
 // corners are noted.
 struct Dedup {
   TempBuf buf;
-  uint8_t* used = nullptr;  // bytes that note points
+  uint8_t* used = nullptr;  // null: no room for the tables, sort
   DedupState* state = nullptr;
   uint32_t *count = nullptr, *sizes = nullptr, *ptile = nullptr, *n_list = nullptr,
            *n_edges = nullptr;
@@ -956,7 +956,8 @@ struct Dedup {
   int64_t nw = 0, npt = 0, n_tiles = 0;
   explicit Dedup(hipStream_t s) : buf(s) {}
 
-  // 60 bytes a triangle and a byte and a quarter a point.
+  // 60 bytes a triangle and a byte and a quarter a point; where there is no such
+  // memory the sort is left, which takes 48 a triangle.
   int begin(int64_t n_tris, int64_t n_points, hipStream_t s) {
     const int64_t n = 3 * n_tris;
     nw = ceil_div(n_points, 64);
@@ -976,6 +977,7 @@ struct Dedup {
     const size_t rp_at = take((size_t)n * sizeof(uint2));
     const size_t list_at = take((size_t)n * sizeof(TileCorner));
     const int rc = buf.alloc(at);
+    if (rc == DAX_HIP_OOM) return DAX_HIP_OK;
     if (rc) return rc;
     char* p = (char*)buf.p;
     used = (uint8_t*)(p + used_at);

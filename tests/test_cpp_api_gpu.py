@@ -11,7 +11,7 @@ BIN = Path(__file__).resolve().parent / "cpp" / "bin"
 TESTS = ["UnitTestDeviceAdapterHip", "UnitTestWorkletMarchingCubesHip",
          "UnitTestWorkletCellGradientHip", "UnitTestWorkletSliceHip",
          "UnitTestWorkletMarchingTetrahedraHip", "UnitTestWorkletThresholdHip",
-         "UnitTestHostSlotHip"]
+         "UnitTestHostSlotHip", "UnitTestCellsDedupHip"]
 
 
 @pytest.mark.parametrize("name", TESTS)
