@@ -68,3 +68,49 @@ def test_ids_out_of_range(V, bad):
         topology.generate_topology(counts, cells=cd, points=pd)
     counts[150] = 0
     assert topology.generate_topology(counts, cells=cd, points=pd).num_cells == 199
+
+
+@pytest.mark.parametrize("C", [2**17, 2**18])
+@pytest.mark.parametrize("where", [0, -1])
+def test_totals_of_many_counts(C, where):
+    """Counts beyond one turn of the blocks that add them up: the sum is exact to
+    the last cell, and a negative count is seen wherever it stands."""
+    rng = np.random.default_rng(C)
+    cells = torch.from_numpy(rng.integers(0, 99, (C, 8)).astype(np.int32)).cuda()
+    points = torch.zeros((99, 3), device="cuda")
+    counts = torch.full((C,), 2**28 // C, dtype=torch.int32, device="cuda")  # 2^31 ids
+    with pytest.raises(_lib.ErrorControlBadValue):
+        topology.generate_topology(counts, cells=cells, points=points)
+    counts.zero_()
+    counts[where] = -1
+    counts[C // 2] = 2
+    with pytest.raises(_lib.ErrorControlBadValue):
+        topology.generate_topology(counts, cells=cells, points=points)
+    counts[where] = 3
+    out = topology.generate_topology(counts, cells=cells, points=points)
+    kept = torch.repeat_interleave(torch.arange(C, device="cuda"), counts.long())
+    used, ids = torch.unique(cells[kept], return_inverse=True)
+    assert torch.equal(out.connectivity, ids.to(torch.int32))
+    assert torch.equal(torch.nonzero(out.point_mask).reshape(-1), used.long())
+
+
+def test_any_counts_take_no_longer_for_the_words():
+    """Counts above 1 among 1.7 M cells, which are found while the cells' words
+    are made: adding them up took as long as all the rest of the call."""
+    cells, points = orc.voxel_hexes((121, 121, 121))
+    cd, pd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (cells, points))
+    counts = torch.zeros(len(cells), dtype=torch.int32, device="cuda")
+
+    def best_of(above):
+        counts[5::50] = above
+        best = float("inf")
+        start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        for _ in range(12):
+            start.record()
+            topology.generate_topology(counts, cells=cd, points=pd)
+            stop.record()
+            stop.synchronize()
+            best = min(best, start.elapsed_time(stop))
+        return best
+
+    assert best_of(2) < 2.8 * best_of(1)
