@@ -22,6 +22,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "mc_kernels.h"
@@ -347,9 +348,12 @@ bool valid_tuning(const Tuning& t) {
 // row words: one load instruction brings all their neighbour words (lane
 // 8u+v holds neighbour v of word u) and their bases, each word then reads its
 // eight from the lanes and writes its 64 cells (lane = cell).  Words without
-// a mixed cell need no case lookup.  Bound by the stores (9 bytes a cell):
-// 253x241x230 (125 MB) took 48 us with a lookup, a scan and a dependent base
-// load in every word, this 42; with scalar loads of the neighbours 78.
+// a mixed cell need no case lookup, but testing every word for it keeps the
+// words' chains from overlapping: where over a quarter of the neighbour words
+// are mixed (rows of one word have half of them) all are looked up.  253x241x230
+// (125 MB) of a sphere took 43 us with lookups only, 37 with tests only, this
+// 38; 300^3 of noise 84, 87, 80.  Bound by the number of stores, 64 cells each
+// wherever they start (3.3 TB/s); with scalar loads of the neighbours 78 us.
 constexpr int kCellWords = 8;
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
@@ -384,32 +388,38 @@ __global__ __launch_bounds__(256) void k_cell_outputs(VolGeom g, const uint64_t*
     }
   }
   const int64_t cx = g.nx - 1, cy = g.ny - 1;
+  auto store_words = [&](auto look_up_all) {
 #pragma unroll
-  for (int u = 0; u < kCellWords; ++u) {
-    const int64_t w = w0 + u;
-    const WordPos p = word_pos(g, w < g.nwords ? w : w0);
-    if (w >= g.nwords || !(p.has_y && p.has_z)) continue;  // wave-uniform: no cells
-    uint64_t nb[8];
+    for (int u = 0; u < kCellWords; ++u) {
+      const int64_t w = w0 + u;
+      const WordPos p = word_pos(g, w < g.nwords ? w : w0);
+      if (w >= g.nwords || !(p.has_y && p.has_z)) continue;  // wave-uniform: no cells
+      uint64_t nb[8];
 #pragma unroll
-    for (int v = 0; v < 8; ++v) nb[v] = readlane64(mine, 8 * u + v);
-    CellPlanes cp;
-    cell_planes(p, nb[0], nb[1], nb[2], nb[3], nb[4], nb[5], nb[6], nb[7], cp);
-    const bool valid = ((p.xmask >> lane) & 1ull) != 0;
-    int cs = (nb[0] >> lane) & 1ull ? 255 : 0;  // no mixed corners: no faces
-    uint32_t nf = 0u, incl = 0u;
-    if (cp.active != 0ull) {  // wave-uniform
-      cs = cell_case(cp, lane);
-      nf = valid ? (uint32_t)s_nf[cs] : 0u;
-      incl = offsets ? wave_incl_scan(nf) : 0u;
+      for (int v = 0; v < 8; ++v) nb[v] = readlane64(mine, 8 * u + v);
+      CellPlanes cp;
+      cell_planes(p, nb[0], nb[1], nb[2], nb[3], nb[4], nb[5], nb[6], nb[7], cp);
+      const bool valid = ((p.xmask >> lane) & 1ull) != 0;
+      int cs = (nb[0] >> lane) & 1ull ? 255 : 0;  // no mixed corners: no faces
+      uint32_t nf = 0u, incl = 0u;
+      if (look_up_all.value || cp.active != 0ull) {  // wave-uniform
+        cs = cell_case(cp, lane);
+        nf = valid ? (uint32_t)s_nf[cs] : 0u;
+        incl = offsets ? wave_incl_scan(nf) : 0u;
+      }
+      if (valid) {
+        const int64_t cell = (int64_t)p.q * 64 + cx * (p.j + cy * (int64_t)p.k);
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)base, 8 * u);
+        if (cases) (cases + cell)[lane] = (uint8_t)cs;
+        if (count) (count + cell)[lane] = (int32_t)nf;
+        if (offsets) (offsets + cell)[lane] = (int32_t)(first + incl - nf);
+      }
     }
-    if (valid) {
-      const int64_t cell = (int64_t)p.q * 64 + cx * (p.j + cy * (int64_t)p.k);
-      const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)base, 8 * u);
-      if (cases) (cases + cell)[lane] = (uint8_t)cs;
-      if (count) (count + cell)[lane] = (int32_t)nf;
-      if (offsets) (offsets + cell)[lane] = (int32_t)(first + incl - nf);
-    }
-  }
+  };
+  if (__popcll(__ballot(mine != 0ull && mine != ~0ull)) > 16)
+    store_words(std::true_type{});
+  else
+    store_words(std::false_type{});
 }
 
 __global__ void k_interpolate_scalar(const float* __restrict__ in, const int32_t* __restrict__ first,

@@ -96,12 +96,17 @@ def test_more_planes_than_blocks_of_a_launch():
                        want.nan_to_num(nan=-7.0, posinf=7e9, neginf=-7e9))
 
 
-@pytest.mark.parametrize("dims", [(2, 2, 2), (66, 9, 7), (200, 12, 5)])
-def test_cell_outputs_quiet_and_mixed_words(dims):
+@pytest.mark.parametrize("noise", [0.0, 0.2, 0.6, 1.0])
+@pytest.mark.parametrize("dims", [(2, 2, 2), (3, 70, 9), (66, 9, 7), (200, 12, 5), (600, 9, 9)])
+def test_cell_outputs_quiet_and_mixed_words(dims, noise):
+    """Groups of words of which few, some or all are mixed (noise: in how many
+    of the rows)."""
     nx, ny, nz = dims
     f = np.zeros((nz, ny, nx), np.float32)
     f[:, :, nx // 2:] = 1.0          # whole words in and out
     f[nz // 2, ny // 2, 0] = 1.0     # and mixed ones
+    rng = np.random.default_rng(nx)
+    f = np.where(rng.random((nz, ny, 1)) < noise, rng.random(f.shape), f).astype(np.float32)
     field = torch.from_numpy(f).cuda()
     ws, _ = mc.classify(field, 0.5)
     C = (nx - 1) * (ny - 1) * (nz - 1)
