@@ -71,10 +71,6 @@ struct HostSlot {
     if (_e != hipSuccess) return ::daxhip::check_hip(_e, what); \
   } while (0)
 
-constexpr int kWave = 64;
-
-__device__ __forceinline__ int lane_id() { return __lane_id(); }
-
 // Inclusive prefix sum over the 64 lanes of a wavefront with DPP row shifts
 // and the GFX9 row broadcasts (row_shr:1/2/4/8, row_bcast:15, row_bcast:31).
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
@@ -93,17 +89,6 @@ __device__ __forceinline__ uint32_t wave_last(uint32_t v) {
 }
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return wave_last(wave_incl_scan(v)); }
-
-__device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
-  // two 32-bit halves scanned separately, recombined with the carry of the
-  // low half accumulated in 64 bits
-  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-  // sum of lows can exceed 32 bits: split further into 16-bit pieces
-  uint32_t l0 = lo & 0xffffu, l1 = lo >> 16;
-  uint64_t s = (uint64_t)wave_sum(l0) + ((uint64_t)wave_sum(l1) << 16) +
-               ((uint64_t)wave_sum(hi) << 32);
-  return s;
-}
 
 // Exclusive scan of one value per thread over the block (thread order);
 // returns the thread's offset and the block total.
@@ -198,8 +183,6 @@ __device__ __forceinline__ void store_prefixes(uint32_t* __restrict__ v, int64_t
     }
   }
 }
-
-__device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -211,16 +211,7 @@ __device__ __forceinline__ int cell_case(const CellPlanes& cp, int i) {
   return c;
 }
 
-// Rank of the edge (bit i, axis a) among the active edges of a word.
-__device__ __forceinline__ int edge_rank(uint64_t fx, uint64_t fy, uint64_t fz, int i, int a) {
-  const uint64_t lo = (1ull << i) - 1ull;
-  int r = popc(fx & lo) + popc(fy & lo) + popc(fz & lo);
-  if (a > 0) r += (int)((fx >> i) & 1ull);
-  if (a > 1) r += (int)((fy >> i) & 1ull);
-  return r;
-}
-
-// Inverse of edge_rank: the k-th active edge of a word in (bit, axis x<y<z)
+// The k-th active edge of a word in (bit, axis x<y<z)
 // order (k < popc(fx) + popc(fy) + popc(fz)): the 32-bit half that holds
 // it, then halving steps, each counting the three flag sets below the split.
 __device__ __forceinline__ void edge_select(uint64_t fx, uint64_t fy, uint64_t fz, int k, int& bit,
