@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from daxtoolkit_amd import _lib, fields, mc
+from daxtoolkit_amd import fields, mc
 from mc_autograd import MarchingCubesFunction, torch_reference_loss
 from oracle import oracle as orc
 
@@ -134,10 +134,9 @@ def test_backward_deterministic_and_fd_256():
 
 def test_backward_dense_surface():
     """A field with surface everywhere (sum of short-period sines, 64^3 and a
-    ragged 70x45x38): most gather tiles then hold more stencil endpoints than
-    their LDS record space and take the direct per-point path, the others the
-    shared per-endpoint path.  Checked against the oracle's FP64 adjoint and
-    for run-to-run determinism."""
+    ragged 70x45x38): most words then hold many endpoints, which share their
+    edges' records.  Checked against the oracle's FP64 adjoint and for
+    run-to-run determinism."""
     for dims in ((64, 64, 64), (70, 45, 38)):
         nx, ny, nz = dims
         z, y, x = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
@@ -148,18 +147,7 @@ def test_backward_dense_surface():
         field = torch.from_numpy(f).cuda()
         out = mc.forward(field, iso, edges=True)
         U = out.num_points
-        # endpoints (points with an active incident edge) per 16384 points
-        b = f > iso
-        ends = np.zeros_like(b)
-        for ax in range(3):
-            d = np.diff(b, axis=ax) != 0
-            sl_lo = [slice(None)] * 3
-            sl_hi = [slice(None)] * 3
-            sl_lo[ax] = slice(0, -1)
-            sl_hi[ax] = slice(1, None)
-            ends[tuple(sl_lo)] |= d
-            ends[tuple(sl_hi)] |= d
-        assert ends.sum() / f.size * 16384 > 2048
+        assert _endpoints(f, iso).sum() > f.size / 8
         gen = torch.Generator().manual_seed(7)
         dx = torch.randn((U, 3), generator=gen, dtype=torch.float32)
         dn = torch.randn((U, 3), generator=gen, dtype=torch.float32)
@@ -176,12 +164,8 @@ def test_backward_dense_surface():
         assert _close(got, ref, 1e-4, 1e-3) <= 1e-4
 
 
-def _gather_tile_endpoints(f, iso, rows):
-    """Endpoint slots of a gather tile of `rows` full rows (one plane) and of
-    its 2^lg spans: the endpoints (points with an active incident edge) of
-    its rows, of the row before and after it, and of its rows in the planes
-    below and above."""
-    nz, ny, _ = f.shape
+def _endpoints(f, iso):
+    """The points with an active incident edge."""
     b = f > iso
     ends = np.zeros_like(b)
     for ax in range(3):
@@ -190,35 +174,16 @@ def _gather_tile_endpoints(f, iso, rows):
         d = a[1:] != a[:-1]
         e[1:] |= d
         e[:-1] |= d
-    rc = ends.sum(axis=2)
-
-    def slots(k, j0, j1):
-        s = rc[k, j0:j1].sum() + (rc[k, j0 - 1] if j0 > 0 else 0) + (rc[k, j1] if j1 < ny else 0)
-        return int(s + (rc[k - 1, j0:j1].sum() if k > 0 else 0) +
-                   (rc[k + 1, j0:j1].sum() if k + 1 < nz else 0))
-
-    tiles = []
-    for k in range(nz):
-        for j0 in range(0, ny, rows):
-            n = slots(k, j0, j0 + rows)
-            lg = 1
-            while lg < 4 and (1536 << lg) < n:
-                lg += 1
-            sub = rows >> lg
-            tiles.append((n, lg, [slots(k, j0 + s * sub, j0 + (s + 1) * sub) for s in range(1 << lg)]))
-    return tiles
+    return ends
 
 
-@pytest.mark.parametrize("tiles_per_cu", [16, 0])
-def test_backward_dense_tiles_in_spans(tiles_per_cu):
-    """Gather tiles (256 row words: here one 64 x 256 plane) with more
-    endpoint slots than their 2048 records.  With few tiles per CU every
-    such tile is listed for the span pass; with threshold 0 a tile of up to
-    6144 slots runs as 2 or 4 spans in its own block, listing only a span
-    that still does not fit, and a denser tile is listed whole.  The field
-    (zero, with a noisy strip, a noisy half plane and a box face) holds
-    every kind; the adjoint is checked bit for bit against the oracle and
-    for determinism."""
+def test_backward_dense_and_empty_words():
+    """Endpoint words of every kind beside each other: a tile is 256 row words
+    (here a 64 x 256 plane), a wave's share of it 8 (two rows).  The field
+    (zero, with a noisy strip, a noisy half plane and a box face) has tiles
+    and waves without an endpoint, waves that are nearly full and tiles of
+    both; the adjoint is checked bit for bit against the oracle and for
+    determinism."""
     nx, ny, nz = 256, 64, 12
     rng = np.random.default_rng(3)
     f = np.zeros((nz, ny, nx), np.float32)
@@ -226,28 +191,21 @@ def test_backward_dense_tiles_in_spans(tiles_per_cu):
     f[5, :, :128] = rng.integers(0, 2, (ny, 128))
     f[8, :, :20] = 1.0
     iso = 0.5
-    tiles = _gather_tile_endpoints(f, iso, 64)
-    in_block = [t for t in tiles if 2048 < t[0] <= 6144]
-    assert any(t[1] == 1 and max(t[2]) <= 2048 for t in in_block)
-    assert any(t[1] == 2 and max(t[2]) <= 2048 for t in in_block)
-    assert any(max(t[2]) > 2048 for t in in_block)  # a span listed from its block
-    assert any(t[0] > 6144 for t in tiles)          # tiles listed whole
-    print(f"[case] adjoint dense tiles in spans {(nx, ny, nz)} threshold {tiles_per_cu}",
-          flush=True)
+    ends = _endpoints(f, iso)
+    waves = ends.reshape(nz, ny // 2, -1).sum(-1)  # of 512 points
+    assert any((w == 0).all() for w in waves) and waves.max() > 450
+    assert any((w == 0).any() and (w > 450).any() for w in waves)
+    words = ends.reshape(nz, ny, -1, 64).sum(-1)
+    assert any((w == 0).any() and (w == 64).any() for w in words.reshape(-1, 8))
+    print(f"[case] adjoint dense and empty words {(nx, ny, nz)}", flush=True)
     field = torch.from_numpy(f).cuda()
     out = mc.forward(field, iso, edges=True)
     U = out.num_points
     gen = torch.Generator().manual_seed(11)
     dx = torch.randn((U, 3), generator=gen, dtype=torch.float32)
     dn = torch.randn((U, 3), generator=gen, dtype=torch.float32)
-    lib = _lib.load()
-    assert lib.dax_hip_mc_backward_set_span_threshold(tiles_per_cu) == 0
-    try:
-        g1 = mc.backward(field, iso, out, dx.cuda(), dn.cuda())
-        g2 = mc.backward(field, iso, out, dx.cuda(), dn.cuda())
-        torch.cuda.synchronize()
-    finally:
-        assert lib.dax_hip_mc_backward_set_span_threshold(16) == 0
+    g1 = mc.backward(field, iso, out, dx.cuda(), dn.cuda())
+    g2 = mc.backward(field, iso, out, dx.cuda(), dn.cuda())
     assert torch.equal(g1, g2)
     r = orc.generate(f, iso)
     assert r["n_pts"] == U
@@ -257,8 +215,8 @@ def test_backward_dense_tiles_in_spans(tiles_per_cu):
 
 @pytest.mark.parametrize("dims", [(4000, 3, 4), (15872, 2, 3)])
 def test_backward_wide_rows(dims):
-    """Rows of 63 and 248 words (the widest the adjoint takes): a gather tile then
-    spans few rows and its LDS exceeds 64 KiB.  A smooth field; bit for bit
+    """Rows of 63 and 248 words (the widest the adjoint takes): the words of a
+    wave and of a tile are then parts of a row.  A smooth field; bit for bit
     against the oracle's FP32 restatement, and against its FP64 adjoint within
     1e-3 (near-tangent crossings, with active-edge differences down to 4e-3,
     put the FP32 rounding itself at up to 3e-4 relative here)."""
