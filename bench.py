@@ -65,10 +65,11 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, GB/s
 
 
 def _kernel_variants(n, tuned):
-    """Template names of the three forward kernels a tuning launches."""
+    """Template names of the forward kernels a tuning launches at 512^3 (generate
+    with a thread per tile word)."""
     unroll, vec, sub, tile = tuned[0], tuned[1], tuned[2], tuned[3]
     cls = f"k_classify_v4<{unroll}>" if vec == 4 else f"k_classify<{unroll}>"
-    return cls, f"k_count<{sub}>", f"k_generate<{tile}, FieldArray>"
+    return cls, f"k_count<{sub}>", f"k_generate<{tile}, {tile}, FieldArray, true>"
 
 
 def kernel_sources_sha256():

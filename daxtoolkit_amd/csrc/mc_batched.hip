@@ -44,9 +44,10 @@ constexpr int64_t kLaunchTiles = 1 << 23;
 
 // Launch shapes of the batch forward, picked by dax_hip_mc_batch_autotune
 // and cached per batch shape class: classify unroll (row words per wave
-// step, a float4 load in flight per thread for two of them) and persistent blocks per CU, threads per count block (a wave per
-// tile), generate's XCD-contiguous tile order.  gen_blocks is kept for callers
-// that set it: generate runs a block per tile.
+// step, a float4 load in flight per thread for two of them) and persistent
+// blocks per CU, threads per count block (a wave per tile), generate's
+// XCD-contiguous tile order.  gen_blocks has no effect (generate runs a block
+// per tile) and is kept, and checked, for callers that set it.
 struct BatchTuning {
   int32_t cls_unroll, cls_blocks, scan_threads, gen_blocks, gen_xcd, pad;
 };
@@ -881,9 +882,10 @@ int dax_hip_graph_end_capture(void* stream, void** h_graph_exec) {
 }
 
 // Baseline of the batched path: the same volumes, one single-volume forward
-// (three launches) and, when upstream gradients are given, one single-volume
-// backward (two launches) per volume, written at the offsets of the batched
-// outputs (h_vol_offsets, as the batched forward reports them).
+// (four launches) and, when upstream gradients are given, one single-volume
+// backward (three launches, four on large volumes) per volume, written at the
+// offsets of the batched outputs (h_vol_offsets, as the batched forward reports
+// them).
 int dax_hip_mc_volume_loop(int64_t n_volumes, const int64_t* h_dims3,
                            const int64_t* h_field_offsets, const float* h_isos,
                            const float* h_origins3, const float* h_spacings3,

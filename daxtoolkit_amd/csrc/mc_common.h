@@ -211,9 +211,9 @@ __device__ __forceinline__ int cell_case(const CellPlanes& cp, int i) {
   return c;
 }
 
-// The k-th active edge of a word in (bit, axis x<y<z)
-// order (k < popc(fx) + popc(fy) + popc(fz)): the 32-bit half that holds
-// it, then halving steps, each counting the three flag sets below the split.
+// The k-th active edge of a word in (bit, axis x<y<z) order (k < popc(fx) +
+// popc(fy) + popc(fz)): the 32-bit half that holds it, then halving steps, each
+// counting the three flag sets below the split.
 __device__ __forceinline__ void edge_select(uint64_t fx, uint64_t fy, uint64_t fz, int k, int& bit,
                                             int& axis) {
   const int nlo = __popc((uint32_t)fx) + __popc((uint32_t)fy) + __popc((uint32_t)fz);

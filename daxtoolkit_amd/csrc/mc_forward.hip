@@ -12,9 +12,10 @@
 // (classify).  Everything topological after that works on the bits: 64 cells
 // per 64-bit word op.  Vertex numbering uses active-edge flags in
 // (point id, axis) order, which is the order the reference's sort/unique
-// produces, so no sort is needed.  The count/scan kernel is a single pass
-// with decoupled look-back; the generate kernel revisits only tiles that
-// have output and touches the field only around the surface.
+// produces, so no sort is needed.  The count kernel writes prefixes within
+// its blocks and one block scans the blocks' sums; the generate kernel
+// revisits only tiles that have output and touches the field only around the
+// surface.
 //
 // Tile shapes (classify unroll and load width, scan sub-tiles, generate tile
 // words) are chosen per grid shape by the autotuner at the end of this file.
@@ -309,13 +310,16 @@ std::map<std::tuple<int64_t, int64_t, int64_t>, Tuning> g_tune_cache;
 
 // The launch shape of a volume without a choice of its own, while no caller has
 // set the default.  Generate tiles: 64 words (spread over the waves
-// launch_generate_src gives them) up to 2^20 words, 256 beyond, where the
-// dispatch order of tiles of at least a count tile pays (forward, 64 / 256
-// words: 256^3 points 59 / 65 us, 384^3 105 / 109, 512^3 194 / 176; dense
-// 640^3 367 / 375).  A tile stages two rows beyond its own, so rows of more
-// than 32 words take tiles of at least two rows.  Count blocks: one wave up to
-// 2^16 words, to spread over more CUs (100 x 90 x 110 points: forward 37 / 38
-// / 40 us with 1 / 4 / 8 waves), four beyond (256^3: 68 / 67 / 69).
+// launch_generate_src gives them) up to 2^20 words.  Beyond, tiles of 256 words
+// can be dispatched in an order of their work, which pays where the surface
+// takes few of the tiles (forward, 64 / 256 words: 256^3 points 59 / 65 us,
+// 384^3 105 / 109, 512^3 194 / 176) and costs where most have output (dense
+// 640^3 367 / 375, 1024^3 of 12.7 M vertices 1420 / 1435).  Which it is depends
+// on the field, not on the shape, and the first gains more than the second
+// loses; the autotuner times both.  A tile stages two rows beyond its own, so
+// rows of more than 32 words take tiles of at least two rows.  Count blocks: one
+// wave up to 2^16 words, to spread over more CUs (100 x 90 x 110 points: forward
+// 37 / 38 / 40 us with 1 / 4 / 8 waves), four beyond (256^3: 68 / 67 / 69).
 Tuning shape_tuning(int64_t nx, int64_t ny, int64_t nz) {
   Tuning t;
   const int64_t wpr = ceil_div(nx, 64), words = wpr * ny * nz;
@@ -864,7 +868,7 @@ int launch_bits_plane(const VolGeom& g, const FieldPlane& pl, char* ws, const Wo
   return DAX_HIP_OK;
 }
 
-// The three kernels of a forward over the whole volume.
+// The kernels of a forward over the whole volume.
 int launch_forward(const VolGeom& g, const float* field, char* ws, const Workspace& L,
                    unsigned flags, const OutPtrs& o, int64_t cap_points, int64_t cap_tris,
                    int64_t* counts, const Tuning& tu, hipStream_t s) {
@@ -1030,8 +1034,9 @@ int dax_hip_mc_forward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
 // ---- forward without allocation -------------------------------------------
 // dax_hip_mc_forward with its workspace in a file-scope device array, for
 // callers that cannot allocate (code under graph capture, serving loops):
-// grids of up to kNoAllocMaxWords row words (512^3 points have 2^21).  Every GPU the library runs on holds the array until the process
-// ends.  Calls that overlap on one GPU share the array and race.
+// grids of up to kNoAllocMaxWords row words (512^3 points have 2^21).  Every GPU
+// the library runs on holds the array until the process ends.  Calls that
+// overlap on one GPU share the array and race.
 constexpr int64_t kNoAllocMaxWords = 2484927;
 constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;  // 12.3 bytes a word
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];

@@ -1,6 +1,5 @@
 // Device bodies of the marching-cubes kernels, shared by the single-volume
-// launches (mc_forward.hip) and the batched persistent launches
-// (mc_batched.hip).
+// launches (mc_forward.hip) and the batched launches (mc_batched.hip).
 //
 //   classify   : field -> inside-bits                         (one pass over f)
 //   count/scan : per-word edge and triangle counts, prefixes within count

@@ -157,11 +157,11 @@ int dax_hip_timer_elapsed(void* timer, void* stream, double* h_seconds);
  * (dax/Extent.h:104-112), coordinates origin + spacing*ijk
  * (dax/cont/UniformGrid.h:82-89).  Cells (nx-1)(ny-1)(nz-1), x fastest.
  *
- * The forward runs as three kernels over a caller-provided workspace:
+ * The forward runs as four kernels over a caller-provided workspace:
  *   classify: field -> one inside-bit per point (f > iso, strict, as
  *             GetHexahedronClassification, dax/worklet/MarchingCubes.h:36-48)
- *   count+scan: per 64-point row word, active-edge and triangle counts, and a
- *             single-pass decoupled look-back exclusive scan
+ *   count, scan: per 64-point row word, active-edge and triangle counts and
+ *             their prefixes within blocks, then an exclusive scan of the blocks
  *             (replaces ScanInclusive at DispatcherGenerateInterpolatedCells.h:180-183)
  *   generate: vertices, normals, connectivity (MarchingCubesGenerate,
  *             MarchingCubes.h:90-169, plus ResolveCoordinates
@@ -272,7 +272,9 @@ int dax_hip_mc_slice_generate(int64_t nx, int64_t ny, int64_t nz, const float* h
  * (the reference's Sort/Unique/LowerBounds, :261-301), d_first/second/
  * weight optional.  d_vertices [3T][3] and d_conn [3T] (3T is the most
  * points there can be); *h_points = U.  Dedup needs
- * dax_hip_mt_scratch_bytes(T) bytes of d_scratch. */
+ * dax_hip_mt_scratch_bytes(T) bytes of d_scratch, and takes 60 bytes a
+ * triangle and 1.25 a point of temporaries (the general sort, where those
+ * cannot be had and for very uneven meshes, 48 a triangle). */
 int dax_hip_mt_count(const int32_t* d_tets, int64_t n_tets, const float* d_field,
                      int64_t n_points, float iso, int32_t* d_counts, int32_t* d_offsets,
                      int64_t* h_tris, void* stream);
@@ -466,10 +468,9 @@ int dax_hip_mc_read_counts(const int64_t* d_counts, int64_t cap_points, int64_t 
  * workspace, in this order:
  *   dax_hip_mc_bits      classify: field -> inside-bits (one kernel)
  *   dax_hip_mc_scan      per-word vertex / triangle counts, then the scan
- *                        of the 256-word count tiles' sums (two kernels)
- *   dax_hip_mc_generate  outputs, as dax_hip_mc_forward (d_counts written),
- *                        and every row word's vertex / triangle base in the
- *                        workspace (one kernel)
+ *                        of the count blocks' sums (two kernels)
+ *   dax_hip_mc_generate  outputs, as dax_hip_mc_forward (d_counts written;
+ *                        one kernel)
  * Together they replace DispatcherMapCell<MarchingCubesCount>
  * (dax/cont/DispatcherMapCell.h:27-64), the ScanInclusive/UpperBounds of
  * DispatcherGenerateInterpolatedCells.h:180-223 and its generate/resolve
@@ -584,11 +585,10 @@ int dax_hip_mc_batch_graph_create(const float* d_fields, const void* h_header, v
                                   int64_t* d_vol_offsets, void* stream, void** h_graph_exec);
 /* Launch shapes of the batch forward, held in the header:
  * {classify unroll 8|16|32, classify blocks per CU 2|4|8, threads per count
- * block 256|512|1024, generate blocks per CU 2|4|8 (no
- * longer used: generate runs a block per tile), generate XCD-contiguous tile
- * order 0|1}.  prepare starts from the shape cached for
- * the batch's class (volume count, ceil(log2(row words)), widest row) or the
- * default {16, 4, 256, 4, 1}.  Every shape gives the same outputs.
+ * block 256|512|1024, generate blocks per CU 2|4|8 (checked, but without
+ * effect: generate runs a block per tile), generate XCD-contiguous tile order
+ * 0|1}.  prepare starts from the shape cached for the batch's class (volume
+ * count, ceil(log2(row words)), widest row) or the default {16, 4, 256, 4, 1}.  Every shape gives the same outputs.
  *   dax_hip_mc_batch_set_tuning / _get_tuning  write / read the header's
  *   dax_hip_mc_batch_autotune  times each phase's shapes on this batch (reps
  *       launches each, synchronous), keeps the fastest in the header and the
@@ -651,10 +651,10 @@ int dax_hip_graph_destroy(void* graph_exec);
  * interpolants (t, endpoint gradients) are recomputed from the field.
  * U = min(d_counts[1], n_points) if d_counts is given (device {T, U} of the
  * forward), else n_points.  d_scratch needs
- * dax_hip_mc_backward_scratch_bytes(n_points) bytes (a 32-byte record per
- * vertex and the sums of its two endpoints).  Deterministic: every sum has a
- * fixed order, so the result is bitwise reproducible.  Rows of at most 15872 points (nx).  d_dl_dfield [P]
- * f32 is fully written. */
+ * dax_hip_mc_backward_scratch_bytes(n_points) bytes, 64 a vertex and 16 (a
+ * 32-byte record per vertex and the sums of its two endpoints).  Deterministic:
+ * every sum has a fixed order, so the result is bitwise reproducible.  Rows of
+ * at most 15872 points (nx).  d_dl_dfield [P] f32 is fully written. */
 size_t dax_hip_mc_backward_scratch_bytes(int64_t n_points);
 int dax_hip_mc_backward(const float* d_field, int64_t nx, int64_t ny, int64_t nz,
                         const float* h_origin3, const float* h_spacing3, float iso,

@@ -42,7 +42,7 @@ def test_workspace_size_is_host_only():
     lib = daxtoolkit_amd.load_library()
     assert lib.dax_hip_mc_workspace_bytes(0, 1, 1) == 0
     b = lib.dax_hip_mc_workspace_bytes(512, 512, 512)
-    # bit words (P/8) + two 32-bit bases per word + tile states
+    # bit words (P/8), prefixes (4 bytes a word), endpoint words and prefixes (10)
     assert 512**3 // 8 <= b < 512**3 // 8 * 3
 
 
